@@ -20,6 +20,8 @@
 //      a value passes if approx <= thr, thr = kth^2 (1 + 8e-6) + M with the
 //      rigorous FP32 bound M = 64 u (|q|^2 + max|x|^2) (u = 2^-24) on the
 //      cancellation error, so no point of the exact result is ever dropped.
+//   (This full scan serves what the spatial index of nn_tree.hip does not:
+//   use_tree below.)
 //   3. Passing points get the exact FP32 distance (the oracle's formula) and
 //      enter the lane's sorted register top-k; the two lanes of a query merge
 //      their lists at the end (wave-level merge), DB splits merge in a second
@@ -33,7 +35,8 @@
 #include <cstdint>
 #include <vector>
 
-#include "fp32_math.hpp"
+#include "nn_device.hpp"
+#include "nn_tree.hpp"
 #include "runtime.hpp"
 
 namespace ompl_amd {
@@ -52,9 +55,14 @@ struct NNIndex {
     float *pts = nullptr;      // [cap][dim]
     float *xt = nullptr;       // [cap/32][ksteps][64] tiled augmented points
     uint8_t *removed = nullptr;
-    uint32_t *xn_max = nullptr; // max |x|^2 as FP32 bits (non-negative)
+    uint32_t *xn_max = nullptr; // max |x|^2 as FP32 bits (non-negative), then the extents (kStatWords words)
     int64_t n_removed = 0;
     std::vector<uint8_t> removed_host;
+    // spatial index of the first tree.m points; the stream of its last use,
+    // and whether it was used on others since it was built
+    NNTree tree;
+    hipStream_t tree_stream = nullptr;
+    bool tree_mixed = false;
     // per-call scratch (grow-only)
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
@@ -76,55 +84,6 @@ __device__ __forceinline__ float l2_exact(const float *__restrict__ e, const flo
         dist += diff * diff;
     }
     return __builtin_sqrtf(dist);
-}
-
-template <int METRIC, int DIM>
-__device__ __forceinline__ float exact_dist(const float *__restrict__ e, const float q[DIM])
-{
-    if (METRIC == OMPL_AMD_METRIC_L2) {
-        float dist = 0.0f;
-#pragma unroll
-        for (int i = 0; i < DIM; ++i) {
-            const float diff = e[i] - q[i];
-            dist += diff * diff;
-        }
-        return __builtin_sqrtf(dist);
-    } else {
-        float t = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            const float diff = e[i] - q[i];
-            t += diff * diff;
-        }
-        const float dt = __builtin_sqrtf(t);
-        const float dq = fabsf(((e[3] * q[3] + e[4] * q[4]) + e[5] * q[5]) + e[6] * q[6]);
-        const float dr = dq > 1.0f ? 0.0f : acos_as(dq);
-        float dist = 0.0f;
-        dist += 1.0f * dt;
-        dist += 1.0f * dr;
-        return dist;
-    }
-}
-
-// SE3: true when the point's distance is certainly above `bound` (a finite
-// distance), from a lower bound that skips the acos: acos(x) >= sqrt(2 (1 - x))
-// on [0, 1] (2 sin(t / 2) <= t), so d >= d_t + sqrt(2 (1 - |q.x|)).  The margin
-// (relative 1e-5 plus 1e-5) covers the FP32 rounding of both sides and
-// acos_as's error, so a point this skips is one whose exact distance is above
-// the bound.  Other metrics: never.
-template <int METRIC, int DIM>
-__device__ __forceinline__ bool certainly_above(const float *__restrict__ e, const float q[DIM], float bound)
-{
-    if (METRIC != OMPL_AMD_METRIC_SE3) return false;
-    float t = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        const float diff = e[i] - q[i];
-        t += diff * diff;
-    }
-    const float dq = fabsf(((e[3] * q[3] + e[4] * q[4]) + e[5] * q[5]) + e[6] * q[6]);
-    const float lb = __builtin_amdgcn_sqrtf(t) + __builtin_amdgcn_sqrtf(2.0f * (1.0f - dq));
-    return lb > bound * (1.0f + 1e-5f) + 1e-5f; // false for NaN (dq > 1) or an infinite bound
 }
 
 struct Key {
@@ -230,11 +189,6 @@ template <int KMAX>
 struct KnnGroup {
     static constexpr int kMaxWaves = KMAX <= 16 ? 16 : 4;
 };
-
-__device__ __forceinline__ unsigned long long pack_key(float d, int i)
-{
-    return ((unsigned long long)__float_as_uint(d) << 32) | (uint32_t)i;
-}
 
 // Row of the 32x32 MFMA output held in element j of a lane in half h.
 __device__ __forceinline__ int mfma_row(int j, int h)
@@ -708,27 +662,69 @@ __global__ void radius_unpack_kernel(const uint64_t *__restrict__ keys, int64_t 
 }
 
 // Writes tiled augmented rows for points [from, to) and the padding of the
-// last tile; tracks max |x|^2.
-__global__ void build_xt_kernel(const float *__restrict__ pts, int dim, int tdim, int ksteps, int64_t from,
-                                int64_t to, int64_t n_total, float *__restrict__ xt, uint32_t *__restrict__ xn_max)
+// last tile; tracks max |x|^2 and the extents of the first coordinates
+// (stats: kStatNorm, kStatLo, kStatHi).  The figures meet in LDS, and a block
+// makes a device-wide atomic only for one that it improves (one atomic per
+// point took 187 us of adding 1,000,000).
+constexpr int kStatNorm = 0, kStatLo = 8, kStatHi = 16, kStatWords = 24;
+
+__global__ void __launch_bounds__(256) build_xt_kernel(const float *__restrict__ pts, int dim, int tdim, int ksteps,
+                                                       int64_t from, int64_t to, int64_t n_total,
+                                                       float *__restrict__ xt, uint32_t *__restrict__ stats)
 {
+    __shared__ uint32_t blk[kStatWords];
+    if (threadIdx.x < kStatWords) blk[threadIdx.x] = threadIdx.x >= kStatLo && threadIdx.x < kStatHi ? ~0u : 0u;
+    __syncthreads();
     const int64_t p = from + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= to) return;
-    const bool real = p < n_total;
+    const bool real = p < n_total && p < to;
     float xn = 0.0f;
     if (real)
         for (int i = 0; i < tdim; ++i) xn += pts[p * dim + i] * pts[p * dim + i];
-    const int64_t t = p >> 5;
-    const int row = (int)(p & 31);
-    for (int kk = 0; kk < 2 * ksteps; ++kk) {
-        float v;
-        if (kk < tdim) v = real ? pts[p * dim + kk] : 0.0f;
-        else if (kk == tdim) v = 1.0f;
-        else if (kk == tdim + 1) v = real ? xn : kPadNorm;
-        else v = 0.0f;
-        xt[t * (ksteps * 64) + (kk >> 1) * 64 + (kk & 1) * 32 + row] = v;
+    if (p < to) {
+        const int64_t t = p >> 5;
+        const int row = (int)(p & 31);
+        for (int kk = 0; kk < 2 * ksteps; ++kk) {
+            float v;
+            if (kk < tdim) v = real ? pts[p * dim + kk] : 0.0f;
+            else if (kk == tdim) v = 1.0f;
+            else if (kk == tdim + 1) v = real ? xn : kPadNorm;
+            else v = 0.0f;
+            xt[t * (ksteps * 64) + (kk >> 1) * 64 + (kk & 1) * 32 + row] = v;
+        }
     }
-    if (real) atomicMax(xn_max, __float_as_uint(xn));
+    uint32_t norm = real ? __float_as_uint(xn) : 0u;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) norm = max(norm, (uint32_t)__shfl_xor((int)norm, d));
+    if ((threadIdx.x & 63) == 0) atomicMax(&blk[kStatNorm], norm);
+    for (int j = 0; j < tdim && j < 8; ++j) {
+        const float v = real ? pts[p * dim + j] : INFINITY;
+        const bool fin = fabsf(v) < 3e38f; // finite
+        uint32_t lo = fin ? ordered_bits(v) : ~0u, hi = fin ? ordered_bits(v) : 0u;
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            lo = min(lo, (uint32_t)__shfl_xor((int)lo, d));
+            hi = max(hi, (uint32_t)__shfl_xor((int)hi, d));
+        }
+        if ((threadIdx.x & 63) == 0) {
+            atomicMin(&blk[kStatLo + j], lo);
+            atomicMax(&blk[kStatHi + j], hi);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < kStatWords) {
+        const uint32_t v = blk[threadIdx.x];
+        const uint32_t have = __hip_atomic_load(&stats[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (threadIdx.x >= kStatLo && threadIdx.x < kStatHi) {
+            if (v < have) atomicMin(&stats[threadIdx.x], v);
+        } else if (v > have) {
+            atomicMax(&stats[threadIdx.x], v);
+        }
+    }
+}
+
+__global__ void clear_stats_kernel(uint32_t *__restrict__ stats)
+{
+    if (threadIdx.x < kStatWords) stats[threadIdx.x] = threadIdx.x >= kStatLo && threadIdx.x < kStatHi ? ~0u : 0u;
 }
 
 // Each query's radius keys (distance bits << 32 | index; unique per query)
@@ -775,10 +771,44 @@ __global__ void __launch_bounds__(256) radius_sort_kernel(const uint64_t *__rest
     for (int i = lane; i < m; i += 64) out[b + i] = sb[i];
 }
 
-__global__ void max_i64_kernel(const int64_t *__restrict__ v, int64_t n, unsigned long long *__restrict__ out)
+// Largest of v[0, n): one atomic per wave (one per value on one address took
+// 15.7 us for 65,536 values).
+__global__ void __launch_bounds__(256) max_i64_kernel(const int64_t *__restrict__ v, int64_t n,
+                                                      unsigned long long *__restrict__ out)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) atomicMax(out, (unsigned long long)v[i]);
+    unsigned long long m = 0;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        m = max(m, (unsigned long long)v[i]);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) m = max(m, __shfl_xor(m, d));
+    if ((threadIdx.x & 63) == 0 && m) atomicMax(out, m);
+}
+
+// The two figures the host waits for, into its own (mapped) memory.
+__global__ void report_kernel(const int64_t *__restrict__ total, const unsigned long long *__restrict__ longest,
+                              int64_t *__restrict__ host)
+{
+    if (threadIdx.x == 0) {
+        host[0] = *total;
+        host[1] = (int64_t)*longest;
+    }
+}
+
+// Results of the one-pass search from the queries' sorted slots into the CSR
+// arrays, 16 lanes per query (a query of the RRT* schedule has about ten).
+__global__ void __launch_bounds__(256) radius_place_kernel(const uint64_t *__restrict__ slots, int slot_cap,
+                                                           const int64_t *__restrict__ off, int64_t nq,
+                                                           int32_t *__restrict__ idx, float *__restrict__ dist)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t q = t >> 4;
+    if (q >= nq) return;
+    const int64_t b = off[q], m = off[q + 1] - b;
+    for (int64_t i = t & 15; i < m; i += 16) {
+        const uint64_t k = slots[q * slot_cap + i];
+        if (idx) idx[b + i] = (int32_t)(uint32_t)k;
+        if (dist) dist[b + i] = __uint_as_float((uint32_t)(k >> 32));
+    }
 }
 
 __global__ void fill_i64_kernel(int64_t *p, int64_t n, int64_t v)
@@ -820,6 +850,12 @@ static void *scratch_keep(NNIndex &x, size_t bytes, size_t keep, hipStream_t s)
     return x.scratch;
 }
 
+// Points from which on the spatial index is kept, and up to which (its places
+// and counts are 32-bit words; beyond, the working space of a build would be
+// more than a gigabyte).
+constexpr int64_t kTreeMinPoints = 2048;
+constexpr int64_t kTreeMaxPoints = (int64_t)1 << 25;
+
 static void reserve(NNIndex &x, int64_t need, hipStream_t s)
 {
     if (need <= x.cap) return;
@@ -847,6 +883,48 @@ static void reserve(NNIndex &x, int64_t need, hipStream_t s)
     x.removed = rem;
     x.cap = cap;
     x.removed_host.resize((size_t)cap, 0);
+    if (tree_supported(x.metric, x.dim) && cap >= kTreeMinPoints && cap <= kTreeMaxPoints)
+        tree_reserve(x.tree, cap, x.dim, x.tdim);
+    else
+        tree_free(x.tree);
+}
+
+// Notes a use of the index on stream s.
+static void tree_used(NNIndex &x, hipStream_t s)
+{
+    if (x.tree_stream != s) x.tree_mixed = true;
+}
+
+// Brings the index up to date once a tail of 512 points, or of 1/128 of the
+// indexed ones, waits: every query scans the tail (512 points are 8 tiles, a
+// fifth of the tiles that a 10-NN query of 100,000 points looks at), and a
+// build takes about 80 us at 5,000 to 100,000 points, 370 at 1,000,000.
+static void tree_update(NNIndex &x, hipStream_t s)
+{
+    if (!x.tree.mem || x.n < kTreeMinPoints || x.n - x.tree.m < std::max<int64_t>(512, x.tree.m / 128)) return;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return; // the tail grows
+    // the arrays are rewritten: wait for readers on other streams
+    if (x.tree.m > 0 && (x.tree_mixed || x.tree_stream != s)) OA_HIP(hipDeviceSynchronize());
+    tree_build(x.tree, x.pts, x.removed, x.xn_max + kStatLo, x.xn_max + kStatHi, x.n, x.dim, x.tdim, s);
+    x.tree_stream = s;
+    x.tree_mixed = false;
+}
+
+// The index serves a search when the tail it leaves to a scan is small; below
+// kTreeMinPoints everything is tail.  Else (8 and more L2 dimensions, where
+// boxes exclude little, or a tail grown under stream capture) the full scan on
+// the matrix cores does.  Measured, index against full scan, k = 10, one query
+// to 65,536: 2,048 points of R^7 12.9 / 175 us against 46 / 266; 5,000 of SE3
+// 12.6 / 118 against 54 / 418 (the smallest are the call itself).
+static bool use_tree(const NNIndex &x)
+{
+    return tree_supported(x.metric, x.dim) && x.n - x.tree.m <= std::max<int64_t>(kTreeMinPoints, x.tree.m / 8);
+}
+
+static TreeView tree_view(const NNIndex &x)
+{
+    return TreeView{x.tree.sp, x.tree.sid, x.tree.b0, x.tree.b1, x.tree.b2, x.tree.m, x.n, x.pts, x.removed};
 }
 
 static void append(NNIndex &x, const float *src, int64_t n, bool src_dev, hipStream_t s)
@@ -862,6 +940,7 @@ static void append(NNIndex &x, const float *src, int64_t n, bool src_dev, hipStr
     hipLaunchKernelGGL(build_xt_kernel, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, x.pts, x.dim, x.tdim,
                        x.ksteps, from, to_pad, x.n, x.xt, x.xn_max);
     OA_HIP(hipGetLastError());
+    tree_update(x, s);
     if (!src_dev) OA_HIP(hipStreamSynchronize(s)); // host source may be freed after return
 }
 
@@ -963,6 +1042,15 @@ __global__ void packed_counts_kernel(const int32_t *__restrict__ kq, int64_t nq,
     cnt[i] = v < 0 ? 0 : (v > kmax ? kmax : v);
 }
 
+// CSR offsets of a packed batch: the exclusive scan of the clamped k.
+static void packed_offsets(const int32_t *kq, int64_t nq, int kmax, int64_t *cnt, void *tmp, size_t tmp_bytes,
+                           int64_t *out_off, hipStream_t s)
+{
+    hipLaunchKernelGGL(packed_counts_kernel, dim3((unsigned)((nq + 1 + 255) / 256)), dim3(256), 0, s, kq, nq, kmax,
+                       cnt);
+    OA_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tmp_bytes, cnt, out_off, (int)(nq + 1), s));
+}
+
 // k nearest of nq queries.  Uniform k (kq null): results [nq][k].  Packed
 // batch (kq non-null, per-query k clamped to [0, k]): results CSR at
 // out_off, which this call writes (exclusive scan of the clamped k).
@@ -978,6 +1066,21 @@ static void knn(NNIndex &x, const float *q, int64_t nq, int k, const int32_t *kq
     }
     OA_REQUIRE(q && out_i && out_d, OMPL_AMD_ERR_ARG, "null pointer");
     OA_REQUIRE(x.n < INT32_MAX, OMPL_AMD_ERR_ARG, "too many points for int32 ids");
+    if (use_tree(x)) {
+        size_t cub_bytes = 0;
+        if (kq)
+            OA_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, cub_bytes, (int64_t *)nullptr, (int64_t *)nullptr,
+                                                    (int)(nq + 1), s));
+        const size_t counts_bytes = kq ? ((size_t)(nq + 1) * sizeof(int64_t) + 255) / 256 * 256 : 0;
+        const size_t head = counts_bytes + (cub_bytes + 255) / 256 * 256;
+        char *buf = head ? (char *)scratch(x, head) : nullptr;
+        ProfScope ps("nn_knn", s);
+        if (kq) packed_offsets(kq, nq, k, (int64_t *)buf, buf + counts_bytes, cub_bytes, out_off, s);
+        tree_used(x, s);
+        tree_knn(x.metric, x.dim,
+                 TreeKnnArgs{tree_view(x), q, nq, k, kq, kq ? out_off : nullptr, out_d, out_i}, s);
+        return;
+    }
     const int kmax = k <= 16 ? 16 : (k <= 32 ? 32 : 64);
     // the search keeps a 10-slot list for k <= 10 (PRM's default k): fewer
     // slots per insertion; the split merge keeps its 16
@@ -1008,12 +1111,7 @@ static void knn(NNIndex &x, const float *q, int64_t nq, int k, const int32_t *kq
     const size_t per = splits > 1 ? (size_t)splits * nq * k : 0;
     char *buf = (char *)scratch(x, counts_bytes + cub_span + per * (sizeof(float) + sizeof(int32_t)) + 256);
     ProfScope ps("nn_knn", s);
-    if (kq) {
-        int64_t *cnt = (int64_t *)buf;
-        hipLaunchKernelGGL(packed_counts_kernel, dim3((unsigned)((nq + 1 + 255) / 256)), dim3(256), 0, s, kq, nq, k,
-                           cnt);
-        OA_HIP(hipcub::DeviceScan::ExclusiveSum(buf + counts_bytes, cub_bytes, cnt, out_off, (int)(nq + 1), s));
-    }
+    if (kq) packed_offsets(kq, nq, k, (int64_t *)buf, buf + counts_bytes, cub_bytes, out_off, s);
     if (splits == 1) {
         // one split (or an empty structure: every slot is (-1, +inf))
         A.out_d = out_d;
@@ -1050,6 +1148,9 @@ static void knn(NNIndex &x, const float *q, int64_t nq, int k, const int32_t *kq
 constexpr int kRadiusSlotCap = 64;
 constexpr size_t kRadiusSlotBytesMax = (size_t)256 << 20;
 
+// Word of the thread's pinned slot (runtime.hpp) that a radius search reports in.
+constexpr int kRadiusReportAt = 512;
+
 // Radius search of nq queries, at radius r or, in a packed batch (rq
 // non-null), at each query's own radius.
 static void radius(NNIndex &x, const float *q, int64_t nq, float r, const float *rq, int64_t *offsets, int32_t *out_i,
@@ -1068,6 +1169,13 @@ static void radius(NNIndex &x, const float *q, int64_t nq, float r, const float 
     A.radius = r;
     A.rq = rq;
     const int64_t n_tiles = A.n_tiles;
+    const bool tree = use_tree(x);
+    if (tree) tree_used(x, s);
+    const size_t order_bytes = tree ? tree_order_bytes(x.tree, nq) : 0;
+    const uint32_t *order = nullptr;
+    auto tree_search = [&](int64_t *cnt, const int64_t *off, int slot_cap, uint64_t *keys) {
+        tree_radius(x.metric, x.dim, TreeRadiusArgs{tree_view(x), q, order, nq, r, rq, cnt, off, slot_cap, keys}, s);
+    };
     // more splits than k-NN: a radius wave keeps no list, so the launch gains
     // from more waves to hide its latency (SE3 1M x 65,536: 15.8 ms at 16
     // waves per CU, 13.9 at 32, 13.1 at 64, 12.7 at 128)
@@ -1086,7 +1194,8 @@ static void radius(NNIndex &x, const float *q, int64_t nq, float r, const float 
     const size_t counts_bytes = ((size_t)(nq + 2) * sizeof(int64_t) + 255) / 256 * 256;
     const size_t cub_span = (cub_bytes + 255) / 256 * 256;
     const size_t slot_bytes = one_pass ? (size_t)nq * kRadiusSlotCap * sizeof(uint64_t) : 0;
-    char *buf = (char *)scratch(x, counts_bytes + cub_span + slot_bytes);
+    // (the query order is scratch of the first pass alone)
+    char *buf = (char *)scratch(x, counts_bytes + cub_span + slot_bytes + order_bytes);
     int64_t *counts = (int64_t *)buf;
     unsigned long long *max_count = (unsigned long long *)(counts + nq + 1);
     void *cub_tmp = buf + counts_bytes;
@@ -1095,19 +1204,27 @@ static void radius(NNIndex &x, const float *q, int64_t nq, float r, const float 
     hipLaunchKernelGGL(fill_i64_kernel, dim3((unsigned)((nq + 2 + 255) / 256)), dim3(256), 0, s, counts, nq + 2,
                        (int64_t)0);
     A.counts = counts;
-    if (one_pass) {
+    if (tree) {
+        if (order_bytes)
+            order = tree_order(x.tree, q, nq, x.dim, x.tdim, buf + counts_bytes + cub_span + slot_bytes, s);
+        tree_search(counts, nullptr, one_pass ? kRadiusSlotCap : 0, slots);
+    } else if (one_pass) {
         A.slot_cap = kRadiusSlotCap;
         dispatch_search<2>(x, A, 16, slots, qtiles * splits, s, true);
     } else if (n_tiles) {
         dispatch_search<0>(x, A, 16, nullptr, qtiles * splits, s, true);
     }
-    hipLaunchKernelGGL(max_i64_kernel, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, s, counts, nq, max_count);
+    hipLaunchKernelGGL(max_i64_kernel, dim3((unsigned)std::min<int64_t>((nq + 255) / 256, 64)), dim3(256), 0, s,
+                       counts, nq, max_count);
     OA_HIP(hipcub::DeviceScan::ExclusiveSum(cub_tmp, cub_bytes, counts, offsets, (int)(nq + 1), s));
-    int64_t tot = 0;
-    unsigned long long longest = 0;
-    OA_HIP(hipMemcpyAsync(&tot, offsets + nq, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    OA_HIP(hipMemcpyAsync(&longest, max_count, sizeof(longest), hipMemcpyDeviceToHost, s));
+    ThreadResources &host = thread_resources();
+    volatile int64_t *seen = reinterpret_cast<volatile int64_t *>(host.pinned + kRadiusReportAt);
+    hipLaunchKernelGGL(report_kernel, dim3(1), dim3(64), 0, s, offsets + nq, max_count,
+                       reinterpret_cast<int64_t *>(host.pinned_dev + kRadiusReportAt));
+    OA_HIP(hipGetLastError());
     OA_HIP(hipStreamSynchronize(s));
+    const int64_t tot = seen[0];
+    const unsigned long long longest = (unsigned long long)seen[1];
     *total = tot;
     if (!want || tot == 0) return;
     OA_REQUIRE(capacity >= tot, OMPL_AMD_ERR_ARG, "radius output capacity %lld < %lld results", (long long)capacity,
@@ -1116,6 +1233,12 @@ static void radius(NNIndex &x, const float *q, int64_t nq, float r, const float 
     // keys (dist bits << 32 | idx) sorted per query: one wave per query when
     // every query holds at most kRadiusSortMax keys, else a segmented radix sort
     const bool from_slots = one_pass && longest <= (unsigned long long)kRadiusSlotCap;
+    if (from_slots && tree) { // the tree search leaves its slots sorted
+        hipLaunchKernelGGL(radius_place_kernel, dim3((unsigned)((nq * 16 + 255) / 256)), dim3(256), 0, s, slots,
+                           kRadiusSlotCap, offsets, nq, out_i, out_d);
+        OA_HIP(hipGetLastError());
+        return;
+    }
     const bool wave_sort = longest <= (unsigned long long)kRadiusSortMax;
     size_t sort_bytes = 0;
     if (!wave_sort)
@@ -1136,11 +1259,16 @@ static void radius(NNIndex &x, const float *q, int64_t nq, float r, const float 
     } else {
         // a query overflowed its slot (or no slots): write every key into
         // its CSR span, then sort
-        hipLaunchKernelGGL(fill_i64_kernel, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, s, counts, nq,
-                           (int64_t)0);
-        A.counts = counts;
-        A.offsets = offsets;
-        dispatch_search<1>(x, A, 16, keys, qtiles * splits, s, true);
+        if (tree) {
+            order = nullptr;
+            tree_search(nullptr, offsets, 0, keys);
+        } else {
+            hipLaunchKernelGGL(fill_i64_kernel, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, s, counts, nq,
+                               (int64_t)0);
+            A.counts = counts;
+            A.offsets = offsets;
+            dispatch_search<1>(x, A, 16, keys, qtiles * splits, s, true);
+        }
         if (wave_sort)
             hipLaunchKernelGGL(radius_sort_kernel, dim3((unsigned)((nq + 3) / 4)), dim3(256), 0, s, keys, offsets,
                                nq, (int64_t)0, keys_sorted);
@@ -1200,8 +1328,9 @@ int ompl_amd_nn_create(int metric, int dim, ompl_amd_nn *out)
         x.dim = dim;
         x.tdim = metric == OMPL_AMD_METRIC_SE3 ? 3 : dim;
         x.ksteps = (x.tdim + 2 + 1) / 2;
-        OA_HIP(hipMalloc(&x.xn_max, sizeof(uint32_t)));
-        OA_HIP(hipMemset(x.xn_max, 0, sizeof(uint32_t)));
+        OA_HIP(hipMalloc(&x.xn_max, kStatWords * sizeof(uint32_t)));
+        hipLaunchKernelGGL(clear_stats_kernel, dim3(1), dim3(64), 0, default_stream(), x.xn_max);
+        OA_HIP(hipStreamSynchronize(default_stream()));
         *out = h;
     });
 }
@@ -1216,6 +1345,7 @@ int ompl_amd_nn_destroy(ompl_amd_nn h)
         if (x.removed) OA_HIP(hipFree(x.removed));
         if (x.xn_max) OA_HIP(hipFree(x.xn_max));
         if (x.scratch) OA_HIP(hipFree(x.scratch));
+        tree_free(x.tree);
         delete h;
     });
 }
@@ -1226,11 +1356,12 @@ int ompl_amd_nn_clear(ompl_amd_nn h)
         NNIndex &x = nn_of(h);
         hipStream_t s = default_stream();
         if (x.n && x.removed) OA_HIP(hipMemsetAsync(x.removed, 0, (size_t)x.n, s));
-        OA_HIP(hipMemsetAsync(x.xn_max, 0, sizeof(uint32_t), s));
+        hipLaunchKernelGGL(clear_stats_kernel, dim3(1), dim3(64), 0, s, x.xn_max);
         OA_HIP(hipStreamSynchronize(s));
         std::fill(x.removed_host.begin(), x.removed_host.end(), 0);
         x.n = 0;
         x.n_removed = 0;
+        x.tree.m = 0;
     });
 }
 
@@ -1264,6 +1395,7 @@ int ompl_amd_nn_remove(ompl_amd_nn h, int64_t id, int *removed)
             const uint8_t one = 1;
             hipStream_t s = default_stream();
             OA_HIP(hipMemcpyAsync(x.removed + id, &one, 1, hipMemcpyHostToDevice, s));
+            tree_remove(x.tree, id, s);
             OA_HIP(hipStreamSynchronize(s));
             ++x.n_removed;
             ok = 1;
