@@ -165,24 +165,12 @@ struct LaneSpheres<7> {
     float cx, cy, cz;
 };
 
-// FK of the link layout (GS lanes per state, GS >= 8 a power of two): lane
-// i < 7 of the state's group evaluates sincos of joint i once and the group
-// reads the seven results (readlane when the group is the whole wave); the
-// rotation chain is the one arm_fk_slots evaluates, and the lane keeps the
-// frame (p, Z) of its link g, so its sphere centres are the same bits as
-// arm_fk_slots's.
+// Frame (P, W) of link g from the sines and cosines that lanes 0 .. 6 of the
+// state's GS lanes hold, one joint each; the rotation chain is the one
+// arm_fk_slots evaluates.
 template <int GS>
-__device__ __forceinline__ void arm_fk_links(const float q[kDof], int g, LaneSpheres<7> &S)
+__device__ __forceinline__ void link_chain(float sm, float cm, int g, float P[3], float W[3])
 {
-    const int j = threadIdx.x & 7;
-    float qj = q[0];
-#pragma unroll
-    for (int i = 1; i < kDof; ++i) {
-        qj = (j == i) ? q[i] : qj;
-        asm volatile("" : "+v"(qj)); // keep the selects (not an indexed private-memory load)
-    }
-    float sm, cm;
-    sincos_pl(qj, sm, cm);
     float sj[kDof], cj[kDof];
 #pragma unroll
     for (int i = 0; i < kDof; ++i) {
@@ -227,16 +215,52 @@ __device__ __forceinline__ void arm_fk_links(const float q[kDof], int g, LaneSph
         p1 = p1 + Z1 * kLink;
         p2 = p2 + Z2 * kLink;
     }
+    P[0] = P0;
+    P[1] = P1;
+    P[2] = P2;
+    W[0] = W0;
+    W[1] = W1;
+    W[2] = W2;
+}
+
+// FK of the link layout (GS lanes per state, GS >= 8 a power of two): lane
+// i < 7 of the state's group evaluates sincos of joint i once and the group
+// reads the seven results (readlane when the group is the whole wave); the
+// rotation chain is the one arm_fk_slots evaluates, and the lane keeps the
+// frame (p, Z) of its link g, so its sphere centres (p + Z off) are the same
+// bits as arm_fk_slots's.
+template <int GS>
+__device__ __forceinline__ void link_frame(const float q[kDof], int g, float P[3], float W[3])
+{
+    const int j = threadIdx.x & 7;
+    float qj = q[0];
+#pragma unroll
+    for (int i = 1; i < kDof; ++i) {
+        qj = (j == i) ? q[i] : qj;
+        asm volatile("" : "+v"(qj)); // keep the selects (not an indexed private-memory load)
+    }
+    float sm, cm;
+    sincos_pl(qj, sm, cm);
+    link_chain<GS>(sm, cm, g, P, W);
+}
+
+// The link layout's spheres of link g: its frame's four sphere centres and the
+// centre of their bounding sphere.
+template <int GS>
+__device__ __forceinline__ void arm_fk_links(const float q[kDof], int g, LaneSpheres<7> &S)
+{
+    float P[3], W[3];
+    link_frame<GS>(q, g, P, W);
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
         const float off = sphere_offset(m);
-        S.x[m] = P0 + W0 * off;
-        S.y[m] = P1 + W1 * off;
-        S.z[m] = P2 + W2 * off;
+        S.x[m] = P[0] + W[0] * off;
+        S.y[m] = P[1] + W[1] * off;
+        S.z[m] = P[2] + W[2] * off;
     }
-    S.cx = P0 + W0 * kLinkCentre;
-    S.cy = P1 + W1 * kLinkCentre;
-    S.cz = P2 + W2 * kLinkCentre;
+    S.cx = P[0] + W[0] * kLinkCentre;
+    S.cy = P[1] + W[1] * kLinkCentre;
+    S.cz = P[2] + W[2] * kLinkCentre;
 }
 
 // With LPS = 8 the eight lanes of an aligned lane octet always hold the same

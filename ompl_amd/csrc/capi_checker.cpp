@@ -17,6 +17,9 @@ Env &env_of(ompl_amd_env e)
     return e->env;
 }
 
+// Word of the thread's pinned slot that an environment's build reports in.
+constexpr int kEnvBaseAt = 520;
+
 // Staging order of an obstacle list: increasing distance from the arm's base
 // (the world origin) to the obstacle's nearest point, ties in the caller's
 // order.  Every check result is "any obstacle hit", so the order leaves results
@@ -61,7 +64,11 @@ void ompl_amd::check_motions_tuned(const Tuning &t, const Env &env, const double
     const int LE = t.validity_lanes_per_state, OE = t.validity_obstacle_parts;
     const int LW = t.motion_lanes_per_state, OW = t.motion_obstacle_parts;
     const int64_t persistent_waves = (int64_t)num_cus() * t.motion_waves_per_cu;
-    if (t.motion_strategy == 3 || t.motion_strategy == 4) {
+    if (own_validity_shape(t) && own_walk_shape(t)) {
+        std::unique_lock<std::mutex> lk; // held until this batch's launches are enqueued
+        Workspace &w = own ? *own : workspace(s, (size_t)n, lk);
+        launch_grid_motions(env.grid, A, grid_scratch(w), s);
+    } else if (t.motion_strategy == 3 || t.motion_strategy == 4) {
         // Strategy 4 walks chunks with each position's FK computed once per
         // wave and shared across the obstacle partitions; the s2 pass shares
         // its FK when validity_shared_fk is set.  The survivors' booleans are
@@ -168,10 +175,7 @@ struct ompl_amd_motion_graph_s {
             if (graph[i]) hipGraphDestroy(graph[i]);
         }
         for (auto &w : ws) {
-            if (w->list) hipFree(w->list);
-            if (w->first_bad) hipFree(w->first_bad);
-            if (w->surv_nd) hipFree(w->surv_nd);
-            if (w->surv_ab) hipFree(w->surv_ab);
+            free_workspace_arrays(*w);
             if (w->counters) hipFree(w->counters);
         }
         for (hipStream_t st : side) hipStreamDestroy(st);
@@ -186,11 +190,7 @@ void graph_workspace(Workspace &w, int64_t n)
     const size_t cap = (size_t)n < 1024 ? 1024 : (size_t)n;
     OA_HIP(hipMalloc(&w.counters, 64 * sizeof(int32_t)));
     OA_HIP(hipMemset(w.counters, 0, 64 * sizeof(int32_t)));
-    OA_HIP(hipMalloc(&w.list, cap * sizeof(int32_t)));
-    OA_HIP(hipMalloc(&w.first_bad, cap * sizeof(int32_t)));
-    OA_HIP(hipMalloc(&w.surv_nd, cap * sizeof(int32_t)));
-    OA_HIP(hipMalloc(&w.surv_ab, cap * 14 * sizeof(double)));
-    w.list_cap = cap;
+    alloc_workspace_arrays(w, cap);
     w.parity = 0;
 }
 
@@ -295,28 +295,66 @@ int ompl_amd_env_create(const float *spheres, int n_spheres, const float *boxes,
         }
         both[h.size() - 1] = h[h.size() - 1];
         std::copy(h.begin(), h.end(), both.begin() + h.size());
+        // the grid's obstacle table: every obstacle as a box with a squared
+        // contact distance (a sphere is the box lo = hi = centre)
+        const int n_obs = n_spheres + n_boxes;
+        std::vector<float4> tab;
+        double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+        for (int i = 0; i < n_obs; ++i) {
+            const bool sphere = i < n_spheres;
+            float4 l = sphere ? both[i] : both[2 * i - n_spheres], u = sphere ? l : both[2 * i - n_spheres + 1];
+            if (!sphere) l.w = kRobotR * kRobotR;
+            u.w = 0.0f;
+            tab.push_back(l);
+            tab.push_back(u);
+            const double r = std::sqrt((double)l.w) * 1.00002 + 2e-4;
+            const float a[3] = {l.x, l.y, l.z}, c[3] = {u.x, u.y, u.z};
+            for (int k = 0; k < 3; ++k) {
+                lo[k] = std::min(lo[k], (double)a[k] - r);
+                hi[k] = std::max(hi[k], (double)c[k] + r);
+            }
+        }
         auto *e = new ompl_amd_env_s();
-        e->env.ns = n_spheres;
-        e->env.nb = n_boxes;
-        e->env.bytes = both.size() * sizeof(float4);
-        hipError_t err = hipMalloc(&e->env.obs, e->env.bytes);
+        Env &env = e->env;
+        env.ns = n_spheres;
+        env.nb = n_boxes;
+        env.grid.n_obs = n_obs;
+        grid_extent(env.grid, lo, hi, n_obs == 0);
+        // one allocation: obstacles (both orders) and table, link layout, cells, lists, build counter
+        auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+        const size_t n_both = both.size();
+        both.insert(both.end(), tab.begin(), tab.end());
+        const size_t obs_b = up(both.size() * sizeof(float4)), links_b = up(links_bytes(env.view()) + sizeof(float4)),
+                     cells_b = grid_cells_bytes(env.grid), lists_b = grid_lists_bytes(env.grid);
+        env.bytes = obs_b + links_b + cells_b + lists_b + 256;
+        char *mem = nullptr;
+        const hipError_t err = hipMalloc((void **)&mem, env.bytes);
         if (err != hipSuccess) {
             delete e;
             fail(OMPL_AMD_ERR_NOMEM, "environment allocation failed: %s", hipGetErrorString(err));
         }
-        e->env.obs_input = e->env.obs + h.size();
-        OA_HIP(hipMemcpy(e->env.obs, both.data(), e->env.bytes, hipMemcpyHostToDevice));
-        const size_t lb = links_bytes(e->env.view()) + sizeof(float4);
-        err = hipMalloc(&e->env.obs_links, lb);
-        if (err != hipSuccess) {
-            (void)hipFree(e->env.obs);
+        env.obs = (float4 *)mem;
+        try {
+            env.obs_input = env.obs + h.size();
+            env.obs_links = (float4 *)(mem + obs_b);
+            uint32_t *cells = (uint32_t *)(mem + obs_b + links_b);
+            uint16_t *lists = (uint16_t *)(mem + obs_b + links_b + cells_b);
+            uint32_t *counter = (uint32_t *)(mem + obs_b + links_b + cells_b + lists_b);
+            env.grid.tab = env.obs + n_both;
+            env.grid.cells = cells;
+            env.grid.lists = lists;
+            ThreadResources &r = thread_resources();
+            OA_HIP(hipMemcpyAsync(env.obs, both.data(), both.size() * sizeof(float4), hipMemcpyHostToDevice,
+                                  r.stream));
+            launch_stage_links(env.view(), env.obs_links, r.stream);
+            launch_grid_build(env.grid, cells, lists, counter, r.pinned_dev + kEnvBaseAt, r.stream);
+            OA_HIP(hipStreamSynchronize(r.stream));
+            env.grid.base_hit = r.pinned[kEnvBaseAt];
+        } catch (...) {
+            (void)hipFree(mem);
             delete e;
-            fail(OMPL_AMD_ERR_NOMEM, "environment allocation failed: %s", hipGetErrorString(err));
+            throw;
         }
-        e->env.bytes += lb;
-        ThreadResources &r = thread_resources();
-        launch_stage_links(e->env.view(), e->env.obs_links, r.stream);
-        OA_HIP(hipStreamSynchronize(r.stream));
         *out = e;
     });
 }
@@ -330,7 +368,6 @@ int ompl_amd_env_destroy(ompl_amd_env e)
                    "environment still in use by %d queued or running server request(s); destroy it after they finish",
                    users);
         if (e->env.obs) OA_HIP(hipFree(e->env.obs));
-        if (e->env.obs_links) OA_HIP(hipFree(e->env.obs_links));
         delete e;
     });
 }
@@ -351,6 +388,10 @@ int ompl_amd_validate_states_dev(ompl_amd_env e, const float *q, int64_t n, uint
         if (n == 0) return;
         OA_REQUIRE(q && out, OMPL_AMD_ERR_ARG, "null state or output pointer");
         const Tuning t = tuning_for(*e);
+        if (own_validity_shape(t)) {
+            launch_grid_validate<float>(env.grid, q, n, out, resolve_stream(stream));
+            return;
+        }
         launch_validate<float>(env.view(), q, n, out, t.validity_lanes_per_state, t.validity_obstacle_parts,
                                t.validity_block, resolve_stream(stream), t.validity_shared_fk != 0);
     });
@@ -364,6 +405,10 @@ int ompl_amd_validate_states_f64_dev(ompl_amd_env e, const double *q, int64_t n,
         if (n == 0) return;
         OA_REQUIRE(q && out, OMPL_AMD_ERR_ARG, "null state or output pointer");
         const Tuning t = tuning_for(*e);
+        if (own_validity_shape(t)) {
+            launch_grid_validate<double>(env.grid, q, n, out, resolve_stream(stream));
+            return;
+        }
         launch_validate<double>(env.view(), q, n, out, t.validity_lanes_per_state, t.validity_obstacle_parts,
                                 t.validity_block, resolve_stream(stream), t.validity_shared_fk != 0);
     });
@@ -424,6 +469,10 @@ int ompl_amd_check_motions_last_valid_dev(ompl_amd_env e, const double *a, const
         const hipStream_t st = resolve_stream(stream);
         std::unique_lock<std::mutex> lk; // held until the launches are enqueued
         Workspace &w = workspace(st, (size_t)n, lk);
+        if (own_walk_shape(t)) {
+            launch_grid_last_valid(env.grid, A, last_t, grid_scratch(w), st);
+            return;
+        }
         A.list = w.list;
         A.first_bad = w.first_bad;
         A.surv_nd = w.surv_nd;
@@ -467,6 +516,11 @@ int ompl_amd_check_state_lists_dev(ompl_amd_env e, const double *q_soa, int64_t 
         const hipStream_t st = resolve_stream(stream);
         std::unique_lock<std::mutex> lk; // held until the launches are enqueued
         Workspace &w = workspace(st, (size_t)n_lists, lk);
+        if (own_walk_shape(t)) {
+            launch_grid_state_lists(env.grid, q_soa, n_states, offsets, n_lists, out, first_invalid, grid_scratch(w),
+                                    st);
+            return;
+        }
         launch_state_lists(env.view(), q_soa, n_states, offsets, n_lists, out, first_invalid,
                            t.motion_lanes_per_state, t.motion_obstacle_parts,
                            (int64_t)num_cus() * t.motion_waves_per_cu, w.list, w.first_bad, w.counters + 2, st);
@@ -492,7 +546,13 @@ int ompl_amd_check_states(ompl_amd_env e, const double *states, int count, int *
         {
             std::unique_lock<std::mutex> lk; // held until the launches are enqueued
             Workspace &w = workspace(r.stream, 1, lk);
-            launch_state_lists(env.view(), reinterpret_cast<const double *>(r.stage_dev + head), count,
+            if (own_walk_shape(t))
+                launch_grid_state_lists(env.grid, reinterpret_cast<const double *>(r.stage_dev + head), count,
+                                        reinterpret_cast<const int64_t *>(r.stage_dev), 1,
+                                        reinterpret_cast<uint8_t *>(r.stage_dev + 16),
+                                        reinterpret_cast<int32_t *>(r.stage_dev + 32), grid_scratch(w), r.stream);
+            else
+                launch_state_lists(env.view(), reinterpret_cast<const double *>(r.stage_dev + head), count,
                                reinterpret_cast<const int64_t *>(r.stage_dev), 1,
                                reinterpret_cast<uint8_t *>(r.stage_dev + 16),
                                reinterpret_cast<int32_t *>(r.stage_dev + 32), t.motion_lanes_per_state,
@@ -541,7 +601,10 @@ int ompl_amd_check_motion_last_valid(ompl_amd_env e, const double *a, const doub
             A.list_count = w.counters + 2;
             A.max_m = w.counters + 3;
             const Tuning t = tuning_for(*e);
-            launch_motion_last_valid(A, dev_pd + 2 * kDof, t.motion_lanes_per_state, t.motion_obstacle_parts,
+            if (own_walk_shape(t))
+                launch_grid_last_valid(env.grid, A, dev_pd + 2 * kDof, grid_scratch(w), r.stream);
+            else
+                launch_motion_last_valid(A, dev_pd + 2 * kDof, t.motion_lanes_per_state, t.motion_obstacle_parts,
                                      (int64_t)num_cus() * t.motion_waves_per_cu, r.stream);
         }
         OA_HIP(hipStreamSynchronize(r.stream));

@@ -7,6 +7,7 @@
 
 #include "arm_device.hpp"
 #include "common.hpp"
+#include "grid.hpp"
 
 namespace ompl_amd {
 
@@ -68,6 +69,21 @@ void launch_motion_last_valid(const MotionArgs &A, double *last_t, int lps, int 
 void launch_state_lists(const EnvView &env, const double *q_soa, int64_t n_states, const int64_t *offsets,
                         int64_t n_lists, uint8_t *out, int32_t *first_invalid, int lps, int ops, int64_t waves,
                         int32_t *unres, int32_t *unres_fb, int32_t *counters, hipStream_t s);
+// Survivor workspace of the checks over the cell grid (grid_check.hip).
+struct GridScratch {
+    int32_t *list, *surv_nd, *rest, *long_slot, *long_bad, *ticket; // an entry per edge or list
+    double *surv_ab;                                                 // 14 per edge
+    int32_t *counts;                                                 // two words, zero
+    int32_t *next;                                                   // two words, cleared for the next batch
+};
+template <typename T>
+void launch_grid_validate(const GridView &g, const T *q, int64_t n, uint8_t *out, hipStream_t s);
+void launch_grid_motions(const GridView &g, const MotionArgs &m, const GridScratch &w, hipStream_t s);
+void launch_grid_last_valid(const GridView &g, const MotionArgs &m, double *last_t, const GridScratch &w,
+                            hipStream_t s);
+void launch_grid_state_lists(const GridView &g, const double *q_soa, int64_t n_states, const int64_t *offsets,
+                             int64_t n_lists, uint8_t *out, int32_t *first_invalid, const GridScratch &w,
+                             hipStream_t s);
 void launch_arm_spheres(const float *q, int64_t n, float *out, hipStream_t s);
 
 } // namespace ompl_amd

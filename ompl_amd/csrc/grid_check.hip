@@ -1,0 +1,772 @@
+// State validity, motion validation, lastValid and state lists over an
+// environment's cell grid (grid.hpp).
+//
+// A state is 28 sphere centres; the base link's four never move and are
+// decided when the environment is made.  Each of the other six links looks up
+// the cell of its second sphere: "far" clears the whole link, "clear" all but
+// its last sphere, else the cells of the other three are looked up as well.  Only spheres in a cell that some
+// obstacle's surface passes near are tested, against the obstacles the cell
+// lists, with the exact predicate (arm_device.hpp), so results are the same
+// bits as a test against every obstacle.  On the 128 + 128 obstacle scene that
+// is 6 to 24 reads of a 1 MiB table and a few exact tests per state where the
+// full test has 28 x 256.
+//
+// Lane mapping: one state per lane (no redundant forward kinematics: the
+// fastest where there are states enough), or eight lanes per state, one link
+// each (a third of the latency, twice the instructions).
+//
+// Measured against the kernels that test every obstacle, in the launch shapes
+// the library starts with: 65,536 states, 64 spheres 35.7 -> 8.7 us; 16,384
+// edges, 16 + 16 obstacles, checked counts 384 -> 68 us; 4,099 edges' lastValid
+// 110 -> 31 us; 61 edges, 128 + 128 obstacles 38 -> 11.7 us.  Against shapes
+// tuned for the scene: 16,384 edges, 128 + 128 obstacles 31 -> 22 us on one
+// stream, 12.4 -> 11.3 us a batch on four; 16 + 16 obstacles 77 -> 53 us (no
+// counts).  Large batches are bound by VALU instructions (about 1,100 a wave of
+// 64 states, half of them the forward kinematics), small ones by the chain of
+// dependent reads (counts, record, cells, cells, obstacles) and by fetching
+// the code once.
+#include <hip/hip_runtime.h>
+
+#include <climits>
+
+#include "check_device.hpp"
+#include "checker.hpp"
+#include "grid.hpp"
+#include "motion_device.hpp"
+#include "walk_device.hpp"
+
+namespace ompl_amd {
+
+__device__ __forceinline__ uint32_t cell_word(const GridView &g, float x, float y, float z)
+{
+    // outside the grid: the border cell (for NaN: some cell)
+    const int ix = (int)__builtin_amdgcn_fmed3f(__builtin_fmaf(x, g.inv, g.sx), 0.0f, (float)(g.nx - 1));
+    const int iy = (int)__builtin_amdgcn_fmed3f(__builtin_fmaf(y, g.inv, g.sy), 0.0f, (float)(g.ny - 1));
+    const int iz = (int)__builtin_amdgcn_fmed3f(__builtin_fmaf(z, g.inv, g.sz), 0.0f, (float)(g.nz - 1));
+    return g.cells[(ix * g.ny + iy) * g.nz + iz];
+}
+
+// Exact test of a sphere against one obstacle.
+__device__ __forceinline__ bool obstacle_hit(const GridView &g, int o, float x, float y, float z)
+{
+    const float4 lo = g.tab[2 * o], hi = g.tab[2 * o + 1];
+    const float dx = x - clamp_box(x, lo.x, hi.x), dy = y - clamp_box(y, lo.y, hi.y), dz = z - clamp_box(z, lo.z, hi.z);
+    return (dx * dx + dy * dy) + dz * dz < lo.w;
+}
+
+// Pending exact tests of one wave, in LDS: a state has a few, at different
+// spheres in different lanes, so tested where they arise they would cost the
+// wave a round trip for each of its 24 spheres; collected, 64 of them share one.
+struct WaveTests {
+    static constexpr int kRoom = 64 + 4 * 64; // fewer than 64 waiting, and one link's four spheres
+    float4 item[kRoom];                       // centre, cell word
+    uint8_t owner[kRoom];                     // lane
+    uint32_t hit[2];                          // lanes with a hit
+};
+
+struct Tests {
+    const GridView &g;
+    WaveTests &w;
+    int n = 0; // wave-uniform
+    __device__ __forceinline__ Tests(const GridView &grid, WaveTests &lds) : g(grid), w(lds)
+    {
+        if (lane_id() < 2) w.hit[lane_id()] = 0;
+    }
+    __device__ __forceinline__ void sync()
+    {
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    // Runs the waiting tests, one per lane; true for the lanes that have had a hit.
+    __device__ __forceinline__ bool drain()
+    {
+        const int lane = lane_id();
+        sync();
+#pragma unroll 1
+        for (int i = lane; i < n; i += 64) {
+            const float4 t = w.item[i];
+            const uint32_t wd = __float_as_uint(t.w), owner = w.owner[i];
+            const bool scan = wd == kCellScan;
+            const int m = scan ? g.n_obs : (int)(wd & 255u);
+#pragma unroll 1
+            for (int k = 0; k < m; ++k) { // once, but for a cell in twenty
+                int o = (int)(wd >> (k == 0 ? 8 : 20)) & 0xfff;
+                if (m > 2) o = scan ? k : (int)g.lists[(wd >> 8) + k];
+                if (obstacle_hit(g, o, t.x, t.y, t.z)) {
+                    atomicOr(&w.hit[owner >> 5], 1u << (owner & 31));
+                    break;
+                }
+            }
+        }
+        n = 0;
+        sync();
+        return (w.hit[lane >> 5] >> (lane & 31)) & 1u;
+    }
+    // One sphere (at p + Z off) of each `look` lane in a cell with word wd.
+    __device__ __forceinline__ void sphere(bool look, uint32_t wd, const float p[3], const float Z[3], float off)
+    {
+        const bool c = look && (wd & 255u) != 0;
+        const uint64_t m = wave_ballot(c);
+        if (m == 0) return;
+        const int lane = lane_id();
+        if (c) {
+            const int at = n + __popcll(m & (((uint64_t)1 << lane) - 1));
+            w.item[at] = make_float4(p[0] + Z[0] * off, p[1] + Z[1] * off, p[2] + Z[2] * off, __uint_as_float(wd));
+            w.owner[at] = (uint8_t)lane;
+        }
+        n += __popcll(m);
+    }
+};
+
+// The cells speak for centres within the workspace: sincos_pl is a sine and
+// cosine below 6000 rad only, so a state beyond (or not a number) is tested
+// against every obstacle.
+__device__ __forceinline__ bool odd_state(const float q[kDof])
+{
+    float m = 0.0f;
+    bool nan = false;
+#pragma unroll
+    for (int j = 0; j < kDof; ++j) {
+        m = fmaxf(m, fabsf(q[j]));
+        nan = nan || q[j] != q[j];
+    }
+    return nan || !(m < 6000.0f);
+}
+
+// One state per lane.
+__device__ __forceinline__ bool state_hit1(const GridView &g, const float q[kDof], bool live, WaveTests &lds)
+{
+    if (g.base_hit) return live;
+    const bool odd = odd_state(q);
+    float X[3] = {1.0f, 0.0f, 0.0f}, Y[3] = {0.0f, 1.0f, 0.0f}, Z[3] = {0.0f, 0.0f, 1.0f}, p[3] = {0.0f, 0.0f, 0.0f};
+    float P[kDof - 1][3], W[kDof - 1][3];
+    uint32_t w[kDof - 1];
+#pragma unroll
+    for (int i = 0; i < kDof; ++i) {
+        float s, c;
+        sincos_pl(q[i], s, c);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            if ((i & 1) == 0) {
+                const float nx = X[k] * c + Y[k] * s, ny = Y[k] * c - X[k] * s;
+                X[k] = nx;
+                Y[k] = ny;
+            } else {
+                const float nx = X[k] * c - Z[k] * s, nz = X[k] * s + Z[k] * c;
+                X[k] = nx;
+                Z[k] = nz;
+            }
+        }
+        if (i > 0) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                P[i - 1][k] = p[k];
+                W[i - 1][k] = Z[k];
+            }
+            // the reads of all links are in flight together
+            w[i - 1] = cell_word(g, p[0] + Z[0] * sphere_offset(1), p[1] + Z[1] * sphere_offset(1),
+                                 p[2] + Z[2] * sphere_offset(1));
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) p[k] = p[k] + Z[k] * kLink;
+    }
+    bool hit = false;
+#pragma unroll
+    for (int i = 0; i + 1 < kDof; ++i) {
+        if (odd) w[i] = kCellScan;
+        hit = hit || w[i] == kCellHit;
+    }
+    if (wave_ballot(live && !hit) == 0) return hit && live;
+    // the other spheres of the links that are not far from everything
+    uint32_t v[kDof - 1][4];
+#pragma unroll
+    for (int i = 0; i + 1 < kDof; ++i) {
+        const bool look = live && !hit && w[i] != kCellFar;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            v[i][m] = m == 1 ? w[i] : kCellFree;
+            if (m != 1 && look && (m == 3 || w[i] != kCellClear))
+                v[i][m] = odd ? kCellScan
+                              : cell_word(g, P[i][0] + W[i][0] * sphere_offset(m),
+                                          P[i][1] + W[i][1] * sphere_offset(m),
+                                          P[i][2] + W[i][2] * sphere_offset(m));
+        }
+    }
+#pragma unroll
+    for (int i = 0; i + 1 < kDof; ++i) hit = hit || v[i][0] == kCellHit || v[i][2] == kCellHit || v[i][3] == kCellHit;
+    if (wave_ballot(live && !hit) == 0) return hit && live;
+    // the few centres that are tested are made again from the frames: kept, all
+    // 24 would take 72 registers
+#pragma unroll
+    for (int i = 0; i + 1 < kDof; ++i)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) asm volatile("" : "+v"(P[i][k]), "+v"(W[i][k]));
+    Tests T(g, lds);
+#pragma unroll
+    for (int i = 0; i + 1 < kDof; ++i) {
+        const bool look = live && !hit;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) T.sphere(look, v[i][m], P[i], W[i], sphere_offset(m));
+        if (T.n >= 64 || (i + 2 == kDof && T.n > 0)) hit = T.drain() || hit;
+    }
+    return hit && live;
+}
+
+// Eight lanes per state, lane j of the group holding joint j (qj) and link j:
+// the lane's result (the state's is the OR over the group).
+__device__ __forceinline__ bool state_hit8(const GridView &g, float qj, bool live, WaveTests &lds)
+{
+    if (g.base_hit) return live;
+    const int j = threadIdx.x & 7, group = threadIdx.x & 56;
+    const bool odd = ((wave_ballot(j < kDof && !(fabsf(qj) < 6000.0f)) >> group) & 0x7f) != 0;
+    float sm, cm, p[3], Z[3];
+    sincos_pl(qj, sm, cm);
+    link_chain<8>(sm, cm, j, p, Z);
+    const bool mine = live && j > 0 && j < kDof;
+    uint32_t w[4];
+    // the link's cells are read together: one round trip
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        w[m] = kCellFar;
+        if (mine)
+            w[m] = odd ? kCellScan
+                       : cell_word(g, p[0] + Z[0] * sphere_offset(m), p[1] + Z[1] * sphere_offset(m),
+                                   p[2] + Z[2] * sphere_offset(m));
+    }
+    bool hit = w[0] == kCellHit || w[1] == kCellHit || w[2] == kCellHit || w[3] == kCellHit;
+    const bool done = ((wave_ballot(hit) >> group) & 0xff) != 0;
+    if (wave_ballot(mine && !done) == 0) return hit;
+    Tests T(g, lds);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) T.sphere(mine && !done, w[m], p, Z, sphere_offset(m));
+    if (T.n) hit = T.drain() || hit;
+    return hit;
+}
+
+// ---------------------------------------------------------------------------
+// validity
+// ---------------------------------------------------------------------------
+template <int LANES, typename T>
+__global__ void __launch_bounds__(256) grid_validate_kernel(GridView g, const T *__restrict__ q_soa, int64_t n,
+                                                            uint8_t *__restrict__ out)
+{
+    __shared__ WaveTests tests[4];
+    const int64_t st = (xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x) / LANES;
+    const bool live = st < n;
+    bool hit;
+    if constexpr (LANES == 1) {
+        float q[kDof];
+        load_config(q_soa, n, st, live, q);
+        hit = state_hit1(g, q, live, tests[threadIdx.x >> 6]);
+    } else {
+        const int j = min((int)threadIdx.x & 7, kDof - 1);
+        hit = state_hit8(g, (float)q_soa[(int64_t)j * n + (live ? st : 0)], live, tests[threadIdx.x >> 6]);
+    }
+    const uint64_t H = fold_groups<LANES>(wave_ballot(hit));
+    const int lane = lane_id();
+    if (live && lane % LANES == 0) out[st] = ((H >> lane) & 1) ? 0 : 1;
+}
+
+// ---------------------------------------------------------------------------
+// motions, lastValid, state lists
+// ---------------------------------------------------------------------------
+// What is walked: kBisect, an edge's positions 1 .. nd-1 in bisection order
+// (position 0, its s2, first where the walk starts there); kSequence, positions
+// 1 .. nd in order, nd being s2 (DiscreteMotionValidator.cpp:48-91); kList, the
+// states of a precomputed list in order (SpaceInformation.cpp:288-299).
+enum class Walk { kBisect, kSequence, kList };
+
+// Workspace use (Workspace in runtime.hpp): the first kernel says in rest[slot]
+// whether it left an item unfinished (a list of them would take a device-wide
+// atomic each: on one address they are 6 ns apart, 60 us for 10,000); those
+// with more than kLongWalk positions left are listed in long_slot, with a
+// first_bad and a ticket each.
+constexpr int kLongWalk = 16384;
+
+struct GridWalkArgs {
+    GridView g;
+    MotionArgs m;      // edges: env unused; list / list_count / surv_nd / surv_ab as for the chunk walk
+    double *last_t;    // kSequence
+    const double *q;   // kList: dof-major states
+    int64_t n_states;
+    const int64_t *offsets;
+    int32_t *rest;      // [cap]
+    int32_t *long_slot; // [cap]
+    int32_t *long_bad;  // [cap]
+    int32_t *ticket;    // [cap]
+    int32_t *counts;    // [0] survivors, [1] long items; zero at the batch's start
+    int32_t *next;     // the set the next batch uses, cleared by the first kernel after the s2 pass
+};
+
+// One item: its id (edge or list) and what is needed to make its states.
+template <Walk MODE>
+struct Item {
+    int64_t id;
+    double a[kDof], b[kDof];
+    int64_t lo;
+    int nd, total; // positions are below `total`
+    __device__ __forceinline__ void edge(const MotionArgs &A, int64_t e)
+    {
+        id = e;
+#pragma unroll
+        for (int j = 0; j < kDof; ++j) {
+            a[j] = A.a[(int64_t)j * A.n + e];
+            b[j] = A.b[(int64_t)j * A.n + e];
+        }
+        nd = valid_segment_count<kDof>(a, b, A.lvs, A.factor);
+        total = MODE == Walk::kBisect ? max(nd, 1) : max(nd, 1) + 1;
+    }
+    // slot is wave-uniform; the record was written by an earlier kernel, so it
+    // is read into scalar registers (28 vector registers fewer: a wave more per SIMD)
+    __device__ __forceinline__ void survivor(const MotionArgs &A, int slot_any)
+    {
+        using Const = const __attribute__((address_space(4))) double;
+        const int slot = __builtin_amdgcn_readfirstlane(slot_any);
+        Const *ab = (Const *)(A.surv_ab + (int64_t)slot * 2 * kDof);
+#pragma unroll
+        for (int j = 0; j < kDof; ++j) {
+            a[j] = ab[j];
+            b[j] = ab[kDof + j];
+        }
+        nd = A.surv_nd[slot];
+        id = A.list[slot];
+        total = MODE == Walk::kBisect ? max(nd, 1) : max(nd, 1) + 1;
+    }
+    __device__ __forceinline__ bool nd_too_many() const { return MODE != Walk::kList && nd > kMaxSegments; }
+    __device__ __forceinline__ void list(const GridWalkArgs &A, int64_t l)
+    {
+        id = l;
+        lo = min(max(A.offsets[l], (int64_t)0), A.n_states);
+        total = (int)(max(min(A.offsets[l + 1], A.n_states), lo) - lo);
+    }
+    __device__ __forceinline__ void state(const GridWalkArgs &A, int p, float q[kDof]) const
+    {
+        if (MODE == Walk::kBisect) {
+            walk_state(a, b, nd, p, q);
+        } else if (MODE == Walk::kSequence) {
+            if (p >= total - 1) {
+#pragma unroll
+                for (int j = 0; j < kDof; ++j) q[j] = (float)b[j];
+            } else {
+                interpolate_f32<kDof>(a, b, (double)p / (double)nd, q);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < kDof; ++j) q[j] = (float)A.q[(int64_t)j * A.n_states + lo + p];
+        }
+    }
+    // Result from the lowest invalid position (INT_MAX: none); one lane.
+    __device__ __forceinline__ void result(const GridWalkArgs &A, int bad) const
+    {
+        const bool ok = bad == INT_MAX;
+        A.m.out[id] = ok ? 1 : 0;
+        if (MODE == Walk::kBisect) {
+            if (A.m.checked) A.m.checked[id] = ok ? total : bad + 1;
+        } else if (MODE == Walk::kSequence) {
+            // an interior position j: (j - 1) / nd; s2: (nd - 1) / nd
+            if (!ok) A.last_t[id] = bad < total - 1 ? (double)(bad - 1) / (double)nd : (double)(nd - 1) / (double)nd;
+        } else {
+            if (A.m.checked) A.m.checked[id] = ok ? -1 : bad;
+        }
+    }
+};
+
+// Lowest invalid of the positions base + lane below `total` (one state per
+// lane), or INT_MAX; wave-uniform.
+template <Walk MODE>
+__device__ __forceinline__ int wave_walk(const GridWalkArgs &A, const Item<MODE> &I, int base, int total,
+                                         WaveTests *tests)
+{
+    if (base >= total) return INT_MAX;
+    const int p = base + lane_id();
+    const bool live = p < total;
+    float q[kDof];
+    I.state(A, live ? p : base, q);
+    const uint64_t H = wave_ballot(state_hit1(A.g, q, live, tests[threadIdx.x >> 6]));
+    return H ? base + lowest_bit(H) : INT_MAX;
+}
+
+// The walk of one item by a block (from .. total-1, a block's positions at a
+// time) or, with `wide` false, by each wave for itself (the first 64).  The
+// kernels below have one call of it each: the code of a state check is 10 KB,
+// and a short launch waits for every line of it.  bad: the block's LDS word.
+// Returns the lowest invalid position or INT_MAX, uniform over the walkers.
+template <Walk MODE>
+__device__ __forceinline__ int walk_item(const GridWalkArgs &A, const Item<MODE> &I, int from, int total, bool wide,
+                                         int *bad, WaveTests *tests)
+{
+    if (wide) {
+        if (threadIdx.x == 0) *bad = INT_MAX;
+        __syncthreads();
+    }
+    int64_t base = from + (wide ? (int)(threadIdx.x & ~63u) : 0);
+    for (int64_t round = from;;) {
+        const int b = wave_walk<MODE>(A, I, (int)min(base, (int64_t)INT_MAX), total, tests);
+        if (!wide) return b;
+        if (b != INT_MAX && lane_id() == 0) atomicMin(bad, b);
+        __syncthreads();
+        const int found = *bad;
+        __syncthreads(); // every wave has read it before the next round (or walk) writes it
+        round += blockDim.x;
+        base += blockDim.x;
+        if (found != INT_MAX || round >= total) return found; // block-uniform
+    }
+}
+
+// Leaves an item's positions from `from` on to grid_rest_kernel (one lane).
+__device__ __forceinline__ void leave_rest(const GridWalkArgs &A, int slot, int total, int from)
+{
+    const bool is_long = total - from > kLongWalk;
+    A.rest[slot] = is_long ? 0 : 1;
+    if (is_long) {
+        const int l = atomicAdd(&A.counts[1], 1);
+        A.long_slot[l] = slot;
+        A.long_bad[l] = INT_MAX;
+        A.ticket[l] = 0;
+    }
+}
+
+// Keeps an edge for grid_rest_kernel under `slot` (one lane).
+template <Walk MODE>
+__device__ __forceinline__ void keep_edge(const GridWalkArgs &A, const Item<MODE> &I, int slot)
+{
+    A.m.list[slot] = (int32_t)I.id;
+    A.m.surv_nd[slot] = I.nd;
+    double *ab = A.m.surv_ab + (int64_t)slot * 2 * kDof;
+#pragma unroll
+    for (int j = 0; j < kDof; ++j) {
+        ab[j] = I.a[j];
+        ab[kDof + j] = I.b[j];
+    }
+}
+
+__device__ __forceinline__ void clear_next(const GridWalkArgs &A)
+{
+    if (blockIdx.x == 0 && threadIdx.x < 2) A.next[threadIdx.x] = 0;
+}
+
+// s2 of every edge; survivors (s2 valid, 2 <= nd) go to the list.  One lane
+// per edge: large batches.
+__global__ void __launch_bounds__(256) grid_endpoint1_kernel(GridWalkArgs A)
+{
+    __shared__ WaveTests tests[4];
+    const MotionArgs &M = A.m;
+    const int64_t e = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    const bool live = e < M.n;
+    float q[kDof];
+    load_config(M.b, M.n, e, live, q);
+    const uint64_t H = wave_ballot(state_hit1(A.g, q, live, tests[threadIdx.x >> 6]));
+    int m = 0;
+    double a[kDof], b[kDof];
+    const bool survivor = endpoint_finish<1>(M, e, live, H, m, a, b);
+    append_survivor(M, e, survivor, m, a, b);
+}
+
+// As above with eight lanes per edge: lane j reads joint j of both ends (two
+// reads in flight in place of 7 and then 14) and writes it to a survivor's
+// record.
+__global__ void __launch_bounds__(256) grid_endpoint8_kernel(GridWalkArgs A)
+{
+    __shared__ WaveTests tests[4];
+    __shared__ int blk_count, blk_base;
+    const MotionArgs &M = A.m;
+    if (threadIdx.x == 0) blk_count = 0;
+    const int64_t e = (xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x) >> 3;
+    const bool live = e < M.n;
+    const int lane = lane_id(), j = lane & 7;
+    const int64_t at = (int64_t)min(j, kDof - 1) * M.n + (live ? e : 0);
+    const double bj = M.b[at], aj = M.a[at];
+    const bool hit = state_hit8(A.g, (float)bj, live, tests[threadIdx.x >> 6]);
+    const uint64_t H = fold_groups<8>(wave_ballot(hit));
+    const bool bad = ((H >> (lane & 56)) & 1) != 0;
+    int nd = 0;
+    if (wave_ballot(live && !bad)) {
+        const double diff = aj - bj, sq = diff * diff;
+        double dist2 = 0.0;
+#pragma unroll
+        for (int i = 0; i < kDof; ++i) dist2 += __shfl(sq, (lane & 56) + i);
+        nd = segments_of(dist2, M.lvs, M.factor);
+    }
+    const bool survivor = live && !bad && nd >= 2 && nd <= kMaxSegments;
+    if (live && j == 0) {
+        M.out[e] = !bad && nd <= kMaxSegments ? 1 : 0; // a survivor's until the walk finds an invalid position
+        if (M.checked && !survivor) M.checked[e] = !bad && nd > kMaxSegments ? 0 : 1;
+    }
+    // the block's survivors take consecutive slots
+    const uint64_t sm = wave_ballot(survivor && j == 0);
+    __syncthreads();
+    int woff = 0;
+    if (sm) {
+        if (lane == lowest_bit(sm)) woff = atomicAdd(&blk_count, __popcll(sm));
+        woff = __shfl(woff, lowest_bit(sm));
+    }
+    __syncthreads();
+    if (blk_count == 0) return; // block-uniform
+    if (threadIdx.x == 0) blk_base = atomicAdd(M.list_count, blk_count);
+    __syncthreads();
+    if (survivor) {
+        const int slot = blk_base + woff + __popcll(sm & (((uint64_t)1 << (lane & 56)) - 1));
+        if (j == 0) {
+            M.list[slot] = (int32_t)e;
+            M.surv_nd[slot] = nd;
+        }
+        if (j < kDof) {
+            double *ab = M.surv_ab + (int64_t)slot * 2 * kDof;
+            ab[j] = aj;
+            ab[kDof + j] = bj;
+        }
+    }
+}
+
+// Survivors of the s2 pass: when there are no more than blocks, a block walks
+// each to its end; else a wave walks the first 64 positions of each and leaves
+// the rest to grid_rest_kernel (an edge that fails does so early, and one wave
+// finds out without the other three).
+__global__ void __launch_bounds__(256, 4) grid_survivors_kernel(GridWalkArgs A)
+{
+    __shared__ int bad;
+    __shared__ WaveTests tests[4];
+    clear_next(A);
+    const int n = A.counts[0];
+    const bool wide = n <= (int)gridDim.x;
+    const int wave = threadIdx.x >> 6;
+    Item<Walk::kBisect> I;
+    for (int s = wide ? blockIdx.x : blockIdx.x * 4 + wave; s < n; s += wide ? gridDim.x : 4 * gridDim.x) {
+        I.survivor(A.m, s);
+        const int done = !wide || I.total - 65 > kLongWalk ? min(I.total, 65) : I.total;
+        const int b = walk_item(A, I, 1, done, wide, &bad, tests);
+        if (wide ? threadIdx.x == 0 : lane_id() == 0) {
+            if (b != INT_MAX || done == I.total) {
+                I.result(A, b);
+                A.rest[s] = 0;
+            } else {
+                leave_rest(A, s, I.total, done);
+            }
+        }
+    }
+}
+
+// First walk of edges (kBisect with s2 as position 0, kSequence) and lists:
+// WIDE, a block walks each item to its end (small batches: one launch, every
+// position in flight at once); else a wave walks the first 64 positions.
+template <Walk MODE, bool WIDE>
+__global__ void __launch_bounds__(256, 4) grid_first_kernel(GridWalkArgs A)
+{
+    __shared__ int bad;
+    __shared__ WaveTests tests[4];
+    clear_next(A);
+    const int64_t id = WIDE ? blockIdx.x : (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (id >= A.m.n) return;
+    constexpr int from = MODE == Walk::kSequence ? 1 : 0;
+    const bool writer = WIDE ? threadIdx.x == 0 : lane_id() == 0;
+    Item<MODE> I;
+    if (MODE == Walk::kList) {
+        I.list(A, id);
+    } else {
+        I.edge(A.m, id);
+    }
+    const int slot = (int)id;
+    int done = I.total;
+    if (WIDE ? I.total - from > kLongWalk : true) done = min(I.total, from + (WIDE ? 256 : 64));
+    if (I.nd_too_many()) done = 1; // its s2 alone
+    const int b = walk_item(A, I, I.nd_too_many() && MODE == Walk::kSequence ? done : from, done, WIDE, &bad, tests);
+    if (!writer) return;
+    if (I.nd_too_many()) { // reported invalid without a walk
+        A.m.out[id] = 0;
+        if (A.m.checked) A.m.checked[id] = b == 0 ? 1 : 0;
+        A.rest[slot] = 0;
+        return;
+    }
+    if (b != INT_MAX || done == I.total) {
+        I.result(A, b);
+        if (!WIDE) A.rest[slot] = 0;
+    } else {
+        if (MODE != Walk::kList) keep_edge(A, I, slot);
+        leave_rest(A, slot, I.total, done);
+    }
+}
+
+// What the first kernel left of `items` slots (-1: of the survivors, when there
+// were more than blocks): a block per item from position `from` on; then all
+// blocks together walk the long ones, and the last to finish one writes its
+// result.
+template <Walk MODE>
+__global__ void __launch_bounds__(256, 4) grid_rest_kernel(GridWalkArgs A, int from, int64_t items)
+{
+    __shared__ int bad;
+    __shared__ WaveTests tests[4];
+    const int n_long = A.counts[1];
+    int64_t n = items;
+    if (items < 0) {
+        n = A.counts[0];
+        if (n <= (int64_t)gridDim.x) n = 0;
+    }
+    Item<MODE> I;
+    const int lane = lane_id();
+    // the block's slots are blockIdx.x + i gridDim.x (every wave reads the same
+    // 64 flags at a time), then all blocks' long items
+    int64_t i0 = -64;
+    uint64_t open = 0;
+    int l = -1;
+    for (;;) {
+        int slot = -1;
+        if (l < 0) {
+            while (open == 0) {
+                i0 += 64;
+                if (blockIdx.x + i0 * gridDim.x >= n) break;
+                const int64_t mine = blockIdx.x + (i0 + lane) * gridDim.x;
+                open = wave_ballot(mine < n && A.rest[mine < n ? mine : 0] != 0);
+            }
+            if (open) {
+                slot = (int)(blockIdx.x + (i0 + lowest_bit(open)) * gridDim.x);
+                open &= open - 1;
+            }
+        }
+        const bool is_long = slot < 0;
+        if (is_long) {
+            if (++l >= n_long) break;
+            slot = A.long_slot[l];
+        }
+        if (MODE == Walk::kList) I.list(A, slot);
+        else I.survivor(A.m, slot);
+        // a block's positions at a time: all of a short item's, every gridDim-th
+        // of a long one's until an earlier position is known invalid
+        int64_t at = from + (is_long ? (int64_t)blockIdx.x * blockDim.x : 0);
+        int b = INT_MAX;
+        for (; at < I.total; at += (int64_t)gridDim.x * blockDim.x) {
+            if (is_long && __hip_atomic_load(&A.long_bad[l], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < at) break;
+            b = walk_item(A, I, (int)at, is_long ? (int)min(at + blockDim.x, (int64_t)I.total) : I.total, true, &bad,
+                          tests);
+            if (!is_long || b != INT_MAX) break;
+        }
+        if (!is_long) {
+            if (threadIdx.x == 0) I.result(A, b);
+            continue;
+        }
+        if (threadIdx.x == 0) {
+            if (b != INT_MAX) atomicMin(&A.long_bad[l], b);
+            __threadfence(); // the minimum is made before the ticket is taken
+            if (atomicAdd(&A.ticket[l], 1) == (int)gridDim.x - 1) {
+                __threadfence();
+                I.result(A, __hip_atomic_load(&A.long_bad[l], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// host launchers
+// ---------------------------------------------------------------------------
+static unsigned grid_of(int64_t units, int64_t per)
+{
+    return (unsigned)((units + per - 1) / per);
+}
+
+// States (or edges) from which on one lane per state beats eight: 131,072 fill
+// every SIMD with two waves of 64 states; below, eight lanes have more in flight.
+constexpr int64_t kLaneStates = 131072;
+// Edges or lists up to which a block each walks them in one launch: 1,024
+// blocks of four waves are one wave per SIMD, so the speculative positions of
+// edges that fail at once cost no time; more edges go through the s2 pass.
+constexpr int64_t kWideItems = 1024;
+
+template <typename T>
+void launch_grid_validate(const GridView &g, const T *q, int64_t n, uint8_t *out, hipStream_t s)
+{
+    if (n <= 0) return;
+    ProfScope ps("validate_states", s);
+    if (n >= kLaneStates)
+        hipLaunchKernelGGL((grid_validate_kernel<1, T>), dim3(grid_of(n, 256)), dim3(256), 0, s, g, q, n, out);
+    else
+        hipLaunchKernelGGL((grid_validate_kernel<8, T>), dim3(grid_of(n, 32)), dim3(256), 0, s, g, q, n, out);
+    OA_HIP(hipGetLastError());
+}
+template void launch_grid_validate<float>(const GridView &, const float *, int64_t, uint8_t *, hipStream_t);
+template void launch_grid_validate<double>(const GridView &, const double *, int64_t, uint8_t *, hipStream_t);
+
+static GridWalkArgs walk_args(const GridView &g, const MotionArgs &m, const GridScratch &w)
+{
+    GridWalkArgs A{};
+    A.g = g;
+    A.m = m;
+    A.m.list = w.list;
+    A.m.surv_nd = w.surv_nd;
+    A.m.surv_ab = w.surv_ab;
+    A.m.list_count = w.counts;
+    A.m.max_m = nullptr;
+    A.m.first_bad = nullptr;
+    A.rest = w.rest;
+    A.long_slot = w.long_slot;
+    A.long_bad = w.long_bad;
+    A.ticket = w.ticket;
+    A.counts = w.counts;
+    A.next = w.next;
+    return A;
+}
+
+template <Walk MODE>
+static void launch_first_and_rest(const GridWalkArgs &A, hipStream_t s)
+{
+    constexpr int from = MODE == Walk::kSequence ? 1 : 0;
+    const int64_t n = A.m.n;
+    if (n <= kWideItems)
+        hipLaunchKernelGGL((grid_first_kernel<MODE, true>), dim3((unsigned)n), dim3(256), 0, s, A);
+    else
+        hipLaunchKernelGGL((grid_first_kernel<MODE, false>), dim3(grid_of(n, 4)), dim3(256), 0, s, A);
+    hipLaunchKernelGGL((grid_rest_kernel<MODE>), dim3((unsigned)num_cus() * 4), dim3(256), 0, s, A,
+                       n <= kWideItems ? from + 256 : from + 64, n <= kWideItems ? (int64_t)0 : n);
+    OA_HIP(hipGetLastError());
+}
+
+void launch_grid_motions(const GridView &g, const MotionArgs &m, const GridScratch &w, hipStream_t s)
+{
+    if (m.n <= 0) return;
+    const GridWalkArgs A = walk_args(g, m, w);
+    if (m.n <= kWideItems) {
+        ProfScope ps("motion_walk", s);
+        launch_first_and_rest<Walk::kBisect>(A, s);
+        return;
+    }
+    {
+        ProfScope ps("motion_endpoint", s);
+        if (m.n >= kLaneStates)
+            hipLaunchKernelGGL(grid_endpoint1_kernel, dim3(grid_of(m.n, 256)), dim3(256), 0, s, A);
+        else
+            hipLaunchKernelGGL(grid_endpoint8_kernel, dim3(grid_of(m.n, 32)), dim3(256), 0, s, A);
+    }
+    ProfScope ps("motion_chunk", s);
+    const unsigned blocks = (unsigned)num_cus() * 8;
+    hipLaunchKernelGGL(grid_survivors_kernel, dim3(blocks), dim3(256), 0, s, A);
+    hipLaunchKernelGGL((grid_rest_kernel<Walk::kBisect>), dim3(blocks), dim3(256), 0, s, A, 65,
+                       (int64_t)-1);
+    OA_HIP(hipGetLastError());
+}
+
+void launch_grid_last_valid(const GridView &g, const MotionArgs &m, double *last_t, const GridScratch &w,
+                            hipStream_t s)
+{
+    if (m.n <= 0) return;
+    GridWalkArgs A = walk_args(g, m, w);
+    A.last_t = last_t;
+    ProfScope ps("motion_last_valid", s);
+    launch_first_and_rest<Walk::kSequence>(A, s);
+}
+
+void launch_grid_state_lists(const GridView &g, const double *q_soa, int64_t n_states, const int64_t *offsets,
+                             int64_t n_lists, uint8_t *out, int32_t *first_invalid, const GridScratch &w,
+                             hipStream_t s)
+{
+    if (n_lists <= 0) return;
+    MotionArgs m{};
+    m.n = n_lists;
+    m.out = out;
+    m.checked = first_invalid;
+    GridWalkArgs A = walk_args(g, m, w);
+    A.q = q_soa;
+    A.n_states = n_states;
+    A.offsets = offsets;
+    ProfScope ps("state_lists", s);
+    launch_first_and_rest<Walk::kList>(A, s);
+}
+
+} // namespace ompl_amd

@@ -67,6 +67,16 @@ __host__ __device__ __forceinline__ int bisection_index(int p, int nd)
 
 // StateSpace::validSegmentCount (base/src/StateSpace.cpp:851-854) over
 // RealVectorStateSpace::distance (base/spaces/src/RealVectorStateSpace.cpp:230-242).
+// segments_of: from the squared distance.
+__host__ __device__ __forceinline__ int segments_of(double dist2, double lvs, unsigned factor)
+{
+    const double d = __builtin_sqrt(dist2);
+    const double segs = __builtin_ceil(d / lvs);
+    // out of range (or NaN): more than kMaxSegments, flagged to the caller
+    if (!(segs * (double)factor <= (double)kMaxSegments)) return kMaxSegments + 1;
+    return (int)(factor * (unsigned)segs);
+}
+
 template <int DIM>
 __host__ __device__ __forceinline__ int valid_segment_count(const double a[DIM], const double b[DIM], double lvs,
                                                             unsigned factor)
@@ -77,11 +87,7 @@ __host__ __device__ __forceinline__ int valid_segment_count(const double a[DIM],
         double diff = a[i] - b[i];
         dist += diff * diff;
     }
-    const double d = __builtin_sqrt(dist);
-    const double segs = __builtin_ceil(d / lvs);
-    // out of range (or NaN): more than kMaxSegments, flagged to the caller
-    if (!(segs * (double)factor <= (double)kMaxSegments)) return kMaxSegments + 1;
-    return (int)(factor * (unsigned)segs);
+    return segments_of(dist, lvs, factor);
 }
 
 // RealVectorStateSpace::interpolate then the FP64 -> FP32 cast of

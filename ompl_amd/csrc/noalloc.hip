@@ -23,8 +23,8 @@ constexpr int64_t kNoAllocMaxEdges = 65536;
 constexpr size_t kNoAllocCounterBytes = 256; // 64 int32 counters
 constexpr size_t kNoAllocListBytes = (size_t)kNoAllocMaxEdges * sizeof(int32_t);
 constexpr size_t kNoAllocEndpointBytes = (size_t)kNoAllocMaxEdges * 14 * sizeof(double);
-// counters | list | first_bad | surv_nd | surv_ab  (every part 256-byte aligned)
-constexpr size_t kNoAllocScratchBytes = kNoAllocCounterBytes + 3 * kNoAllocListBytes + kNoAllocEndpointBytes;
+// counters | list | first_bad | surv_nd | surv_ab | longs  (every part 256-byte aligned)
+constexpr size_t kNoAllocScratchBytes = kNoAllocCounterBytes + 6 * kNoAllocListBytes + kNoAllocEndpointBytes;
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
@@ -75,6 +75,8 @@ extern "C" int ompl_amd_check_motions_noalloc_dev(ompl_amd_env e, const double *
         w.first_bad = reinterpret_cast<int32_t *>(base + kNoAllocCounterBytes + kNoAllocListBytes);
         w.surv_nd = reinterpret_cast<int32_t *>(base + kNoAllocCounterBytes + 2 * kNoAllocListBytes);
         w.surv_ab = reinterpret_cast<double *>(base + kNoAllocCounterBytes + 3 * kNoAllocListBytes);
+        w.longs = reinterpret_cast<int32_t *>(base + kNoAllocCounterBytes + 3 * kNoAllocListBytes +
+                                              kNoAllocEndpointBytes);
         w.list_cap = (size_t)kNoAllocMaxEdges;
         w.parity = 0;
         launch_zero(w.counters, (int)(kNoAllocCounterBytes / sizeof(int32_t)), s);

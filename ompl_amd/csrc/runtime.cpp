@@ -101,6 +101,42 @@ hipStream_t default_stream()
     return g_stream;
 }
 
+void alloc_workspace_arrays(Workspace &w, size_t cap)
+{
+    OA_HIP(hipMalloc(&w.list, cap * sizeof(int32_t)));
+    OA_HIP(hipMalloc(&w.first_bad, cap * sizeof(int32_t)));
+    OA_HIP(hipMalloc(&w.surv_nd, cap * sizeof(int32_t)));
+    OA_HIP(hipMalloc(&w.longs, 3 * cap * sizeof(int32_t)));
+    OA_HIP(hipMalloc(&w.surv_ab, cap * 14 * sizeof(double)));
+    w.list_cap = cap;
+}
+
+void free_workspace_arrays(Workspace &w)
+{
+    for (void *p : {(void *)w.list, (void *)w.first_bad, (void *)w.surv_nd, (void *)w.longs, (void *)w.surv_ab})
+        if (p) (void)hipFree(p);
+    w.list = w.first_bad = w.surv_nd = w.longs = nullptr;
+    w.surv_ab = nullptr;
+    w.list_cap = 0;
+}
+
+GridScratch grid_scratch(Workspace &w)
+{
+    int32_t *sets = w.counters + 16;
+    const size_t cap = w.list_cap;
+    GridScratch g{w.list,
+                  w.surv_nd,
+                  w.first_bad,
+                  w.longs,
+                  w.longs + cap,
+                  w.longs + 2 * cap,
+                  w.surv_ab,
+                  sets + 4 * w.grid_parity,
+                  sets + 4 * (1 - w.grid_parity)};
+    w.grid_parity ^= 1;
+    return g;
+}
+
 Workspace &workspace(hipStream_t s, size_t list_entries, std::unique_lock<std::mutex> &lock)
 {
     Workspace *w = nullptr;
@@ -120,16 +156,8 @@ Workspace &workspace(hipStream_t s, size_t list_entries, std::unique_lock<std::m
     if (w->list_cap < list_entries) {
         // the stream may still use the old arrays
         OA_HIP(hipStreamSynchronize(s));
-        if (w->list) OA_HIP(hipFree(w->list));
-        if (w->first_bad) OA_HIP(hipFree(w->first_bad));
-        if (w->surv_nd) OA_HIP(hipFree(w->surv_nd));
-        if (w->surv_ab) OA_HIP(hipFree(w->surv_ab));
-        size_t cap = list_entries < 1024 ? 1024 : list_entries;
-        OA_HIP(hipMalloc(&w->list, cap * sizeof(int32_t)));
-        OA_HIP(hipMalloc(&w->first_bad, cap * sizeof(int32_t)));
-        OA_HIP(hipMalloc(&w->surv_nd, cap * sizeof(int32_t)));
-        OA_HIP(hipMalloc(&w->surv_ab, cap * 14 * sizeof(double)));
-        w->list_cap = cap;
+        free_workspace_arrays(*w);
+        alloc_workspace_arrays(*w, list_entries < 1024 ? 1024 : list_entries);
     }
     return *w;
 }

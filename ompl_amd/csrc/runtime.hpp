@@ -25,14 +25,18 @@ struct Workspace {
     int32_t *first_bad = nullptr; // per survivor (chunk-parallel walk)
     int32_t *surv_nd = nullptr;   // per survivor segment count (chunk-parallel walk)
     double *surv_ab = nullptr;    // per survivor endpoints a, b (14 doubles)
+    int32_t *longs = nullptr;     // three words per survivor (grid walk: long items)
     size_t list_cap = 0;
     // [0] survivor count, [1] walk queue (strategy 1, cleared per call);
     // strategies 3 and 4: two sets of (survivor count, max positions) at
     // [8..9] and [10..11], zero at creation.  A batch uses set `parity`; either
     // its results kernel clears that set, or (no results kernel) its phase-1
     // walk clears the other set and the next batch uses that one.
+    // The checks over the cell grid: two sets of two at [16..17] and
+    // [20..21], used in turn by grid_parity, each cleared by the batch before.
     int32_t *counters = nullptr;
     int parity = 0;
+    int grid_parity = 0;
     // Held by a batch from choosing its counter set to enqueuing its launches
     // (and around resizing), so host threads that share a stream cannot pick
     // the same set or see arrays being replaced.
@@ -41,6 +45,11 @@ struct Workspace {
 // The stream's workspace with room for list_entries survivors.  The caller
 // must hold the returned workspace's mu while it uses the workspace (lock
 // passes that lock back, already taken, before any resize).
+// Arrays of a workspace for `cap` survivors (counters excepted); freed with free_workspace_arrays.
+void alloc_workspace_arrays(Workspace &w, size_t cap);
+void free_workspace_arrays(Workspace &w);
+// The next grid batch's view of a workspace (its lock held).
+GridScratch grid_scratch(Workspace &w);
 Workspace &workspace(hipStream_t s, size_t list_entries, std::unique_lock<std::mutex> &lock);
 
 // Per-thread stream and pinned result slot of the blocking single-call entry
@@ -70,6 +79,21 @@ struct Tuning {
     int validity_shared_fk = 0;
 };
 
+// The launch shapes the library starts with stand for its own choice: batched
+// validity, motion, lastValid and list checks with these run over the
+// environment's cell grid (grid_check.hip), with shapes chosen by batch size.
+// Any other shapes ask for the kernels of checker.hip in those shapes.  The
+// block sizes and the waves per CU do not matter here: the grid kernels have
+// their own.
+inline bool own_validity_shape(const Tuning &t)
+{
+    return t.validity_lanes_per_state == 8 && t.validity_obstacle_parts == 2 && t.validity_shared_fk == 0;
+}
+inline bool own_walk_shape(const Tuning &t)
+{
+    return t.motion_lanes_per_state == 8 && t.motion_obstacle_parts == 1 && t.motion_strategy == 3;
+}
+
 Tuning get_tuning();
 // Rejects (OA_REQUIRE) a tuning whose shapes or limits are not built.
 void check_tuning(const Tuning &t);
@@ -94,6 +118,7 @@ struct Env {
     // the same obstacles in the link layout's staging (spheres (x,y,z,bound^2),
     // boxes, then the spheres' rr as floats), for kernels that read them from HBM
     float4 *obs_links = nullptr;
+    GridView grid{}; // cell grid (grid.hpp), in the same allocation
     int ns = 0;
     int nb = 0;
     size_t bytes = 0;
