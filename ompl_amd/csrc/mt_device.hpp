@@ -2,14 +2,12 @@
 // libstdc++'s generate_canonical<double, 53> over it (the 0-1 distribution
 // of RNG::uniformReal, util/RandomNumbers.h:72-76, :191).
 //
-// The 624-word state lives in LDS.  A twist is done by the whole block in the
-// four dependency phases of the in-place recurrence
+// The 624-word state lives in LDS.  The in-place recurrence
 //   new[i] = src[i+397] ^ twist(old[i], old[i+1])   (indices mod 624)
-// phase A: i in [0,227)   src = old,
-// phase B: i in [227,454) src = new (phase A),
-// phase C: i in [454,623) src = new (phase B),
-// phase D: i = 623        old[624 mod 624] = new[0], src = new[396],
-// each phase reading its inputs before any thread writes.
+// reads src from the new words from i = 227 on: new[i] then needs new[i-227].
+// So the chain t, t+227, t+454 depends on no other chain: one thread computes
+// it from old words alone, the block needs no barrier within a twist, and only
+// word 623 wants a word of another chain (new[0]), which it makes again.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -48,28 +46,33 @@ __device__ __forceinline__ void mt_seed_serial(uint32_t *mt, uint32_t v)
     }
 }
 
-// One phase: words [lo, hi) from (old[i], old[i+1], mt[i + off]), all read
-// before any is written.
-__device__ __forceinline__ void mt_twist_phase(uint32_t *mt, int lo, int hi, int off)
-{
-    for (int i0 = lo; i0 < hi; i0 += blockDim.x) {
-        const int i = i0 + threadIdx.x;
-        uint32_t v = 0;
-        if (i < hi) v = mt_twist_word(mt[i], mt[i + 1], mt[i + off]);
-        __syncthreads();
-        if (i < hi) mt[i] = v;
-        __syncthreads();
-    }
-}
-
-// Twist of the LDS state by the whole block (any block size; every thread
-// must call it).
+// Twist of the LDS state by the whole block (at least 64 threads; every thread
+// must call it): every old word is read before any new one is written, two
+// barriers in all.
 __device__ __forceinline__ void mt_twist_block(uint32_t *mt)
 {
-    mt_twist_phase(mt, 0, 227, kMtM);
-    mt_twist_phase(mt, 227, 454, -227);
-    mt_twist_phase(mt, 454, 623, -227);
-    if (threadIdx.x == 0) mt[623] = mt_twist_word(mt[623], mt[0], mt[396]);
+    constexpr int kChains = 227, kMost = (kChains + 63) / 64;
+    uint32_t v[kMost][3];
+#pragma unroll
+    for (int i = 0; i < kMost; ++i) {
+        const int t = threadIdx.x + i * blockDim.x;
+        if (t < kChains) {
+            v[i][0] = mt_twist_word(mt[t], mt[t + 1], mt[t + kMtM]);
+            v[i][1] = mt_twist_word(mt[t + 227], mt[t + 228], v[i][0]);
+            if (t < 169) v[i][2] = mt_twist_word(mt[t + 454], mt[t + 455], v[i][1]);
+            else if (t == 169) v[i][2] = mt_twist_word(mt[623], mt_twist_word(mt[0], mt[1], mt[kMtM]), v[i][1]);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kMost; ++i) {
+        const int t = threadIdx.x + i * blockDim.x;
+        if (t < kChains) {
+            mt[t] = v[i][0];
+            mt[t + 227] = v[i][1];
+            if (t < 170) mt[t + 454] = v[i][2];
+        }
+    }
     __syncthreads();
 }
 

@@ -6,13 +6,14 @@
 // (w1 + w2*2^32) / 2^64, values rounding to 1 replaced by the largest double
 // below 1), then (hi - lo) * u + lo per dimension in order.
 //
-// One wave per generator; the 624-word state lives in LDS and is twisted by
-// the block in the recurrence's four dependency phases (mt_device.hpp).
+// One workgroup per generator; the 624-word state lives in LDS and is twisted
+// by the block (mt_device.hpp).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <vector>
 
+#include "grid_device.hpp"
 #include "mt_device.hpp"
 #include "runtime.hpp"
 
@@ -20,79 +21,25 @@ namespace ompl_amd {
 
 constexpr int kDim7 = OMPL_AMD_ARM_DOF;
 
-struct SampleArgs {
-    const uint32_t *seeds;
-    int n_streams;
-    int64_t n_per_stream;
-    int dim;
-    const double *lo;
-    const double *hi;
-    double *out;       // [stream][n_per_stream][dim]
-    float *out_f32;    // [dim][n_streams * n_per_stream] or null
+// A call's bounds, by value (they are host arrays of at most 16 entries).
+struct Bounds {
+    double lo[16], span[16];
 };
 
-__global__ void __launch_bounds__(64) sample_uniform_kernel(SampleArgs A)
+static Bounds bounds_of(const double *lo, const double *hi, int dim)
 {
-    __shared__ uint32_t mt[kMtN];
-    __shared__ double lo[16], span[16];
-    const int s = blockIdx.x;
-    const int t = threadIdx.x;
-    if (t < A.dim) {
-        lo[t] = A.lo[t];
-        span[t] = A.hi[t] - A.lo[t];
+    Bounds b{};
+    for (int d = 0; d < dim; ++d) {
+        b.lo[d] = lo[d];
+        b.span[d] = hi[d] - lo[d];
     }
-    if (t == 0) {
-        uint32_t v = A.seeds[s];
-        mt[0] = v;
-        for (int i = 1; i < kMtN; ++i) {
-            v = 1812433253u * (v ^ (v >> 30)) + (uint32_t)i;
-            mt[i] = v;
-        }
-    }
-    __syncthreads();
-    const int64_t total_pairs = A.n_per_stream * A.dim;
-    const int64_t total_states = (int64_t)A.n_streams * A.n_per_stream;
-    double *out = A.out + (int64_t)s * total_pairs;
-    for (int64_t base = 0; base < total_pairs; base += kMtN / 2) {
-        mt_twist_block(mt);
-        for (int p = t; p < kMtN / 2; p += 64) {
-            const int64_t z = base + p;
-            if (z >= total_pairs) break;
-            const uint32_t w1 = mt_temper(mt[2 * p]);
-            const uint32_t w2 = mt_temper(mt[2 * p + 1]);
-            const int d = (int)(z % A.dim);
-            const double v = span[d] * canonical53(w1, w2) + lo[d];
-            out[z] = v;
-            if (A.out_f32) {
-                const int64_t st = (int64_t)s * A.n_per_stream + z / A.dim;
-                A.out_f32[(int64_t)d * total_states + st] = (float)v;
-            }
-        }
-        __syncthreads();
-    }
+    return b;
 }
-
-// ---------------------------------------------------------------------------
-// UniformValidStateSampler::sample (base/samplers/src/UniformValidStateSampler.cpp:
-// 46-57), batched over streams: each stream is one sampler making successive
-// sample() calls; a call draws uniform states until one is valid or `attempts`
-// draws were made.  The draws of a stream depend on the validity of earlier
-// ones, so the batch runs in rounds: every unfinished stream draws C more
-// states (its generator resumes where it stopped), all are checked in one
-// batched validity launch, and one thread per stream hands them out to its
-// calls in order.
 
 struct MtState {
     uint32_t mt[kMtN];
     int32_t idx; // next word; kMtN = twist before the next draw
     int32_t pad[3];
-};
-
-struct ValidCursor {
-    int64_t call;     // next call of this stream
-    int64_t used;     // draws consumed from the generator by the calls so far
-    int32_t attempts; // draws made by the current call
-    int32_t pad;
 };
 
 __global__ void mt_seed_kernel(const uint32_t *__restrict__ seeds, int n, MtState *__restrict__ st)
@@ -108,127 +55,214 @@ __global__ void mt_seed_kernel(const uint32_t *__restrict__ seeds, int n, MtStat
     st[s].idx = kMtN;
 }
 
-// One wave per listed stream: resumes the generator and writes C states of
-// `dim` doubles ([a][C][dim]) and, when out_f32 is given, their FP32 copy
-// ([dim][n_active * C]); `active` lists the streams (all of them, or the
-// unfinished ones of a valid-sampling round).
-__global__ void __launch_bounds__(64) resume_uniform_kernel(MtState *__restrict__ st, const int32_t *__restrict__ active,
-                                                            int n_active, int64_t C, int dim,
-                                                            const double *__restrict__ lo_g,
-                                                            const double *__restrict__ hi_g, double *__restrict__ out,
-                                                            float *__restrict__ out_f32)
+// The block's generator into LDS: seeded (seeds: a device or host-mapped
+// array) or resumed.  Ends with a barrier.
+__device__ __forceinline__ int load_generator(uint32_t *mt, const uint32_t *seeds, const MtState *gen)
 {
-    __shared__ uint32_t mt[kMtN];
-    __shared__ double lo[16], span[16];
-    const int a = blockIdx.x;
-    const int t = threadIdx.x;
-    MtState &S = st[active ? active[a] : a];
-    for (int i = t; i < kMtN; i += 64) mt[i] = S.mt[i];
-    if (t < dim) {
-        lo[t] = lo_g[t];
-        span[t] = hi_g[t] - lo_g[t];
+    int idx = kMtN;
+    if (seeds) {
+        if (threadIdx.x == 0) mt_seed_serial(mt, seeds[blockIdx.x]);
+    } else {
+        for (int i = threadIdx.x; i < kMtN; i += blockDim.x) mt[i] = gen[blockIdx.x].mt[i];
+        idx = gen[blockIdx.x].idx;
     }
-    int idx = S.idx;
     __syncthreads();
-    const int64_t total = C * dim;
-    const int64_t n_f32 = (int64_t)n_active * C;
-    double *o = out + (int64_t)a * total;
+    return idx;
+}
+
+__device__ __forceinline__ void store_generator(const uint32_t *mt, int idx, MtState *gen)
+{
+    for (int i = threadIdx.x; i < kMtN; i += blockDim.x) gen[blockIdx.x].mt[i] = mt[i];
+    if (threadIdx.x == 0) gen[blockIdx.x].idx = idx;
+}
+
+// The next `total` canonical draws of the block's generator, draw z handed to
+// use(z, value) by one thread.
+template <class Use>
+__device__ __forceinline__ void draw_block(uint32_t *mt, int &idx, int64_t total, Use use)
+{
     for (int64_t z = 0; z < total;) {
         if (idx >= kMtN) {
             mt_twist_block(mt);
             idx = 0;
         }
-        const int64_t cnt = min((int64_t)((kMtN - idx) / 2), total - z);
-        for (int p = t; p < cnt; p += 64) {
-            const uint32_t w1 = mt_temper(mt[idx + 2 * p]);
-            const uint32_t w2 = mt_temper(mt[idx + 2 * p + 1]);
-            const int64_t zz = z + p;
-            const int d = (int)(zz % dim);
-            const double v = span[d] * canonical53(w1, w2) + lo[d];
-            o[zz] = v;
-            if (out_f32) out_f32[(int64_t)d * n_f32 + (int64_t)a * C + zz / dim] = (float)v;
-        }
-        __syncthreads();
-        idx += 2 * (int)cnt;
+        const int cnt = (int)min((int64_t)((kMtN - idx) / 2), total - z);
+        for (int p = threadIdx.x; p < cnt; p += blockDim.x)
+            use(z + p, canonical53(mt_temper(mt[idx + 2 * p]), mt_temper(mt[idx + 2 * p + 1])));
+        idx += 2 * cnt;
         z += cnt;
+        __syncthreads(); // the words are read before the next twist writes them
     }
-    for (int i = t; i < kMtN; i += 64) S.mt[i] = mt[i];
-    if (t == 0) S.idx = idx;
 }
 
-// One wave per stream: st = saved advanced by the cursor's consumed draws
-// (2 words per coordinate), i.e. the generator exactly after the last draw
-// the calls used; the draws of the last round past that point are dropped.
-__global__ void __launch_bounds__(64) mt_advance_kernel(MtState *__restrict__ st, const MtState *__restrict__ saved,
-                                                        const ValidCursor *__restrict__ cur, int dim)
+// n_per_stream states of `dim` doubles per generator ([stream][n][dim]) and,
+// when out_f32 is given, their FP32 copy ([dim][n_streams * n]).  Bound by the
+// twists (one per 312 coordinates, a chain): 256 generators x 782 states of 7
+// take 36 us; with 64 threads and eight barriers a twist they took 58.
+__global__ void __launch_bounds__(256) sample_uniform_kernel(const uint32_t *__restrict__ seeds,
+                                                             MtState *__restrict__ gen, int64_t n_per_stream, int dim,
+                                                             Bounds B, double *__restrict__ out,
+                                                             float *__restrict__ out_f32)
 {
     __shared__ uint32_t mt[kMtN];
-    const int s = blockIdx.x;
-    const int t = threadIdx.x;
-    for (int i = t; i < kMtN; i += 64) mt[i] = saved[s].mt[i];
-    int idx = saved[s].idx;
-    __syncthreads();
-    int64_t skip = cur[s].used * 2 * dim;
-    while (skip > 0) {
-        if (idx >= kMtN) {
-            mt_twist_block(mt);
-            idx = 0;
-        }
-        const int take = (int)min((int64_t)(kMtN - idx), skip);
-        idx += take;
-        skip -= take;
+    __shared__ double lo[16], span[16];
+    if (threadIdx.x < 16) {
+        lo[threadIdx.x] = B.lo[threadIdx.x];
+        span[threadIdx.x] = B.span[threadIdx.x];
     }
-    for (int i = t; i < kMtN; i += 64) st[s].mt[i] = mt[i];
-    if (t == 0) st[s].idx = idx;
+    int idx = load_generator(mt, seeds, gen);
+    const int64_t n_all = (int64_t)gridDim.x * n_per_stream;
+    double *o = out + (int64_t)blockIdx.x * n_per_stream * dim;
+    const bool small = n_per_stream * dim <= (int64_t)UINT32_MAX;
+    draw_block(mt, idx, n_per_stream * dim, [&](int64_t z, double u) {
+        const int64_t st = small ? (int64_t)((uint32_t)z / (uint32_t)dim) : z / dim;
+        const int d = (int)(z - st * dim);
+        const double v = span[d] * u + lo[d];
+        o[z] = v;
+        if (out_f32) out_f32[(int64_t)d * n_all + (int64_t)blockIdx.x * n_per_stream + st] = (float)v;
+    });
+    if (gen && !seeds) store_generator(mt, idx, gen);
 }
 
-// One thread per active stream: hands the round's draws to its calls in order.
-__global__ void assign_valid_kernel(ValidCursor *__restrict__ cur, const int32_t *__restrict__ active, int n_active,
-                                    int64_t C, const uint8_t *__restrict__ valid, const double *__restrict__ cand,
-                                    int64_t n_calls, int attempts, double *__restrict__ out,
-                                    uint8_t *__restrict__ found, int32_t *__restrict__ draws,
-                                    unsigned long long *__restrict__ stats)
+// ---------------------------------------------------------------------------
+// UniformValidStateSampler::sample (base/samplers/src/UniformValidStateSampler.cpp:
+// 46-57), batched over streams: each stream is one sampler making successive
+// sample() calls; a call draws uniform states until one is valid or `attempts`
+// draws were made.  One workgroup per stream runs all its calls: it draws a
+// batch, one state per thread, checks the batch over the cell grid, and finds
+// where calls end.  Draw j ends a call when it is valid or when the draws since
+// the last valid one (or since the call under way began) are a multiple of
+// `attempts`, so every thread decides its own draw from the batch's valid bits.
+// A batch may draw past the last call's end; the generator is then put back to
+// the batch's start and advanced by the draws that were used.
+//
+// 256 samplers x 64 calls, one draw in eighty valid: 198 us, bound by the
+// batches' chain (a twist per 44 draws, then the check); in rounds of one launch
+// per step it took 3.9 ms (a host round trip, a serial hand-out of 867 us and a
+// rewind pass per round).
+constexpr int kValidThreads = 512;
+// Batches of one launch: a call whose calls could take more (many attempts in a
+// scene with nothing valid) goes on in another, from its cursors.
+constexpr int kValidBatches = 4096;
+
+struct ValidCursor {
+    int64_t call, drawn; // calls made; draws seen by them
+    uint32_t carry;      // draws of the call under way
+    uint32_t pad;
+};
+
+struct ValidArgs {
+    GridView g;
+    const uint32_t *seeds; // or null: resume gen
+    MtState *gen;          // or null: the generators are not kept
+    int64_t n_calls;
+    int attempts;
+    Bounds b;
+    double *out;
+    uint8_t *found;
+    int32_t *draws;
+    ValidCursor *cursor; // or null: one launch is enough
+    int32_t *open;       // with cursor: streams that are not done
+};
+
+__global__ void __launch_bounds__(kValidThreads) sample_valid_kernel(ValidArgs A)
 {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= n_active) return;
-    const int s = active[a];
-    ValidCursor c = cur[s];
-    int64_t used = 0, used_valid = 0;
-    for (int64_t j = 0; j < C && c.call < n_calls; ++j) {
-        const bool v = valid[(int64_t)a * C + j] != 0;
-        ++c.attempts;
-        ++used;
-        used_valid += v;
-        if (v || c.attempts >= attempts) {
-            const int64_t o = (int64_t)s * n_calls + c.call;
+    constexpr int kWaves = kValidThreads / 64;
+    __shared__ uint32_t mt[kMtN], mt0[kMtN];
+    // the batch's draws, until each thread has its state; then the exact tests
+    __shared__ union {
+        double u[kValidThreads * kDim7];
+        WaveTests tests[kWaves];
+    } w;
+    __shared__ uint64_t valid_bits[kWaves], end_bits[kWaves];
+    __shared__ int used;
+    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    int idx = load_generator(mt, A.seeds, A.gen);
+    int64_t call = 0, calls_drawn = 0;
+    uint32_t carry = 0; // draws of the call under way (fewer than attempts)
+    if (A.cursor) {
+        call = A.cursor[blockIdx.x].call;
+        calls_drawn = A.cursor[blockIdx.x].drawn;
+        carry = A.cursor[blockIdx.x].carry;
+        if (call >= A.n_calls) return;
+    }
+    for (int batch = 0; call < A.n_calls && !(A.cursor && batch == kValidBatches); ++batch) {
+        // a batch that should finish the calls, by the draws a call took so far
+        const int64_t left = A.n_calls - call;
+        const double want = call > 0 ? 1.125 * (double)left * (double)calls_drawn / (double)call
+                                     : (calls_drawn ? (double)kValidThreads : 1.25 * (double)left) + 16.0;
+        const int m = (int)fmin((double)kValidThreads, fmax(64.0, want));
+        for (int i = t; i < kMtN; i += kValidThreads) mt0[i] = mt[i];
+        const int idx0 = idx;
+        __syncthreads();
+        draw_block(mt, idx, (int64_t)m * kDim7, [&](int64_t z, double u) { w.u[z] = u; });
+        double v[kDim7];
+        float q[kDof];
 #pragma unroll
-            for (int d = 0; d < kDim7; ++d) out[o * kDim7 + d] = cand[((int64_t)a * C + j) * kDim7 + d];
-            found[o] = v ? 1 : 0;
-            if (draws) draws[o] = c.attempts;
-            ++c.call;
-            c.attempts = 0;
+        for (int d = 0; d < kDim7; ++d) {
+            v[d] = A.b.span[d] * (t < m ? w.u[t * kDim7 + d] : 0.0) + A.b.lo[d];
+            q[d] = (float)v[d];
         }
+        __syncthreads(); // the draws are read: their room is free
+        const bool live = t < m;
+        const bool valid = live && !state_hit1(A.g, q, live, w.tests[wave]);
+        const uint64_t vb = __ballot(valid);
+        if (lane == 0) valid_bits[wave] = vb;
+        __syncthreads();
+        int last = -1; // the last valid draw before this one
+        for (int i = 0; i < wave; ++i)
+            if (valid_bits[i]) last = i * 64 + 63 - __builtin_clzll(valid_bits[i]);
+        const uint64_t below = vb & (((uint64_t)1 << lane) - 1);
+        if (below) last = wave * 64 + 63 - __builtin_clzll(below);
+        const uint32_t since = last >= 0 ? (uint32_t)(t - last) : (uint32_t)t + 1u + carry;
+        const bool end = live && (valid || since % (uint32_t)A.attempts == 0);
+        const uint64_t eb = __ballot(end);
+        if (lane == 0) end_bits[wave] = eb;
+        if (t == 0) used = m;
+        __syncthreads();
+        int before = 0, all = 0, last_end = -1;
+        for (int i = 0; i < kWaves; ++i) {
+            const uint64_t e = end_bits[i];
+            if (i < wave) before += __popcll(e);
+            all += __popcll(e);
+            if (e) last_end = i * 64 + 63 - __builtin_clzll(e);
+        }
+        const int64_t c = call + before + __popcll(eb & (((uint64_t)1 << lane) - 1));
+        if (end && c < A.n_calls) {
+            const int64_t o = (int64_t)blockIdx.x * A.n_calls + c;
+#pragma unroll
+            for (int d = 0; d < kDim7; ++d) A.out[o * kDim7 + d] = v[d];
+            A.found[o] = valid ? 1 : 0;
+            if (A.draws) A.draws[o] = (int32_t)((since - 1) % (uint32_t)A.attempts) + 1;
+            if (c == A.n_calls - 1) used = t + 1;
+        }
+        __syncthreads();
+        carry = last_end >= 0 ? (uint32_t)(m - 1 - last_end) : carry + (uint32_t)m;
+        calls_drawn += m;
+        call = min(call + all, A.n_calls);
+        if (call == A.n_calls && A.gen) {
+            // back to the batch's start, then past the draws that were used
+            const int take = used;
+            for (int i = t; i < kMtN; i += kValidThreads) mt[i] = mt0[i];
+            __syncthreads();
+            idx = idx0;
+            for (int skip = take * 2 * kDim7; skip > 0;) {
+                if (idx >= kMtN) {
+                    mt_twist_block(mt);
+                    idx = 0;
+                }
+                const int n = min(kMtN - idx, skip);
+                idx += n;
+                skip -= n;
+            }
+        }
+        __syncthreads(); // `used` and the bits are read before the next batch writes them
     }
-    c.used += used;
-    cur[s] = c;
-    atomicAdd(&stats[0], (unsigned long long)used);
-    atomicAdd(&stats[1], (unsigned long long)used_valid);
-    if (c.call < n_calls) atomicMax(&stats[2], (unsigned long long)(n_calls - c.call));
-}
-
-__global__ void next_active_kernel(const ValidCursor *__restrict__ cur, int n_streams, int64_t n_calls,
-                                   int32_t *__restrict__ active, unsigned long long *__restrict__ stats)
-{
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool open = s < n_streams && cur[s].call < n_calls;
-    const uint64_t m = __ballot(open);
-    int base = 0;
-    const int lane = threadIdx.x & 63;
-    if (m) {
-        if (lane == __ffsll((unsigned long long)m) - 1) base = (int)atomicAdd(&stats[3], (unsigned long long)__popcll(m));
-        base = __shfl(base, __ffsll((unsigned long long)m) - 1);
+    if (A.gen) store_generator(mt, idx, A.gen);
+    if (A.cursor && t == 0) {
+        A.cursor[blockIdx.x] = ValidCursor{call, calls_drawn, carry, 0};
+        if (call < A.n_calls) atomicAdd(A.open, 1);
     }
-    if (open) active[base + __popcll(m & (((uint64_t)1 << lane) - 1))] = s;
 }
 
 // SE3StateSampler::sampleUniform (a compound sampler: the R^3 component's
@@ -238,8 +272,7 @@ __global__ void next_active_kernel(const ValidCursor *__restrict__ cur, int n_st
 // t2 = 2 pi u5, q = (sin t1 sqrt(1-x0), cos t1 sqrt(1-x0), sin t2 sqrt(x0),
 // cos t2 sqrt(x0)) in FP64 (the device's sin/cos are within an ulp or two of
 // the host's).  Output rows (x, y, z, qx, qy, qz, qw) as FP64 and FP32.
-__global__ void se3_from_uniform_kernel(const double *__restrict__ u, int64_t n, const double *__restrict__ lo,
-                                        const double *__restrict__ hi, double *__restrict__ out,
+__global__ void se3_from_uniform_kernel(const double *__restrict__ u, int64_t n, Bounds B, double *__restrict__ out,
                                         float *__restrict__ out_f32)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -247,7 +280,7 @@ __global__ void se3_from_uniform_kernel(const double *__restrict__ u, int64_t n,
     const double *v = u + i * 6;
     double r[7];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) r[k] = (hi[k] - lo[k]) * v[k] + lo[k];
+    for (int k = 0; k < 3; ++k) r[k] = B.span[k] * v[k] + B.lo[k];
     const double pi = 3.141592653589793238462643383279502884;
     const double x0 = v[3];
     const double r1 = sqrt(1.0 - x0), r2 = sqrt(x0);
@@ -263,103 +296,67 @@ __global__ void se3_from_uniform_kernel(const double *__restrict__ u, int64_t n,
     }
 }
 
-// Device bounds of a sampling call (host arrays staged per call).
-struct Bounds {
-    double *lo, *hi;
-};
-
-static Bounds stage_bounds(const double *lo, const double *hi, int dim, hipStream_t s)
+// The seeds of a call in the thread's host-mapped staging, which the kernel
+// reads; the call waits for the stream before it returns.
+static const uint32_t *stage_seeds(const uint32_t *seeds, int n)
 {
-    double *d = nullptr;
-    OA_HIP(hipMallocAsync((void **)&d, 32 * sizeof(double), s));
-    OA_HIP(hipMemcpyAsync(d, lo, dim * sizeof(double), hipMemcpyHostToDevice, s));
-    OA_HIP(hipMemcpyAsync(d + 16, hi, dim * sizeof(double), hipMemcpyHostToDevice, s));
-    return Bounds{d, d + 16};
+    ThreadResources &r = thread_resources();
+    stage_reserve(r, (size_t)n * sizeof(uint32_t));
+    std::copy(seeds, seeds + n, reinterpret_cast<uint32_t *>(r.stage));
+    return reinterpret_cast<const uint32_t *>(r.stage_dev);
 }
 
-// UniformValidStateSampler::sample x n_calls on each of n_streams generators
-// (gen, device), continuing them; on return every generator stands exactly
-// after the last draw its calls consumed.  Blocking.
-static void sample_valid_rounds(ompl_amd_env env, MtState *gen, int n_streams, int64_t n_calls, int attempts,
-                                const double *lo, const double *hi, double *out_dev, uint8_t *found_dev,
-                                int32_t *draws_dev, hipStream_t s)
+static void sample_uniform(const uint32_t *seeds, MtState *gen, int n_streams, int64_t n_per_stream, int dim,
+                           const double *lo, const double *hi, double *out, float *out_f32, hipStream_t s)
 {
-    const size_t head = 256;
-    const size_t bytes = head + (size_t)n_streams * (sizeof(MtState) + sizeof(ValidCursor) + sizeof(int32_t));
-    char *base = nullptr;
-    OA_HIP(hipMallocAsync((void **)&base, bytes, s));
-    unsigned long long *stats = (unsigned long long *)base; // [0] used [1] valid [2] max remaining [3] active
-    MtState *saved = (MtState *)(base + head);
-    ValidCursor *cur = (ValidCursor *)(saved + n_streams);
-    int32_t *active = (int32_t *)(cur + n_streams);
-    const Bounds bd = stage_bounds(lo, hi, kDim7, s);
-    OA_HIP(hipMemcpyAsync(saved, gen, (size_t)n_streams * sizeof(MtState), hipMemcpyDeviceToDevice, s));
-    OA_HIP(hipMemsetAsync(cur, 0, (size_t)n_streams * sizeof(ValidCursor), s));
-    std::vector<int32_t> all((size_t)n_streams);
-    for (int i = 0; i < n_streams; ++i) all[(size_t)i] = i;
-    OA_HIP(hipMemcpyAsync(active, all.data(), all.size() * sizeof(int32_t), hipMemcpyHostToDevice, s));
-    int n_active = n_streams;
-    int64_t remaining = n_calls;
-    double draws_per_call = 1.0; // refined from every round
-    double *cand = nullptr;
-    float *cand32 = nullptr;
-    uint8_t *valid = nullptr;
-    size_t cap = 0;
-    const int64_t max_round = ((int64_t)64 << 20) / ((int64_t)n_streams * kDim7 * 8) + 16; // ~64 MiB of draws
-    int64_t rounds = 0;
-    const int64_t round_limit = n_calls * (int64_t)attempts + 2;
-    while (n_active > 0) {
-        if (++rounds > round_limit) fail(OMPL_AMD_ERR_INTERNAL, "valid sampler did not finish");
-        const double want = (double)remaining * std::min((double)attempts, draws_per_call) * 1.25 + 16.0;
-        const int64_t C = std::max<int64_t>(
-            16, std::min<int64_t>((int64_t)want, std::min<int64_t>(max_round, remaining * (int64_t)attempts)));
-        const size_t need = (size_t)n_active * (size_t)C;
-        if (need > cap) {
-            if (cand) {
-                OA_HIP(hipFreeAsync(cand, s));
-                OA_HIP(hipFreeAsync(cand32, s));
-                OA_HIP(hipFreeAsync(valid, s));
-            }
-            cap = need;
-            OA_HIP(hipMallocAsync((void **)&cand, cap * kDim7 * sizeof(double), s));
-            OA_HIP(hipMallocAsync((void **)&cand32, cap * kDim7 * sizeof(float), s));
-            OA_HIP(hipMallocAsync((void **)&valid, cap, s));
-        }
-        {
-            ProfScope ps("sample_valid", s);
-            hipLaunchKernelGGL(resume_uniform_kernel, dim3(n_active), dim3(64), 0, s, gen, active, n_active, C, kDim7,
-                               bd.lo, bd.hi, cand, cand32);
-            OA_HIP(hipGetLastError());
-        }
-        const int rc = ompl_amd_validate_states_dev(env, cand32, (int64_t)need, valid, s);
-        if (rc != OMPL_AMD_OK) fail(rc, "%s", last_error());
-        OA_HIP(hipMemsetAsync(stats, 0, 4 * sizeof(unsigned long long), s));
-        hipLaunchKernelGGL(assign_valid_kernel, dim3((n_active + 63) / 64), dim3(64), 0, s, cur, active, n_active, C,
-                           valid, cand, n_calls, attempts, out_dev, found_dev, draws_dev, stats);
-        hipLaunchKernelGGL(next_active_kernel, dim3((n_streams + 255) / 256), dim3(256), 0, s, cur, n_streams,
-                           n_calls, active, stats);
-        OA_HIP(hipGetLastError());
-        unsigned long long h[4];
-        OA_HIP(hipMemcpyAsync(h, stats, sizeof(h), hipMemcpyDeviceToHost, s));
-        OA_HIP(hipStreamSynchronize(s));
-        n_active = (int)h[3];
-        remaining = (int64_t)h[2];
-        if (h[1] > 0)
-            draws_per_call = std::max(1.0, (double)h[0] / (double)h[1]);
-        else
-            draws_per_call = (double)attempts;
-    }
-    // drop the draws of the last round that no call used
-    hipLaunchKernelGGL(mt_advance_kernel, dim3(n_streams), dim3(64), 0, s, gen, saved, cur, kDim7);
+    ProfScope ps("sample_uniform", s);
+    hipLaunchKernelGGL(sample_uniform_kernel, dim3(n_streams), dim3(256), 0, s, seeds, gen, n_per_stream, dim,
+                       bounds_of(lo, hi, dim), out, out_f32);
     OA_HIP(hipGetLastError());
-    if (cand) {
-        OA_HIP(hipFreeAsync(cand, s));
-        OA_HIP(hipFreeAsync(cand32, s));
-        OA_HIP(hipFreeAsync(valid, s));
+}
+
+static void sample_valid(ompl_amd_env env, const uint32_t *seeds, MtState *gen, int n_streams, int64_t n_calls,
+                         int attempts, const double *lo, const double *hi, double *out_dev, uint8_t *found_dev,
+                         int32_t *draws_dev, hipStream_t s)
+{
+    ValidArgs A{env->env.grid, seeds,     gen,       n_calls, attempts, bounds_of(lo, hi, kDim7), out_dev,
+                found_dev,     draws_dev, nullptr, nullptr};
+    auto launch = [&] {
+        ProfScope ps("sample_valid", s);
+        hipLaunchKernelGGL(sample_valid_kernel, dim3(n_streams), dim3(kValidThreads), 0, s, A);
+        OA_HIP(hipGetLastError());
+    };
+    // no batch holds fewer than 64 draws
+    if ((double)n_calls * attempts <= 64.0 * (kValidBatches - 1)) {
+        launch();
+        OA_HIP(hipStreamSynchronize(s));
+        return;
     }
-    OA_HIP(hipFreeAsync(bd.lo, s));
-    OA_HIP(hipFreeAsync(base, s));
-    OA_HIP(hipStreamSynchronize(s));
+    struct Scratch { // generators of a seeded call, cursors and the count
+        hipStream_t s;
+        char *p = nullptr;
+        ~Scratch()
+        {
+            if (p) (void)hipFreeAsync(p, s);
+            (void)hipStreamSynchronize(s);
+        }
+    } room{s};
+    const size_t cursors = (size_t)n_streams * sizeof(ValidCursor), gens = seeds ? (size_t)n_streams * sizeof(MtState) : 0;
+    OA_HIP(hipMallocAsync((void **)&room.p, cursors + gens + 256, s));
+    A.cursor = (ValidCursor *)room.p;
+    A.open = (int32_t *)(room.p + cursors + gens);
+    OA_HIP(hipMemsetAsync(A.cursor, 0, cursors, s));
+    if (seeds) {
+        A.gen = (MtState *)(room.p + cursors);
+        A.seeds = nullptr;
+        hipLaunchKernelGGL(mt_seed_kernel, dim3((n_streams + 63) / 64), dim3(64), 0, s, seeds, n_streams, A.gen);
+    }
+    for (int32_t open = 1; open > 0;) {
+        OA_HIP(hipMemsetAsync(A.open, 0, sizeof(int32_t), s));
+        launch();
+        OA_HIP(hipMemcpyAsync(&open, A.open, sizeof(open), hipMemcpyDeviceToHost, s));
+        OA_HIP(hipStreamSynchronize(s));
+    }
 }
 
 } // namespace ompl_amd
@@ -376,23 +373,9 @@ extern "C" int ompl_amd_sample_uniform_dev(const uint32_t *seeds, int n_streams,
         if (n_streams == 0 || n_per_stream == 0) return;
         OA_REQUIRE(seeds && lo && hi && out_dev, OMPL_AMD_ERR_ARG, "null pointer");
         hipStream_t s = resolve_stream(stream);
-        // bounds and seeds are small host arrays: stage them on the device
-        char *stage = nullptr;
-        const size_t bytes = (size_t)n_streams * sizeof(uint32_t) + 2 * 16 * sizeof(double);
-        OA_HIP(hipMallocAsync((void **)&stage, bytes, s));
-        double *dlo = (double *)stage, *dhi = dlo + 16;
-        uint32_t *dseeds = (uint32_t *)(dhi + 16);
-        OA_HIP(hipMemcpyAsync(dlo, lo, dim * sizeof(double), hipMemcpyHostToDevice, s));
-        OA_HIP(hipMemcpyAsync(dhi, hi, dim * sizeof(double), hipMemcpyHostToDevice, s));
-        OA_HIP(hipMemcpyAsync(dseeds, seeds, n_streams * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-        SampleArgs A{dseeds, n_streams, n_per_stream, dim, dlo, dhi, out_dev, out_f32};
-        {
-            ProfScope ps("sample_uniform", s);
-            hipLaunchKernelGGL(sample_uniform_kernel, dim3(n_streams), dim3(64), 0, s, A);
-            OA_HIP(hipGetLastError());
-        }
-        OA_HIP(hipFreeAsync(stage, s));
-        OA_HIP(hipStreamSynchronize(s)); // host arrays were staged with async copies
+        sample_uniform(stage_seeds(seeds, n_streams), nullptr, n_streams, n_per_stream, dim, lo, hi, out_dev, out_f32,
+                       s);
+        OA_HIP(hipStreamSynchronize(s)); // the seeds are read from host memory
     });
 }
 
@@ -433,16 +416,8 @@ int ompl_amd_sample_valid_dev(ompl_amd_env env, const uint32_t *seeds, int n_str
         if (n_streams == 0 || n_calls == 0) return;
         OA_REQUIRE(seeds && lo && hi && out_dev && found_dev, OMPL_AMD_ERR_ARG, "null pointer");
         hipStream_t s = resolve_stream(stream);
-        MtState *gen = seed_generators(seeds, n_streams, s);
-        try {
-            sample_valid_rounds(env, gen, n_streams, n_calls, attempts, lo, hi, out_dev, found_dev, draws_dev, s);
-        } catch (...) {
-            hipStreamSynchronize(s);
-            hipFree(gen);
-            throw;
-        }
-        OA_HIP(hipFreeAsync(gen, s));
-        OA_HIP(hipStreamSynchronize(s));
+        sample_valid(env, stage_seeds(seeds, n_streams), nullptr, n_streams, n_calls, attempts, lo, hi, out_dev,
+                     found_dev, draws_dev, s);
     });
 }
 
@@ -480,15 +455,8 @@ int ompl_amd_rng_sample_uniform_dev(ompl_amd_rng rng, int64_t n_per_stream, int 
         if (n_per_stream == 0) return;
         OA_REQUIRE(lo && hi && out_dev, OMPL_AMD_ERR_ARG, "null pointer");
         hipStream_t s = resolve_stream(stream);
-        const Bounds bd = stage_bounds(lo, hi, dim, s);
-        {
-            ProfScope ps("sample_uniform", s);
-            hipLaunchKernelGGL(resume_uniform_kernel, dim3(rng->n), dim3(64), 0, s, rng->gen, (const int32_t *)nullptr,
-                               rng->n, n_per_stream, dim, bd.lo, bd.hi, out_dev, out_f32_soa_dev);
-            OA_HIP(hipGetLastError());
-        }
-        OA_HIP(hipFreeAsync(bd.lo, s));
-        OA_HIP(hipStreamSynchronize(s)); // host bounds were staged with async copies
+        sample_uniform(nullptr, rng->gen, rng->n, n_per_stream, dim, lo, hi, out_dev, out_f32_soa_dev, s);
+        OA_HIP(hipStreamSynchronize(s));
     });
 }
 
@@ -502,23 +470,18 @@ int ompl_amd_rng_sample_se3_dev(ompl_amd_rng rng, int64_t n_per_stream, const do
         OA_REQUIRE(lo && hi && out_dev, OMPL_AMD_ERR_ARG, "null pointer");
         hipStream_t s = resolve_stream(stream);
         const double zero[6] = {0, 0, 0, 0, 0, 0}, one[6] = {1, 1, 1, 1, 1, 1};
-        const Bounds unit = stage_bounds(zero, one, 6, s);
-        const Bounds box = stage_bounds(lo, hi, 3, s);
         const int64_t n = (int64_t)rng->n * n_per_stream;
         double *u = nullptr;
         OA_HIP(hipMallocAsync((void **)&u, (size_t)n * 6 * sizeof(double), s));
         {
             ProfScope ps("sample_se3", s);
-            hipLaunchKernelGGL(resume_uniform_kernel, dim3(rng->n), dim3(64), 0, s, rng->gen, (const int32_t *)nullptr,
-                               rng->n, n_per_stream, 6, unit.lo, unit.hi, u, (float *)nullptr);
+            sample_uniform(nullptr, rng->gen, rng->n, n_per_stream, 6, zero, one, u, nullptr, s);
             hipLaunchKernelGGL(se3_from_uniform_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, u, n,
-                               box.lo, box.hi, out_dev, out_f32_dev);
+                               bounds_of(lo, hi, 3), out_dev, out_f32_dev);
             OA_HIP(hipGetLastError());
         }
         OA_HIP(hipFreeAsync(u, s));
-        OA_HIP(hipFreeAsync(unit.lo, s));
-        OA_HIP(hipFreeAsync(box.lo, s));
-        OA_HIP(hipStreamSynchronize(s)); // host bounds were staged with async copies
+        OA_HIP(hipStreamSynchronize(s));
     });
 }
 
@@ -531,8 +494,8 @@ int ompl_amd_rng_sample_valid_dev(ompl_amd_rng rng, ompl_amd_env env, int64_t n_
         OA_REQUIRE(n_calls >= 0 && attempts >= 1, OMPL_AMD_ERR_ARG, "bad sizes");
         if (n_calls == 0) return;
         OA_REQUIRE(lo && hi && out_dev && found_dev, OMPL_AMD_ERR_ARG, "null pointer");
-        sample_valid_rounds(env, rng->gen, rng->n, n_calls, attempts, lo, hi, out_dev, found_dev, draws_dev,
-                            resolve_stream(stream));
+        sample_valid(env, nullptr, rng->gen, rng->n, n_calls, attempts, lo, hi, out_dev, found_dev, draws_dev,
+                     resolve_stream(stream));
     });
 }
 
