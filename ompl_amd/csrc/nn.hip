@@ -66,6 +66,8 @@ struct NNIndex {
     // per-call scratch (grow-only)
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
+    // the library's device blocks behind pts, xt, removed and xn_max
+    DeviceBlock blocks[4];
 };
 
 } // namespace ompl_amd
@@ -864,9 +866,13 @@ static void reserve(NNIndex &x, int64_t need, hipStream_t s)
     cap = (cap + 31) / 32 * 32;
     float *pts = nullptr, *xt = nullptr;
     uint8_t *rem = nullptr;
-    OA_HIP(hipMalloc(&pts, (size_t)cap * x.dim * sizeof(float)));
-    OA_HIP(hipMalloc(&xt, (size_t)cap * x.ksteps * 2 * sizeof(float)));
-    OA_HIP(hipMalloc(&rem, (size_t)cap));
+    DeviceBlock fresh[3];
+    fresh[0] = take_block((size_t)cap * x.dim * sizeof(float));
+    fresh[1] = take_block((size_t)cap * x.ksteps * 2 * sizeof(float));
+    fresh[2] = take_block((size_t)cap);
+    pts = (float *)fresh[0].p;
+    xt = (float *)fresh[1].p;
+    rem = (uint8_t *)fresh[2].p;
     OA_HIP(hipMemsetAsync(rem, 0, (size_t)cap, s));
     if (x.n) {
         OA_HIP(hipMemcpyAsync(pts, x.pts, (size_t)x.n * x.dim * sizeof(float), hipMemcpyDeviceToDevice, s));
@@ -875,9 +881,11 @@ static void reserve(NNIndex &x, int64_t need, hipStream_t s)
         OA_HIP(hipMemcpyAsync(rem, x.removed, (size_t)x.n, hipMemcpyDeviceToDevice, s));
     }
     OA_HIP(hipStreamSynchronize(s));
-    if (x.pts) OA_HIP(hipFree(x.pts));
-    if (x.xt) OA_HIP(hipFree(x.xt));
-    if (x.removed) OA_HIP(hipFree(x.removed));
+    if (x.pts) OA_HIP(hipDeviceSynchronize()); // searches on other streams may read the old arrays
+    for (int i = 0; i < 3; ++i) {
+        give_block(x.blocks[i]);
+        x.blocks[i] = fresh[i];
+    }
     x.pts = pts;
     x.xt = xt;
     x.removed = rem;
@@ -1328,7 +1336,8 @@ int ompl_amd_nn_create(int metric, int dim, ompl_amd_nn *out)
         x.dim = dim;
         x.tdim = metric == OMPL_AMD_METRIC_SE3 ? 3 : dim;
         x.ksteps = (x.tdim + 2 + 1) / 2;
-        OA_HIP(hipMalloc(&x.xn_max, kStatWords * sizeof(uint32_t)));
+        x.blocks[3] = take_block(kStatWords * sizeof(uint32_t));
+        x.xn_max = (uint32_t *)x.blocks[3].p;
         hipLaunchKernelGGL(clear_stats_kernel, dim3(1), dim3(64), 0, default_stream(), x.xn_max);
         OA_HIP(hipStreamSynchronize(default_stream()));
         *out = h;
@@ -1340,10 +1349,8 @@ int ompl_amd_nn_destroy(ompl_amd_nn h)
     return guarded([&] {
         if (!h) return;
         NNIndex &x = h->idx;
-        if (x.pts) OA_HIP(hipFree(x.pts));
-        if (x.xt) OA_HIP(hipFree(x.xt));
-        if (x.removed) OA_HIP(hipFree(x.removed));
-        if (x.xn_max) OA_HIP(hipFree(x.xn_max));
+        OA_HIP(hipDeviceSynchronize()); // searches on any stream may use the arrays
+        for (const DeviceBlock &b : x.blocks) give_block(b);
         if (x.scratch) OA_HIP(hipFree(x.scratch));
         tree_free(x.tree);
         delete h;

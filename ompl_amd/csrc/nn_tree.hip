@@ -786,8 +786,8 @@ void tree_reserve(NNTree &t, int64_t cap, int dim, int tdim)
     const size_t sp = up256((size_t)tiles * dim * kTile * sizeof(float)), sid = up256((size_t)tiles * kTile * 4),
                  pos = up256((size_t)cap * 4), b0 = up256((size_t)nodes * box), b1 = up256((size_t)supers * box),
                  b2 = up256((size_t)ceil_div(supers, kTile) * box);
-    const hipError_t e = hipMalloc((void **)&t.mem, sp + sid + pos + b0 + b1 + b2 + build_bytes(cap));
-    if (e != hipSuccess) fail(OMPL_AMD_ERR_NOMEM, "nearest-neighbour index allocation failed (%lld points)", (long long)cap);
+    t.block = take_block(sp + sid + pos + b0 + b1 + b2 + build_bytes(cap));
+    t.mem = (char *)t.block.p;
     char *at = t.mem;
     auto take = [&](size_t b) {
         char *r = at;
@@ -806,7 +806,7 @@ void tree_reserve(NNTree &t, int64_t cap, int dim, int tdim)
 
 void tree_free(NNTree &t)
 {
-    if (t.mem) OA_HIP(hipFree(t.mem));
+    give_block(t.block);
     t = NNTree{};
 }
 

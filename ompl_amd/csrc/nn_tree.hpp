@@ -8,6 +8,8 @@
 #include <cstddef>
 #include <cstdint>
 
+#include "runtime.hpp"
+
 namespace ompl_amd {
 
 constexpr int kTile = 64;   // points per tile, tiles per node, nodes per supernode
@@ -17,7 +19,8 @@ constexpr int kTreeDimMax = 7;
 struct NNTree {
     int64_t m = 0;   // points in the index: ids [0, m); later ids are its tail
     int64_t cap = 0; // points the arrays have room for
-    char *mem = nullptr;
+    DeviceBlock block;
+    char *mem = nullptr; // block's
     float *sp = nullptr;       // [tiles][dim][64] coordinates
     int32_t *sid = nullptr;    // [tiles][64] ids; -1: no point, or a removed one
     int32_t *pos = nullptr;    // [cap] place of an id in sid
@@ -71,7 +74,7 @@ struct TreeRadiusArgs {
 bool tree_supported(int metric, int dim);
 // Allocates the arrays for `cap` points (the old ones are dropped: m = 0).
 void tree_reserve(NNTree &t, int64_t cap, int dim, int tdim);
-void tree_free(NNTree &t);
+void tree_free(NNTree &t); // nothing on the device uses the arrays any more
 // Indexes points [0, n) of pts ([n][dim]); removed ones get no entry.  ext_lo,
 // ext_hi: extents of the first tdim coordinates (device, ordered_bits).
 void tree_build(NNTree &t, const float *pts, const uint8_t *removed, const uint32_t *ext_lo, const uint32_t *ext_hi,

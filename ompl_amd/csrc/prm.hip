@@ -10,7 +10,7 @@
 //   5. every candidate motion checked (DiscreteMotionValidator semantics,
 //      direction: lower milestone index -> higher)
 //   6. connected components of the valid edges (union-find: root hooking by
-//      atomicCAS + pointer jumping)
+//      atomicCAS with path halving, one launch)
 //
 // The reference connects each new milestone to its k nearest *existing*
 // milestones as they are added (incremental); this batch form connects every
@@ -42,27 +42,28 @@ struct PrmRoadmap {
     float *nodes_f32 = nullptr;    // [nv][7]
     int32_t *knn = nullptr;        // [nv][k+1]
     float *knn_d = nullptr;
-    uint64_t *keys = nullptr;      // candidate (u << 32 | v), u < v
+    uint64_t *keys = nullptr;      // candidate edges, packed (edge_keys_kernel)
     int32_t *eu = nullptr, *ev = nullptr;
     uint8_t *evalid = nullptr;
     int32_t *label = nullptr;      // component root per milestone
     int64_t *csr_off = nullptr;    // [nv + 1] symmetric adjacency of the valid edges
     int32_t *csr_adj = nullptr;    // [2 * valid_edges], ascending per row
     ompl_amd_prm_stats stats{};
-    std::vector<void *> allocs;
+    std::vector<DeviceBlock> allocs;
+    hipStream_t stream = nullptr; // the build's
 
     template <class T>
     T *alloc(size_t count)
     {
-        void *p = nullptr;
-        hipError_t e = hipMalloc(&p, (count ? count : 1) * sizeof(T));
-        if (e != hipSuccess) fail(OMPL_AMD_ERR_NOMEM, "roadmap allocation (%zu bytes) failed", count * sizeof(T));
-        allocs.push_back(p);
-        return (T *)p;
+        allocs.push_back(take_block((count ? count : 1) * sizeof(T)));
+        return (T *)allocs.back().p;
     }
+    // the blocks go back to the library's store (about 35 hipMalloc and hipFree
+    // calls of a roadmap took 6 ms): nothing may still use them
     ~PrmRoadmap()
     {
-        for (void *p : allocs) (void)hipFree(p);
+        if (!allocs.empty()) (void)hipStreamSynchronize(stream);
+        for (const DeviceBlock &b : allocs) give_block(b);
     }
 };
 
@@ -82,7 +83,9 @@ __global__ void gather_nodes_kernel(const int32_t *__restrict__ milestone, int64
 }
 
 // Candidate keys: the first k neighbours of milestone i other than i itself.
-__global__ void edge_keys_kernel(const int32_t *__restrict__ knn, int64_t nv, int kk, int k,
+// (u << bits | v, u < v; bits: of a milestone number.  Packed keys sort in 5
+// radix passes at 135,000 milestones, u << 32 | v in 8.)
+__global__ void edge_keys_kernel(const int32_t *__restrict__ knn, int64_t nv, int kk, int k, int bits,
                                  uint64_t *__restrict__ keys)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -92,20 +95,20 @@ __global__ void edge_keys_kernel(const int32_t *__restrict__ knn, int64_t nv, in
         const int nb = knn[i * kk + j];
         if (taken < k && nb >= 0 && nb != (int)i) {
             const uint64_t u = (uint64_t)min((int64_t)nb, i), v = (uint64_t)max((int64_t)nb, i);
-            keys[i * k + taken] = (u << 32) | v;
+            keys[i * k + taken] = (u << bits) | v;
             ++taken;
         }
     }
     for (int t = taken; t < k; ++t) keys[i * k + t] = ~(uint64_t)0;
 }
 
-__global__ void edge_endpoints_kernel(const uint64_t *__restrict__ keys, int64_t ne, const double *__restrict__ nodes,
+__global__ void edge_endpoints_kernel(const uint64_t *__restrict__ keys, int64_t ne, int bits, const double *__restrict__ nodes,
                                       int32_t *__restrict__ eu, int32_t *__restrict__ ev, double *__restrict__ a_soa,
                                       double *__restrict__ b_soa)
 {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= ne) return;
-    const int32_t u = (int32_t)(keys[e] >> 32), v = (int32_t)(keys[e] & 0xffffffffu);
+    const int32_t u = (int32_t)(keys[e] >> bits), v = (int32_t)(keys[e] & (((uint64_t)1 << bits) - 1));
     eu[e] = u;
     ev[e] = v;
 #pragma unroll
@@ -121,55 +124,95 @@ __global__ void iota_kernel(int32_t *__restrict__ p, int64_t n)
     if (i < n) p[i] = (int32_t)i;
 }
 
-__device__ __forceinline__ int32_t find_root(const int32_t *parent, int32_t x)
+// Through the caches: a stale pointer is an older ancestor, which is as good
+// (agent-scope reads, past the XCD's L2, made this 2.5 ms of a roadmap of
+// 135,000 milestones).  Only atomicCAS, at the device's scope, decides who is a
+// root.
+__device__ __forceinline__ int32_t parent_of(const int32_t *parent, int32_t x)
 {
-    int32_t p = __hip_atomic_load(&parent[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __hip_atomic_load(&parent[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Root of x, halving the path on the way: a node's pointer moves to its
+// grandparent, which stays an ancestor whatever other threads do (pointers only
+// ever go down, and only a root is ever hooked).
+__device__ __forceinline__ int32_t find_root(int32_t *parent, int32_t x)
+{
+    int32_t p = parent_of(parent, x);
     while (p != x) {
+        const int32_t g = parent_of(parent, p);
+        if (g != p) __hip_atomic_store(&parent[x], g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         x = p;
-        p = __hip_atomic_load(&parent[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        p = g;
     }
     return x;
 }
 
-// Hooks the higher root under the lower one for every valid edge whose ends
-// are in different trees; sets *changed when any hook succeeded.
-__global__ void hook_kernel(const int32_t *__restrict__ eu, const int32_t *__restrict__ ev,
-                            const uint8_t *__restrict__ evalid, int64_t ne, int32_t *parent, int32_t *changed)
+// Every milestone starts under its lowest neighbour below it (edges have u < v):
+// most of the forest in one step, before any path is followed.
+__global__ void lowest_neighbour_kernel(const int32_t *__restrict__ eu, const int32_t *__restrict__ ev,
+                                        const uint8_t *__restrict__ evalid, int64_t ne, int32_t *parent)
 {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < ne && evalid[e]) atomicMin(&parent[ev[e]], eu[e]);
+}
+
+// Joins the ends of every `stride`-th valid edge: the higher root goes under the
+// lower one.  A thread whose root was hooked meanwhile goes on from where that
+// root went, so the launch over all edges joins everything, and the root of a
+// component is its lowest milestone.  The launches over a few edges before it
+// (each followed by jump_kernel) leave it almost none to join: with all edges at
+// once, thousands of threads try the same roots, one atomic after the other
+// (589,000 edges of 135,000 milestones: 1.9 ms; rounds of single attempts
+// without path halving: 3 to 4 ms).
+__global__ void hook_kernel(const int32_t *__restrict__ eu, const int32_t *__restrict__ ev,
+                            const uint8_t *__restrict__ evalid, int64_t ne, int64_t stride, int32_t *parent)
+{
+    const int64_t e = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * stride;
     if (e >= ne || !evalid[e]) return;
-    const int32_t ru = find_root(parent, eu[e]), rv = find_root(parent, ev[e]);
-    if (ru == rv) return;
-    const int32_t hi = max(ru, rv), lo = min(ru, rv);
-    if (atomicCAS(&parent[hi], hi, lo) == hi) *changed = 1;
+    int32_t u = find_root(parent, eu[e]), v = find_root(parent, ev[e]);
+    // every failed attempt lowers the higher of the two, so this ends
+    while (u != v) {
+        const int32_t hi = max(u, v), lo = min(u, v);
+        const int32_t was = atomicCAS(&parent[hi], hi, lo);
+        if (was == hi) break;
+        u = find_root(parent, was);
+        v = lo;
+    }
 }
 
 __global__ void jump_kernel(int32_t *parent, int64_t nv)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nv) return;
-    parent[i] = find_root(parent, (int32_t)i);
+    // no halving here: a late store would put a grandparent over a written root
+    int32_t x = (int32_t)i, p = parent_of(parent, x);
+    while (p != x) {
+        x = p;
+        p = parent_of(parent, x);
+    }
+    __hip_atomic_store(&parent[i], x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Both directions of every valid edge as (row << 32 | col) keys, at the
+// Both directions of every valid edge as (row << bits | col) keys, at the
 // positions given by the exclusive scan of evalid.
 __global__ void csr_keys_kernel(const int32_t *__restrict__ eu, const int32_t *__restrict__ ev,
                                 const uint8_t *__restrict__ evalid, const int32_t *__restrict__ pos, int64_t ne,
-                                uint64_t *__restrict__ keys, int32_t *__restrict__ degree)
+                                int bits, uint64_t *__restrict__ keys, int32_t *__restrict__ degree)
 {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= ne || !evalid[e]) return;
     const uint64_t u = (uint32_t)eu[e], v = (uint32_t)ev[e];
-    keys[2 * (int64_t)pos[e]] = (u << 32) | v;
-    keys[2 * (int64_t)pos[e] + 1] = (v << 32) | u;
+    keys[2 * (int64_t)pos[e]] = (u << bits) | v;
+    keys[2 * (int64_t)pos[e] + 1] = (v << bits) | u;
     atomicAdd(&degree[u], 1);
     atomicAdd(&degree[v], 1);
 }
 
-__global__ void csr_cols_kernel(const uint64_t *__restrict__ keys, int64_t n, int32_t *__restrict__ adj)
+__global__ void csr_cols_kernel(const uint64_t *__restrict__ keys, int64_t n, int bits, int32_t *__restrict__ adj)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) adj[i] = (int32_t)(keys[i] & 0xffffffffu);
+    if (i < n) adj[i] = (int32_t)(keys[i] & (((uint64_t)1 << bits) - 1));
 }
 
 __global__ void widen_kernel(const int32_t *__restrict__ in, int64_t n, int64_t *__restrict__ out)
@@ -211,6 +254,7 @@ void build(PrmRoadmap &R, ompl_amd_env env, uint32_t seed, int n_streams, int64_
     auto check = [](int rc) {
         if (rc != OMPL_AMD_OK) fail(rc, "%s", last_error());
     };
+    R.stream = s;
     // 1. samples
     auto t0 = Clock::now();
     const int64_t per = (n_samples + n_streams - 1) / n_streams;
@@ -302,15 +346,17 @@ void build(PrmRoadmap &R, ompl_amd_env env, uint32_t seed, int n_streams, int64_
     // 4. candidate edges: sort + unique of (min, max) keys
     t0 = Clock::now();
     const int64_t nk = nv * k;
+    int bits = 1;
+    while (((int64_t)1 << bits) < nv) ++bits;
     uint64_t *keys = R.alloc<uint64_t>((size_t)nk);
     uint64_t *sorted = R.alloc<uint64_t>((size_t)nk);
     R.keys = R.alloc<uint64_t>((size_t)nk);
-    hipLaunchKernelGGL(edge_keys_kernel, dim3(blocks_for(nv)), dim3(256), 0, s, R.knn, nv, kk, k, keys);
+    hipLaunchKernelGGL(edge_keys_kernel, dim3(blocks_for(nv)), dim3(256), 0, s, R.knn, nv, kk, k, bits, keys);
     size_t sort_bytes = 0, uniq_bytes = 0;
-    OA_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, sort_bytes, keys, sorted, (int)nk, 0, 64, s));
+    OA_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, sort_bytes, keys, sorted, (int)nk, 0, 2 * bits, s));
     OA_HIP(hipcub::DeviceSelect::Unique(nullptr, uniq_bytes, sorted, R.keys, d_nv, (int)nk, s));
     void *tmp2 = R.alloc<char>(std::max(sort_bytes, uniq_bytes));
-    OA_HIP(hipcub::DeviceRadixSort::SortKeys(tmp2, sort_bytes, keys, sorted, (int)nk, 0, 64, s));
+    OA_HIP(hipcub::DeviceRadixSort::SortKeys(tmp2, sort_bytes, keys, sorted, (int)nk, 0, 2 * bits, s));
     OA_HIP(hipcub::DeviceSelect::Unique(tmp2, uniq_bytes, sorted, R.keys, d_nv, (int)nk, s));
     int64_t nu = 0;
     OA_HIP(hipMemcpyAsync(&nu, d_nv, sizeof(int64_t), hipMemcpyDeviceToHost, s));
@@ -327,7 +373,7 @@ void build(PrmRoadmap &R, ompl_amd_env env, uint32_t seed, int n_streams, int64_
     R.evalid = R.alloc<uint8_t>((size_t)nu);
     double *a_soa = R.alloc<double>((size_t)nu * kDim), *b_soa = R.alloc<double>((size_t)nu * kDim);
     if (nu > 0)
-        hipLaunchKernelGGL(edge_endpoints_kernel, dim3(blocks_for(nu)), dim3(256), 0, s, R.keys, nu, R.nodes, R.eu,
+        hipLaunchKernelGGL(edge_endpoints_kernel, dim3(blocks_for(nu)), dim3(256), 0, s, R.keys, nu, bits, R.nodes, R.eu,
                            R.ev, a_soa, b_soa);
     OA_HIP(hipStreamSynchronize(s));
     R.stats.ms_candidates = ms(t0);
@@ -336,7 +382,7 @@ void build(PrmRoadmap &R, ompl_amd_env env, uint32_t seed, int n_streams, int64_
         const int64_t nt = std::min<int64_t>(nu, 32768);
         double *ta = R.alloc<double>((size_t)nt * kDim), *tb = R.alloc<double>((size_t)nt * kDim);
         int32_t *teu = R.alloc<int32_t>((size_t)nt), *tev = R.alloc<int32_t>((size_t)nt);
-        hipLaunchKernelGGL(edge_endpoints_kernel, dim3(blocks_for(nt)), dim3(256), 0, s, R.keys, nt, R.nodes, teu,
+        hipLaunchKernelGGL(edge_endpoints_kernel, dim3(blocks_for(nt)), dim3(256), 0, s, R.keys, nt, bits, R.nodes, teu,
                            tev, ta, tb);
         OA_HIP(hipStreamSynchronize(s));
         // the winner becomes the environment's own launch shapes; the
@@ -355,20 +401,15 @@ void build(PrmRoadmap &R, ompl_amd_env env, uint32_t seed, int n_streams, int64_
     // 6. components
     t0 = Clock::now();
     hipLaunchKernelGGL(iota_kernel, dim3(blocks_for(nv)), dim3(256), 0, s, R.label, nv);
-    // Every round with a successful hook removes at least one root, so at
-    // most nv - 1 rounds change anything; the round after the last change
-    // sees every valid edge inside one tree and ends the loop.
-    int32_t *changed = R.alloc<int32_t>(1);
-    for (int64_t round = 0; nu > 0; ++round) {
-        if (round > nv) fail(OMPL_AMD_ERR_INTERNAL, "union-find did not converge");
-        OA_HIP(hipMemsetAsync(changed, 0, sizeof(int32_t), s));
-        hipLaunchKernelGGL(hook_kernel, dim3(blocks_for(nu)), dim3(256), 0, s, R.eu, R.ev, R.evalid, nu, R.label,
-                           changed);
+    if (nu > 0) {
+        hipLaunchKernelGGL(lowest_neighbour_kernel, dim3(blocks_for(nu)), dim3(256), 0, s, R.eu, R.ev, R.evalid, nu,
+                           R.label);
         hipLaunchKernelGGL(jump_kernel, dim3(blocks_for(nv)), dim3(256), 0, s, R.label, nv);
-        int32_t h = 0;
-        OA_HIP(hipMemcpyAsync(&h, changed, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        OA_HIP(hipStreamSynchronize(s));
-        if (!h) break;
+        for (const int64_t stride : {(int64_t)32, (int64_t)6, (int64_t)1}) {
+            hipLaunchKernelGGL(hook_kernel, dim3(blocks_for((nu + stride - 1) / stride)), dim3(256), 0, s, R.eu, R.ev,
+                               R.evalid, nu, stride, R.label);
+            hipLaunchKernelGGL(jump_kernel, dim3(blocks_for(nv)), dim3(256), 0, s, R.label, nv);
+        }
     }
     unsigned long long *cnt = R.alloc<unsigned long long>(1);
     OA_HIP(hipMemsetAsync(cnt, 0, sizeof(unsigned long long), s));
@@ -401,12 +442,12 @@ void build(PrmRoadmap &R, ompl_amd_env env, uint32_t seed, int n_streams, int64_
     int32_t *off32 = R.alloc<int32_t>((size_t)nv + 1);
     if (nd) {
         hipLaunchKernelGGL(csr_keys_kernel, dim3(blocks_for(nu)), dim3(256), 0, s, R.eu, R.ev, R.evalid, pos, nu,
-                           dkeys, degree);
+                           bits, dkeys, degree);
         size_t b1 = 0;
-        OA_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, b1, dkeys, dsorted, (int)nd, 0, 64, s));
+        OA_HIP(hipcub::DeviceRadixSort::SortKeys(nullptr, b1, dkeys, dsorted, (int)nd, 0, 2 * bits, s));
         void *tmp4 = R.alloc<char>(b1);
-        OA_HIP(hipcub::DeviceRadixSort::SortKeys(tmp4, b1, dkeys, dsorted, (int)nd, 0, 64, s));
-        hipLaunchKernelGGL(csr_cols_kernel, dim3(blocks_for(nd)), dim3(256), 0, s, dsorted, nd, R.csr_adj);
+        OA_HIP(hipcub::DeviceRadixSort::SortKeys(tmp4, b1, dkeys, dsorted, (int)nd, 0, 2 * bits, s));
+        hipLaunchKernelGGL(csr_cols_kernel, dim3(blocks_for(nd)), dim3(256), 0, s, dsorted, nd, bits, R.csr_adj);
     }
     size_t b2 = 0;
     OA_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, b2, degree, off32, (int)(nv + 1), s));

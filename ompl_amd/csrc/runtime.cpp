@@ -2,6 +2,7 @@
 // per-stream workspaces and per-thread resources of the blocking entry points.
 #include "runtime.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -135,6 +136,63 @@ GridScratch grid_scratch(Workspace &w)
                   sets + 4 * (1 - w.grid_parity)};
     w.grid_parity ^= 1;
     return g;
+}
+
+namespace {
+std::mutex g_blocks_mutex;
+std::multimap<size_t, void *> g_blocks;
+size_t g_blocks_bytes = 0;
+} // namespace
+
+DeviceBlock take_block(size_t bytes)
+{
+    // sizes in steps of an eighth of their power of two, so that calls of about
+    // the same size find each other's blocks
+    size_t step = 256;
+    while (step * 16 <= bytes) step *= 2;
+    const size_t want = (std::max<size_t>(bytes, 1) + step - 1) / step * step;
+    {
+        std::lock_guard<std::mutex> lk(g_blocks_mutex);
+        const auto it = g_blocks.lower_bound(want);
+        if (it != g_blocks.end() && it->first <= want + want / 4) {
+            const DeviceBlock b{it->second, it->first};
+            g_blocks_bytes -= it->first;
+            g_blocks.erase(it);
+            return b;
+        }
+    }
+    DeviceBlock b{nullptr, want};
+    hipError_t e = hipMalloc(&b.p, want);
+    if (e == hipErrorOutOfMemory) {
+        std::multimap<size_t, void *> kept;
+        {
+            std::lock_guard<std::mutex> lk(g_blocks_mutex);
+            kept.swap(g_blocks);
+            g_blocks_bytes = 0;
+        }
+        for (const auto &k : kept) (void)hipFree(k.second);
+        (void)hipGetLastError();
+        e = hipMalloc(&b.p, want);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        fail(OMPL_AMD_ERR_NOMEM, "device allocation of %zu bytes failed: %s", want, hipGetErrorString(e));
+    }
+    return b;
+}
+
+void give_block(const DeviceBlock &b)
+{
+    if (!b.p) return;
+    {
+        std::lock_guard<std::mutex> lk(g_blocks_mutex);
+        if (g_blocks_bytes + b.bytes <= kKeptBlocksBytes) {
+            g_blocks.emplace(b.bytes, b.p);
+            g_blocks_bytes += b.bytes;
+            return;
+        }
+    }
+    (void)hipFree(b.p);
 }
 
 Workspace &workspace(hipStream_t s, size_t list_entries, std::unique_lock<std::mutex> &lock)

@@ -19,6 +19,19 @@ void init_device(int dev);
 // (once per device, with that device current).
 void init_noalloc_scratch(int dev);
 
+// Device memory of objects that come and go (roadmaps, nearest-neighbour
+// structures): a block given back is kept for the next taker, up to
+// kKeptBlocksBytes in all, and kept blocks go back to the device when an
+// allocation fails.  The giver sees to it that nothing on the device still
+// uses the block.  Safe from any thread.
+struct DeviceBlock {
+    void *p = nullptr;
+    size_t bytes = 0;
+};
+constexpr size_t kKeptBlocksBytes = (size_t)768 << 20;
+DeviceBlock take_block(size_t bytes);
+void give_block(const DeviceBlock &b);
+
 // Per-stream scratch of the batched motion path: survivor list + counters.
 struct Workspace {
     int32_t *list = nullptr;
