@@ -416,10 +416,9 @@ typedef struct {
                                 creation); a request is admitted when its region fits */
     int max_active;          /* concurrent requests */
     int max_nodes;           /* largest nodes per tree of a request */
-    int check_obstacle_parts; /* lanes splitting the environment's obstacle list in a motion
-                                 check (link layout): 1, 2, 4 or 9 (8, 4, 2 or 1 positions
-                                 per wave); 0 = chosen per motion from its length */
-    int check_lanes_per_state; /* 0 or 7 (the link layout with bounding-sphere culling) */
+    int check_obstacle_parts; /* 0, 1, 2, 4 or 9; without effect (checks look their obstacles
+                                 up in the environment's cell grid) */
+    int check_lanes_per_state; /* 0 or 7; without effect */
     int slice_us;            /* device time per slice before the host admits and retires
                                 (at least one growTree step per request); 0 = 200 */
     int block_threads;       /* threads of each request's workgroup: 512 or 1024 (0 = 512) */

@@ -18,13 +18,20 @@
 // does not depend on the slices it ran in or the requests it shared them
 // with.
 //
-// Inside a block: the nearest neighbour is a thread-strided FP64 scan of the
-// tree (first strict minimum), reduced by (distance, index); a motion check
-// takes the block's waves over its positions in rounds (the link layout
-// with bounding-sphere culling, the environment staged in LDS once per
-// slice), with a block-wide OR after each round as the early exit; the
-// sampler's words are tempered from the LDS state and the state is twisted
-// by the whole block.
+// Inside a block: the nearest neighbour is an FP64 scan of the tree (first
+// strict minimum), its first nodes in LDS, reduced by (distance, index); states
+// are checked over the environment's cell grid (grid_device.hpp), eight lanes
+// each where few are wanted at once and one lane each for the rest of a long
+// motion; the sampler's draws are made a generator block at a time.
+//
+// A request is one chain of steps, so it is bound by latency: what counts is
+// how many steps share one pass of it.  Most sampling steps are trapped, and a
+// trapped step changes nothing but the draws, so up to 32 of them run at once
+// (16 lanes each), the first valid one is committed, and the pass costs about
+// 9 us.  64 requests over eight scenes of up to 128 obstacles, 48,900 steps,
+// the longest request 2,128 of them: 4.1 ms (11.3 before: eight at
+// a time, each tested against every obstacle, and copies of commands, results, end states and
+// paths around every slice, which the kernel now reads and writes in pinned memory).
 //
 // Plain counterpart: ompl_amd_plan_plain runs the same RRT-Connect on the host
 // with host nearest neighbours and one GPU launch + synchronisation per
@@ -44,6 +51,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "grid_device.hpp"
 #include "mt_device.hpp"
 #include "runtime.hpp"
 #include "walk_device.hpp"
@@ -54,10 +62,9 @@ enum GrowStatus { kTrapped = 0, kAdvanced = 1, kReached = 2 };
 
 constexpr double kPi = 3.141592653589793238462643383279502884;
 constexpr double kEqualEps = 2.220446049250313080847e-16 * 2.0; // StateSpace::equalStates (RealVector)
-// Obstacle staging padding shared by the motion check's four partitionings
-// (whole passes of 8, 16, 32 and 144 obstacles): their least common multiple.
+// Largest environment a request may name, as the bytes of its obstacles in
+// lists padded to kPlanPad (60 KiB: 2,880 spheres or 1,728 boxes).
 constexpr int kPlanPad = 288;
-// Dynamic LDS of one planner block (the staged environment).
 constexpr size_t kPlanMaxEnvBytes = 60 * 1024;
 // Start / goal states a request may list (each).
 constexpr int kMaxEnds = OMPL_AMD_MAX_ENDPOINTS;
@@ -129,11 +136,10 @@ static size_t footprint(int max_nodes)
     return region_ptrs(nullptr, max_nodes).bytes;
 }
 
-// Per active request and slice (device copy of a host array).
+// Per active request and slice (a host array that the kernel reads once).
 struct PlanCmd {
-    const float4 *obs; // environment, staging order (spheres, then boxes as lo/hi pairs)
+    GridView grid; // the environment
     char *region;
-    int32_t ns, nb;
     int32_t cap;       // nodes per tree
     int32_t max_iters;
     double maxd;       // maxDistance_
@@ -141,9 +147,10 @@ struct PlanCmd {
     uint32_t factor;
     uint32_t seed;
     int32_t init;      // 1: first slice (seed the sampler, plant the roots)
-    int32_t ops;       // obstacle partitions of the motion check (0: by motion length)
     int32_t n_starts, n_goals; // rows of the region's start and goal states
     int32_t inter;     // addIntermediateStates
+    const double *ends; // first slice: the start and goal rows, as in the region (host memory)
+    double *path;       // where a solution of at most SliceArgs::path_rows rows goes (host memory), else the region
 };
 
 // Per active request, written at the end of each slice.  t_*: device
@@ -155,9 +162,15 @@ struct PlanOut {
     int64_t t_sample, t_nearest, t_check, t_step;
 };
 
+// Longest solution written to pinned memory by the slice that finds it (a longer
+// one is copied from its region), within kPathBytes for all active requests.
+constexpr int kPathRows = 128;
+constexpr size_t kPathBytes = (size_t)16 << 20;
+
 struct SliceArgs {
-    const PlanCmd *cmds;
+    const PlanCmd *cmds; // host memory, as is out: read and written once, no copies around a slice
     PlanOut *out;
+    int path_rows;
     int64_t budget; // wall-clock ticks per slice (at least one step is always made)
 };
 
@@ -166,152 +179,220 @@ static size_t env_stage_bytes(int ns, int nb)
     return (size_t)(pad_to(ns, kPlanPad) + 2 * pad_to(nb, kPlanPad)) * sizeof(float4) + (size_t)ns * sizeof(float);
 }
 
-// Obstacle partitions for a motion of npos positions: the widest split whose
-// round (NW waves x states per wave) still covers the motion, else one.
-template <int NW>
-__device__ __forceinline__ int auto_ops(int npos)
-{
-    return npos <= NW * 1 ? 9 : npos <= NW * 2 ? 4 : npos <= NW * 4 ? 2 : 1;
-}
+// Candidate nearest node: its distance and index; the lower index wins a tie.
+struct Near {
+    double d = INFINITY;
+    int i = INT_MAX;
+    __device__ __forceinline__ void take(double od, int oi)
+    {
+        if (od < d || (od == d && oi < i)) {
+            d = od;
+            i = oi;
+        }
+    }
+    template <int CTRL>
+    __device__ __forceinline__ void dpp()
+    {
+        const long long u = __double_as_longlong(d);
+        const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)u, CTRL, 0xf, 0xf, true);
+        const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), CTRL, 0xf, 0xf, true);
+        const int oi = __builtin_amdgcn_update_dpp(0, i, CTRL, 0xf, 0xf, true);
+        take(__longlong_as_double((long long)(((unsigned long long)hi << 32) | lo)), oi);
+    }
+    // The best of each group of `lanes` (16 or 64) in all its lanes.
+    __device__ __forceinline__ void share(int lanes)
+    {
+        dpp<0x128>(); // row_ror 8, 4, 2, 1: rows of 16 lanes
+        dpp<0x124>();
+        dpp<0x122>();
+        dpp<0x121>();
+        if (lanes == 64) {
+            take(__shfl_xor(d, 16), __shfl_xor(i, 16));
+            take(__shfl_xor(d, 32), __shfl_xor(i, 32));
+        }
+    }
+};
 
-// Nearest node of tree T (n nodes, dof-major with stride cap) to tgt: first
-// strict minimum of distance(node, tgt) (NearestNeighborsLinear::nearest
-// order).  Every thread returns the same index.
-template <int NT>
-__device__ __forceinline__ int block_nearest(const double *__restrict__ T, int cap, int n, const double tgt[kDof],
-                                             double *s_wd, int *s_wi)
+constexpr int kKeptNodes = 256; // of each tree, in LDS
+
+// A tree: its nodes (dof-major with stride cap), the first `kept` of them also
+// in LDS (stride kept).
+struct Tree {
+    double *T, *lds;
+    int cap;
+    static constexpr int kept = kKeptNodes;
+    __device__ __forceinline__ double at(int k, int i) const
+    {
+        return i < kept ? lds[k * kept + i] : T[(int64_t)k * cap + i];
+    }
+    __device__ __forceinline__ void set(int k, int i, double v) const
+    {
+        T[(int64_t)k * cap + i] = v;
+        if (i < kept) lds[k * kept + i] = v;
+    }
+};
+
+// Nearest of n nodes to tgt among nodes first, first + stride, ..: first strict
+// minimum of distance(node, tgt) (NearestNeighborsLinear::nearest order).
+__device__ __forceinline__ Near scan_nearest(const Tree &t, int n, const double tgt[kDof], int first, int stride)
 {
-    double best = INFINITY;
-    int bi = INT_MAX;
-    for (int i = threadIdx.x; i < n; i += NT) {
+    Near best;
+    double best2 = INFINITY; // a squared distance no smaller has no smaller root
+    auto distance2 = [&](int i, const double *T, int64_t step) {
         double dist = 0.0;
 #pragma unroll
         for (int k = 0; k < kDof; ++k) {
-            const double diff = T[(int64_t)k * cap + i] - tgt[k];
+            const double diff = T[k * step + i] - tgt[k];
             dist += diff * diff;
         }
-        const double d = __builtin_sqrt(dist);
-        if (d < best) { // a thread's indices increase: strict < keeps its lowest
-            best = d;
-            bi = i;
+        return dist;
+    };
+    auto take = [&](int i, double dist) {
+        if (dist < best2) {
+            const double d = __builtin_sqrt(dist);
+            best2 = dist;
+            if (d < best.d) { // indices increase: strict < keeps the lowest
+                best.d = d;
+                best.i = i;
+            }
         }
-    }
+    };
+    int i = first;
+    for (; i < min(n, t.kept); i += stride) take(i, distance2(i, t.lds, t.kept));
+    constexpr int kAtOnce = 4; // nodes whose reads are in flight together
+    for (; i < n; i += kAtOnce * stride) {
+        double d2[kAtOnce];
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const double od = __shfl_xor(best, off);
-        const int oi = __shfl_xor(bi, off);
-        if (od < best || (od == best && oi < bi)) {
-            best = od;
-            bi = oi;
-        }
+        for (int u = 0; u < kAtOnce; ++u) d2[u] = distance2(min(i + u * stride, n - 1), t.T, t.cap);
+#pragma unroll
+        for (int u = 0; u < kAtOnce; ++u)
+            if (i + u * stride < n) take(i + u * stride, d2[u]);
     }
+    return best;
+}
+
+// The same over the whole tree by the whole block; every thread returns it.
+template <int NT>
+__device__ __forceinline__ Near block_nearest(const Tree &t, int n, const double tgt[kDof], double *s_wd, int *s_wi)
+{
+    Near best = scan_nearest(t, n, tgt, threadIdx.x, NT);
+    best.share(64);
     if (lane_id() == 0) {
-        s_wd[threadIdx.x >> 6] = best;
-        s_wi[threadIdx.x >> 6] = bi;
+        s_wd[threadIdx.x >> 6] = best.d;
+        s_wi[threadIdx.x >> 6] = best.i;
     }
     __syncthreads();
-    best = s_wd[0];
-    bi = s_wi[0];
+    best.d = s_wd[0];
+    best.i = s_wi[0];
 #pragma unroll
-    for (int w = 1; w < NT / 64; ++w)
-        if (s_wd[w] < best || (s_wd[w] == best && s_wi[w] < bi)) {
-            best = s_wd[w];
-            bi = s_wi[w];
-        }
-    return bi;
+    for (int w = 1; w < NT / 64; ++w) best.take(s_wd[w], s_wi[w]);
+    return best;
 }
 
-// Positions [first, npos) of the motion by the whole block, in rounds of NT/64 waves x G
-// states: with `extra`, position 0 is isValid(dst) and position p >= 1 the
-// DiscreteMotionValidator position p-1 of (a, b) (0 = b, then the bisection
-// order); without, position p is the validator's position p.  Returns false
-// at the first round holding an invalid position.  Validity of the whole
-// motion does not depend on the order positions are visited in.  a, b and
-// dst are in LDS (read per round; no registers held across the rounds);
-// `stop` is an LDS flag, zero on entry, that lets the other waves of a round
-// leave once one has found an invalid position.
-template <int NT, int OPS>
-__device__ __forceinline__ bool block_check(const double *a, const double *b, const double *dst, int nd, int first,
-                                            int npos, bool extra, const float4 *env, int ns, int nb, int *stop)
-{
-    using Shape = GroupShape<7, OPS>;
-    constexpr int G = Shape::STATES;
-    const int wave = threadIdx.x >> 6;
-    const Shape sh(lane_id());
-    for (int base = first; base < npos; base += NT / 64 * G) {
-        const int p = base + wave * G + sh.group;
-        const bool live = p < npos;
-        float q[kDof];
-        if (extra && p == 0) {
-#pragma unroll
-            for (int k = 0; k < kDof; ++k) q[k] = (float)dst[k];
-        } else {
-            const int mp = extra ? p - 1 : p;
-            walk_state(a, b, nd, live ? mp : 0, q);
-        }
-        LaneSpheres<7> S;
-        arm_fk<7, Shape::GS>(q, sh.slot, S);
-        const bool hit = collide_links<OPS, Exit::kAnyGroup, true, kPlanPad>(S, env, ns, nb, live, sh.part, stop);
-        if (__syncthreads_or(hit && live)) return false;
-    }
-    return true;
-}
-
-// Nearest node of tree T to tgt by one wave (the speculative sampling steps):
-// the same first strict minimum as block_nearest; every lane returns it.
-__device__ __forceinline__ int wave_nearest(const double *__restrict__ T, int cap, int n, const double tgt[kDof])
-{
-    double best = INFINITY;
-    int bi = INT_MAX;
-    for (int i = lane_id(); i < n; i += 64) {
+// growTree's new state (RRTConnect.cpp:116-135): the nearest node nst (made
+// node 0 where no distance is finite), the target or, farther than maxd, the
+// state maxd from nst towards it.
+struct Steer {
+    double nst[kDof], x[kDof];
+    int nm;
+    bool reach, moved; // not moved: no progress, TRAPPED without a check
+    __device__ __forceinline__ void run(const Tree &t, int n, const Near &best, const double tgt[kDof], double maxd)
+    {
+        nm = best.i < n ? best.i : 0;
+        double dd = best.d;
         double dist = 0.0;
 #pragma unroll
         for (int k = 0; k < kDof; ++k) {
-            const double diff = T[(int64_t)k * cap + i] - tgt[k];
-            dist += diff * diff;
+            nst[k] = t.at(k, nm);
+            x[k] = tgt[k];
         }
-        const double d = __builtin_sqrt(dist);
-        if (d < best) {
-            best = d;
-            bi = i;
-        }
-    }
+        if (best.i >= n) {
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const double od = __shfl_xor(best, off);
-        const int oi = __shfl_xor(bi, off);
-        if (od < best || (od == best && oi < bi)) {
-            best = od;
-            bi = oi;
+            for (int k = 0; k < kDof; ++k) {
+                const double diff = nst[k] - tgt[k];
+                dist += diff * diff;
+            }
+            dd = __builtin_sqrt(dist);
+        }
+        reach = moved = true;
+        if (dd > maxd) {
+            const double s = maxd / dd;
+            bool equal = true;
+#pragma unroll
+            for (int k = 0; k < kDof; ++k) {
+                x[k] = nst[k] + (tgt[k] - nst[k]) * s;
+                if (fabs(nst[k] - x[k]) > kEqualEps) equal = false;
+            }
+            moved = !equal;
+            reach = false;
         }
     }
-    return bi;
+};
+
+// A growTree step's motion: npos positions, the DiscreteMotionValidator's of
+// (a, b) (0 = b, then the bisection order), or with `extra`, where b is a tree
+// node, isValid(dst) first and b last.  a, b and dst are in LDS (read per
+// round; no registers held across).  Validity of the whole motion does not
+// depend on the order positions are visited in.
+struct StepMotion {
+    const double *a, *b, *dst;
+    int nd, npos;
+    bool extra;
+    static __device__ __forceinline__ int positions(int nd, bool extra)
+    {
+        return 1 + (nd >= 2 ? nd - 1 : 0) + (extra ? 1 : 0);
+    }
+    // the state of position p if it is one of the motion's ends, else null
+    __device__ __forceinline__ const double *end(int p) const
+    {
+        return !extra ? (p == 0 ? b : nullptr) : p == 0 ? dst : p == npos - 1 ? b : nullptr;
+    }
+    __device__ __forceinline__ double fraction(int p) const
+    {
+        return (double)bisection_index(p - 1, nd) / (double)nd;
+    }
+    // Eight lanes per position: joint j of position p.
+    __device__ __forceinline__ float joint(int p, int j) const
+    {
+        if (const double *e = end(p)) return (float)e[j];
+        const double t = fraction(p);
+        return (float)(a[j] + (b[j] - a[j]) * t);
+    }
+    // One lane per position.
+    __device__ __forceinline__ void state(int p, float q[kDof]) const
+    {
+        if (const double *e = end(p)) {
+#pragma unroll
+            for (int k = 0; k < kDof; ++k) q[k] = (float)e[k];
+        } else {
+            interpolate_f32<kDof>(a, b, fraction(p), q);
+        }
+    }
+};
+
+// Eight lanes per position: whether the lane finds position p (if there is
+// one) invalid.
+__device__ __forceinline__ bool wave_hit8(const GridView &g, const StepMotion &M, int p, WaveTests &tests)
+{
+    const bool live = p < M.npos;
+    return state_hit8(g, M.joint(live ? p : 0, min(lane_id() & 7, kDof - 1)), live, tests);
 }
 
-// Positions [first, last) of a motion (numbered as in block_check) by one
-// wave; false at the first round holding an invalid position.
-template <int OPS>
-__device__ __forceinline__ bool wave_check(const double *a, const double *b, const double *dst, int nd, int first,
-                                           int last, bool extra, const float4 *env, int ns, int nb)
+// Positions from `first` on of a motion by the whole block, one lane each:
+// false at the first round holding an invalid position.
+template <int NT>
+__device__ __forceinline__ bool block_check(const GridView &g, const StepMotion &M, int first, WaveTests *tests)
 {
-    using Shape = GroupShape<7, OPS>;
-    constexpr int G = Shape::STATES;
-    const Shape sh(lane_id());
-    for (int base = first; base < last; base += G) {
-        const int p = base + sh.group;
-        const bool live = p < last;
-        float q[kDof];
-        if (extra && p == 0) {
-#pragma unroll
-            for (int k = 0; k < kDof; ++k) q[k] = (float)dst[k];
-        } else {
-            const int mp = extra ? p - 1 : p;
-            walk_state(a, b, nd, live ? mp : 0, q);
+    for (int base = first; base < M.npos; base += NT) {
+        const int p = base + (int)threadIdx.x;
+        const bool live = p < M.npos;
+        bool hit = false;
+        if (wave_ballot(live)) {
+            float q[kDof];
+            M.state(live ? p : 0, q);
+            hit = state_hit1(g, q, live, tests[threadIdx.x >> 6]);
         }
-        LaneSpheres<7> S;
-        arm_fk<7, Shape::GS>(q, sh.slot, S);
-        const bool hit = collide_links<OPS, Exit::kAnyGroup, true, kPlanPad>(S, env, ns, nb, live, sh.part);
-        if (wave_ballot(hit && live)) return false;
+        if (__syncthreads_or(hit)) return false;
     }
     return true;
 }
@@ -319,13 +400,10 @@ __device__ __forceinline__ bool wave_check(const double *a, const double *b, con
 // SpaceInformation::satisfiesBounds && isValid of state q (global memory) by
 // the whole block (PlannerInputStates, base/src/Planner.cpp:243-245): within
 // machine epsilon of [-pi, pi] per joint (RealVectorStateSpace.cpp:200-208),
-// then the checker.  q is staged in sx; sa / sb are any LDS states.
-template <int NT>
-__device__ bool endpoint_usable(const double *q, double *sx, const double *sa, const double *sb, const float4 *env,
-                                int ns, int nb, int *stop)
+// then the checker.  q is staged in sx.
+__device__ __forceinline__ bool endpoint_usable(const GridView &g, const double *q, double *sx, WaveTests *tests)
 {
     if (threadIdx.x < kDof) sx[threadIdx.x] = q[threadIdx.x];
-    if (threadIdx.x == 0) *stop = 0;
     __syncthreads();
     const double eps = 2.220446049250313080847e-16;
     bool in = true;
@@ -333,10 +411,12 @@ __device__ bool endpoint_usable(const double *q, double *sx, const double *sa, c
     for (int k = 0; k < kDof; ++k)
         if (sx[k] - eps > kPi || sx[k] + eps < -kPi) in = false;
     if (!in) return false; // block-uniform: every thread read the same state
-    return block_check<NT, 9>(sa, sb, sx, 0, 0, 1, true, env, ns, nb, stop);
+    // every wave checks the one state
+    const StepMotion M{sx, sx, sx, 0, 1, true};
+    return wave_ballot(wave_hit8(g, M, lane_id() >> 3, tests[threadIdx.x >> 6])) == 0;
 }
 
-// Appends a valid growTree step to tree (T, P) after node nm: the new state x,
+// Appends a valid growTree step to tree (t, P) after node nm: the new state x,
 // or with addIntermediateStates (RRTConnect.cpp:148-183) the states of
 // getMotionStates(a, b, validSegmentCount(a, b) = nd, endpoints) --
 // a + (b - a) j / (nd + 1) -- without the tree's own end: from the start tree
@@ -344,18 +424,18 @@ __device__ bool endpoint_usable(const double *q, double *sx, const double *sa, c
 // nearest) states nd .. 0, each the parent of the next.  Returns the index of
 // the last (the new state), or -1 when the tree cannot hold them.
 template <int NT>
-__device__ int append_step(double *T, int32_t *P, int cap, int &n, int nm, const double *a, const double *b,
+__device__ int append_step(const Tree &t, int32_t *P, int &n, int nm, const double *a, const double *b,
                            const double *x, int nd, bool from_start, bool inter)
 {
     const int tid = threadIdx.x;
     if (!inter) {
-        if (n + 1 > cap) return -1;
-        if (tid < kDof) T[(int64_t)tid * cap + n] = x[tid];
+        if (n + 1 > t.cap) return -1;
+        if (tid < kDof) t.set(tid, n, x[tid]);
         if (tid == 0) P[n] = nm;
         return n++;
     }
     const int seg = nd + 1;
-    if (n + seg > cap) return -1;
+    if (n + seg > t.cap) return -1;
     for (int i = tid; i < seg * kDof; i += NT) {
         const int r = i / kDof, k = i - r * kDof; // chain element r (0-based)
         const int j = from_start ? r + 1 : seg - 1 - r;
@@ -363,20 +443,24 @@ __device__ int append_step(double *T, int32_t *P, int cap, int &n, int nm, const
         if (j == 0) v = a[k];
         else if (j == seg) v = b[k];
         else v = a[k] + (b[k] - a[k]) * ((double)j / (double)seg);
-        T[(int64_t)k * cap + n + r] = v;
+        t.set(k, n + r, v);
     }
     for (int r = tid; r < seg; r += NT) P[n + r] = r == 0 ? nm : n + r - 1;
     n += seg;
     return n - 1;
 }
 
-// Outcome of a speculative sampling step's own check.
-enum SpecResult { kSpecTrapped = 0, kSpecValid = 1, kSpecUndecided = 2 };
-// Positions a speculative step checks with its own wave: the new state (or
-// s2) with the obstacle list split nine ways, then the next eight with one
-// state per link group; a motion still valid after them is finished by the
-// whole block if its step is the next one to commit.
-constexpr int kSpecPositions = 9;
+// Lanes of a speculative step, by the larger tree's size; it checks a position
+// (the new state or s2 and what follows) with eight lanes each; those still
+// open after them get a few more from whole waves, and the first that is then
+// open is finished by the whole block.  While the nodes are in LDS a step costs
+// the same in 16 lanes as in 64, and four times as many run at once; of a large
+// tree's scan, the steps behind the first valid one would be wasted work.
+__device__ __forceinline__ int spec_lanes(int nodes)
+{
+    return nodes <= kKeptNodes ? 16 : 64;
+}
+constexpr int kDraws = kMtN / 2; // 0-1 draws of a generator's block
 
 // Runs request blockIdx.x's RRTConnect::solve loop for one slice.  Control
 // flow is block-uniform: every thread holds the loop's variables and updates
@@ -385,28 +469,38 @@ constexpr int kSpecPositions = 9;
 template <int NT>
 __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
 {
-    extern __shared__ float4 s_env[];
+    __shared__ WaveTests s_tests[NT / 64];
+    __shared__ double s_nodes[2][kDof * kKeptNodes];
     __shared__ uint32_t s_mt[kMtN];
     __shared__ double s_rstate[kDof];
     __shared__ double s_wd[NT / 64];
     __shared__ int s_wi[NT / 64];
     __shared__ double s_a[kDof], s_b[kDof], s_x[kDof]; // the step's motion and new state
-    __shared__ double s_u[kMtN / 2]; // the 0-1 draws of the generator's current 624-word block
-    __shared__ int s_stop, s_hit, s_n1, s_len;
-    // speculative sampling steps, one per wave: samples, motions, outcomes
-    __shared__ double s_samp[NT / 64 * kDof], s_ga[NT / 64 * kDof], s_gb[NT / 64 * kDof], s_gx[NT / 64 * kDof];
-    __shared__ int s_res[NT / 64], s_nm[NT / 64], s_reach[NT / 64], s_chk[NT / 64], s_nd[NT / 64],
-        s_npos[NT / 64];
+    // the 0-1 draws of the generator's current 624-word block and, with `ahead`, of the next; s_mt is the last
+    // block made, s_prev then the one before
+    __shared__ double s_u[2 * kDraws];
+    __shared__ uint32_t s_prev[kMtN];
+    __shared__ int s_stop, s_n1, s_len;
+    // speculative sampling steps: samples, motions, outcomes
+    constexpr int kSpec = NT / 16 < 44 ? NT / 16 : 44; // their draws fit in one block
+    static_assert(kSpec < 64 && kSpec * kDof <= NT && kSpec * kDof <= kDraws, "one lane an outcome, one thread a draw");
+    __shared__ double s_samp[kSpec * kDof], s_ga[kSpec * kDof], s_gb[kSpec * kDof], s_gx[kSpec * kDof];
+    __shared__ int s_open[kSpec], s_bad[kSpec], s_nm[kSpec], s_reach[kSpec], s_chk[kSpec], s_nd[kSpec], s_npos[kSpec];
     const int tid = threadIdx.x;
     const int64_t t0 = wall_clock64();
-    const PlanCmd &C = A.cmds[blockIdx.x];
+    const PlanCmd C = A.cmds[blockIdx.x];
+    const GridView &g = C.grid;
     const RegionPtrs R = region_ptrs(C.region, C.cap);
     PlanState *st = R.state;
+    // (selected, not indexed: an indexed local array lives in memory)
+    auto tree = [&](int t) { return Tree{t ? R.tree_s[1] : R.tree_s[0], s_nodes[t], C.cap}; };
+    auto parents = [&](int t) { return t ? R.parent[1] : R.parent[0]; };
 
     int mti, status, iteration, n0, n1, start_tree, tgi_start, grow_tree, phase, added, xmotion, path_len;
     int sampled_goals;
     int64_t steps, checks;
     if (C.init) {
+        if (tid < 2 * kMaxEnds * kDof) R.ends[tid] = C.ends[tid];
         if (tid == 0) mt_seed_serial(s_mt, C.seed);
         if (tid < kDof) s_rstate[tid] = 0.0;
         mti = kMtN;
@@ -439,24 +533,52 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
         sampled_goals = st->sampled_goals;
         steps = st->steps;
         checks = st->checks;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+            for (int i = tid; i < kDof * kKeptNodes; i += NT) {
+                const int k = i / kKeptNodes, node = i % kKeptNodes;
+                if (node < (t ? n1 : n0)) s_nodes[t][i] = R.tree_s[t][(int64_t)k * C.cap + node];
+            }
     }
     __syncthreads();
-    // the draws of the current block (consecutive word pairs; a sample's seven
-    // draws are seven consecutive pairs, so a pair never spans two twists)
-    auto refill_draws = [&]() {
-        for (int i = tid; i < kMtN / 2; i += NT) s_u[i] = canonical53(mt_temper(s_mt[2 * i]), mt_temper(s_mt[2 * i + 1]));
+    // words are consumed in pairs (mti is even); draw i is the i-th after the last one taken
+    int pidx = mti / 2, cur = 0;
+    bool ahead = false;
+    auto make_draws = [&](int which) {
+        for (int i = tid; i < kDraws; i += NT)
+            s_u[which * kDraws + i] = canonical53(mt_temper(s_mt[2 * i]), mt_temper(s_mt[2 * i + 1]));
     };
-    if (mti < kMtN) refill_draws();
-    int pidx = mti / 2; // next draw (words are consumed in pairs: mti is even)
-    stage_env<true, kPlanPad>(EnvView{C.obs, C.ns, C.nb}, s_env); // ends with a barrier
+    auto to_current = [&]() { // the block made ahead becomes the current one when that is used up
+        if (ahead && pidx >= kDraws) {
+            pidx -= kDraws;
+            cur ^= 1;
+            ahead = false;
+        }
+    };
+    auto need_draws = [&](int need) { // need <= kDraws; whole block, a barrier before the draws are read
+        to_current();
+        if (!ahead && pidx + need > kDraws) {
+            for (int i = tid; i < kMtN; i += NT) s_prev[i] = s_mt[i];
+            mt_twist_block(s_mt); // reads the old words before its first barrier
+            make_draws(cur ^ 1);
+            ahead = true;
+            to_current();
+            __syncthreads();
+        }
+    };
+    auto draw = [&](int i) {
+        const int at = pidx + i;
+        return s_u[at < kDraws ? cur * kDraws + at : (cur ^ 1) * kDraws + at - kDraws];
+    };
+    if (pidx < kDraws) make_draws(0);
+    __syncthreads();
     if (C.init) {
         // PlannerInputStates::nextStart (Planner.cpp:228-256): the start
         // states in order; those in bounds and valid become the start tree's
         // roots
         for (int i = 0; i < C.n_starts; ++i) {
-            if (endpoint_usable<NT>(R.ends + (size_t)i * kDof, s_x, s_a, s_b, s_env, C.ns, C.nb, &s_hit) &&
-                n0 < C.cap) {
-                if (tid < kDof) R.tree_s[0][(int64_t)tid * C.cap + n0] = s_x[tid];
+            if (endpoint_usable(g, R.ends + (size_t)i * kDof, s_x, s_tests) && n0 < C.cap) {
+                if (tid < kDof) tree(0).set(tid, n0, s_x[tid]);
                 if (tid == 0) R.parent[0][n0] = -1;
                 ++n0;
             }
@@ -481,132 +603,124 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
         // ---- speculative sampling steps.  A sampling step (phase 0) that is
         // TRAPPED changes neither tree, and the samples of the next steps are
         // the generator's next draws whatever happens, so the next m steps can
-        // run at once, one per wave, against the current trees (step j grows
-        // the start tree iff start_tree ^ (j & 1)); they are then taken in order
-        // up to the first that is not TRAPPED, which is committed, and the rest
-        // are dropped (their draws are not consumed).  Same steps, same results
-        // as one at a time.  m stays within the generator's current block of
-        // draws and the iterations left.
+        // run at once, a few lanes each, against the current trees (step j
+        // grows the start tree iff start_tree ^ (j & 1)); they are then taken in
+        // order up to the first that is not TRAPPED, which is committed, and the
+        // rest are dropped (their draws are not consumed).  Same steps, same
+        // results as one at a time.  m stays within the iterations left.
         // (not while a goal state is due: the goal tree would change between
         // the steps)
         const bool goal_due = n1 == 0 || (sampled_goals < C.n_goals && sampled_goals < n1 / 2);
-        const int m_spec =
-            phase == 0 && !goal_due ? min(NT / 64, min((kMtN / 2 - pidx) / kDof, C.max_iters - iteration)) : 0;
-        if (m_spec >= 2) {
-            const int m = m_spec;
-            if (tid < kDof * m) s_samp[tid] = (kPi - -kPi) * s_u[pidx + tid] + -kPi;
+        const int lanes = spec_lanes(max(n0, n1));
+        const int m = phase == 0 && !goal_due ? min(min(kSpec, NT / lanes), C.max_iters - iteration) : 0;
+        if (m >= 2) {
+            need_draws(kDof * m);
+            if (tid < kDof * m) s_samp[tid] = (kPi - -kPi) * draw(tid) + -kPi;
             __syncthreads();
             if (tid == 0) {
                 c1 = wall_clock64();
                 t_sample += c1 - c0;
             }
             const int wave = tid >> 6, lane = tid & 63;
-            if (wave < m) {
-                const int st_j = start_tree ^ (wave & 1);
+            if (wave * 64 < m * lanes) {
+                const int step = lanes == 64 ? wave : tid / 16, sub = tid & (lanes - 1), j = min(step, m - 1);
+                const int st_j = start_tree ^ (j & 1);
                 const int tree_j = st_j ? 0 : 1;
-                const double *Tj = R.tree_s[tree_j];
+                const Tree Tj = tree(tree_j);
                 double tgt[kDof];
 #pragma unroll
-                for (int k = 0; k < kDof; ++k) tgt[k] = s_samp[kDof * wave + k];
-                const int nm = wave_nearest(Tj, C.cap, tree_j ? n1 : n0, tgt);
+                for (int k = 0; k < kDof; ++k) tgt[k] = s_samp[kDof * j + k];
+                const int n_j = tree_j ? n1 : n0;
+                Near best = scan_nearest(Tj, n_j, tgt, sub, lanes);
+                best.share(lanes);
                 if (tid == 0) {
                     const int64_t c2 = wall_clock64();
                     t_nearest += c2 - c1;
                 }
-                double nst[kDof], x[kDof];
-                double dist = 0.0;
+                Steer S;
+                S.run(Tj, n_j, best, tgt, C.maxd);
+                double a[kDof], b[kDof];
 #pragma unroll
                 for (int k = 0; k < kDof; ++k) {
-                    nst[k] = Tj[(int64_t)k * C.cap + nm];
-                    const double diff = nst[k] - tgt[k];
-                    dist += diff * diff;
+                    a[k] = st_j ? S.nst[k] : S.x[k];
+                    b[k] = st_j ? S.x[k] : S.nst[k];
                 }
-                const double dd = __builtin_sqrt(dist);
-                bool reach = true, moved = true;
-#pragma unroll
-                for (int k = 0; k < kDof; ++k) x[k] = tgt[k];
-                if (dd > C.maxd) {
-                    const double t = C.maxd / dd;
-                    bool equal = true;
+                const int nd = valid_segment_count<kDof>(a, b, C.lvs, C.factor);
+                // no progress, or too many segments: TRAPPED without a check
+                const int npos = S.moved && nd <= kMaxSegments ? StepMotion::positions(nd, !st_j) : 0;
+                if (sub == 0 && step < m) {
 #pragma unroll
                     for (int k = 0; k < kDof; ++k) {
-                        x[k] = nst[k] + (tgt[k] - nst[k]) * t;
-                        if (fabs(nst[k] - x[k]) > kEqualEps) equal = false;
+                        s_ga[kDof * j + k] = a[k];
+                        s_gb[kDof * j + k] = b[k];
+                        s_gx[kDof * j + k] = S.x[k];
                     }
-                    moved = !equal;
-                    reach = false;
+                    s_nm[j] = S.nm;
+                    s_reach[j] = S.reach ? 1 : 0;
+                    s_chk[j] = S.moved ? 1 : 0;
+                    s_nd[j] = nd;
+                    s_npos[j] = npos;
+                    s_bad[j] = 0;
                 }
-                int res = kSpecTrapped, nd = 0, npos = 0;
-                if (moved) {
-                    double *ga = s_ga + kDof * wave, *gb = s_gb + kDof * wave, *gx = s_gx + kDof * wave;
-                    double a[kDof], b[kDof];
-#pragma unroll
-                    for (int k = 0; k < kDof; ++k) {
-                        a[k] = st_j ? nst[k] : x[k];
-                        b[k] = st_j ? x[k] : nst[k];
-                    }
-                    nd = valid_segment_count<kDof>(a, b, C.lvs, C.factor);
-                    if (lane == 0)
-                        for (int k = 0; k < kDof; ++k) {
-                            ga[k] = a[k];
-                            gb[k] = b[k];
-                            gx[k] = x[k];
-                        }
-                    // lane 0's LDS writes before the wave's reads
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                    if (nd <= kMaxSegments) {
-                        const bool extra = !st_j;
-                        npos = 1 + (nd >= 2 ? nd - 1 : 0) + (extra ? 1 : 0);
-                        bool valid = wave_check<9>(ga, gb, gx, nd, 0, 1, extra, s_env, C.ns, C.nb);
-                        if (valid && npos > 1)
-                            valid = wave_check<1>(ga, gb, gx, nd, 1, min(npos, kSpecPositions), extra, s_env, C.ns,
-                                                  C.nb);
-                        res = !valid ? kSpecTrapped : (npos <= kSpecPositions ? kSpecValid : kSpecUndecided);
-                    }
-                }
-                if (lane == 0) {
-                    s_res[wave] = res;
-                    s_nm[wave] = nm;
-                    s_reach[wave] = reach ? 1 : 0;
-                    s_chk[wave] = moved ? 1 : 0;
-                    s_nd[wave] = nd;
-                    s_npos[wave] = npos;
-                }
+                // the steps' LDS writes before the wave's reads
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                const StepMotion M{s_ga + kDof * j, s_gb + kDof * j, s_gx + kDof * j, nd, step < m ? npos : 0, !st_j};
+                const uint64_t H = wave_ballot(wave_hit8(g, M, sub >> 3, s_tests[wave])) >> lane;
+                if (sub == 0 && step < m) s_open[j] = npos > 0 && (lanes == 64 ? H : H & 0xffff) == 0;
             }
             __syncthreads();
-            // take the steps in order
-            for (int j = 0; j < m; ++j) {
-                const int st_j = start_tree;
-                int res = s_res[j];
-                ++steps;
-                checks += s_chk[j];
-                if (res == kSpecUndecided) { // the rest of the motion by the whole block
-                    if (tid == 0) s_hit = 0;
-                    __syncthreads();
-                    const int nd = s_nd[j], npos = s_npos[j];
-                    const double *ga = s_ga + kDof * j, *gb = s_gb + kDof * j, *gx = s_gx + kDof * j;
-                    const bool extra = !st_j;
-                    const int ops = C.ops ? C.ops : auto_ops<NT / 64>(npos - kSpecPositions);
-                    bool valid;
-                    if (ops == 9)
-                        valid = block_check<NT, 9>(ga, gb, gx, nd, kSpecPositions, npos, extra, s_env, C.ns, C.nb,
-                                                   &s_hit);
-                    else if (ops == 4)
-                        valid = block_check<NT, 4>(ga, gb, gx, nd, kSpecPositions, npos, extra, s_env, C.ns, C.nb,
-                                                   &s_hit);
-                    else if (ops == 2)
-                        valid = block_check<NT, 2>(ga, gb, gx, nd, kSpecPositions, npos, extra, s_env, C.ns, C.nb,
-                                                   &s_hit);
-                    else
-                        valid = block_check<NT, 1>(ga, gb, gx, nd, kSpecPositions, npos, extra, s_env, C.ns, C.nb,
-                                                   &s_hit);
-                    res = valid ? kSpecValid : kSpecTrapped;
+            uint64_t open = wave_ballot(lane < m && s_open[min(lane, m - 1)] != 0);
+            const uint64_t moved_steps = wave_ballot(lane < m && s_chk[min(lane, m - 1)] != 0);
+            // the next positions of the open steps (those after the NT/64-th are
+            // dropped with what follows them), the block's waves shared out
+            int steps_here = m, checked = lanes / 8;
+            if (open) {
+                uint64_t more = open;
+                int c = 0;
+                for (; more && c < NT / 64; ++c) more &= more - 1;
+                if (more) steps_here = lowest_bit(more);
+                const int each = NT / 64 / c;
+                if (wave < c * each) {
+                    uint64_t rest = open;
+                    for (int r = wave / each; r > 0; --r) rest &= rest - 1;
+                    const int j = lowest_bit(rest);
+                    const StepMotion M{s_ga + kDof * j, s_gb + kDof * j, s_gx + kDof * j, s_nd[j], s_npos[j],
+                                       ((start_tree ^ j) & 1) == 0};
+                    const int p = checked + 8 * (wave % each) + (lane >> 3);
+                    if (wave_ballot(wave_hit8(g, M, p, s_tests[wave])) && lane == 0) s_bad[j] = 1;
                 }
-                start_tree = !start_tree; // RRTConnect.cpp:249
-                pidx += kDof;             // this step's sample is consumed
-                if (res == kSpecTrapped) {
+                checked += 8 * each;
+                __syncthreads();
+                if (steps_here < m) open &= ((uint64_t)1 << steps_here) - 1;
+                open &= ~wave_ballot(lane < m && s_bad[min(lane, m - 1)] != 0);
+            }
+            // take the steps in order: those before the first open one together
+            // (all TRAPPED), then that one
+            for (int taken = 0; taken < steps_here;) {
+                const int j = open ? lowest_bit(open) : steps_here;
+                const uint64_t before = ((uint64_t)1 << j) - 1;
+                steps += j - taken;
+                checks += __popcll(moved_steps & before & ~(((uint64_t)1 << taken) - 1));
+                pidx += kDof * (j - taken);
+                start_tree ^= (j - taken) & 1; // RRTConnect.cpp:249
+                iteration += j - taken;
+                taken = j;
+                if (j == steps_here) {
+                    if (iteration >= C.max_iters) status = OMPL_AMD_PLAN_FAILED;
+                    break;
+                }
+                const int st_j = start_tree;
+                ++steps;
+                ++checks; // an open step has moved
+                const StepMotion M{s_ga + kDof * j, s_gb + kDof * j, s_gx + kDof * j, s_nd[j], s_npos[j], !st_j};
+                const bool valid = block_check<NT>(g, M, checked, s_tests); // what is left of it
+                start_tree = !start_tree;
+                pidx += kDof; // this step's sample is consumed
+                ++taken;
+                open &= open - 1;
+                if (!valid) {
                     ++iteration;
                     if (iteration >= C.max_iters) {
                         status = OMPL_AMD_PLAN_FAILED;
@@ -616,7 +730,7 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
                 }
                 // commit step j: append its new state, then connect (phase 1)
                 const int tree_j = st_j ? 0 : 1;
-                const int last = append_step<NT>(R.tree_s[tree_j], R.parent[tree_j], C.cap, tree_j ? n1 : n0, s_nm[j],
+                const int last = append_step<NT>(tree(tree_j), parents(tree_j), tree_j ? n1 : n0, s_nm[j],
                                                  s_ga + kDof * j, s_gb + kDof * j, s_gx + kDof * j, s_nd[j], st_j != 0,
                                                  C.inter != 0);
                 if (last < 0) {
@@ -651,13 +765,12 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
             if (n1 == 0 || sampled_goals < n1 / 2) {
                 const bool empty = n1 == 0;
                 while (sampled_goals < C.n_goals) {
-                    const int g = sampled_goals++;
-                    if (endpoint_usable<NT>(R.ends + (size_t)(kMaxEnds + g) * kDof, s_x, s_a, s_b, s_env, C.ns, C.nb,
-                                            &s_hit)) {
+                    const int goal = sampled_goals++;
+                    if (endpoint_usable(g, R.ends + (size_t)(kMaxEnds + goal) * kDof, s_x, s_tests)) {
                         if (n1 >= C.cap) {
                             status = OMPL_AMD_PLAN_TREE_FULL;
                         } else {
-                            if (tid < kDof) R.tree_s[1][(int64_t)tid * C.cap + n1] = s_x[tid];
+                            if (tid < kDof) tree(1).set(tid, n1, s_x[tid]);
                             if (tid == 0) R.parent[1][n1] = -1;
                             ++n1;
                         }
@@ -671,19 +784,10 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
                 if (status != OMPL_AMD_PLAN_RUNNING) break;
             }
             // sampler_->sampleUniform(rstate): RNG::uniformReal(-pi, pi) per joint,
-            // from the next seven draws (twisting when the block runs out)
-            for (int d0 = 0; d0 < kDof;) {
-                if (pidx >= kMtN / 2) {
-                    mt_twist_block(s_mt);
-                    refill_draws();
-                    __syncthreads();
-                    pidx = 0;
-                }
-                const int take = min(kDof - d0, kMtN / 2 - pidx);
-                if (tid < take) s_rstate[d0 + tid] = (kPi - -kPi) * s_u[pidx + tid] + -kPi;
-                pidx += take;
-                d0 += take;
-            }
+            // from the next seven draws
+            need_draws(kDof);
+            if (tid < kDof) s_rstate[tid] = (kPi - -kPi) * draw(tid) + -kPi;
+            pidx += kDof;
             __syncthreads();
             if (tid == 0) {
                 c1 = wall_clock64();
@@ -696,91 +800,50 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
 #pragma unroll
         for (int k = 0; k < kDof; ++k) tgt[k] = s_rstate[k];
         const int nt = grow_tree ? n1 : n0;
-        double *T = R.tree_s[grow_tree];
-        const int nm = block_nearest<NT>(T, C.cap, nt, tgt, s_wd, s_wi);
+        const Tree T = tree(grow_tree);
+        const Near best = block_nearest<NT>(T, nt, tgt, s_wd, s_wi);
         if (tid == 0) {
             const int64_t c2 = wall_clock64();
             t_nearest += c2 - c1;
             c1 = c2;
         }
-        double nst[kDof], x[kDof];
-        double dist = 0.0;
-#pragma unroll
-        for (int k = 0; k < kDof; ++k) {
-            nst[k] = T[(int64_t)k * C.cap + nm];
-            const double diff = nst[k] - tgt[k];
-            dist += diff * diff;
-        }
-        const double dd = __builtin_sqrt(dist);
-        bool reach = true, moved = true;
-#pragma unroll
-        for (int k = 0; k < kDof; ++k) x[k] = tgt[k];
-        if (dd > C.maxd) {
-            const double t = C.maxd / dd;
-            bool equal = true;
-#pragma unroll
-            for (int k = 0; k < kDof; ++k) {
-                x[k] = nst[k] + (tgt[k] - nst[k]) * t;
-                if (fabs(nst[k] - x[k]) > kEqualEps) equal = false;
-            }
-            moved = !equal; // no progress: TRAPPED without a check
-            reach = false;
-        }
+        Steer S;
+        S.run(T, nt, best, tgt, C.maxd);
         int gs = kTrapped;
-        if (moved) {
+        if (S.moved) {
             // tgi.start ? checkMotion(nearest, dst) : isValid(dst) && checkMotion(dst, nearest)
             const bool from_start = tgi_start != 0;
             double a[kDof], b[kDof];
 #pragma unroll
             for (int k = 0; k < kDof; ++k) {
-                a[k] = from_start ? nst[k] : x[k];
-                b[k] = from_start ? x[k] : nst[k];
+                a[k] = from_start ? S.nst[k] : S.x[k];
+                b[k] = from_start ? S.x[k] : S.nst[k];
             }
             const int nd = valid_segment_count<kDof>(a, b, C.lvs, C.factor);
             if (tid == 0) {
                 for (int k = 0; k < kDof; ++k) {
                     s_a[k] = a[k];
                     s_b[k] = b[k];
-                    s_x[k] = x[k];
+                    s_x[k] = S.x[k];
                 }
-                s_hit = 0;
             }
             __syncthreads();
             ++checks;
             bool valid = false;
             if (nd <= kMaxSegments) { // longer motions are reported invalid
-                const int npos = 1 + (nd >= 2 ? nd - 1 : 0) + (from_start ? 0 : 1);
-                // First round: one position per wave, the obstacle list split nine
-                // ways (a failing motion -- most are -- usually fails at the new
-                // state or an early bisection point, found within a pass or two);
-                // then the rest in rounds shaped by the configured or auto split.
-                const int nfirst = min(npos, NT / 64);
-                valid = block_check<NT, 9>(s_a, s_b, s_x, nd, 0, nfirst, !from_start, s_env, C.ns, C.nb, &s_hit);
-                if (valid && nfirst < npos) {
-                    const int ops = C.ops ? C.ops : auto_ops<NT / 64>(npos - nfirst);
-                    if (ops == 9)
-                        valid = block_check<NT, 9>(s_a, s_b, s_x, nd, nfirst, npos, !from_start, s_env, C.ns, C.nb,
-                                                   &s_hit);
-                    else if (ops == 4)
-                        valid = block_check<NT, 4>(s_a, s_b, s_x, nd, nfirst, npos, !from_start, s_env, C.ns, C.nb,
-                                                   &s_hit);
-                    else if (ops == 2)
-                        valid = block_check<NT, 2>(s_a, s_b, s_x, nd, nfirst, npos, !from_start, s_env, C.ns, C.nb,
-                                                   &s_hit);
-                    else
-                        valid = block_check<NT, 1>(s_a, s_b, s_x, nd, nfirst, npos, !from_start, s_env, C.ns, C.nb,
-                                                   &s_hit);
-                }
+                const StepMotion M{s_a, s_b, s_x, nd, StepMotion::positions(nd, !from_start), !from_start};
+                valid = !__syncthreads_or(wave_hit8(g, M, tid >> 3, s_tests[tid >> 6])) &&
+                        block_check<NT>(g, M, NT / 8, s_tests);
             }
             if (valid) {
-                const int last = append_step<NT>(T, R.parent[grow_tree], C.cap, grow_tree ? n1 : n0, nm, s_a, s_b, s_x,
+                const int last = append_step<NT>(T, parents(grow_tree), grow_tree ? n1 : n0, S.nm, s_a, s_b, s_x,
                                                  nd, from_start, C.inter != 0);
                 if (last < 0) {
                     status = OMPL_AMD_PLAN_TREE_FULL;
                     break;
                 }
                 xmotion = last;
-                gs = reach ? kReached : kAdvanced;
+                gs = S.reach ? kReached : kAdvanced;
             }
         }
         ++steps;
@@ -820,10 +883,11 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
                 }
                 __syncthreads();
                 const int c1 = s_n1, len = s_len;
+                double *path = len <= A.path_rows ? C.path : R.path;
                 for (int r = tid; r < len * kDof; r += NT) {
                     const int row = r / kDof, k = r - row * kDof;
-                    R.path[r] = row < c1 ? R.tree_s[0][(int64_t)k * C.cap + R.path_idx[c1 - 1 - row]]
-                                         : R.tree_s[1][(int64_t)k * C.cap + R.path_idx[row]];
+                    path[r] = row < c1 ? R.tree_s[0][(int64_t)k * C.cap + R.path_idx[c1 - 1 - row]]
+                                       : R.tree_s[1][(int64_t)k * C.cap + R.path_idx[row]];
                 }
                 path_len = len;
                 status = OMPL_AMD_PLAN_SOLVED;
@@ -841,7 +905,8 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
     }
 
     __syncthreads();
-    for (int i = tid; i < kMtN; i += NT) st->mt[i] = s_mt[i];
+    to_current();
+    for (int i = tid; i < kMtN; i += NT) st->mt[i] = ahead ? s_prev[i] : s_mt[i];
     if (tid < kDof) st->rstate[tid] = s_rstate[tid];
     if (tid == 0) {
         st->mti = 2 * pidx;
@@ -967,8 +1032,12 @@ struct Server {
     hipStream_t stream = nullptr;
     char *pool = nullptr;
     PoolAlloc alloc;
-    PlanCmd *cmd_host = nullptr, *cmd_dev = nullptr;
-    PlanOut *out_host = nullptr, *out_dev = nullptr;
+    // pinned, one per active request: the slice kernel reads and writes them in place
+    PlanCmd *cmd_host = nullptr;
+    PlanOut *out_host = nullptr;
+    double *ends_host = nullptr; // [max_active][2 kMaxEnds][kDof]
+    double *path_host = nullptr; // [max_active][path_rows][kDof]
+    int path_rows = 0;
     int64_t budget_ticks = 0;
 
     std::mutex mu;
@@ -1149,15 +1218,12 @@ void Server::run()
             }
             if (batch.empty()) continue;
             const int n = (int)batch.size();
-            size_t lds = 0;
             for (int i = 0; i < n; ++i) {
                 Planner &p = *batch[i];
                 const Env &env = p.req.env->env;
                 PlanCmd &c = cmd_host[i];
-                c.obs = env.obs;
+                c.grid = env.grid;
                 c.region = pool + p.off;
-                c.ns = env.ns;
-                c.nb = env.nb;
                 c.cap = p.req.max_nodes;
                 c.max_iters = p.req.max_iters;
                 c.maxd = p.maxd;
@@ -1165,30 +1231,23 @@ void Server::run()
                 c.factor = p.req.factor;
                 c.seed = p.req.seed;
                 c.init = p.init ? 1 : 0;
-                c.ops = cfg.check_obstacle_parts;
                 c.n_starts = p.req.n_starts;
                 c.n_goals = p.req.n_goals;
                 c.inter = p.req.intermediate_states ? 1 : 0;
-                if (p.init) {
-                    // the request's start and goal states into its region
-                    const RegionPtrs Rp = region_ptrs(pool + p.off, p.req.max_nodes);
-                    OA_HIP(hipMemcpyAsync(Rp.ends, p.ends.data(), p.ends.size() * sizeof(double),
-                                          hipMemcpyHostToDevice, stream));
-                }
-                lds = std::max(lds, env_stage_bytes(env.ns, env.nb));
+                c.ends = ends_host + (size_t)i * 2 * kMaxEnds * kDof;
+                c.path = path_host + (size_t)i * path_rows * kDof;
+                if (p.init) std::copy(p.ends.begin(), p.ends.end(), ends_host + (size_t)i * 2 * kMaxEnds * kDof);
                 p.init = false;
             }
-            OA_HIP(hipMemcpyAsync(cmd_dev, cmd_host, n * sizeof(PlanCmd), hipMemcpyHostToDevice, stream));
             {
                 ProfScope ps("serve_slice", stream);
-                const SliceArgs args{cmd_dev, out_dev, budget_ticks};
+                const SliceArgs args{cmd_host, out_host, path_rows, budget_ticks};
                 if (cfg.block_threads == 1024)
-                    hipLaunchKernelGGL(plan_slice_kernel<1024>, dim3(n), dim3(1024), lds, stream, args);
+                    hipLaunchKernelGGL(plan_slice_kernel<1024>, dim3(n), dim3(1024), 0, stream, args);
                 else
-                    hipLaunchKernelGGL(plan_slice_kernel<512>, dim3(n), dim3(512), lds, stream, args);
+                    hipLaunchKernelGGL(plan_slice_kernel<512>, dim3(n), dim3(512), 0, stream, args);
                 OA_HIP(hipGetLastError());
             }
-            OA_HIP(hipMemcpyAsync(out_host, out_dev, n * sizeof(PlanOut), hipMemcpyDeviceToHost, stream));
             OA_HIP(hipStreamSynchronize(stream));
             ++slices;
             // solution paths of the requests that solved in this slice
@@ -1198,6 +1257,11 @@ void Server::run()
                 const PlanOut &o = out_host[i];
                 if (o.status != OMPL_AMD_PLAN_SOLVED || o.path_len <= 0) continue;
                 paths[i].resize((size_t)o.path_len * kDof);
+                if (o.path_len <= path_rows) {
+                    const double *path = cmd_host[i].path;
+                    std::copy(path, path + paths[i].size(), paths[i].begin());
+                    continue;
+                }
                 const RegionPtrs Rp = region_ptrs(pool + batch[i]->off, batch[i]->req.max_nodes);
                 OA_HIP(hipMemcpyAsync(paths[i].data(), Rp.path, paths[i].size() * sizeof(double),
                                       hipMemcpyDeviceToHost, stream));
@@ -1513,8 +1577,11 @@ int ompl_amd_server_create(const ompl_amd_server_config *cfg, ompl_amd_server *o
         S.alloc.reset(cfg->hbm_budget_bytes);
         OA_HIP(hipHostMalloc((void **)&S.cmd_host, sizeof(PlanCmd) * cfg->max_active, hipHostMallocDefault));
         OA_HIP(hipHostMalloc((void **)&S.out_host, sizeof(PlanOut) * cfg->max_active, hipHostMallocDefault));
-        OA_HIP(hipMalloc(&S.cmd_dev, sizeof(PlanCmd) * cfg->max_active));
-        OA_HIP(hipMalloc(&S.out_dev, sizeof(PlanOut) * cfg->max_active));
+        OA_HIP(hipHostMalloc((void **)&S.ends_host, sizeof(double) * 2 * kMaxEnds * kDof * cfg->max_active,
+                             hipHostMallocDefault));
+        S.path_rows = std::max(1, std::min(kPathRows, (int)(kPathBytes / (sizeof(double) * kDof * cfg->max_active))));
+        OA_HIP(hipHostMalloc((void **)&S.path_host, sizeof(double) * kDof * S.path_rows * cfg->max_active,
+                             hipHostMallocDefault));
         OA_HIP(hipStreamCreateWithFlags(&S.prm_stream, hipStreamNonBlocking));
         S.th = std::thread([&S] { S.run(); });
         S.prm_th = std::thread([&S] { S.run_prm(); });
@@ -1542,10 +1609,10 @@ int ompl_amd_server_destroy(ompl_amd_server h)
         // teardown: release everything even if one release reports an error
         (void)hipStreamSynchronize(S.stream);
         if (S.pool) (void)hipFree(S.pool);
-        (void)hipFree(S.cmd_dev);
-        (void)hipFree(S.out_dev);
         (void)hipHostFree(S.cmd_host);
         (void)hipHostFree(S.out_host);
+        (void)hipHostFree(S.ends_host);
+        (void)hipHostFree(S.path_host);
         (void)hipStreamDestroy(S.stream);
         (void)hipStreamSynchronize(S.prm_stream);
         (void)hipStreamDestroy(S.prm_stream);
