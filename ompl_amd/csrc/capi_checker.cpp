@@ -188,8 +188,8 @@ namespace {
 void graph_workspace(Workspace &w, int64_t n)
 {
     const size_t cap = (size_t)n < 1024 ? 1024 : (size_t)n;
-    OA_HIP(hipMalloc(&w.counters, 64 * sizeof(int32_t)));
-    OA_HIP(hipMemset(w.counters, 0, 64 * sizeof(int32_t)));
+    OA_HIP(hipMalloc(&w.counters, kWorkspaceCounters * sizeof(int32_t)));
+    OA_HIP(hipMemset(w.counters, 0, kWorkspaceCounters * sizeof(int32_t)));
     alloc_workspace_arrays(w, cap);
     w.parity = 0;
 }

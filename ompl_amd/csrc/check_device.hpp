@@ -68,12 +68,13 @@ __device__ __forceinline__ bool endpoint_finish(const MotionArgs &A, int64_t e, 
 
 // Block-aggregated append of the survivors to the list (with their segment
 // count and, when kept, their endpoints contiguous for the chunk walk).
-// Every thread of the block calls it (it holds three barriers).  The waves'
+// Every thread of the block calls it (it holds three barriers); a survivor's
+// slot is returned.  The waves'
 // counts and largest segment counts meet in LDS, and one thread per block
 // makes the two device-wide atomics: device-scope atomics on one address
 // from every CU serialise, and with many survivors (a sparse scene) one
 // atomic per survivor cost more than the s2 checks themselves.
-__device__ __forceinline__ void append_survivor(const MotionArgs &A, int64_t e, bool survivor, int m,
+__device__ __forceinline__ int append_survivor(const MotionArgs &A, int64_t e, bool survivor, int m,
                                                 const double a[kDof], const double b[kDof])
 {
     __shared__ int blk_count, blk_max, blk_base;
@@ -101,8 +102,8 @@ __device__ __forceinline__ void append_survivor(const MotionArgs &A, int64_t e, 
         if (A.max_m) atomicMax(A.max_m, blk_max);
     }
     __syncthreads();
+    const int slot = blk_base + woff + __popcll(sm & (((uint64_t)1 << lane) - 1));
     if (survivor) {
-        const int slot = blk_base + woff + __popcll(sm & (((uint64_t)1 << lane) - 1));
         A.out[e] = 1; // until the walk finds an invalid position
         A.list[slot] = (int32_t)e;
         if (A.first_bad) A.first_bad[slot] = INT_MAX;
@@ -116,6 +117,7 @@ __device__ __forceinline__ void append_survivor(const MotionArgs &A, int64_t e, 
             }
         }
     }
+    return slot;
 }
 
 } // namespace ompl_amd

@@ -69,10 +69,17 @@ void launch_motion_last_valid(const MotionArgs &A, double *last_t, int lps, int 
 void launch_state_lists(const EnvView &env, const double *q_soa, int64_t n_states, const int64_t *offsets,
                         int64_t n_lists, uint8_t *out, int32_t *first_invalid, int lps, int ops, int64_t waves,
                         int32_t *unres, int32_t *unres_fb, int32_t *counters, hipStream_t s);
+// Edges or lists up to which a block each walks them in one launch: 1,024
+// blocks of four waves are one wave per SIMD, so the speculative positions of
+// edges that fail at once cost no time; more edges go through the s2 pass.
+constexpr int kWideItems = 1024;
+// Ints of a workspace's counters, zero at its creation.
+constexpr int kWorkspaceCounters = 64 + 2 * kWideItems;
 // Survivor workspace of the checks over the cell grid (grid_check.hip).
 struct GridScratch {
     int32_t *list, *surv_nd, *rest, *long_slot, *long_bad, *ticket; // an entry per edge or list
     double *surv_ab;                                                 // 14 per edge
+    int32_t *wide;                                                   // 2 kWideItems words, zero between batches
     int32_t *counts;                                                 // two words, zero
     int32_t *next;                                                   // two words, cleared for the next batch
 };

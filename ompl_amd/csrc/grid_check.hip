@@ -17,14 +17,18 @@
 //
 // Measured against the kernels that test every obstacle, in the launch shapes
 // the library starts with: 65,536 states, 64 spheres 35.7 -> 8.7 us; 16,384
-// edges, 16 + 16 obstacles, checked counts 384 -> 68 us; 4,099 edges' lastValid
-// 110 -> 31 us; 61 edges, 128 + 128 obstacles 38 -> 11.7 us.  Against shapes
-// tuned for the scene: 16,384 edges, 128 + 128 obstacles 31 -> 22 us on one
-// stream, 12.4 -> 11.3 us a batch on four; 16 + 16 obstacles 77 -> 53 us (no
+// edges, 16 + 16 obstacles, checked counts 384 -> 62 us; 4,099 edges' lastValid
+// 110 -> 29 us; 61 edges, 128 + 128 obstacles 38 -> 8.8 us.  Against shapes
+// tuned for the scene: 16,384 edges, 128 + 128 obstacles 31 -> 19.3 us on one
+// stream, 12.6 -> 8.7 us a batch on four; 16 + 16 obstacles 77 -> 49 us (no
 // counts).  Large batches are bound by VALU instructions (about 1,100 a wave of
 // 64 states, half of them the forward kinematics), small ones by the chain of
-// dependent reads (counts, record, cells, cells, obstacles) and by fetching
-// the code once.
+// dependent reads (counts, record, cells, cells, obstacles), by fetching the
+// code once and by the launches: a kernel that only walked what the one before
+// had left cost 3 to 4 us, so the survivors' kernel walks its own leftovers
+// (16,384 dense edges 22.2 -> 19.3 us, 11.3 -> 8.7 on four streams; 16 + 16
+// obstacles 68 -> 62) and a one-launch batch finds its own long items (61
+// edges 11.7 -> 8.8 us).
 #include <hip/hip_runtime.h>
 
 #include <climits>
@@ -70,12 +74,13 @@ __global__ void __launch_bounds__(256) grid_validate_kernel(GridView g, const T 
 // states of a precomputed list in order (SpaceInformation.cpp:288-299).
 enum class Walk { kBisect, kSequence, kList };
 
-// Workspace use (Workspace in runtime.hpp): the first kernel says in rest[slot]
-// whether it left an item unfinished (a list of them would take a device-wide
-// atomic each: on one address they are 6 ns apart, 60 us for 10,000); those
-// with more than kLongWalk positions left are listed in long_slot, with a
-// first_bad and a ticket each.
+// Items with more than kLongWalk positions are long: walked by many blocks
+// together, each every so-manyth 256 of its positions.  A long item has a word
+// for the lowest position found invalid (INT_MAX minus it, 0: none) and a
+// ticket; the last block to finish it writes its result.
 constexpr int kLongWalk = 16384;
+// Blocks that look for long items beside up to kWideItems blocks of an item each.
+constexpr int kHelpers = 256;
 
 struct GridWalkArgs {
     GridView g;
@@ -84,12 +89,16 @@ struct GridWalkArgs {
     const double *q;   // kList: dof-major states
     int64_t n_states;
     const int64_t *offsets;
-    int32_t *rest;      // [cap]
-    int32_t *long_slot; // [cap]
+    int32_t *rest;      // [cap] lists of a wave each: whether the item is unfinished (listing
+                        // them would take a device-wide atomic each: on one address they
+                        // are 6 ns apart, 60 us for 10,000)
+    int32_t *long_slot; // [cap] long items
     int32_t *long_bad;  // [cap]
     int32_t *ticket;    // [cap]
+    int32_t *wide_bad;  // [kWideItems] by item, zero between batches
+    int32_t *wide_ticket;
     int32_t *counts;    // [0] survivors, [1] long items; zero at the batch's start
-    int32_t *next;     // the set the next batch uses, cleared by the first kernel after the s2 pass
+    int32_t *next;      // the set the next batch uses, cleared by the first kernel after the s2 pass
 };
 
 // One item: its id (edge or list) and what is needed to make its states.
@@ -110,8 +119,23 @@ struct Item {
         nd = valid_segment_count<kDof>(a, b, A.lvs, A.factor);
         total = MODE == Walk::kBisect ? max(nd, 1) : max(nd, 1) + 1;
     }
-    // slot is wave-uniform; the record was written by an earlier kernel, so it
-    // is read into scalar registers (28 vector registers fewer: a wave more per SIMD)
+    // As edge() for a wave-uniform e.  The edges, as a survivor's record below,
+    // were written by earlier kernels, so they are read into scalar registers (28
+    // vector registers fewer: a wave more per SIMD).
+    __device__ __forceinline__ void one_edge(const MotionArgs &A, int e_any)
+    {
+        using Const = const __attribute__((address_space(4))) double;
+        const int e = __builtin_amdgcn_readfirstlane(e_any);
+        id = e;
+#pragma unroll
+        for (int j = 0; j < kDof; ++j) {
+            a[j] = ((Const *)A.a)[(int64_t)j * A.n + e];
+            b[j] = ((Const *)A.b)[(int64_t)j * A.n + e];
+        }
+        nd = valid_segment_count<kDof>(a, b, A.lvs, A.factor);
+        total = MODE == Walk::kBisect ? max(nd, 1) : max(nd, 1) + 1;
+    }
+    // slot is wave-uniform
     __device__ __forceinline__ void survivor(const MotionArgs &A, int slot_any)
     {
         using Const = const __attribute__((address_space(4))) double;
@@ -177,47 +201,70 @@ __device__ __forceinline__ int wave_walk(const GridWalkArgs &A, const Item<MODE>
     float q[kDof];
     I.state(A, live ? p : base, q);
     const uint64_t H = wave_ballot(state_hit1(A.g, q, live, tests[threadIdx.x >> 6]));
-    return H ? base + lowest_bit(H) : INT_MAX;
+    return H ? base + lowest_bit(H) : INT_MAX; // wave-uniform
 }
 
-// The walk of one item by a block (from .. total-1, a block's positions at a
-// time) or, with `wide` false, by each wave for itself (the first 64).  The
-// kernels below have one call of it each: the code of a state check is 10 KB,
-// and a short launch waits for every line of it.  bad: the block's LDS word.
-// Returns the lowest invalid position or INT_MAX, uniform over the walkers.
+__device__ __forceinline__ int known_bad(const int32_t *p)
+{
+    return INT_MAX - __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// What the waves of a block tell each other after a round, twice over so that
+// one barrier a round is enough.
+struct Rounds {
+    int bad[2][4];
+    int known[2];
+};
+
+// The walk of one item by a block: its positions below `end` from `first` on, a
+// block's at a time, `step` apart; or (own) by each wave for itself its item's
+// first 64 from `first` on.  The kernels below have one call of it each: the
+// code of a state check is 10 KB, and a short launch waits for every line of it.
+// known: a long item's word (else null), which ends the walk once an earlier
+// position is known invalid.  Returns the lowest invalid position seen or
+// INT_MAX, uniform over the walkers.
 template <Walk MODE>
-__device__ __forceinline__ int walk_item(const GridWalkArgs &A, const Item<MODE> &I, int from, int total, bool wide,
-                                         int *bad, WaveTests *tests)
+__device__ __forceinline__ int walk_item(const GridWalkArgs &A, const Item<MODE> &I, int64_t first, int end, bool own,
+                                         int64_t step, const int32_t *known, Rounds &R, int &turn, WaveTests *tests)
 {
-    if (wide) {
-        if (threadIdx.x == 0) *bad = INT_MAX;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int64_t round = first;;) {
+        const int64_t base = round + (own ? 0 : wave * 64);
+        const int b = wave_walk<MODE>(A, I, (int)min(base, (int64_t)INT_MAX), end, tests);
+        if (own) return b;
+        if (lane_id() == 0) R.bad[turn][wave] = b;
+        if (threadIdx.x == 0) R.known[turn] = known ? known_bad(known) : INT_MAX;
         __syncthreads();
-    }
-    int64_t base = from + (wide ? (int)(threadIdx.x & ~63u) : 0);
-    for (int64_t round = from;;) {
-        const int b = wave_walk<MODE>(A, I, (int)min(base, (int64_t)INT_MAX), total, tests);
-        if (!wide) return b;
-        if (b != INT_MAX && lane_id() == 0) atomicMin(bad, b);
-        __syncthreads();
-        const int found = *bad;
-        __syncthreads(); // every wave has read it before the next round (or walk) writes it
-        round += blockDim.x;
-        base += blockDim.x;
-        if (found != INT_MAX || round >= total) return found; // block-uniform
+        const int found = __builtin_amdgcn_readfirstlane(
+            min(min(R.bad[turn][0], R.bad[turn][1]), min(R.bad[turn][2], R.bad[turn][3])));
+        const int earlier = __builtin_amdgcn_readfirstlane(R.known[turn]);
+        turn ^= 1;
+        round += step;
+        if (found != INT_MAX || round >= end || earlier < round) return found; // block-uniform
     }
 }
 
-// Leaves an item's positions from `from` on to grid_rest_kernel (one lane).
-__device__ __forceinline__ void leave_rest(const GridWalkArgs &A, int slot, int total, int from)
+// A block's share of a long item is done (one thread); `blocks` of them.
+template <Walk MODE>
+__device__ __forceinline__ void finish_long(const GridWalkArgs &A, const Item<MODE> &I, int b, int32_t *bad,
+                                            int32_t *ticket, int blocks)
 {
-    const bool is_long = total - from > kLongWalk;
-    A.rest[slot] = is_long ? 0 : 1;
-    if (is_long) {
-        const int l = atomicAdd(&A.counts[1], 1);
-        A.long_slot[l] = slot;
-        A.long_bad[l] = INT_MAX;
-        A.ticket[l] = 0;
-    }
+    if (b != INT_MAX) atomicMax(bad, INT_MAX - b);
+    __threadfence(); // the minimum is made before the ticket is taken
+    if (atomicAdd(ticket, 1) != blocks - 1) return;
+    __threadfence();
+    I.result(A, known_bad(bad));
+    *bad = 0; // as the next batch finds them
+    *ticket = 0;
+}
+
+// Lists a long item (one lane).
+__device__ __forceinline__ void list_long(const GridWalkArgs &A, int slot)
+{
+    const int l = atomicAdd(&A.counts[1], 1);
+    A.long_slot[l] = slot;
+    A.long_bad[l] = 0;
+    A.ticket[l] = 0;
 }
 
 // Keeps an edge for grid_rest_kernel under `slot` (one lane).
@@ -253,7 +300,8 @@ __global__ void __launch_bounds__(256) grid_endpoint1_kernel(GridWalkArgs A)
     int m = 0;
     double a[kDof], b[kDof];
     const bool survivor = endpoint_finish<1>(M, e, live, H, m, a, b);
-    append_survivor(M, e, survivor, m, a, b);
+    const int slot = append_survivor(M, e, survivor, m, a, b);
+    if (survivor && m > kLongWalk) list_long(A, slot);
 }
 
 // As above with eight lanes per edge: lane j reads joint j of both ends (two
@@ -303,6 +351,7 @@ __global__ void __launch_bounds__(256) grid_endpoint8_kernel(GridWalkArgs A)
         if (j == 0) {
             M.list[slot] = (int32_t)e;
             M.surv_nd[slot] = nd;
+            if (nd - 1 > kLongWalk) list_long(A, slot);
         }
         if (j < kDof) {
             double *ab = M.surv_ab + (int64_t)slot * 2 * kDof;
@@ -313,95 +362,160 @@ __global__ void __launch_bounds__(256) grid_endpoint8_kernel(GridWalkArgs A)
 }
 
 // Survivors of the s2 pass: when there are no more than blocks, a block walks
-// each to its end; else a wave walks the first 64 positions of each and leaves
-// the rest to grid_rest_kernel (an edge that fails does so early, and one wave
-// finds out without the other three).
+// each to its end; else its waves walk the first 64 positions of one each (an
+// edge that fails does so early, and one wave finds out without the other
+// three), then the block what is left of them.  Last, all blocks together walk
+// the long ones.
 __global__ void __launch_bounds__(256, 4) grid_survivors_kernel(GridWalkArgs A)
 {
-    __shared__ int bad;
+    __shared__ Rounds R;
     __shared__ WaveTests tests[4];
     clear_next(A);
-    const int n = A.counts[0];
+    const int n = A.counts[0], n_long = A.counts[1];
     const bool wide = n <= (int)gridDim.x;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), groups = wide ? n : (n + 3) / 4;
+    int turn = 0, group = 0, l = -1;
+    int64_t next = blockIdx.x;
+    unsigned open = 0; // items of the group that are unfinished
     Item<Walk::kBisect> I;
-    for (int s = wide ? blockIdx.x : blockIdx.x * 4 + wave; s < n; s += wide ? gridDim.x : 4 * gridDim.x) {
-        I.survivor(A.m, s);
-        const int done = !wide || I.total - 65 > kLongWalk ? min(I.total, 65) : I.total;
-        const int b = walk_item(A, I, 1, done, wide, &bad, tests);
-        if (wide ? threadIdx.x == 0 : lane_id() == 0) {
-            if (b != INT_MAX || done == I.total) {
-                I.result(A, b);
-                A.rest[s] = 0;
-            } else {
-                leave_rest(A, s, I.total, done);
+    for (;;) {
+        int slot, from = 1;
+        bool own = false, is_long = false;
+        if (open) {
+            slot = 4 * group + __builtin_ctz(open);
+            open &= open - 1;
+            from = 65;
+        } else if (next < groups) {
+            group = (int)next;
+            next += gridDim.x;
+            own = !wide;
+            slot = wide ? group : 4 * group + wave;
+        } else if (++l < n_long) {
+            slot = A.long_slot[l];
+            is_long = true;
+        } else {
+            break;
+        }
+        I.survivor(A.m, min(slot, n - 1));
+        const bool mine = slot < n && (is_long || I.total - 1 <= kLongWalk);
+        if (!own && !mine) continue; // a long item's turn comes (block-uniform)
+        const int end = !mine ? 0 : own ? min(I.total, 65) : I.total;
+        const int b = walk_item(A, I, from + (is_long ? (int64_t)blockIdx.x * 256 : 0), end, own,
+                                is_long ? (int64_t)gridDim.x * 256 : 256, is_long ? &A.long_bad[l] : nullptr, R, turn,
+                                tests);
+        if (own) {
+            const bool left = mine && b == INT_MAX && end < I.total;
+            if (lane_id() == 0) {
+                if (mine && !left) I.result(A, b);
+                R.bad[turn][wave] = left ? 1 : 0;
             }
+            __syncthreads();
+            open = __builtin_amdgcn_readfirstlane(R.bad[turn][0] | R.bad[turn][1] << 1 | R.bad[turn][2] << 2 |
+                                                  R.bad[turn][3] << 3);
+            turn ^= 1;
+        } else if (threadIdx.x == 0) {
+            if (is_long) finish_long(A, I, b, &A.long_bad[l], &A.ticket[l], gridDim.x);
+            else I.result(A, b);
         }
     }
 }
 
-// First walk of edges (kBisect with s2 as position 0, kSequence) and lists:
-// WIDE, a block walks each item to its end (small batches: one launch, every
-// position in flight at once); else a wave walks the first 64 positions.
-template <Walk MODE, bool WIDE>
+// Up to kWideItems edges (kBisect with s2 as position 0, kSequence) or lists: a
+// block walks each to its end, in one launch with every position in flight at
+// once.  The kHelpers blocks after them look through all items for long ones
+// (a few loads a thread, while the others walk) and walk those together.
+template <Walk MODE>
+__global__ void __launch_bounds__(256, 4) grid_wide_kernel(GridWalkArgs A)
+{
+    __shared__ Rounds R;
+    __shared__ WaveTests tests[4];
+    __shared__ int longs[kWideItems], n_longs;
+    clear_next(A);
+    constexpr int from = MODE == Walk::kSequence ? 1 : 0;
+    const int n = (int)A.m.n, helper = (int)blockIdx.x - n;
+    Item<MODE> I;
+    int turn = 0, left = 1;
+    if (helper >= 0) {
+        if (threadIdx.x == 0) n_longs = 0;
+        __syncthreads();
+        for (int i = threadIdx.x; i < n; i += 256) {
+            if (MODE == Walk::kList) I.list(A, i);
+            else I.edge(A.m, i);
+            if (!I.nd_too_many() && I.total - from > kLongWalk) longs[atomicAdd(&n_longs, 1)] = i;
+        }
+        __syncthreads();
+        left = n_longs;
+    }
+    for (; left > 0; --left) { // block-uniform
+        const int id = helper < 0 ? (int)blockIdx.x : longs[left - 1];
+        if (MODE == Walk::kList) I.list(A, id);
+        else I.one_edge(A.m, id);
+        const bool none = I.nd_too_many(); // reported invalid without a walk (its s2 is looked at)
+        if (helper < 0 && !none && I.total - from > kLongWalk) return;
+        const int end = none ? (MODE == Walk::kBisect ? 1 : 0) : I.total;
+        const int b = walk_item(A, I, from + (int64_t)max(helper, 0) * 256, end, false,
+                                helper < 0 ? 256 : (int64_t)kHelpers * 256, helper < 0 ? nullptr : &A.wide_bad[id], R,
+                                turn, tests);
+        if (threadIdx.x != 0) continue;
+        if (none) {
+            A.m.out[id] = 0;
+            if (A.m.checked) A.m.checked[id] = b == 0 ? 1 : 0;
+        } else if (helper < 0) {
+            I.result(A, b);
+        } else {
+            finish_long(A, I, b, &A.wide_bad[id], &A.wide_ticket[id], kHelpers);
+        }
+    }
+}
+
+// More edges (kSequence) or lists: a wave walks the first 64 positions of each.
+template <Walk MODE>
 __global__ void __launch_bounds__(256, 4) grid_first_kernel(GridWalkArgs A)
 {
-    __shared__ int bad;
     __shared__ WaveTests tests[4];
     clear_next(A);
-    const int64_t id = WIDE ? blockIdx.x : (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t id = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (id >= A.m.n) return;
     constexpr int from = MODE == Walk::kSequence ? 1 : 0;
-    const bool writer = WIDE ? threadIdx.x == 0 : lane_id() == 0;
     Item<MODE> I;
     if (MODE == Walk::kList) {
         I.list(A, id);
     } else {
         I.edge(A.m, id);
     }
-    const int slot = (int)id;
-    int done = I.total;
-    if (WIDE ? I.total - from > kLongWalk : true) done = min(I.total, from + (WIDE ? 256 : 64));
-    if (I.nd_too_many()) done = 1; // its s2 alone
-    const int b = walk_item(A, I, I.nd_too_many() && MODE == Walk::kSequence ? done : from, done, WIDE, &bad, tests);
-    if (!writer) return;
+    const int slot = (int)id, done = I.nd_too_many() ? 0 : min(I.total, from + 64);
+    const int b = wave_walk(A, I, from, done, tests);
+    if (lane_id() != 0) return;
+    bool left = false;
     if (I.nd_too_many()) { // reported invalid without a walk
         A.m.out[id] = 0;
-        if (A.m.checked) A.m.checked[id] = b == 0 ? 1 : 0;
-        A.rest[slot] = 0;
-        return;
-    }
-    if (b != INT_MAX || done == I.total) {
+    } else if (b != INT_MAX || done == I.total) {
         I.result(A, b);
-        if (!WIDE) A.rest[slot] = 0;
     } else {
         if (MODE != Walk::kList) keep_edge(A, I, slot);
-        leave_rest(A, slot, I.total, done);
+        left = I.total - done <= kLongWalk;
+        if (!left) list_long(A, slot);
     }
+    A.rest[slot] = left;
 }
 
-// What the first kernel left of `items` slots (-1: of the survivors, when there
-// were more than blocks): a block per item from position `from` on; then all
-// blocks together walk the long ones, and the last to finish one writes its
-// result.
+// What the first kernel left: a block per item; then all blocks together the
+// long ones.
 template <Walk MODE>
-__global__ void __launch_bounds__(256, 4) grid_rest_kernel(GridWalkArgs A, int from, int64_t items)
+__global__ void __launch_bounds__(256, 4) grid_rest_kernel(GridWalkArgs A)
 {
-    __shared__ int bad;
+    __shared__ Rounds R;
     __shared__ WaveTests tests[4];
+    constexpr int from = (MODE == Walk::kSequence ? 1 : 0) + 64;
     const int n_long = A.counts[1];
-    int64_t n = items;
-    if (items < 0) {
-        n = A.counts[0];
-        if (n <= (int64_t)gridDim.x) n = 0;
-    }
+    const int64_t n = A.m.n;
     Item<MODE> I;
     const int lane = lane_id();
     // the block's slots are blockIdx.x + i gridDim.x (every wave reads the same
     // 64 flags at a time), then all blocks' long items
     int64_t i0 = -64;
     uint64_t open = 0;
-    int l = -1;
+    int turn = 0, l = -1;
     for (;;) {
         int slot = -1;
         if (l < 0) {
@@ -423,28 +537,12 @@ __global__ void __launch_bounds__(256, 4) grid_rest_kernel(GridWalkArgs A, int f
         }
         if (MODE == Walk::kList) I.list(A, slot);
         else I.survivor(A.m, slot);
-        // a block's positions at a time: all of a short item's, every gridDim-th
-        // of a long one's until an earlier position is known invalid
-        int64_t at = from + (is_long ? (int64_t)blockIdx.x * blockDim.x : 0);
-        int b = INT_MAX;
-        for (; at < I.total; at += (int64_t)gridDim.x * blockDim.x) {
-            if (is_long && __hip_atomic_load(&A.long_bad[l], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < at) break;
-            b = walk_item(A, I, (int)at, is_long ? (int)min(at + blockDim.x, (int64_t)I.total) : I.total, true, &bad,
-                          tests);
-            if (!is_long || b != INT_MAX) break;
-        }
-        if (!is_long) {
-            if (threadIdx.x == 0) I.result(A, b);
-            continue;
-        }
-        if (threadIdx.x == 0) {
-            if (b != INT_MAX) atomicMin(&A.long_bad[l], b);
-            __threadfence(); // the minimum is made before the ticket is taken
-            if (atomicAdd(&A.ticket[l], 1) == (int)gridDim.x - 1) {
-                __threadfence();
-                I.result(A, __hip_atomic_load(&A.long_bad[l], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-            }
-        }
+        const int b = walk_item(A, I, from + (is_long ? (int64_t)blockIdx.x * 256 : 0), I.total, false,
+                                is_long ? (int64_t)gridDim.x * 256 : 256, is_long ? &A.long_bad[l] : nullptr, R, turn,
+                                tests);
+        if (threadIdx.x != 0) continue;
+        if (is_long) finish_long(A, I, b, &A.long_bad[l], &A.ticket[l], gridDim.x);
+        else I.result(A, b);
     }
 }
 
@@ -459,11 +557,6 @@ static unsigned grid_of(int64_t units, int64_t per)
 // States (or edges) from which on one lane per state beats eight: 131,072 fill
 // every SIMD with two waves of 64 states; below, eight lanes have more in flight.
 constexpr int64_t kLaneStates = 131072;
-// Edges or lists up to which a block each walks them in one launch: 1,024
-// blocks of four waves are one wave per SIMD, so the speculative positions of
-// edges that fail at once cost no time; more edges go through the s2 pass.
-constexpr int64_t kWideItems = 1024;
-
 template <typename T>
 void launch_grid_validate(const GridView &g, const T *q, int64_t n, uint8_t *out, hipStream_t s)
 {
@@ -493,22 +586,26 @@ static GridWalkArgs walk_args(const GridView &g, const MotionArgs &m, const Grid
     A.long_slot = w.long_slot;
     A.long_bad = w.long_bad;
     A.ticket = w.ticket;
+    A.wide_bad = w.wide;
+    A.wide_ticket = w.wide + kWideItems;
     A.counts = w.counts;
     A.next = w.next;
     return A;
 }
 
 template <Walk MODE>
-static void launch_first_and_rest(const GridWalkArgs &A, hipStream_t s)
+static void launch_wide(const GridWalkArgs &A, hipStream_t s)
 {
-    constexpr int from = MODE == Walk::kSequence ? 1 : 0;
-    const int64_t n = A.m.n;
-    if (n <= kWideItems)
-        hipLaunchKernelGGL((grid_first_kernel<MODE, true>), dim3((unsigned)n), dim3(256), 0, s, A);
-    else
-        hipLaunchKernelGGL((grid_first_kernel<MODE, false>), dim3(grid_of(n, 4)), dim3(256), 0, s, A);
-    hipLaunchKernelGGL((grid_rest_kernel<MODE>), dim3((unsigned)num_cus() * 4), dim3(256), 0, s, A,
-                       n <= kWideItems ? from + 256 : from + 64, n <= kWideItems ? (int64_t)0 : n);
+    hipLaunchKernelGGL((grid_wide_kernel<MODE>), dim3((unsigned)A.m.n + kHelpers), dim3(256), 0, s, A);
+    OA_HIP(hipGetLastError());
+}
+
+template <Walk MODE>
+static void launch_items(const GridWalkArgs &A, hipStream_t s)
+{
+    if (A.m.n <= kWideItems) return launch_wide<MODE>(A, s);
+    hipLaunchKernelGGL((grid_first_kernel<MODE>), dim3(grid_of(A.m.n, 4)), dim3(256), 0, s, A);
+    hipLaunchKernelGGL((grid_rest_kernel<MODE>), dim3((unsigned)num_cus() * 4), dim3(256), 0, s, A);
     OA_HIP(hipGetLastError());
 }
 
@@ -518,7 +615,7 @@ void launch_grid_motions(const GridView &g, const MotionArgs &m, const GridScrat
     const GridWalkArgs A = walk_args(g, m, w);
     if (m.n <= kWideItems) {
         ProfScope ps("motion_walk", s);
-        launch_first_and_rest<Walk::kBisect>(A, s);
+        launch_wide<Walk::kBisect>(A, s);
         return;
     }
     {
@@ -529,10 +626,7 @@ void launch_grid_motions(const GridView &g, const MotionArgs &m, const GridScrat
             hipLaunchKernelGGL(grid_endpoint8_kernel, dim3(grid_of(m.n, 32)), dim3(256), 0, s, A);
     }
     ProfScope ps("motion_chunk", s);
-    const unsigned blocks = (unsigned)num_cus() * 8;
-    hipLaunchKernelGGL(grid_survivors_kernel, dim3(blocks), dim3(256), 0, s, A);
-    hipLaunchKernelGGL((grid_rest_kernel<Walk::kBisect>), dim3(blocks), dim3(256), 0, s, A, 65,
-                       (int64_t)-1);
+    hipLaunchKernelGGL(grid_survivors_kernel, dim3((unsigned)num_cus() * 8), dim3(256), 0, s, A);
     OA_HIP(hipGetLastError());
 }
 
@@ -543,7 +637,7 @@ void launch_grid_last_valid(const GridView &g, const MotionArgs &m, double *last
     GridWalkArgs A = walk_args(g, m, w);
     A.last_t = last_t;
     ProfScope ps("motion_last_valid", s);
-    launch_first_and_rest<Walk::kSequence>(A, s);
+    launch_items<Walk::kSequence>(A, s);
 }
 
 void launch_grid_state_lists(const GridView &g, const double *q_soa, int64_t n_states, const int64_t *offsets,
@@ -560,7 +654,7 @@ void launch_grid_state_lists(const GridView &g, const double *q_soa, int64_t n_s
     A.n_states = n_states;
     A.offsets = offsets;
     ProfScope ps("state_lists", s);
-    launch_first_and_rest<Walk::kList>(A, s);
+    launch_items<Walk::kList>(A, s);
 }
 
 } // namespace ompl_amd

@@ -15,12 +15,13 @@
 #include <mutex>
 #include <vector>
 
+#include "checker.hpp"
 #include "runtime.hpp"
 
 namespace ompl_amd {
 
 constexpr int64_t kNoAllocMaxEdges = 65536;
-constexpr size_t kNoAllocCounterBytes = 256; // 64 int32 counters
+constexpr size_t kNoAllocCounterBytes = kWorkspaceCounters * sizeof(int32_t);
 constexpr size_t kNoAllocListBytes = (size_t)kNoAllocMaxEdges * sizeof(int32_t);
 constexpr size_t kNoAllocEndpointBytes = (size_t)kNoAllocMaxEdges * 14 * sizeof(double);
 // counters | list | first_bad | surv_nd | surv_ab | longs  (every part 256-byte aligned)

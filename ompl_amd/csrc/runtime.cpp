@@ -132,6 +132,7 @@ GridScratch grid_scratch(Workspace &w)
                   w.longs + cap,
                   w.longs + 2 * cap,
                   w.surv_ab,
+                  w.counters + 64,
                   sets + 4 * w.grid_parity,
                   sets + 4 * (1 - w.grid_parity)};
     w.grid_parity ^= 1;
@@ -203,8 +204,8 @@ Workspace &workspace(hipStream_t s, size_t list_entries, std::unique_lock<std::m
         Workspace *&slot = g_ws[s];
         if (!slot) {
             slot = new Workspace();
-            OA_HIP(hipMalloc(&slot->counters, 64 * sizeof(int32_t)));
-            OA_HIP(hipMemset(slot->counters, 0, 64 * sizeof(int32_t)));
+            OA_HIP(hipMalloc(&slot->counters, kWorkspaceCounters * sizeof(int32_t)));
+            OA_HIP(hipMemset(slot->counters, 0, kWorkspaceCounters * sizeof(int32_t)));
             OA_HIP(hipDeviceSynchronize());
         }
         w = slot;

@@ -46,7 +46,8 @@ struct Workspace {
     // its results kernel clears that set, or (no results kernel) its phase-1
     // walk clears the other set and the next batch uses that one.
     // The checks over the cell grid: two sets of two at [16..17] and
-    // [20..21], used in turn by grid_parity, each cleared by the batch before.
+    // [20..21], used in turn by grid_parity, each cleared by the batch before;
+    // from [64] on a word and a ticket per item of a one-launch batch.
     int32_t *counters = nullptr;
     int parity = 0;
     int grid_parity = 0;
