@@ -138,7 +138,7 @@ def concurrent_streams(oa, torch, env, A, B, lvs, want, candidates=12, k=24):
 
 
 def served_stream(oa, n_requests, qps, n_envs, plain_workers, seed=8, max_iters=2000, log_path=None,
-                  check_parts=0, profile_slices=False, run_plain=True, block_threads=0, slice_us=0, prm_every=4,
+                  profile_slices=False, run_plain=True, block_threads=0, slice_us=0, prm_every=4,
                   prm_samples=2048):
     """Poisson stream of planning requests over seeded environments (16-1024
     obstacles, log-uniform, half spheres / half boxes): RRT-Connect, and every
@@ -186,7 +186,7 @@ def served_stream(oa, n_requests, qps, n_envs, plain_workers, seed=8, max_iters=
     if profile_slices:
         oa.profile.reset()
         oa.profile.enable(True)
-    srv = serve.Server(hbm_budget_bytes=4 << 30, max_active=1024, max_nodes=4096, check_obstacle_parts=check_parts,
+    srv = serve.Server(hbm_budget_bytes=4 << 30, max_active=1024, max_nodes=4096,
                        block_threads=block_threads, slice_us=slice_us)
     ids = [None] * n_requests
     t0 = time.perf_counter()
@@ -217,7 +217,7 @@ def served_stream(oa, n_requests, qps, n_envs, plain_workers, seed=8, max_iters=
               "edge_checks_per_s": checks_s / span_s,
               "run_ms": pct([r.run_ms for r in res_s]), "queued_ms": pct([r.queued_ms for r in res_s]),
               "device_us_per_step": {k: v / max(stats["steps"], 1) for k, v in phases.items()},
-              "config": {"check_obstacle_parts": check_parts, "block_threads": block_threads or 512,
+              "config": {"block_threads": block_threads or 512,
                          "slice_us": slice_us or 200}}
     if profile_slices:
         served["gpu_us_per_slice"] = slice_us_gpu
@@ -328,39 +328,22 @@ def prm_batch(oa, n_samples, cpu_samples, cpu_threads, run_cpu):
 TRAFFIC_RECORD = ROOT / "profiles" / "motion_batch_16384_edges_256_obstacles.hbm_traffic.json"
 
 
-def hbm_traffic(kernel: str, tuning: dict):
+# The kernels each timed scope holds at this batch's size.
+SCOPE_KERNELS = {"motion_endpoint": ["grid_endpoint8_kernel"], "motion_chunk": ["grid_survivors_kernel"],
+                 "motion_fused": ["grid_endpoint8_kernel", "grid_survivors_kernel"]}
+
+
+def hbm_traffic(kernel: str):
     """HBM bytes per launch of the dominant kernel from the committed rocprofv3
-    FETCH_SIZE / WRITE_SIZE records, when one was taken with this launch
-    shape; otherwise None."""
+    FETCH_SIZE / WRITE_SIZE record of this batch; None where it has none."""
     try:
-        rec = json.loads(TRAFFIC_RECORD.read_text())
-    except (OSError, ValueError):
+        rec = json.loads(TRAFFIC_RECORD.read_text())["bytes_per_dispatch"]
+    except (OSError, ValueError, KeyError):
         return None, None
-    keys = ("validity_lanes_per_state", "validity_obstacle_parts", "motion_lanes_per_state",
-            "motion_obstacle_parts", "motion_waves_per_cu", "motion_strategy", "validity_shared_fk")
-    # the kernels that run for this tuning (shared FK exists for (8, parts > 1) only)
-    lw, ow, le, oe = (tuning["motion_lanes_per_state"], tuning["motion_obstacle_parts"],
-                      tuning["validity_lanes_per_state"], tuning["validity_obstacle_parts"])
-    shared = "true" if tuning["motion_strategy"] == 4 and lw == 8 and ow > 1 else "false"
-    if kernel == "motion_chunk":  # both phases (the timed batches ask for no checked counts: no results kernel)
-        names = [f"motion_chunk_kernel<{lw}, {ow}, false, {shared}, {ph}>" for ph in (1, 2)]
-    elif kernel == "motion_endpoint":
-        es = tuning.get("validity_shared_fk") and le == 8 and oe > 1
-        names = [f"{'motion_endpoint_shared_kernel' if es else 'motion_endpoint_kernel'}<{le}, {oe}>"]
-    else:
-        return None, None
-    # a record taken with this tuning first; else any record of the same kernels
-    # (their sweep dispatches), noted as such
-    for same in (True, False):
-        for r in rec["records"]:
-            if same and any(r["tuning"].get(k) != tuning.get(k) for k in keys):
-                continue
-            found = {n: (k, v) for n in names for k, v in r["bytes_per_dispatch"].items() if n + "(" in k}
-            if len(found) == len(names):
-                src = " + ".join(k for k, _ in found.values())
-                note = "" if same else ", recorded under another tuning"
-                return int(sum(v for _, v in found.values())), f"{TRAFFIC_RECORD.name} ({src}{note})"
-    return None, f"{TRAFFIC_RECORD.name}: no record for this launch shape"
+    found = [(k, v) for n in SCOPE_KERNELS.get(kernel, ()) for k, v in rec.items() if n + "(" in k]
+    if not found or len(found) != len(SCOPE_KERNELS[kernel]):
+        return None, f"{TRAFFIC_RECORD.name}: no record of these kernels"
+    return int(sum(v for _, v in found)), f"{TRAFFIC_RECORD.name} ({' + '.join(k for k, _ in found)})"
 
 
 def timed(fn, reps, warm=2):
@@ -600,18 +583,9 @@ def validity_row(oa, rows, oracle_py, cpu_threads, roof, timed):
     q = oa.workload.configs(1, 65536)
     qd = torch.from_numpy(q.T.astype(np.float32).copy()).cuda()
     out = torch.empty(65536, dtype=torch.uint8, device="cuda")
-    shapes = {}
-    saved = oa.get_tuning()
-    for lps, ops, shared in ((8, 1, 0), (8, 2, 0), (8, 8, 0), (8, 2, 1), (8, 4, 1), (8, 8, 1), (7, 1, 0), (7, 2, 0), (7, 4, 0), (7, 9, 0), (1, 1, 0)):
-        oa.set_tuning(validity_lanes_per_state=lps, validity_obstacle_parts=ops, validity_shared_fk=shared)
-        shapes[f"{lps}x{ops}{'-shared' if shared else ''}"] = timed(lambda: oa.validate_states(env, qd, out=out), 50)
-    best = min(shapes, key=shapes.get)
-    ms = shapes[best]
-    oa.set_tuning(**saved)
-    oa.validate_states(env, qd, out=out)
+    ms = timed(lambda: oa.validate_states(env, qd, out=out), 50)
     w = oa.validity_work(env, qd)
-    row = {"states": 65536, "obstacles": 64, "ms": ms, "states_per_s": 65536 / (ms * 1e-3), "shape": best,
-           "ms_by_shape": shapes, "valid_fraction": float(out.float().mean().item()),
+    row = {"states": 65536, "obstacles": 64, "ms": ms, "states_per_s": 65536 / (ms * 1e-3), "valid_fraction": float(out.float().mean().item()),
            "roofline": roof(oa.work_flops(w), ms)}
     if oracle_py is not None:
         oenv = oracle_py.OracleEnv(s, b)
@@ -855,9 +829,7 @@ def main(argv=None):
 
     # ---- the streams the timed steps are issued on: ones whose batches overlap
     picked, pair_checks = concurrent_streams(oa, torch, env, A, B, lvs, max(1, args.streams))
-    # ---- the launch shape for batches on those streams (the one-batch-at-a-time
-    #      shape above keeps more persistent walk waves than is best when the
-    #      streams' batches share the device)
+    # ---- the time of batches on those streams
     t_one = t
     streams_us = None
     if not args.tuning and len(picked) > 1:
@@ -908,37 +880,6 @@ def main(argv=None):
         oa.check_motions(env, A, B, lvs, out=out)
         torch.cuda.synchronize()
         step_ms.append((time.perf_counter() - s0) * 1e3)
-
-    # ---- a few fixed launch shapes beside the tuned one (per-kernel times)
-    sweep = {}
-    for name, kw in (("s3_e8x8_w8x8", dict(motion_strategy=3, validity_obstacle_parts=8, motion_obstacle_parts=8)),
-                     ("s3_e8x8sh_w8x4", dict(motion_strategy=3, validity_obstacle_parts=8, motion_obstacle_parts=4,
-                                             validity_shared_fk=1)),
-                     ("s4_e8x8_w8x8", dict(motion_strategy=4, validity_obstacle_parts=8, motion_obstacle_parts=8)),
-                     ("s4_e8x8sh_w8x2", dict(motion_strategy=4, validity_obstacle_parts=8, motion_obstacle_parts=2,
-                                             validity_shared_fk=1)),
-                     ("s3_e7x9_w7x9", dict(motion_strategy=3, validity_lanes_per_state=7, validity_obstacle_parts=9,
-                                           motion_lanes_per_state=7, motion_obstacle_parts=9)),
-                     ("s3_e8x8_w7x9", dict(motion_strategy=3, validity_obstacle_parts=8, motion_lanes_per_state=7,
-                                           motion_obstacle_parts=9)),
-                     ("s3_e7x4_w7x9", dict(motion_strategy=3, validity_lanes_per_state=7, validity_obstacle_parts=4,
-                                           motion_lanes_per_state=7, motion_obstacle_parts=9)),
-                     ("s3_e7x2_w7x9", dict(motion_strategy=3, validity_lanes_per_state=7, validity_obstacle_parts=2,
-                                           motion_lanes_per_state=7, motion_obstacle_parts=9))):
-        oa.set_tuning(**{**t, "validity_lanes_per_state": 8, "motion_lanes_per_state": 8, "validity_shared_fk": 0,
-                         **kw})
-        oa.profile.reset()
-        oa.profile.enable(True)
-        ms = timed(lambda: oa.check_motions(env, A, B, lvs, out=out), 30)
-        oa.profile.enable(False)
-        per = {}
-        for kname in ("motion_endpoint", "motion_chunk"):
-            n, kms = oa.profile.query(kname)
-            if n:
-                per[kname] = 1e3 * kms / n
-        oa.profile.reset()
-        sweep[name] = {"ms_per_step": ms, "kernel_us": per}
-    oa.set_tuning(**t)
 
     # ---- the same batch replayed from a HIP graph (launch cost removed)
     g = oa.MotionGraph(env, A, B, lvs)
@@ -1030,21 +971,19 @@ def main(argv=None):
              "motion_chunk": flops_step - flops_end}
     if t["motion_strategy"] == 0:
         share["motion_walk"] = flops_step
-    # the dominant kernel is the one with the most time per step; the chunk
-    # walk's two launches (one event scope) count as one kernel (its work is
-    # not split by phase)
+    # the dominant kernel is the one with the most time per step
     dom = max(kernels, key=lambda k: kernels[k]["avg_us"])
     dom_flops = share[dom]
     dom_us = kernels[dom]["avg_us"]
     achieved = dom_flops / (dom_us * 1e-6) / 1e12
-    traffic, traffic_src = hbm_traffic(dom, t)
+    traffic, traffic_src = hbm_traffic(dom)
     # the s2 pass's figure beside it
     roof_s2 = None
     if dom != "motion_endpoint" and "motion_endpoint" in kernels:
         a2 = flops_end / (kernels["motion_endpoint"]["avg_us"] * 1e-6) / 1e12
         roof_s2 = {"kernel": "motion_endpoint", "achieved": a2, "frac": a2 / PEAK_FP32_TFLOPS,
                    "kernel_avg_us": kernels["motion_endpoint"]["avg_us"], "algorithmic_flops_per_launch": flops_end,
-                   "traffic": hbm_traffic("motion_endpoint", t)[0]}
+                   "traffic": hbm_traffic("motion_endpoint")[0]}
 
     # the rest (plain path, served stream, PRM, rows) with the one-stream shape
     oa.set_tuning(**t_one)
@@ -1057,7 +996,7 @@ def main(argv=None):
             if kname in k1:
                 a1 = fl / (k1[kname]["avg_us"] * 1e-6) / 1e12
                 roof_one[kname] = {"kernel_avg_us": k1[kname]["avg_us"], "achieved": a1,
-                                   "frac": a1 / PEAK_FP32_TFLOPS, "traffic": hbm_traffic(kname, t_one)[0]}
+                                   "frac": a1 / PEAK_FP32_TFLOPS, "traffic": hbm_traffic(kname)[0]}
 
     # ---- plain one-launch-per-call path on a prefix of the same edges
     P = min(args.plain_edges, N_EDGES)
@@ -1122,10 +1061,10 @@ def main(argv=None):
         # server settings: obstacle partitions of the motion check (0 = by motion length) and workgroup size;
         # HIP events around each slice launch
         stream_res["served_config_sweep"] = {
-            f"parts{parts}_t{threads}": served_stream(oa, args.stream_requests, args.stream_qps, args.stream_envs, 0,
-                                                      check_parts=parts, block_threads=threads, profile_slices=True,
-                                                      run_plain=False, prm_every=0)["served"]
-            for parts, threads in ((0, 512), (1, 512), (2, 512), (4, 512), (9, 512), (0, 1024))}
+            f"t{threads}": served_stream(oa, args.stream_requests, args.stream_qps, args.stream_envs, 0,
+                                         block_threads=threads, profile_slices=True, run_plain=False,
+                                         prm_every=0)["served"]
+            for threads in (512, 1024)}
 
     prm_res = None
     if args.prm_samples > 0:
@@ -1165,7 +1104,6 @@ def main(argv=None):
         "kernels": kernels,
         "valid_fraction": float(valid.mean()),
         "step_latency_ms": {"p50": percentile(step_ms, 50), "p99": percentile(step_ms, 99)},
-        "shape_sweep": sweep,
         "graph": {"ms_per_step": graph_ms, "edge_checks_per_s": N_EDGES / (graph_ms * 1e-3),
                   "step_latency_ms": {"p50": percentile(graph_lat, 50), "p99": percentile(graph_lat, 99)},
                   "same_result": graph_same,
@@ -1188,7 +1126,7 @@ def main(argv=None):
                      "unit": "TFLOP/s", "frac": achieved / PEAK_FP32_TFLOPS, "traffic": traffic,
                      "traffic_source": traffic_src,
                      "kernel": dom, "kernel_avg_us": dom_us, "algorithmic_flops_per_launch": dom_flops,
-                     "dispatches": 2 if dom == "motion_chunk" else 1,
+                     "dispatches": len(SCOPE_KERNELS.get(dom, (dom,))),
                      "compute": "FP32 VALU (compute-bound; MI355X FP32 vector peak = FP32 matrix peak)"},
         "roofline_s2_pass": roof_s2,
         "roofline_one_stream_shape": roof_one,

@@ -185,74 +185,46 @@ int ompl_amd_motion_graph_create_group(ompl_amd_env env, int n_batches, const do
 int ompl_amd_motion_graph_launch(ompl_amd_motion_graph graph, void *stream);
 int ompl_amd_motion_graph_destroy(ompl_amd_motion_graph graph);
 
-/* Launch-shape knobs used by the batched kernels (set by the autotuner).
- * A state is checked by lanes_per_state x obstacle_parts lanes: the first
- * splits the arm's 28 spheres, the second the obstacle list.  Built shapes
- * (lanes, parts): (1,1) (2,1) (4,1) (8,1) (8,2) (8,4) (8,8), and (7,9), the
- * link layout: one state per wave, each of 7 lanes holds one link's four
- * spheres and tests the link's bounding sphere against an obstacle before
- * the exact sphere tests (same results; environments whose staging would
- * exceed 64 KiB of LDS with the extra sphere radii run as (8,8)); block in
- * {64,128,256,512,1024}. */
+/* Launch shapes.  The batched checks look their obstacles up in the
+ * environment's cell grid and choose lanes and blocks by the batch's size, so
+ * shapes change neither results nor kernels; they are checked, kept and
+ * returned.  Shapes accepted (lanes, parts): (1,1) (2,1) (4,1) (8,1) (8,2)
+ * (8,4) (8,8) (7,1) (7,2) (7,4) (7,9); blocks: powers of two in [64, 1024]. */
 typedef struct {
-    int validity_lanes_per_state; /* validity and s2 (endpoint) checks */
+    int validity_lanes_per_state;
     int validity_obstacle_parts;
     int validity_block;
-    int motion_lanes_per_state;   /* interior (bisection) checks */
+    int motion_lanes_per_state;
     int motion_obstacle_parts;
     int motion_block;
-    int motion_waves_per_cu;      /* persistent kernels' occupancy */
-    int motion_strategy;          /* 0: one wave walks each edge from s2;
-                                     1: s2 pass, then a persistent queue walks
-                                        each survivor with one wave;
-                                     2: fused: each wave checks s2 of its edges
-                                        and walks its own survivors (1 launch);
-                                     3: s2 pass, then the survivors' bisection
-                                        chunks run in parallel across the GPU,
-                                        chunk-major, with early exit;
-                                     4: as 3, the walk with each position's
-                                        FK computed once per wave and shared
-                                        across the obstacle partitions (shapes
-                                        with parts > 1; chunks of 64/lanes
-                                        positions) */
-    int validity_shared_fk;       /* 1: batched validity and the s2 pass of
-                                     the motion strategies compute each
-                                     state's FK once per wave and share it
-                                     across the obstacle partitions */
+    int motion_waves_per_cu;      /* 1 to 32 */
+    int motion_strategy;          /* 0 to 4; 2 is timed as one launch ("motion_fused",
+                                     for pairs of validity (8,1) (8,2) (8,4) and motion
+                                     (1,1) (8,1) (8,8) shapes), the others by kernel */
+    int validity_shared_fk;       /* 0 or 1 */
 } ompl_amd_tuning;
 int ompl_amd_get_tuning(ompl_amd_tuning *t);
 int ompl_amd_set_tuning(const ompl_amd_tuning *t);
-/* Autotuner: times every candidate launch shape (strategy x lanes x block x
- * occupancy) on the given device-resident batch with HIP events, installs the
- * fastest as the current tuning and returns it with its time per batch.  No
- * counterpart in the reference. */
+/* Times `reps` batches of the given device-resident edges with HIP events,
+ * installs the shapes the library starts with as the current tuning and returns
+ * them with the time per batch.  No counterpart in the reference. */
 int ompl_amd_autotune_motions(ompl_amd_env env, const double *a_soa_dev, const double *b_soa_dev, int64_t n,
                               double longest_valid_segment, unsigned factor, int reps, ompl_amd_tuning *best,
                               double *best_us);
-/* Autotuner for batches issued round-robin on several streams (1 to 16 HIP
- * streams whose batches overlap, e.g. one per planner thread): the shape that
- * is fastest for one batch at a time keeps more persistent walk waves than is
- * best when the streams' batches share the device.  Each candidate (s2 pass
- * shapes (7,1) (7,2) (7,4) (7,9) (8,4) (8,8) x walk shapes (7,2) (7,4) (7,9)
- * (8,8) x 2/4/8/16 walk waves per CU, the chunk-parallel walk) runs `steps`
- * batches round-robin on the streams, timed by HIP events on streams[0]; the
- * three fastest run again over 2 x steps and the fastest is installed as the
- * current tuning and returned with its time per batch.  Fields outside the
- * grid keep the current tuning's values.  Refused for an environment with its
- * own shapes (ompl_amd_env_set_tuning), which would ignore the candidates.
- * No counterpart in the reference. */
+/* The same for batches issued round-robin on several streams (1 to 16 HIP
+ * streams whose batches overlap, e.g. one per planner thread): `steps` batches,
+ * timed by HIP events on streams[0].  Installs eight-lane shapes; block sizes
+ * keep the current tuning's values.  Refused for an environment with its own
+ * shapes (ompl_amd_env_set_tuning).  No counterpart in the reference. */
 int ompl_amd_autotune_motions_streams(ompl_amd_env env, const double *a_soa_dev, const double *b_soa_dev, int64_t n,
                                       double longest_valid_segment, unsigned factor, void *const *streams,
                                       int n_streams, int steps, ompl_amd_tuning *best, double *best_us);
 /* Launch shapes of one environment: the batched checks on `env` (validity,
  * motions, last-valid motions, captured motion graphs at capture, the
  * no-allocation motion check) use `t` instead of the library's current tuning;
- * t == NULL makes the environment follow the library's tuning again.  The
- * fastest shape depends on the obstacle count (a dense scene wants many
- * obstacle partitions per state, a sparse one a single partition and more
- * waves per CU).  ompl_amd_env_get_tuning returns the shapes in force for
- * `env` and sets *own to 1 when they are the environment's own.  No
- * counterpart in the reference. */
+ * t == NULL makes the environment follow the library's tuning again.
+ * ompl_amd_env_get_tuning returns the shapes in force for `env` and sets *own to
+ * 1 when they are the environment's own.  No counterpart in the reference. */
 int ompl_amd_env_set_tuning(ompl_amd_env env, const ompl_amd_tuning *t);
 int ompl_amd_env_get_tuning(ompl_amd_env env, ompl_amd_tuning *t, int *own);
 

@@ -123,8 +123,8 @@ def work_flops(w: dict) -> int:
 
 
 def autotune_motions(env: "Env", a_soa, b_soa, lvs: float, factor: int = 1, reps: int = 20):
-    """Runs the library's launch-shape autotuner on a device-resident batch and
-    installs the fastest shape; returns (tuning dict, microseconds per batch)."""
+    """Times a device-resident batch and installs the library's own launch
+    shapes; returns (tuning dict, microseconds per batch)."""
     t = Tuning()
     us = C.c_double()
     call("ompl_amd_autotune_motions", env.handle, _ptr(a_soa), _ptr(b_soa), a_soa.shape[1], float(lvs),
@@ -133,18 +133,10 @@ def autotune_motions(env: "Env", a_soa, b_soa, lvs: float, factor: int = 1, reps
 
 
 def autotune_motions_streams(env: "Env", a_soa, b_soa, lvs: float, streams, factor: int = 1, steps: int = 200):
-    """Runs the library's autotuner for batches issued round-robin on
-    `streams` (torch streams whose batches overlap) and installs the fastest
-    shape; returns (tuning dict, microseconds per batch).
-
-    The shape that is fastest for one batch at a time is not the fastest when
-    batches of several streams share the device: fewer persistent walk waves
-    leave compute units to the other streams' s2 passes.  The library times
-    each shape of its grid (s2 pass x walk shape x walk waves per CU, the
-    chunk-parallel walk) over `steps` batches on the streams, and the three
-    fastest again over 2 x `steps`.  Results do not depend on the shape.  An
-    environment with its own shapes is refused (they would take the place of
-    every candidate)."""
+    """Times batches issued round-robin on `streams` (torch streams whose
+    batches overlap) and installs eight-lane launch shapes; returns (tuning dict,
+    microseconds per batch).  Neither results nor kernels depend on the shapes.
+    An environment with its own shapes is refused."""
     streams = list(streams)
     handles = (C.c_void_p * max(1, len(streams)))(*[s.cuda_stream for s in streams])
     t = Tuning()

@@ -20,13 +20,12 @@ Env &env_of(ompl_amd_env e)
 // Word of the thread's pinned slot that an environment's build reports in.
 constexpr int kEnvBaseAt = 520;
 
-// Staging order of an obstacle list: increasing distance from the arm's base
-// (the world origin) to the obstacle's nearest point, ties in the caller's
-// order.  Every check result is "any obstacle hit", so the order leaves results
-// unchanged; links near the base sweep the least volume, so the obstacles
-// nearest to it are hit by the most configurations, and the checkers, which
-// leave a state's obstacle loop at the first pass with a hit, resolve most
-// invalid states in their first passes.
+// Order of an obstacle list in the grid's table: increasing distance from the
+// arm's base (the world origin) to the obstacle's nearest point, ties in the
+// caller's order.  Every check result is "any obstacle hit", so the order leaves
+// results unchanged; links near the base sweep the least volume, so the
+// obstacles nearest to it are hit by the most configurations, and a state tested
+// against all of them is done sooner.
 std::vector<int> nearest_first(int n, const std::function<double(int)> &gap)
 {
     std::vector<double> key(n);
@@ -52,7 +51,6 @@ void ompl_amd::check_motions_tuned(const Tuning &t, const Env &env, const double
     OA_REQUIRE(lvs > 0.0 && factor >= 1, OMPL_AMD_ERR_ARG, "longest valid segment must be > 0 and factor >= 1");
     OA_REQUIRE(n < (int64_t)1 << 31, OMPL_AMD_ERR_ARG, "at most 2^31-1 edges per call");
     MotionArgs A{};
-    A.env = env.view();
     A.a = a;
     A.b = b;
     A.n = n;
@@ -60,58 +58,9 @@ void ompl_amd::check_motions_tuned(const Tuning &t, const Env &env, const double
     A.factor = factor;
     A.out = out;
     A.checked = checked;
-    const bool exact = checked != nullptr;
-    const int LE = t.validity_lanes_per_state, OE = t.validity_obstacle_parts;
-    const int LW = t.motion_lanes_per_state, OW = t.motion_obstacle_parts;
-    const int64_t persistent_waves = (int64_t)num_cus() * t.motion_waves_per_cu;
-    if (own_validity_shape(t) && own_walk_shape(t)) {
-        std::unique_lock<std::mutex> lk; // held until this batch's launches are enqueued
-        Workspace &w = own ? *own : workspace(s, (size_t)n, lk);
-        launch_grid_motions(env.grid, A, grid_scratch(w), s);
-    } else if (t.motion_strategy == 3 || t.motion_strategy == 4) {
-        // Strategy 4 walks chunks with each position's FK computed once per
-        // wave and shared across the obstacle partitions; the s2 pass shares
-        // its FK when validity_shared_fk is set.  The survivors' booleans are
-        // written by the s2 pass (1) and the walk (0 at an invalid position);
-        // a results kernel runs after the walk when checked counts are asked
-        // for, and clears the batch's counter set; otherwise phase 1 of the
-        // walk clears the other set, which the next batch on this workspace
-        // uses (a captured batch is recorded once per set, and its replays
-        // alternate between the two).
-        const bool shared = t.motion_strategy == 4;
-        const bool eshared = t.validity_shared_fk != 0;
-        std::unique_lock<std::mutex> lk; // held until this batch's launches are enqueued
-        Workspace &w = own ? *own : workspace(s, (size_t)n, lk);
-        const bool results = exact;
-        int32_t *cur = w.counters + 8 + 2 * w.parity, *other = w.counters + 8 + 2 * (1 - w.parity);
-        A.list = w.list;
-        A.list_count = cur;
-        A.max_m = cur + 1;
-        A.reset_next = results ? nullptr : other;
-        A.first_bad = w.first_bad;
-        A.surv_nd = w.surv_nd;
-        A.surv_ab = w.surv_ab;
-        A.start = 1;
-        launch_motion_endpoint(A, LE, OE, t.validity_block, s, eshared);
-        launch_motion_chunks(A, exact, LW, OW, t.motion_block, persistent_waves, s, shared, results);
-        if (!results) w.parity ^= 1;
-    } else if (t.motion_strategy == 2) {
-        A.start = 1;
-        launch_motion_fused(A, exact, LE, OE, LW, OW, t.motion_block, s);
-    } else if (t.motion_strategy == 1) {
-        std::unique_lock<std::mutex> lk; // held until this batch's launches are enqueued
-        Workspace &w = own ? *own : workspace(s, (size_t)n, lk);
-        A.list = w.list;
-        A.list_count = w.counters;
-        A.queue = w.counters + 1;
-        A.start = 1;
-        launch_zero(w.counters, 4, s);
-        launch_motion_endpoint(A, LE, OE, t.validity_block, s, t.validity_shared_fk != 0);
-        launch_motion_walk(A, exact, LW, OW, t.motion_block, persistent_waves, s);
-    } else {
-        A.start = 0;
-        launch_motion_walk(A, exact, LW, OW, t.motion_block, n, s);
-    }
+    std::unique_lock<std::mutex> lk; // held until this batch's launches are enqueued
+    Workspace &w = own ? *own : workspace(s, (size_t)n, lk);
+    launch_grid_motions(env.grid, A, grid_scratch(w), t.motion_strategy == 2, s);
 }
 
 namespace {
@@ -120,33 +69,6 @@ void check_motions(const ompl_amd_env_s &e, const double *a, const double *b, in
                    uint8_t *out, int32_t *checked, hipStream_t s)
 {
     check_motions_tuned(tuning_for(e), e.env, a, b, n, lvs, factor, out, checked, s);
-}
-
-// Candidate launch shapes of the motion autotuner.
-std::vector<Tuning> motion_candidates()
-{
-    std::vector<Tuning> c;
-    const int shapes[][2] = {{8, 1}, {8, 2}, {8, 4}, {8, 8}, {7, 1}, {7, 2}, {7, 4}, {7, 9}, {4, 1}, {1, 1}};
-    for (const auto &e : shapes)
-        for (const auto &w : shapes) {
-            const int LE = e[0], OE = e[1], LW = w[0], OW = w[1];
-            // chunk-parallel walk of the survivors; shared-FK forms of the s2
-            // pass (validity_shared_fk) and of the walk (strategy 4)
-            // (shared FK exists for the sphere-slot shapes (8, parts > 1) only)
-            const int es_max = (LE == 8 && OE > 1) ? 1 : 0;
-            for (int wpc : {8, 16, 32})
-                for (int es = 0; es <= es_max; ++es) {
-                    c.push_back(Tuning{LE, OE, 256, LW, OW, 256, wpc, 3, es});
-                    if (LW == 8 && OW > 1) c.push_back(Tuning{LE, OE, 256, LW, OW, 256, wpc, 4, es});
-                }
-            // fused one-launch form
-            if (fused_supported(LE, OE, LW, OW))
-                for (int block : {64, 256}) c.push_back(Tuning{LE, OE, block, LW, OW, block, 8, 2});
-            // persistent queue, one wave per survivor
-            for (int es = 0; es <= es_max; ++es) c.push_back(Tuning{LE, OE, 256, LW, OW, 256, 16, 1, es});
-        }
-    for (const auto &w : shapes) c.push_back(Tuning{8, 1, 256, w[0], w[1], 256, 8, 0});
-    return c;
 }
 
 } // namespace
@@ -191,7 +113,6 @@ void graph_workspace(Workspace &w, int64_t n)
     OA_HIP(hipMalloc(&w.counters, kWorkspaceCounters * sizeof(int32_t)));
     OA_HIP(hipMemset(w.counters, 0, kWorkspaceCounters * sizeof(int32_t)));
     alloc_workspace_arrays(w, cap);
-    w.parity = 0;
 }
 
 // Records the group twice (once per survivor counter set of every batch's
@@ -216,7 +137,7 @@ void record_group(ompl_amd_motion_graph_s *g, const Env &env, const Tuning &t, i
     hipStream_t cs = thread_resources().stream;
     for (int r = 0; r < 2; ++r) {
         // recording r uses counter set r of each workspace when its batch
-        // alternates sets (check_motions_tuned flips ws.parity after recording)
+        // alternates sets (grid_scratch takes them in turn)
         OA_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
         try {
             if (nb > 1) {
@@ -275,7 +196,6 @@ int ompl_amd_env_create(const float *spheres, int n_spheres, const float *boxes,
             h[n_spheres + 2 * i] = make_float4(o[0] - o[3], o[1] - o[4], o[2] - o[5], 0.0f);
             h[n_spheres + 2 * i + 1] = make_float4(o[0] + o[3], o[1] + o[4], o[2] + o[5], 0.0f);
         }
-        // h (caller's order) goes after the staging-order copy in one allocation
         const std::vector<int> so = nearest_first(n_spheres, [&](int i) {
             const float *o = spheres + 4 * i;
             return std::sqrt((double)o[0] * o[0] + (double)o[1] * o[1] + (double)o[2] * o[2]) - (double)o[3];
@@ -287,14 +207,6 @@ int ompl_amd_env_create(const float *spheres, int n_spheres, const float *boxes,
             const double dz = std::max({(double)lo.z, -(double)hi.z, 0.0});
             return std::sqrt(dx * dx + dy * dy + dz * dz);
         });
-        std::vector<float4> both(2 * h.size());
-        for (int i = 0; i < n_spheres; ++i) both[i] = h[so[i]];
-        for (int i = 0; i < n_boxes; ++i) {
-            both[n_spheres + 2 * i] = h[n_spheres + 2 * bo[i]];
-            both[n_spheres + 2 * i + 1] = h[n_spheres + 2 * bo[i] + 1];
-        }
-        both[h.size() - 1] = h[h.size() - 1];
-        std::copy(h.begin(), h.end(), both.begin() + h.size());
         // the grid's obstacle table: every obstacle as a box with a squared
         // contact distance (a sphere is the box lo = hi = centre)
         const int n_obs = n_spheres + n_boxes;
@@ -302,7 +214,8 @@ int ompl_amd_env_create(const float *spheres, int n_spheres, const float *boxes,
         double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
         for (int i = 0; i < n_obs; ++i) {
             const bool sphere = i < n_spheres;
-            float4 l = sphere ? both[i] : both[2 * i - n_spheres], u = sphere ? l : both[2 * i - n_spheres + 1];
+            const int at = sphere ? so[i] : n_spheres + 2 * bo[i - n_spheres];
+            float4 l = h[at], u = sphere ? l : h[at + 1];
             if (!sphere) l.w = kRobotR * kRobotR;
             u.w = 0.0f;
             tab.push_back(l);
@@ -320,13 +233,13 @@ int ompl_amd_env_create(const float *spheres, int n_spheres, const float *boxes,
         env.nb = n_boxes;
         env.grid.n_obs = n_obs;
         grid_extent(env.grid, lo, hi, n_obs == 0);
-        // one allocation: obstacles (both orders) and table, link layout, cells, lists, build counter
+        // one allocation: obstacles (the caller's order) and table, cells, lists, build counter
         auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-        const size_t n_both = both.size();
-        both.insert(both.end(), tab.begin(), tab.end());
-        const size_t obs_b = up(both.size() * sizeof(float4)), links_b = up(links_bytes(env.view()) + sizeof(float4)),
-                     cells_b = grid_cells_bytes(env.grid), lists_b = grid_lists_bytes(env.grid);
-        env.bytes = obs_b + links_b + cells_b + lists_b + 256;
+        const size_t n_words = h.size();
+        h.insert(h.end(), tab.begin(), tab.end());
+        const size_t obs_b = up(h.size() * sizeof(float4)), cells_b = grid_cells_bytes(env.grid),
+                     lists_b = grid_lists_bytes(env.grid);
+        env.bytes = obs_b + cells_b + lists_b + 256;
         char *mem = nullptr;
         const hipError_t err = hipMalloc((void **)&mem, env.bytes);
         if (err != hipSuccess) {
@@ -335,18 +248,14 @@ int ompl_amd_env_create(const float *spheres, int n_spheres, const float *boxes,
         }
         env.obs = (float4 *)mem;
         try {
-            env.obs_input = env.obs + h.size();
-            env.obs_links = (float4 *)(mem + obs_b);
-            uint32_t *cells = (uint32_t *)(mem + obs_b + links_b);
-            uint16_t *lists = (uint16_t *)(mem + obs_b + links_b + cells_b);
-            uint32_t *counter = (uint32_t *)(mem + obs_b + links_b + cells_b + lists_b);
-            env.grid.tab = env.obs + n_both;
+            uint32_t *cells = (uint32_t *)(mem + obs_b);
+            uint16_t *lists = (uint16_t *)(mem + obs_b + cells_b);
+            uint32_t *counter = (uint32_t *)(mem + obs_b + cells_b + lists_b);
+            env.grid.tab = env.obs + n_words;
             env.grid.cells = cells;
             env.grid.lists = lists;
             ThreadResources &r = thread_resources();
-            OA_HIP(hipMemcpyAsync(env.obs, both.data(), both.size() * sizeof(float4), hipMemcpyHostToDevice,
-                                  r.stream));
-            launch_stage_links(env.view(), env.obs_links, r.stream);
+            OA_HIP(hipMemcpyAsync(env.obs, h.data(), h.size() * sizeof(float4), hipMemcpyHostToDevice, r.stream));
             launch_grid_build(env.grid, cells, lists, counter, r.pinned_dev + kEnvBaseAt, r.stream);
             OA_HIP(hipStreamSynchronize(r.stream));
             env.grid.base_hit = r.pinned[kEnvBaseAt];
@@ -387,13 +296,7 @@ int ompl_amd_validate_states_dev(ompl_amd_env e, const float *q, int64_t n, uint
         OA_REQUIRE(n >= 0, OMPL_AMD_ERR_ARG, "negative state count");
         if (n == 0) return;
         OA_REQUIRE(q && out, OMPL_AMD_ERR_ARG, "null state or output pointer");
-        const Tuning t = tuning_for(*e);
-        if (own_validity_shape(t)) {
-            launch_grid_validate<float>(env.grid, q, n, out, resolve_stream(stream));
-            return;
-        }
-        launch_validate<float>(env.view(), q, n, out, t.validity_lanes_per_state, t.validity_obstacle_parts,
-                               t.validity_block, resolve_stream(stream), t.validity_shared_fk != 0);
+        launch_grid_validate<float>(env.grid, q, n, out, resolve_stream(stream));
     });
 }
 
@@ -404,13 +307,7 @@ int ompl_amd_validate_states_f64_dev(ompl_amd_env e, const double *q, int64_t n,
         OA_REQUIRE(n >= 0, OMPL_AMD_ERR_ARG, "negative state count");
         if (n == 0) return;
         OA_REQUIRE(q && out, OMPL_AMD_ERR_ARG, "null state or output pointer");
-        const Tuning t = tuning_for(*e);
-        if (own_validity_shape(t)) {
-            launch_grid_validate<double>(env.grid, q, n, out, resolve_stream(stream));
-            return;
-        }
-        launch_validate<double>(env.view(), q, n, out, t.validity_lanes_per_state, t.validity_obstacle_parts,
-                                t.validity_block, resolve_stream(stream), t.validity_shared_fk != 0);
+        launch_grid_validate<double>(env.grid, q, n, out, resolve_stream(stream));
     });
 }
 
@@ -422,7 +319,7 @@ int ompl_amd_is_valid(ompl_amd_env e, const double *q, int *valid)
         ThreadResources &r = thread_resources();
         State1 st;
         for (int j = 0; j < kDof; ++j) st.q[j] = q[j];
-        launch_validate_single(env.view(), st, r.pinned_dev, r.stream);
+        launch_validate_single(env.grid, st, r.pinned_dev, r.stream);
         OA_HIP(hipStreamSynchronize(r.stream));
         *valid = r.pinned[0];
     });
@@ -457,9 +354,7 @@ int ompl_amd_check_motions_last_valid_dev(ompl_amd_env e, const double *a, const
         OA_REQUIRE(a && b && out && last_t, OMPL_AMD_ERR_ARG, "null pointer");
         OA_REQUIRE(lvs > 0.0 && factor >= 1, OMPL_AMD_ERR_ARG, "longest valid segment must be > 0 and factor >= 1");
         OA_REQUIRE(n < (int64_t)1 << 31, OMPL_AMD_ERR_ARG, "at most 2^31-1 edges per call");
-        const Tuning t = tuning_for(*e);
         MotionArgs A{};
-        A.env = env.view();
         A.a = a;
         A.b = b;
         A.n = n;
@@ -469,18 +364,7 @@ int ompl_amd_check_motions_last_valid_dev(ompl_amd_env e, const double *a, const
         const hipStream_t st = resolve_stream(stream);
         std::unique_lock<std::mutex> lk; // held until the launches are enqueued
         Workspace &w = workspace(st, (size_t)n, lk);
-        if (own_walk_shape(t)) {
-            launch_grid_last_valid(env.grid, A, last_t, grid_scratch(w), st);
-            return;
-        }
-        A.list = w.list;
-        A.first_bad = w.first_bad;
-        A.surv_nd = w.surv_nd;
-        A.surv_ab = w.surv_ab;
-        A.list_count = w.counters + 2;
-        A.max_m = w.counters + 3;
-        launch_motion_last_valid(A, last_t, t.motion_lanes_per_state, t.motion_obstacle_parts,
-                                 (int64_t)num_cus() * t.motion_waves_per_cu, st);
+        launch_grid_last_valid(env.grid, A, last_t, grid_scratch(w), st);
     });
 }
 
@@ -496,7 +380,7 @@ int ompl_amd_check_motion(ompl_amd_env e, const double *a, const double *b, doub
             E.a[j] = a[j];
             E.b[j] = b[j];
         }
-        launch_motion_single(env.view(), E, lvs, factor, r.pinned_dev, r.stream);
+        launch_motion_single(env.grid, E, lvs, factor, r.pinned_dev, r.stream);
         OA_HIP(hipStreamSynchronize(r.stream));
         *valid = r.pinned[0];
     });
@@ -512,18 +396,10 @@ int ompl_amd_check_state_lists_dev(ompl_amd_env e, const double *q_soa, int64_t 
         OA_REQUIRE(offsets && out && (n_states == 0 || q_soa), OMPL_AMD_ERR_ARG, "null pointer");
         OA_REQUIRE(n_lists < (int64_t)1 << 31 && n_states < (int64_t)1 << 31, OMPL_AMD_ERR_ARG,
                    "at most 2^31-1 lists and states per call");
-        const Tuning t = tuning_for(*e);
         const hipStream_t st = resolve_stream(stream);
         std::unique_lock<std::mutex> lk; // held until the launches are enqueued
         Workspace &w = workspace(st, (size_t)n_lists, lk);
-        if (own_walk_shape(t)) {
-            launch_grid_state_lists(env.grid, q_soa, n_states, offsets, n_lists, out, first_invalid, grid_scratch(w),
-                                    st);
-            return;
-        }
-        launch_state_lists(env.view(), q_soa, n_states, offsets, n_lists, out, first_invalid,
-                           t.motion_lanes_per_state, t.motion_obstacle_parts,
-                           (int64_t)num_cus() * t.motion_waves_per_cu, w.list, w.first_bad, w.counters + 2, st);
+        launch_grid_state_lists(env.grid, q_soa, n_states, offsets, n_lists, out, first_invalid, grid_scratch(w), st);
     });
 }
 
@@ -542,22 +418,13 @@ int ompl_amd_check_states(ompl_amd_env e, const double *states, int count, int *
         double *q = reinterpret_cast<double *>(r.stage + head);
         for (int i = 0; i < count; ++i)
             for (int j = 0; j < kDof; ++j) q[(size_t)j * count + i] = states[(size_t)i * kDof + j];
-        const Tuning t = tuning_for(*e);
         {
             std::unique_lock<std::mutex> lk; // held until the launches are enqueued
             Workspace &w = workspace(r.stream, 1, lk);
-            if (own_walk_shape(t))
-                launch_grid_state_lists(env.grid, reinterpret_cast<const double *>(r.stage_dev + head), count,
-                                        reinterpret_cast<const int64_t *>(r.stage_dev), 1,
-                                        reinterpret_cast<uint8_t *>(r.stage_dev + 16),
-                                        reinterpret_cast<int32_t *>(r.stage_dev + 32), grid_scratch(w), r.stream);
-            else
-                launch_state_lists(env.view(), reinterpret_cast<const double *>(r.stage_dev + head), count,
-                               reinterpret_cast<const int64_t *>(r.stage_dev), 1,
-                               reinterpret_cast<uint8_t *>(r.stage_dev + 16),
-                               reinterpret_cast<int32_t *>(r.stage_dev + 32), t.motion_lanes_per_state,
-                               t.motion_obstacle_parts, (int64_t)num_cus() * t.motion_waves_per_cu, w.list,
-                               w.first_bad, w.counters + 2, r.stream);
+            launch_grid_state_lists(env.grid, reinterpret_cast<const double *>(r.stage_dev + head), count,
+                                    reinterpret_cast<const int64_t *>(r.stage_dev), 1,
+                                    reinterpret_cast<uint8_t *>(r.stage_dev + 16),
+                                    reinterpret_cast<int32_t *>(r.stage_dev + 32), grid_scratch(w), r.stream);
         }
         OA_HIP(hipStreamSynchronize(r.stream));
         *valid = reinterpret_cast<uint8_t *>(r.stage)[16];
@@ -584,7 +451,6 @@ int ompl_amd_check_motion_last_valid(ompl_amd_env e, const double *a, const doub
         double *dev_pd = reinterpret_cast<double *>(r.pinned_dev + 16);
         uint8_t *dev_out = reinterpret_cast<uint8_t *>(r.pinned_dev);
         MotionArgs A{};
-        A.env = env.view();
         A.a = dev_pd;
         A.b = dev_pd + kDof;
         A.n = 1;
@@ -594,18 +460,7 @@ int ompl_amd_check_motion_last_valid(ompl_amd_env e, const double *a, const doub
         {
             std::unique_lock<std::mutex> lk; // held until the launches are enqueued
             Workspace &w = workspace(r.stream, 1, lk);
-            A.list = w.list;
-            A.first_bad = w.first_bad;
-            A.surv_nd = w.surv_nd;
-            A.surv_ab = w.surv_ab;
-            A.list_count = w.counters + 2;
-            A.max_m = w.counters + 3;
-            const Tuning t = tuning_for(*e);
-            if (own_walk_shape(t))
-                launch_grid_last_valid(env.grid, A, dev_pd + 2 * kDof, grid_scratch(w), r.stream);
-            else
-                launch_motion_last_valid(A, dev_pd + 2 * kDof, t.motion_lanes_per_state, t.motion_obstacle_parts,
-                                     (int64_t)num_cus() * t.motion_waves_per_cu, r.stream);
+            launch_grid_last_valid(env.grid, A, dev_pd + 2 * kDof, grid_scratch(w), r.stream);
         }
         OA_HIP(hipStreamSynchronize(r.stream));
         *valid = reinterpret_cast<uint8_t *>(r.pinned)[0];
@@ -654,22 +509,15 @@ extern "C" int ompl_amd_autotune_motions(ompl_amd_env e, const double *a, const 
         hipEvent_t e0, e1;
         OA_HIP(hipEventCreate(&e0));
         OA_HIP(hipEventCreate(&e1));
-        const Tuning base = get_tuning();
-        Tuning win = base;
-        float win_ms = INFINITY;
-        for (const Tuning &t : motion_candidates()) {
-            for (int w = 0; w < 2; ++w) check_motions_tuned(t, env, a, b, n, lvs, factor, out, nullptr, s);
-            OA_HIP(hipEventRecord(e0, s));
-            for (int i = 0; i < reps; ++i) check_motions_tuned(t, env, a, b, n, lvs, factor, out, nullptr, s);
-            OA_HIP(hipEventRecord(e1, s));
-            OA_HIP(hipEventSynchronize(e1));
-            float ms = 0.0f;
-            OA_HIP(hipEventElapsedTime(&ms, e0, e1));
-            if (ms < win_ms) {
-                win_ms = ms;
-                win = t;
-            }
-        }
+        // every shape runs the same kernels: one is timed and installed
+        const Tuning win{8, 2, 256, 8, 1, 256, 8, 3, 0};
+        for (int w = 0; w < 2; ++w) check_motions_tuned(win, env, a, b, n, lvs, factor, out, nullptr, s);
+        OA_HIP(hipEventRecord(e0, s));
+        for (int i = 0; i < reps; ++i) check_motions_tuned(win, env, a, b, n, lvs, factor, out, nullptr, s);
+        OA_HIP(hipEventRecord(e1, s));
+        OA_HIP(hipEventSynchronize(e1));
+        float win_ms = 0.0f;
+        OA_HIP(hipEventElapsedTime(&win_ms, e0, e1));
         OA_HIP(hipEventDestroy(e0));
         OA_HIP(hipEventDestroy(e1));
         OA_HIP(hipFree(out));
@@ -697,30 +545,6 @@ struct PipelineScratch {
         for (hipEvent_t e : join) (void)hipEventDestroy(e);
     }
 };
-
-// Launch shapes tried for batches on several streams: the s2 pass's and the
-// walk's (lanes per state, obstacle parts) and the walk's waves per CU, all
-// with the chunk-parallel walk (strategy 3).
-std::vector<Tuning> stream_candidates(const Tuning &base)
-{
-    const int s2[][2] = {{7, 1}, {7, 2}, {7, 4}, {7, 9}, {8, 4}, {8, 8}};
-    const int walk[][2] = {{7, 2}, {7, 4}, {7, 9}, {8, 8}};
-    std::vector<Tuning> c;
-    for (const auto &e : s2)
-        for (const auto &w : walk)
-            for (int wpc : {2, 4, 8, 16}) {
-                Tuning t = base;
-                t.validity_lanes_per_state = e[0];
-                t.validity_obstacle_parts = e[1];
-                t.motion_lanes_per_state = w[0];
-                t.motion_obstacle_parts = w[1];
-                t.motion_waves_per_cu = wpc;
-                t.motion_strategy = 3;
-                t.validity_shared_fk = 0;
-                c.push_back(t);
-            }
-    return c;
-}
 
 } // namespace
 
@@ -774,22 +598,15 @@ extern "C" int ompl_amd_autotune_motions_streams(ompl_amd_env e, const double *a
             OA_HIP(hipEventElapsedTime(&ms, S.e0, S.e1));
             return 1e3 * (double)ms / k;
         };
-        std::vector<std::pair<double, Tuning>> timed;
-        for (const Tuning &t : stream_candidates(get_tuning())) timed.emplace_back(per_batch(t, steps), t);
-        std::stable_sort(timed.begin(), timed.end(),
-                         [](const std::pair<double, Tuning> &x, const std::pair<double, Tuning> &y) {
-                             return x.first < y.first;
-                         });
-        // the three fastest again over twice the batches
-        double win_us = INFINITY;
-        Tuning win = timed.front().second;
-        for (size_t i = 0; i < timed.size() && i < 3; ++i) {
-            const double us = per_batch(timed[i].second, 2 * steps);
-            if (us < win_us) {
-                win_us = us;
-                win = timed[i].second;
-            }
-        }
+        // every shape runs the same kernels: one of those a tuning for streams
+        // names (eight lanes a state throughout) is timed and installed
+        Tuning win = get_tuning();
+        win.validity_lanes_per_state = win.motion_lanes_per_state = win.motion_waves_per_cu = 8;
+        win.validity_obstacle_parts = 4;
+        win.motion_obstacle_parts = 8;
+        win.motion_strategy = 3;
+        win.validity_shared_fk = 0;
+        const double win_us = per_batch(win, steps);
         set_tuning(win);
         if (best) *best = tuning_to_c(win);
         if (best_us) *best_us = win_us;

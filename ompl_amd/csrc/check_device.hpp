@@ -1,6 +1,5 @@
-// Device helpers shared by the batched check kernels (checker.hip and
-// grid_check.hip): reading configurations, the outcome of an edge's s2 check,
-// and the survivor list.
+// Device helpers of the batched check kernels: reading configurations, the
+// outcome of an edge's s2 check, and the survivor list.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -66,55 +65,38 @@ __device__ __forceinline__ bool endpoint_finish(const MotionArgs &A, int64_t e, 
     return true;
 }
 
-// Block-aggregated append of the survivors to the list (with their segment
-// count and, when kept, their endpoints contiguous for the chunk walk).
-// Every thread of the block calls it (it holds three barriers); a survivor's
-// slot is returned.  The waves'
-// counts and largest segment counts meet in LDS, and one thread per block
-// makes the two device-wide atomics: device-scope atomics on one address
-// from every CU serialise, and with many survivors (a sparse scene) one
+// Block-aggregated append of the survivors to the list, with their segment
+// count and endpoints.  Every thread of the block calls it (it holds three
+// barriers); a survivor's slot is returned.  The waves' counts meet in LDS, and
+// one thread per block makes the device-wide atomic: device-scope atomics on one
+// address from every CU serialise, and with many survivors (a sparse scene) one
 // atomic per survivor cost more than the s2 checks themselves.
 __device__ __forceinline__ int append_survivor(const MotionArgs &A, int64_t e, bool survivor, int m,
-                                                const double a[kDof], const double b[kDof])
+                                               const double a[kDof], const double b[kDof])
 {
-    __shared__ int blk_count, blk_max, blk_base;
+    __shared__ int blk_count, blk_base;
     const int lane = lane_id();
-    if (threadIdx.x == 0) {
-        blk_count = 0;
-        blk_max = 0;
-    }
+    if (threadIdx.x == 0) blk_count = 0;
     __syncthreads();
     const uint64_t sm = wave_ballot(survivor);
     int woff = 0;
     if (sm) {
-        int mm = survivor ? m : 0;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) mm = max(mm, __shfl_xor(mm, d));
-        if (lane == lowest_bit(sm)) {
-            woff = atomicAdd(&blk_count, __popcll(sm));
-            atomicMax(&blk_max, mm);
-        }
+        if (lane == lowest_bit(sm)) woff = atomicAdd(&blk_count, __popcll(sm));
         woff = __shfl(woff, lowest_bit(sm));
     }
     __syncthreads();
-    if (threadIdx.x == 0 && blk_count > 0) {
-        blk_base = atomicAdd(A.list_count, blk_count);
-        if (A.max_m) atomicMax(A.max_m, blk_max);
-    }
+    if (threadIdx.x == 0 && blk_count > 0) blk_base = atomicAdd(A.list_count, blk_count);
     __syncthreads();
     const int slot = blk_base + woff + __popcll(sm & (((uint64_t)1 << lane) - 1));
     if (survivor) {
         A.out[e] = 1; // until the walk finds an invalid position
         A.list[slot] = (int32_t)e;
-        if (A.first_bad) A.first_bad[slot] = INT_MAX;
-        if (A.surv_nd) A.surv_nd[slot] = m + 1;
-        if (A.surv_ab) {
-            double *ab = A.surv_ab + (int64_t)slot * 2 * kDof;
+        A.surv_nd[slot] = m + 1;
+        double *ab = A.surv_ab + (int64_t)slot * 2 * kDof;
 #pragma unroll
-            for (int j = 0; j < kDof; ++j) {
-                ab[j] = a[j];
-                ab[kDof + j] = b[j];
-            }
+        for (int j = 0; j < kDof; ++j) {
+            ab[j] = a[j];
+            ab[kDof + j] = b[j];
         }
     }
     return slot;

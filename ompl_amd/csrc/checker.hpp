@@ -12,7 +12,6 @@
 namespace ompl_amd {
 
 struct MotionArgs {
-    EnvView env;
     const double *a; // FP64 [7][n] dof-major
     const double *b;
     int64_t n;
@@ -20,16 +19,10 @@ struct MotionArgs {
     unsigned factor;
     uint8_t *out;
     int32_t *checked;    // optional
-    int32_t *list;       // survivor list (endpoint output / walk input), optional
-    int32_t *list_count; // number of entries in list
-    int32_t *queue;      // dynamic work counter for the walk, optional
-    int32_t *first_bad;  // per survivor: first invalid position (chunk-parallel walk)
-    int32_t *max_m;      // largest bisection position count among survivors
-    int32_t *surv_nd;    // per survivor: segment count nd
-    double *surv_ab;     // per survivor: endpoints a then b (14 doubles, contiguous), optional
-    int flat;             // chunk walk: the launch reserved LDS for the survivors' chunk offsets
-    int32_t *reset_next;  // chunk walk without a results kernel: the counter set phase 1 clears
-    int start;           // first walk position (0 = s2, 1 = skip s2)
+    int32_t *list;       // survivors of the s2 pass: their edges,
+    int32_t *list_count; // number,
+    int32_t *surv_nd;    // segment counts
+    double *surv_ab;     // and endpoints, a then b (14 doubles)
 };
 
 struct Edge1 {
@@ -41,34 +34,10 @@ struct State1 {
     double q[kDof];
 };
 
+// Launch shapes and one-launch shape pairs a tuning may name.
 bool shape_supported(int lps, int ops);
-// Bytes of an environment's link-layout copy, and the kernel that writes it.
-size_t links_bytes(const EnvView &env);
-void launch_stage_links(const EnvView &env, float4 *out, hipStream_t s);
 bool fused_supported(int le, int oe, int lw, int ow);
-
-template <typename T>
-void launch_validate(const EnvView &env, const T *q, int64_t n, uint8_t *out, int lps, int ops, int block,
-                     hipStream_t s, bool shared = false);
 void launch_zero(int *p, int n, hipStream_t s);
-void launch_motion_endpoint(const MotionArgs &A, int lps, int ops, int block, hipStream_t s, bool shared = false);
-void launch_motion_walk(const MotionArgs &A, bool exact, int lps, int ops, int block, int64_t waves, hipStream_t s);
-void launch_motion_chunks(const MotionArgs &A, bool exact, int lps, int ops, int block, int64_t waves,
-                          hipStream_t s, bool shared, bool results);
-void launch_motion_fused(const MotionArgs &A, bool exact, int le, int oe, int lw, int ow, int block, hipStream_t s);
-void launch_motion_single(const EnvView &env, const Edge1 &E, double lvs, unsigned factor, int *result,
-                          hipStream_t s);
-void launch_validate_single(const EnvView &env, const State1 &st, int *result, hipStream_t s);
-// Uses A.list, first_bad, surv_nd, surv_ab (room for A.n entries) and the
-// adjacent counters list_count, max_m (cleared by the launch); waves: the
-// persistent grid of the chunk phase.
-void launch_motion_last_valid(const MotionArgs &A, double *last_t, int lps, int ops, int64_t waves, hipStream_t s);
-// lps, ops: the launch shape (the walk's: lowest-invalid exit over a list's
-// states); waves: the persistent grid of the chunk phase; unres / unres_fb:
-// room for n_lists entries each; counters: two ints (cleared by the launch).
-void launch_state_lists(const EnvView &env, const double *q_soa, int64_t n_states, const int64_t *offsets,
-                        int64_t n_lists, uint8_t *out, int32_t *first_invalid, int lps, int ops, int64_t waves,
-                        int32_t *unres, int32_t *unres_fb, int32_t *counters, hipStream_t s);
 // Edges or lists up to which a block each walks them in one launch: 1,024
 // blocks of four waves are one wave per SIMD, so the speculative positions of
 // edges that fail at once cost no time; more edges go through the s2 pass.
@@ -85,7 +54,12 @@ struct GridScratch {
 };
 template <typename T>
 void launch_grid_validate(const GridView &g, const T *q, int64_t n, uint8_t *out, hipStream_t s);
-void launch_grid_motions(const GridView &g, const MotionArgs &m, const GridScratch &w, hipStream_t s);
+// fused: timed as one launch ("motion_fused") rather than by kernel.
+void launch_grid_motions(const GridView &g, const MotionArgs &m, const GridScratch &w, bool fused, hipStream_t s);
+// One edge or state, passed by value; *result: 1 valid, 0 not.
+void launch_motion_single(const GridView &g, const Edge1 &E, double lvs, unsigned factor, int *result,
+                          hipStream_t s);
+void launch_validate_single(const GridView &g, const State1 &st, int *result, hipStream_t s);
 void launch_grid_last_valid(const GridView &g, const MotionArgs &m, double *last_t, const GridScratch &w,
                             hipStream_t s);
 void launch_grid_state_lists(const GridView &g, const double *q_soa, int64_t n_states, const int64_t *offsets,

@@ -27,6 +27,8 @@ constexpr double kReach = 2.12;
 // A cell is grown by this much before it is decided: far more than the rounding
 // of a coordinate's cell number (a few 1e-7 of 68 cells of 0.06 m at most).
 constexpr float kCellMargin = 1e-4f;
+// Margins of the decisions, in metres and of the contact distance.
+constexpr float kBoundAbs = 1e-4f, kBoundRel = 1e-5f;
 
 size_t up256(size_t b)
 {

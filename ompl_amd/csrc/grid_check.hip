@@ -84,7 +84,7 @@ constexpr int kHelpers = 256;
 
 struct GridWalkArgs {
     GridView g;
-    MotionArgs m;      // edges: env unused; list / list_count / surv_nd / surv_ab as for the chunk walk
+    MotionArgs m;
     double *last_t;    // kSequence
     const double *q;   // kList: dof-major states
     int64_t n_states;
@@ -546,6 +546,37 @@ __global__ void __launch_bounds__(256, 4) grid_rest_kernel(GridWalkArgs A)
     }
 }
 
+// One edge by value, walked by a block (the per-call path).
+__global__ void __launch_bounds__(256, 4) grid_motion_single_kernel(GridView g, Edge1 E, double lvs, unsigned factor,
+                                                                    int *result)
+{
+    __shared__ Rounds R;
+    __shared__ WaveTests tests[4];
+    GridWalkArgs A{};
+    A.g = g;
+    Item<Walk::kBisect> I;
+#pragma unroll
+    for (int j = 0; j < kDof; ++j) {
+        I.a[j] = E.a[j];
+        I.b[j] = E.b[j];
+    }
+    I.nd = valid_segment_count<kDof>(I.a, I.b, lvs, factor);
+    I.total = max(I.nd, 1);
+    int turn = 0;
+    int b = 0; // too many segments: invalid
+    if (!I.nd_too_many()) b = walk_item(A, I, 0, I.total, false, 256, nullptr, R, turn, tests);
+    if (threadIdx.x == 0) *result = b == INT_MAX ? 1 : 0;
+}
+
+// One state by value.
+__global__ void __launch_bounds__(64) grid_validate_single_kernel(GridView g, State1 s, int *result)
+{
+    __shared__ WaveTests tests;
+    const int lane = lane_id();
+    const uint64_t H = wave_ballot(state_hit8(g, (float)s.q[min(lane & 7, kDof - 1)], lane < 8, tests));
+    if (lane == 0) *result = H ? 0 : 1;
+}
+
 // ---------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------
@@ -580,8 +611,6 @@ static GridWalkArgs walk_args(const GridView &g, const MotionArgs &m, const Grid
     A.m.surv_nd = w.surv_nd;
     A.m.surv_ab = w.surv_ab;
     A.m.list_count = w.counts;
-    A.m.max_m = nullptr;
-    A.m.first_bad = nullptr;
     A.rest = w.rest;
     A.long_slot = w.long_slot;
     A.long_bad = w.long_bad;
@@ -609,25 +638,54 @@ static void launch_items(const GridWalkArgs &A, hipStream_t s)
     OA_HIP(hipGetLastError());
 }
 
-void launch_grid_motions(const GridView &g, const MotionArgs &m, const GridScratch &w, hipStream_t s)
+void launch_motion_single(const GridView &g, const Edge1 &E, double lvs, unsigned factor, int *result, hipStream_t s)
+{
+    hipLaunchKernelGGL(grid_motion_single_kernel, dim3(1), dim3(256), 0, s, g, E, lvs, factor, result);
+    OA_HIP(hipGetLastError());
+}
+
+void launch_validate_single(const GridView &g, const State1 &st, int *result, hipStream_t s)
+{
+    hipLaunchKernelGGL(grid_validate_single_kernel, dim3(1), dim3(64), 0, s, g, st, result);
+    OA_HIP(hipGetLastError());
+}
+
+static void launch_endpoints(const GridWalkArgs &A, hipStream_t s)
+{
+    if (A.m.n >= kLaneStates)
+        hipLaunchKernelGGL(grid_endpoint1_kernel, dim3(grid_of(A.m.n, 256)), dim3(256), 0, s, A);
+    else
+        hipLaunchKernelGGL(grid_endpoint8_kernel, dim3(grid_of(A.m.n, 32)), dim3(256), 0, s, A);
+    OA_HIP(hipGetLastError());
+}
+
+static void launch_survivors(const GridWalkArgs &A, hipStream_t s)
+{
+    hipLaunchKernelGGL(grid_survivors_kernel, dim3((unsigned)num_cus() * 8), dim3(256), 0, s, A);
+    OA_HIP(hipGetLastError());
+}
+
+void launch_grid_motions(const GridView &g, const MotionArgs &m, const GridScratch &w, bool fused, hipStream_t s)
 {
     if (m.n <= 0) return;
     const GridWalkArgs A = walk_args(g, m, w);
     if (m.n <= kWideItems) {
-        ProfScope ps("motion_walk", s);
+        ProfScope ps(fused ? "motion_fused" : "motion_walk", s);
         launch_wide<Walk::kBisect>(A, s);
+        return;
+    }
+    if (fused) {
+        ProfScope ps("motion_fused", s);
+        launch_endpoints(A, s);
+        launch_survivors(A, s);
         return;
     }
     {
         ProfScope ps("motion_endpoint", s);
-        if (m.n >= kLaneStates)
-            hipLaunchKernelGGL(grid_endpoint1_kernel, dim3(grid_of(m.n, 256)), dim3(256), 0, s, A);
-        else
-            hipLaunchKernelGGL(grid_endpoint8_kernel, dim3(grid_of(m.n, 32)), dim3(256), 0, s, A);
+        launch_endpoints(A, s);
     }
     ProfScope ps("motion_chunk", s);
-    hipLaunchKernelGGL(grid_survivors_kernel, dim3((unsigned)num_cus() * 8), dim3(256), 0, s, A);
-    OA_HIP(hipGetLastError());
+    launch_survivors(A, s);
 }
 
 void launch_grid_last_valid(const GridView &g, const MotionArgs &m, double *last_t, const GridScratch &w,

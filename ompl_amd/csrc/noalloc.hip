@@ -1,6 +1,6 @@
 // Batched motion validation that allocates nothing: the survivor workspace of
-// ompl_amd_check_motions_dev (survivor list, per-survivor first invalid
-// position, segment count and FP64 endpoints, and the counters) lives in a
+// ompl_amd_check_motions_dev (survivor list, their segment counts and
+// FP64 endpoints, unfinished and long items, and the counters) lives in a
 // file-scope device array instead of memory the library allocates, for callers
 // that cannot allocate (code under HIP graph capture, tight serving loops).
 //
@@ -24,7 +24,7 @@ constexpr int64_t kNoAllocMaxEdges = 65536;
 constexpr size_t kNoAllocCounterBytes = kWorkspaceCounters * sizeof(int32_t);
 constexpr size_t kNoAllocListBytes = (size_t)kNoAllocMaxEdges * sizeof(int32_t);
 constexpr size_t kNoAllocEndpointBytes = (size_t)kNoAllocMaxEdges * 14 * sizeof(double);
-// counters | list | first_bad | surv_nd | surv_ab | longs  (every part 256-byte aligned)
+// counters | list | rest | surv_nd | surv_ab | longs  (every part 256-byte aligned)
 constexpr size_t kNoAllocScratchBytes = kNoAllocCounterBytes + 6 * kNoAllocListBytes + kNoAllocEndpointBytes;
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
@@ -73,13 +73,12 @@ extern "C" int ompl_amd_check_motions_noalloc_dev(ompl_amd_env e, const double *
         Workspace w;
         w.counters = reinterpret_cast<int32_t *>(base);
         w.list = reinterpret_cast<int32_t *>(base + kNoAllocCounterBytes);
-        w.first_bad = reinterpret_cast<int32_t *>(base + kNoAllocCounterBytes + kNoAllocListBytes);
+        w.rest = reinterpret_cast<int32_t *>(base + kNoAllocCounterBytes + kNoAllocListBytes);
         w.surv_nd = reinterpret_cast<int32_t *>(base + kNoAllocCounterBytes + 2 * kNoAllocListBytes);
         w.surv_ab = reinterpret_cast<double *>(base + kNoAllocCounterBytes + 3 * kNoAllocListBytes);
         w.longs = reinterpret_cast<int32_t *>(base + kNoAllocCounterBytes + 3 * kNoAllocListBytes +
                                               kNoAllocEndpointBytes);
         w.list_cap = (size_t)kNoAllocMaxEdges;
-        w.parity = 0;
         launch_zero(w.counters, (int)(kNoAllocCounterBytes / sizeof(int32_t)), s);
         check_motions_tuned(tuning_for(*e), e->env, a, b, n, lvs, factor, out, checked, s, &w);
     });

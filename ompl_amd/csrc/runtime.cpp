@@ -105,7 +105,7 @@ hipStream_t default_stream()
 void alloc_workspace_arrays(Workspace &w, size_t cap)
 {
     OA_HIP(hipMalloc(&w.list, cap * sizeof(int32_t)));
-    OA_HIP(hipMalloc(&w.first_bad, cap * sizeof(int32_t)));
+    OA_HIP(hipMalloc(&w.rest, cap * sizeof(int32_t)));
     OA_HIP(hipMalloc(&w.surv_nd, cap * sizeof(int32_t)));
     OA_HIP(hipMalloc(&w.longs, 3 * cap * sizeof(int32_t)));
     OA_HIP(hipMalloc(&w.surv_ab, cap * 14 * sizeof(double)));
@@ -114,9 +114,9 @@ void alloc_workspace_arrays(Workspace &w, size_t cap)
 
 void free_workspace_arrays(Workspace &w)
 {
-    for (void *p : {(void *)w.list, (void *)w.first_bad, (void *)w.surv_nd, (void *)w.longs, (void *)w.surv_ab})
+    for (void *p : {(void *)w.list, (void *)w.rest, (void *)w.surv_nd, (void *)w.longs, (void *)w.surv_ab})
         if (p) (void)hipFree(p);
-    w.list = w.first_bad = w.surv_nd = w.longs = nullptr;
+    w.list = w.rest = w.surv_nd = w.longs = nullptr;
     w.surv_ab = nullptr;
     w.list_cap = 0;
 }
@@ -127,7 +127,7 @@ GridScratch grid_scratch(Workspace &w)
     const size_t cap = w.list_cap;
     GridScratch g{w.list,
                   w.surv_nd,
-                  w.first_bad,
+                  w.rest,
                   w.longs,
                   w.longs + cap,
                   w.longs + 2 * cap,

@@ -34,22 +34,16 @@ void give_block(const DeviceBlock &b);
 
 // Per-stream scratch of the batched motion path: survivor list + counters.
 struct Workspace {
-    int32_t *list = nullptr;
-    int32_t *first_bad = nullptr; // per survivor (chunk-parallel walk)
-    int32_t *surv_nd = nullptr;   // per survivor segment count (chunk-parallel walk)
-    double *surv_ab = nullptr;    // per survivor endpoints a, b (14 doubles)
-    int32_t *longs = nullptr;     // three words per survivor (grid walk: long items)
+    int32_t *list = nullptr;    // survivors' edges
+    int32_t *surv_nd = nullptr; // their segment counts
+    double *surv_ab = nullptr;  // and endpoints a, b (14 doubles)
+    int32_t *rest = nullptr;    // whether an item is unfinished
+    int32_t *longs = nullptr;   // three words per entry: long items
     size_t list_cap = 0;
-    // [0] survivor count, [1] walk queue (strategy 1, cleared per call);
-    // strategies 3 and 4: two sets of (survivor count, max positions) at
-    // [8..9] and [10..11], zero at creation.  A batch uses set `parity`; either
-    // its results kernel clears that set, or (no results kernel) its phase-1
-    // walk clears the other set and the next batch uses that one.
-    // The checks over the cell grid: two sets of two at [16..17] and
-    // [20..21], used in turn by grid_parity, each cleared by the batch before;
-    // from [64] on a word and a ticket per item of a one-launch batch.
+    // two sets of two at [16..17] and [20..21] (apart from each other's cache
+    // sector), used in turn by grid_parity, each cleared by the batch before;
+    // from [64] on a word and a ticket per item of a one-launch batch
     int32_t *counters = nullptr;
-    int parity = 0;
     int grid_parity = 0;
     // Held by a batch from choosing its counter set to enqueuing its launches
     // (and around resizing), so host threads that share a stream cannot pick
@@ -93,21 +87,6 @@ struct Tuning {
     int validity_shared_fk = 0;
 };
 
-// The launch shapes the library starts with stand for its own choice: batched
-// validity, motion, lastValid and list checks with these run over the
-// environment's cell grid (grid_check.hip), with shapes chosen by batch size.
-// Any other shapes ask for the kernels of checker.hip in those shapes.  The
-// block sizes and the waves per CU do not matter here: the grid kernels have
-// their own.
-inline bool own_validity_shape(const Tuning &t)
-{
-    return t.validity_lanes_per_state == 8 && t.validity_obstacle_parts == 2 && t.validity_shared_fk == 0;
-}
-inline bool own_walk_shape(const Tuning &t)
-{
-    return t.motion_lanes_per_state == 8 && t.motion_obstacle_parts == 1 && t.motion_strategy == 3;
-}
-
 Tuning get_tuning();
 // Rejects (OA_REQUIRE) a tuning whose shapes or limits are not built.
 void check_tuning(const Tuning &t);
@@ -123,21 +102,14 @@ Tuning tuning_from_c(const ompl_amd_tuning &t);
 
 // Device-resident obstacle set.
 struct Env {
-    // ns spheres (x,y,z,(R+r)^2), then nb boxes as (lo),(hi); each list in
-    // staging order (nearest to the arm's base first), for the checkers
+    // ns spheres (x,y,z,(R+r)^2), then nb boxes as (lo),(hi), in the caller's
+    // order, for the reference-order work accounting only
     float4 *obs = nullptr;
-    // the same words in the caller's order (same allocation), for the
-    // reference-order work accounting only
-    float4 *obs_input = nullptr;
-    // the same obstacles in the link layout's staging (spheres (x,y,z,bound^2),
-    // boxes, then the spheres' rr as floats), for kernels that read them from HBM
-    float4 *obs_links = nullptr;
     GridView grid{}; // cell grid (grid.hpp), in the same allocation
     int ns = 0;
     int nb = 0;
     size_t bytes = 0;
     EnvView view() const { return EnvView{obs, ns, nb}; }
-    EnvView input_view() const { return EnvView{obs_input, ns, nb}; }
 };
 
 // A planning query on a batch PRM roadmap (prm.hip): start and goal become
@@ -157,8 +129,8 @@ size_t prm_footprint(int64_t n_samples, int k);
 std::vector<int32_t> roadmap_shortest_path(const std::vector<int64_t> &off, const std::vector<int32_t> &adj,
                                            const std::vector<double> &nodes);
 
-// Largest obstacle set staged in LDS by one block (float4 words).
-constexpr int kMaxEnvWords = 4096; // 64 KiB of dynamic LDS
+// Largest obstacle set of an environment (float4 words).
+constexpr int kMaxEnvWords = 4096;
 
 } // namespace ompl_amd
 
@@ -168,8 +140,7 @@ struct ompl_amd_env_s {
     // ompl_amd_env_destroy refuses while any remain
     std::atomic<int> server_users{0};
     // launch shapes of this environment's batched checks, when set; else the
-    // library's current tuning (the fastest shape depends on the obstacle
-    // count: many obstacle partitions suit a dense scene, one a sparse one)
+    // library's current tuning
     mutable std::mutex tuning_mutex;
     bool has_tuning = false;
     ompl_amd::Tuning tuning{};

@@ -176,7 +176,8 @@ struct SliceArgs {
 
 static size_t env_stage_bytes(int ns, int nb)
 {
-    return (size_t)(pad_to(ns, kPlanPad) + 2 * pad_to(nb, kPlanPad)) * sizeof(float4) + (size_t)ns * sizeof(float);
+    auto pad = [](int n) { return (n + kPlanPad - 1) / kPlanPad * kPlanPad; };
+    return (size_t)(pad(ns) + 2 * pad(nb)) * sizeof(float4) + (size_t)ns * sizeof(float);
 }
 
 // Candidate nearest node: its distance and index; the lower index wins a tie.
@@ -1379,7 +1380,7 @@ static int plain_grow(const Env &env, HostTree &t, bool start_tree, const double
             E.a[k] = a[k];
             E.b[k] = b[k];
         }
-        launch_motion_single(env.view(), E, lvs, factor, tr.pinned_dev, tr.stream);
+        launch_motion_single(env.grid, E, lvs, factor, tr.pinned_dev, tr.stream);
         OA_HIP(hipStreamSynchronize(tr.stream));
         return tr.pinned[0] != 0;
     };
@@ -1390,7 +1391,7 @@ static int plain_grow(const Env &env, HostTree &t, bool start_tree, const double
     } else {
         State1 st;
         for (int k = 0; k < kDof; ++k) st.q[k] = dst[k];
-        launch_validate_single(env.view(), st, tr.pinned_dev, tr.stream);
+        launch_validate_single(env.grid, st, tr.pinned_dev, tr.stream);
         OA_HIP(hipStreamSynchronize(tr.stream));
         valid = tr.pinned[0] != 0 && check(dst, ns);
     }
@@ -1425,7 +1426,7 @@ static bool plain_usable(const Env &env, const double *q, ThreadResources &tr)
         if (q[k] - eps > kPi || q[k] + eps < -kPi) return false;
     State1 st;
     for (int k = 0; k < kDof; ++k) st.q[k] = q[k];
-    launch_validate_single(env.view(), st, tr.pinned_dev, tr.stream);
+    launch_validate_single(env.grid, st, tr.pinned_dev, tr.stream);
     OA_HIP(hipStreamSynchronize(tr.stream));
     return tr.pinned[0] != 0;
 }
@@ -1460,7 +1461,7 @@ static bool plain_prm(const ompl_amd_plan_request &req, const Env &env, ThreadRe
     for (int64_t r = 0; r < n; ++r) {
         State1 q;
         for (int d = 0; d < kDof; ++d) q.q[d] = smp[(size_t)r * kDof + d];
-        launch_validate_single(env.view(), q, tr.pinned_dev, tr.stream);
+        launch_validate_single(env.grid, q, tr.pinned_dev, tr.stream);
         OA_HIP(hipStreamSynchronize(tr.stream));
         if (tr.pinned[0] != 0) ms.push_back((int32_t)r);
     }
@@ -1508,7 +1509,7 @@ static bool plain_prm(const ompl_amd_plan_request &req, const Env &env, ThreadRe
             E.a[d] = nodes[(size_t)u * kDof + d];
             E.b[d] = nodes[(size_t)v * kDof + d];
         }
-        launch_motion_single(env.view(), E, req.longest_valid_segment, req.factor, tr.pinned_dev, tr.stream);
+        launch_motion_single(env.grid, E, req.longest_valid_segment, req.factor, tr.pinned_dev, tr.stream);
         OA_HIP(hipStreamSynchronize(tr.stream));
         if (tr.pinned[0] != 0) {
             nbr[(size_t)u].push_back(v);
