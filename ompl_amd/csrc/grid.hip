@@ -133,6 +133,7 @@ __global__ void __launch_bounds__(256) grid_build_kernel(GridView g, uint32_t *_
     span(z0, 4, g.oz, a[2], b[2]);
     int n = 0;
     bool many = false;
+    float rest = kClearMost; // clearance of the brick from the obstacles not picked
     for (int o0 = 0; o0 < g.n_obs; o0 += 64) {
         const int o = o0 + lane;
         bool near = false;
@@ -140,7 +141,9 @@ __global__ void __launch_bounds__(256) grid_build_kernel(GridView g, uint32_t *_
             const float4 lo = g.tab[2 * o], hi = g.tab[2 * o + 1];
             float least, most;
             box_range(a, b, lo, hi, least, most);
-            near = least <= sqrtf(lo.w) * (1.0f + kBoundRel) + kFarReach + 2.0f * kBoundAbs;
+            const float gap = least - (sqrtf(lo.w) * (1.0f + kBoundRel) + kBoundAbs);
+            near = !(gap > kFarReach + kBoundAbs);
+            if (!near) rest = fminf(rest, gap);
         }
         const uint64_t m = __ballot(near);
         const int at = n + __popcll(m & (((uint64_t)1 << lane) - 1));
@@ -158,7 +161,10 @@ __global__ void __launch_bounds__(256) grid_build_kernel(GridView g, uint32_t *_
     span(x, 1, g.ox, a[0], b[0]);
     span(y, 1, g.oy, a[1], b[1]);
     span(z, 1, g.oz, a[2], b[2]);
-    bool hit = false, far = true, clear = true;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) rest = fminf(rest, __shfl_xor(rest, d));
+    bool hit = false;
+    float clear = rest;
     int count = 0;
     for (int i = 0; i < n; ++i) {
         const int o = picked[w][i];
@@ -168,10 +174,10 @@ __global__ void __launch_bounds__(256) grid_build_kernel(GridView g, uint32_t *_
         const float r = sqrtf(lo.w), up = r * (1.0f + kBoundRel) + kBoundAbs, down = r * (1.0f - kBoundRel) - kBoundAbs;
         hit = hit || most < down;
         count += least <= up ? 1 : 0;
-        far = far && least > up + kFarReach + kBoundAbs;
-        clear = clear && least > up + kClearReach + kBoundAbs;
+        clear = fminf(clear, least - up);
     }
-    uint32_t word = far ? kCellFar : clear ? kCellClear : kCellFree;
+    // (no obstacle within `up`: the least gap is positive)
+    uint32_t word = (uint32_t)(fmaxf(clear, 0.0f) * kClearUnits);
     if (hit) word = kCellHit;
     else if (many || count > kCellList) word = kCellScan;
     const bool named = in && !hit && !many && count > 0 && count <= kCellList;
@@ -203,7 +209,7 @@ __global__ void __launch_bounds__(256) grid_build_kernel(GridView g, uint32_t *_
             else if (room) lists[at + k] = (uint16_t)o;
             ++k;
         }
-        word = want == 0 ? (ids << 8) | (uint32_t)count : room ? (at << 8) | (uint32_t)count : kCellScan;
+        word = want == 0 || room ? (want == 0 ? ids : at) | (uint32_t)count << 24 : kCellScan;
     }
     if (in) cells[((int64_t)x * g.ny + y) * g.nz + z] = word;
 }

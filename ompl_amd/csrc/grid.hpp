@@ -12,18 +12,21 @@
 
 namespace ompl_amd {
 
-// Cell words.  kCellFar, kCellClear: no obstacle touches a robot sphere centred
-// in the cell, nor one centred up to kFarReach, kClearReach from it; kCellFree:
-// none touches one in the cell; kCellHit: some obstacle touches every such sphere;
+// Cell words.  Top byte 0: no obstacle touches a robot sphere centred in the
+// cell, nor one centred up to word / kClearUnits metres from any point of it (the
+// cell's clearance).  kCellHit: some obstacle touches every such sphere;
 // kCellScan: any obstacle may; else the obstacles that may, their count in the
-// low byte (0 for the three clear words): one or two as 12-bit numbers above
-// it (id | id << 12), three to 253 as the offset of their list.  Only those
-// spheres need an exact test.
-constexpr uint32_t kCellFar = 0, kCellClear = 1u << 8, kCellFree = 2u << 8, kCellHit = 0xffffffffu, kCellScan = 0xfffffffeu;
+// top byte: one or two as 12-bit numbers below it (id | id << 12), three to 253
+// as the offset of their list.  Only those spheres need an exact test.
+constexpr uint32_t kCellHit = 0xffffffffu, kCellScan = 0xfe000000u, kCellNamed = 1u << 24;
 constexpr int kCellList = 253; // most obstacles of a list
+constexpr float kClearUnits = 4096.0f, kClearMost = 2.0f;
 // Distances from a link's second sphere to its fourth, the farthest, and to
-// its neighbours.
+// its neighbours; as clearances (units, with 1e-4 m for the rounding of centres)
+// from which a second sphere clears the whole link, and all but its last sphere.
 constexpr float kFarReach = 0.15f, kClearReach = 0.075f;
+constexpr uint32_t kFarUnits = (uint32_t)((kFarReach + 1e-4f) * kClearUnits) + 1,
+                   kClearReachUnits = (uint32_t)((kClearReach + 1e-4f) * kClearUnits) + 1;
 
 struct GridView {
     const uint32_t *cells; // [nx][ny][nz]

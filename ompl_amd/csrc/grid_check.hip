@@ -3,32 +3,39 @@
 //
 // A state is 28 sphere centres; the base link's four never move and are
 // decided when the environment is made.  Each of the other six links looks up
-// the cell of its second sphere: "far" clears the whole link, "clear" all but
-// its last sphere, else the cells of the other three are looked up as well.  Only spheres in a cell that some
-// obstacle's surface passes near are tested, against the obstacles the cell
-// lists, with the exact predicate (arm_device.hpp), so results are the same
-// bits as a test against every obstacle.  On the 128 + 128 obstacle scene that
-// is 6 to 24 reads of a 1 MiB table and a few exact tests per state where the
-// full test has 28 x 256.
+// the cell of its second sphere: its clearance may spare the whole link or all
+// but its last sphere; else the cells of the other three are looked up as well.
+// Only spheres in a cell that some obstacle's surface passes near are tested,
+// against the obstacles the cell lists, with the exact predicate
+// (arm_device.hpp), so results are the same bits as a test against every
+// obstacle.  On the 128 + 128 obstacle scene that is 6 to 24 reads of a 1 MiB
+// table and a few exact tests per state where the full test has 28 x 256.
+//
+// A walk need not look at every position either: the clearances of a state and
+// the joints' levers say how many positions before and after it are certainly
+// valid (with margins of 1e-4 m and more for the rounding of states and
+// centres), so of a roadmap's edges, 126 positions long, 31 are looked at and
+// then 32 more on average (wave_edges).
 //
 // Lane mapping: one state per lane (no redundant forward kinematics: the
 // fastest where there are states enough), or eight lanes per state, one link
 // each (a third of the latency, twice the instructions).
 //
-// Measured against the kernels that test every obstacle, in the launch shapes
+// Measured against the kernels that tested every obstacle, in the launch shapes
 // the library starts with: 65,536 states, 64 spheres 35.7 -> 8.7 us; 16,384
-// edges, 16 + 16 obstacles, checked counts 384 -> 62 us; 4,099 edges' lastValid
+// edges, 16 + 16 obstacles, checked counts 385 -> 44 us; 4,099 edges' lastValid
 // 110 -> 29 us; 61 edges, 128 + 128 obstacles 38 -> 8.8 us.  Against shapes
-// tuned for the scene: 16,384 edges, 128 + 128 obstacles 31 -> 19.3 us on one
-// stream, 12.6 -> 8.7 us a batch on four; 16 + 16 obstacles 77 -> 49 us (no
+// tuned for the scene: 16,384 edges, 128 + 128 obstacles 31 -> 19.0 us on one
+// stream, 12.6 -> 8.3 us a batch on four; 16 + 16 obstacles 77 -> 39 us (no
 // counts).  Large batches are bound by VALU instructions (about 1,100 a wave of
-// 64 states, half of them the forward kinematics), small ones by the chain of
-// dependent reads (counts, record, cells, cells, obstacles), by fetching the
-// code once and by the launches: a kernel that only walked what the one before
-// had left cost 3 to 4 us, so the survivors' kernel walks its own leftovers
-// (16,384 dense edges 22.2 -> 19.3 us, 11.3 -> 8.7 on four streams; 16 + 16
-// obstacles 68 -> 62) and a one-launch batch finds its own long items (61
-// edges 11.7 -> 8.8 us).
+// 64 states, half of them the forward kinematics): 836,000 roadmap edges, 64
+// spheres 4.8 ms with every position looked at, 1.3 ms with the gaps.  Small
+// ones are bound by the chain of dependent reads (counts, record, cells, cells,
+// obstacles), by fetching the code once and by the launches: a kernel that only
+// walked what the one before had left cost 3 to 4 us, so the survivors' kernel
+// walks its own leftovers (16,384 dense edges 22.2 -> 19.0 us, 11.3 -> 8.3 on
+// four streams) and a one-launch batch finds its own long items (61 edges 11.7
+// -> 8.8 us).
 #include <hip/hip_runtime.h>
 
 #include <climits>
@@ -217,21 +224,19 @@ struct Rounds {
 };
 
 // The walk of one item by a block: its positions below `end` from `first` on, a
-// block's at a time, `step` apart; or (own) by each wave for itself its item's
-// first 64 from `first` on.  The kernels below have one call of it each: the
-// code of a state check is 10 KB, and a short launch waits for every line of it.
+// block's at a time, `step` apart.  The kernels below have one call of it each:
+// the code of a state check is 10 KB, and a short launch waits for every line of it.
 // known: a long item's word (else null), which ends the walk once an earlier
 // position is known invalid.  Returns the lowest invalid position seen or
 // INT_MAX, uniform over the walkers.
 template <Walk MODE>
-__device__ __forceinline__ int walk_item(const GridWalkArgs &A, const Item<MODE> &I, int64_t first, int end, bool own,
+__device__ __forceinline__ int walk_item(const GridWalkArgs &A, const Item<MODE> &I, int64_t first, int end,
                                          int64_t step, const int32_t *known, Rounds &R, int &turn, WaveTests *tests)
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (int64_t round = first;;) {
-        const int64_t base = round + (own ? 0 : wave * 64);
+        const int64_t base = round + wave * 64;
         const int b = wave_walk<MODE>(A, I, (int)min(base, (int64_t)INT_MAX), end, tests);
-        if (own) return b;
         if (lane_id() == 0) R.bad[turn][wave] = b;
         if (threadIdx.x == 0) R.known[turn] = known ? known_bad(known) : INT_MAX;
         __syncthreads();
@@ -361,59 +366,240 @@ __global__ void __launch_bounds__(256) grid_endpoint8_kernel(GridWalkArgs A)
     }
 }
 
+// A wave's view of the edges it walks (LDS): a ring of edges, and a ring of the
+// states to look at, each an edge's slot and an index along it.
+struct WaveEdges {
+    static constexpr int kEdges = 8, kStates = 256;
+    struct Edge {
+        double ab[2 * kDof];
+        int32_t id, nd;
+        int bad; // lowest position found invalid
+        int end; // the edge is done when so many states have been looked at
+    } edge[kEdges];
+    int state[kStates]; // slot << 24 | index
+};
+struct BlockEdges {
+    WaveEdges wave[4];
+    int looked[4], held[4]; // of the waves' rings, while the block shares them
+};
+
+// The first 2^levels - 1 positions of the bisection are a complete binary tree
+// over the edge's interior: in order, the s-th of them (from 1) is the one with
+// this number (root 1).
+__device__ __forceinline__ int heap_of_slot(int s, int levels)
+{
+    const int up = __builtin_ctz(s);
+    return (1 << (levels - 1 - up)) + (s >> (up + 1));
+}
+
+// How fast the spheres of links 1 .. 6 move along an edge: a joint moves a
+// sphere by at most its angle times the sphere's distance from its axis, 0.3 m a
+// link between them and 0.2625 m on the last; an even joint turns its own link
+// about itself.  An edge with a coordinate beyond 16 rad, where rounding to FP32
+// would eat into the margin, gets no clearance.
+// `need` positions are worth looking closer for.
+__device__ __forceinline__ void edge_speeds(const double a[kDof], const double b[kDof], int nd, float need,
+                                            Speeds &sp)
+{
+    float d[kDof];
+    bool plain = true;
+#pragma unroll
+    for (int j = 0; j < kDof; ++j) {
+        d[j] = (float)fabs(b[j] - a[j]);
+        plain = plain && fabs(a[j]) <= 16.0 && fabs(b[j]) <= 16.0;
+    }
+    float most = 0.0f;
+#pragma unroll
+    for (int i = 1; i < kDof; ++i) {
+        float v = 0.0f;
+#pragma unroll
+        for (int j = 0; j <= i; ++j) {
+            const int links = (j & 1) ? i - j : i - j - 1;
+            if (links >= 0) v += d[j] * (0.3f * (float)links + 0.2625f);
+        }
+        v = v * 1.0001f + 1e-6f; // metres from end to end
+        most = fmaxf(most, v);
+        sp.steps[i - 1] = plain ? (float)nd / (v * kClearUnits) : 0.0f;
+    }
+    const uint32_t units = (uint32_t)(most * kClearUnits * (need / (float)max(nd, 1)));
+    sp.far = kFarUnits + units;
+    sp.near = kClearReachUnits + units;
+}
+
+// A wave's share of the survivors: pairs of edges first, first + step, ...  It
+// looks at 31 evenly spread positions of two edges at once (the first 31 of the
+// bisection, with s1 beside them for its clearance): how far the arm can move
+// from each before a sphere could touch anything says which of the positions
+// between them are certainly valid.  Only the others are looked at, 64 at a
+// time, from as many edges as that takes.  A wave that has taken its last pair
+// waits for the block's others, and they look at what is left together: a pair
+// of long edges leaves ten passes, which would be the launch's end (16,384
+// edges, 16 + 16 obstacles 56 us with every wave for itself, 39 together).
+// Looking at the middle of each gap and then of what that leaves takes fewer
+// states but more passes: 72 us.
+__device__ __forceinline__ void wave_edges(const GridWalkArgs &A, int n, int first, int step, BlockEdges &B,
+                                           WaveTests &tests)
+{
+    const int lane = lane_id(), half = lane >> 5, s = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    WaveEdges &W = B.wave[wave];
+    const bool counts = A.m.checked != nullptr;
+    int next = first;            // pair
+    int head = 0, tail = 0;      // edges: retired, taken
+    int looked = 0, listed = 0;  // states
+    int from = 1, to = 0;        // indices after the lane's position that are left to list
+    bool open = false;           // the last pair's states are being listed
+    auto sync = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    for (;;) {
+        const bool more = 2 * (int64_t)next < n; // else the waves of the block go on together
+        const int enough = more ? 64 : WaveEdges::kStates - 63;
+        if (open) { // list states until there are enough, or no more
+            if (!counts && W.edge[(tail - 2 + half) % WaveEdges::kEdges].bad != INT_MAX) to = -1;
+            uint64_t m = wave_ballot(from <= to);
+            while (m && listed - looked < enough) {
+                if (from <= to)
+                    W.state[(listed + __popcll(m & (((uint64_t)1 << lane) - 1))) % WaveEdges::kStates] =
+                        (tail - 2 + half) % WaveEdges::kEdges << 24 | from++;
+                listed += __popcll(m);
+                m = wave_ballot(from <= to);
+            }
+            if (m == 0) {
+                open = false;
+                if (s == 0) W.edge[(tail - 2 + half) % WaveEdges::kEdges].end = listed;
+            }
+            sync();
+        }
+        if (!open) { // results of the edges that are done
+            const int slot = (head + lane) % WaveEdges::kEdges;
+            const bool ready = lane < tail - head && W.edge[slot].end <= looked;
+            if (ready && W.edge[slot].id >= 0) {
+                const int id = W.edge[slot].id, bad = W.edge[slot].bad;
+                A.m.out[id] = bad == INT_MAX ? 1 : 0;
+                if (A.m.checked) A.m.checked[id] = bad == INT_MAX ? W.edge[slot].nd : bad + 1;
+            }
+            head += __popcll(wave_ballot(ready));
+        }
+        const bool pair = more && !open && listed - looked < 64 && tail - head + 2 <= WaveEdges::kEdges;
+        int index = 0, position = 0, done = 0;
+        bool live;
+        WaveEdges::Edge *E;
+        if (pair) {
+            const int item = 2 * next + half;
+            E = &W.edge[(tail + half) % WaveEdges::kEdges];
+            if (item < n && s < 2 * kDof) E->ab[s] = A.m.surv_ab[(int64_t)item * 2 * kDof + s];
+            if (s == 2 * kDof) {
+                const int nd = item < n ? A.m.surv_nd[item] : 1;
+                const bool mine = item < n && nd - 1 <= kLongWalk;
+                E->nd = mine ? nd : 1; // a long one's turn comes
+                E->id = mine ? A.m.list[item] : -1;
+                E->bad = INT_MAX;
+                E->end = INT_MAX;
+            }
+            sync();
+            const int nd = E->nd;
+            // slots in order, or (short edges) positions in order
+            position = nd > 32 ? (s ? heap_of_slot(s, 5) : 0) : s;
+            live = position > 0 ? position < nd : nd > 32;
+            index = live && position > 0 ? bisection_index(position - 1, nd) : 0;
+        } else if (more) {
+            // (a ring full of edges whose states are all looked at cannot be: they are retired)
+            done = min(64, listed - looked);
+            live = lane < done;
+            const int st = live ? W.state[(looked + lane) % WaveEdges::kStates] : 0;
+            E = &W.edge[live ? st >> 24 : head % WaveEdges::kEdges];
+            index = st & 0xffffff;
+        } else {
+            if (lane == 0) {
+                B.looked[wave] = looked;
+                B.held[wave] = listed - looked;
+            }
+            __syncthreads();
+            // the block's next 256 states, ring after ring
+            int at = threadIdx.x, ring = -1, before = 0, st = 0;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const int held = __builtin_amdgcn_readfirstlane(B.held[w]);
+                if (w == wave) done = min(max(256 - before, 0), held);
+                if (ring < 0 && at < held) ring = w;
+                if (ring < 0) at -= held;
+                before += held;
+            }
+            if (before == 0) break; // of all four waves
+            live = ring >= 0;
+            if (live) st = B.wave[ring].state[(B.looked[ring] + at) % WaveEdges::kStates];
+            E = &B.wave[live ? ring : 0].edge[live ? st >> 24 : 0];
+            index = st & 0xffffff;
+        }
+        const int nd = live ? E->nd : 1;
+        float q[kDof], steps;
+        Speeds sp;
+        {
+            double a[kDof], b[kDof];
+#pragma unroll
+            for (int j = 0; j < kDof; ++j) {
+                a[j] = E->ab[j];
+                b[j] = E->ab[kDof + j];
+            }
+            interpolate_f32<kDof>(a, b, (double)index / (double)nd, q);
+            sp.far = kFarUnits;
+            sp.near = kClearReachUnits;
+            if (pair) edge_speeds(a, b, nd, (float)nd * (0.5f / 32.0f) + 1.0f, sp);
+        }
+        const bool hit = state_hit1<true>(A.g, q, live, tests, sp, &steps);
+        if (pair) {
+            if (hit && position > 0) atomicMin(&E->bad, position);
+            const int k = hit || !live ? 0 : (int)fminf(steps, 65536.0f);
+            sync();
+            // what neither this position nor the next one reaches
+            const int right = __shfl(index - k, lane + 1);
+            from = index + k + 1;
+            to = s == 31 ? E->nd - 1 : right - 1;
+            if (E->nd <= 32 || E->bad != INT_MAX) to = -1; // all looked at, or invalid: the first positions come first
+            next += step;
+            tail += 2;
+            open = true;
+        } else {
+            if (hit) atomicMin(&E->bad, 1 + bisection_rank(index, nd));
+            looked += done;
+            sync();
+            if (!more) __syncthreads(); // the others have read this ring
+        }
+    }
+}
+
 // Survivors of the s2 pass: when there are no more than blocks, a block walks
-// each to its end; else its waves walk the first 64 positions of one each (an
-// edge that fails does so early, and one wave finds out without the other
-// three), then the block what is left of them.  Last, all blocks together walk
-// the long ones.
+// each to its end; else waves walk pairs of them (an edge that fails does so
+// early, and half a wave finds out).  Last, all blocks together walk the long
+// ones.
 __global__ void __launch_bounds__(256, 4) grid_survivors_kernel(GridWalkArgs A)
 {
     __shared__ Rounds R;
     __shared__ WaveTests tests[4];
+    __shared__ BlockEdges edges;
     clear_next(A);
     const int n = A.counts[0], n_long = A.counts[1];
     const bool wide = n <= (int)gridDim.x;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), groups = wide ? n : (n + 3) / 4;
-    int turn = 0, group = 0, l = -1;
-    int64_t next = blockIdx.x;
-    unsigned open = 0; // items of the group that are unfinished
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (!wide) wave_edges(A, n, blockIdx.x * 4 + wave, gridDim.x * 4, edges, tests[wave]);
+    int turn = 0, l = -1;
     Item<Walk::kBisect> I;
-    for (;;) {
-        int slot, from = 1;
-        bool own = false, is_long = false;
-        if (open) {
-            slot = 4 * group + __builtin_ctz(open);
-            open &= open - 1;
-            from = 65;
-        } else if (next < groups) {
-            group = (int)next;
-            next += gridDim.x;
-            own = !wide;
-            slot = wide ? group : 4 * group + wave;
-        } else if (++l < n_long) {
+    for (int64_t next = wide ? blockIdx.x : n;;) {
+        const bool is_long = next >= n;
+        int slot = (int)next;
+        if (is_long) {
+            if (++l >= n_long) break;
             slot = A.long_slot[l];
-            is_long = true;
-        } else {
-            break;
         }
-        I.survivor(A.m, min(slot, n - 1));
-        const bool mine = slot < n && (is_long || I.total - 1 <= kLongWalk);
-        if (!own && !mine) continue; // a long item's turn comes (block-uniform)
-        const int end = !mine ? 0 : own ? min(I.total, 65) : I.total;
-        const int b = walk_item(A, I, from + (is_long ? (int64_t)blockIdx.x * 256 : 0), end, own,
+        next += gridDim.x;
+        I.survivor(A.m, slot);
+        if (!is_long && I.total - 1 > kLongWalk) continue; // its turn comes (block-uniform)
+        const int b = walk_item(A, I, 1 + (is_long ? (int64_t)blockIdx.x * 256 : 0), I.total,
                                 is_long ? (int64_t)gridDim.x * 256 : 256, is_long ? &A.long_bad[l] : nullptr, R, turn,
                                 tests);
-        if (own) {
-            const bool left = mine && b == INT_MAX && end < I.total;
-            if (lane_id() == 0) {
-                if (mine && !left) I.result(A, b);
-                R.bad[turn][wave] = left ? 1 : 0;
-            }
-            __syncthreads();
-            open = __builtin_amdgcn_readfirstlane(R.bad[turn][0] | R.bad[turn][1] << 1 | R.bad[turn][2] << 2 |
-                                                  R.bad[turn][3] << 3);
-            turn ^= 1;
-        } else if (threadIdx.x == 0) {
+        if (threadIdx.x == 0) { // (no `continue` for the other lanes: they would walk on without this one)
             if (is_long) finish_long(A, I, b, &A.long_bad[l], &A.ticket[l], gridDim.x);
             else I.result(A, b);
         }
@@ -453,17 +639,18 @@ __global__ void __launch_bounds__(256, 4) grid_wide_kernel(GridWalkArgs A)
         const bool none = I.nd_too_many(); // reported invalid without a walk (its s2 is looked at)
         if (helper < 0 && !none && I.total - from > kLongWalk) return;
         const int end = none ? (MODE == Walk::kBisect ? 1 : 0) : I.total;
-        const int b = walk_item(A, I, from + (int64_t)max(helper, 0) * 256, end, false,
+        const int b = walk_item(A, I, from + (int64_t)max(helper, 0) * 256, end,
                                 helper < 0 ? 256 : (int64_t)kHelpers * 256, helper < 0 ? nullptr : &A.wide_bad[id], R,
                                 turn, tests);
-        if (threadIdx.x != 0) continue;
-        if (none) {
-            A.m.out[id] = 0;
-            if (A.m.checked) A.m.checked[id] = b == 0 ? 1 : 0;
-        } else if (helper < 0) {
-            I.result(A, b);
-        } else {
-            finish_long(A, I, b, &A.wide_bad[id], &A.wide_ticket[id], kHelpers);
+        if (threadIdx.x == 0) {
+            if (none) {
+                A.m.out[id] = 0;
+                if (A.m.checked) A.m.checked[id] = b == 0 ? 1 : 0;
+            } else if (helper < 0) {
+                I.result(A, b);
+            } else {
+                finish_long(A, I, b, &A.wide_bad[id], &A.wide_ticket[id], kHelpers);
+            }
         }
     }
 }
@@ -537,12 +724,13 @@ __global__ void __launch_bounds__(256, 4) grid_rest_kernel(GridWalkArgs A)
         }
         if (MODE == Walk::kList) I.list(A, slot);
         else I.survivor(A.m, slot);
-        const int b = walk_item(A, I, from + (is_long ? (int64_t)blockIdx.x * 256 : 0), I.total, false,
+        const int b = walk_item(A, I, from + (is_long ? (int64_t)blockIdx.x * 256 : 0), I.total,
                                 is_long ? (int64_t)gridDim.x * 256 : 256, is_long ? &A.long_bad[l] : nullptr, R, turn,
                                 tests);
-        if (threadIdx.x != 0) continue;
-        if (is_long) finish_long(A, I, b, &A.long_bad[l], &A.ticket[l], gridDim.x);
-        else I.result(A, b);
+        if (threadIdx.x == 0) { // (no `continue` for the other lanes: they would walk on without this one)
+            if (is_long) finish_long(A, I, b, &A.long_bad[l], &A.ticket[l], gridDim.x);
+            else I.result(A, b);
+        }
     }
 }
 
@@ -564,7 +752,7 @@ __global__ void __launch_bounds__(256, 4) grid_motion_single_kernel(GridView g, 
     I.total = max(I.nd, 1);
     int turn = 0;
     int b = 0; // too many segments: invalid
-    if (!I.nd_too_many()) b = walk_item(A, I, 0, I.total, false, 256, nullptr, R, turn, tests);
+    if (!I.nd_too_many()) b = walk_item(A, I, 0, I.total, 256, nullptr, R, turn, tests);
     if (threadIdx.x == 0) *result = b == INT_MAX ? 1 : 0;
 }
 

@@ -61,11 +61,11 @@ struct Tests {
             const float4 t = w.item[i];
             const uint32_t wd = __float_as_uint(t.w), owner = w.owner[i];
             const bool scan = wd == kCellScan;
-            const int m = scan ? g.n_obs : (int)(wd & 255u);
+            const int m = scan ? g.n_obs : (int)(wd >> 24);
 #pragma unroll 1
             for (int k = 0; k < m; ++k) { // once, but for a cell in twenty
-                int o = (int)(wd >> (k == 0 ? 8 : 20)) & 0xfff;
-                if (m > 2) o = scan ? k : (int)g.lists[(wd >> 8) + k];
+                int o = (int)(wd >> (k == 0 ? 0 : 12)) & 0xfff;
+                if (m > 2) o = scan ? k : (int)g.lists[(wd & 0xffffffu) + k];
                 if (obstacle_hit(g, o, t.x, t.y, t.z)) {
                     atomicOr(&w.hit[owner >> 5], 1u << (owner & 31));
                     break;
@@ -79,7 +79,7 @@ struct Tests {
     // One sphere (at p + Z off) of each `look` lane in a cell with word wd.
     __device__ __forceinline__ void sphere(bool look, uint32_t wd, const float p[3], const float Z[3], float off)
     {
-        const bool c = look && (wd & 255u) != 0;
+        const bool c = look && wd >= kCellNamed;
         const uint64_t m = wave_ballot(c);
         if (m == 0) return;
         const int lane = lane_id();
@@ -107,10 +107,32 @@ __device__ __forceinline__ bool odd_state(const float q[kDof])
     return nan || !(m < 6000.0f);
 }
 
-// One state per lane.
-__device__ __forceinline__ bool state_hit1(const GridView &g, const float q[kDof], bool live, WaveTests &lds)
+// Clearance of a cell, in units; 0 where an obstacle may touch a sphere.
+__device__ __forceinline__ uint32_t clearance(uint32_t word)
 {
+    return word < kCellNamed ? word : 0u;
+}
+
+__device__ __forceinline__ bool at_least(uint32_t word, uint32_t clear)
+{
+    return word - clear < kCellNamed - clear;
+}
+
+// How fast a motion's spheres move, for turning clearances into positions.
+struct Speeds {
+    float steps[kDof - 1]; // positions that link 1 .. 6 needs for one unit of clearance
+    uint32_t far, near;    // clearances of a second sphere that spare the look at the others
+};
+
+// One state per lane.  CLEAR: also how many positions before and after this one
+// are certainly valid if it is (`steps`), as far as the cells tell.
+template <bool CLEAR = false>
+__device__ __forceinline__ bool state_hit1(const GridView &g, const float q[kDof], bool live, WaveTests &lds,
+                                           const Speeds &sp = {}, float *steps = nullptr)
+{
+    if (CLEAR) *steps = 0.0f;
     if (g.base_hit) return live;
+    const uint32_t far = CLEAR ? sp.far : kFarUnits, near = CLEAR ? sp.near : kClearReachUnits;
     const bool odd = odd_state(q);
     float X[3] = {1.0f, 0.0f, 0.0f}, Y[3] = {0.0f, 1.0f, 0.0f}, Z[3] = {0.0f, 0.0f, 1.0f}, p[3] = {0.0f, 0.0f, 0.0f};
     float P[kDof - 1][3], W[kDof - 1][3];
@@ -155,11 +177,13 @@ __device__ __forceinline__ bool state_hit1(const GridView &g, const float q[kDof
     uint32_t v[kDof - 1][4];
 #pragma unroll
     for (int i = 0; i + 1 < kDof; ++i) {
-        const bool look = live && !hit && w[i] != kCellFar;
+        const uint32_t c = w[i];
+        const bool look = live && !hit && !at_least(c, far);
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
-            v[i][m] = m == 1 ? w[i] : kCellFree;
-            if (m != 1 && look && (m == 3 || w[i] != kCellClear))
+            // a sphere that is not looked at has at least what is left of the second's
+            v[i][m] = m == 1 ? w[i] : c - (m == 3 ? kFarUnits : kClearReachUnits);
+            if (m != 1 && look && (m == 3 || !at_least(c, near)))
                 v[i][m] = odd ? kCellScan
                               : cell_word(g, P[i][0] + W[i][0] * sphere_offset(m),
                                           P[i][1] + W[i][1] * sphere_offset(m),
@@ -169,6 +193,17 @@ __device__ __forceinline__ bool state_hit1(const GridView &g, const float q[kDof
 #pragma unroll
     for (int i = 0; i + 1 < kDof; ++i) hit = hit || v[i][0] == kCellHit || v[i][2] == kCellHit || v[i][3] == kCellHit;
     if (wave_ballot(live && !hit) == 0) return hit && live;
+    if (CLEAR) {
+        float least = INFINITY;
+#pragma unroll
+        for (int i = 0; i + 1 < kDof; ++i) {
+            uint32_t c = clearance(v[i][0]);
+#pragma unroll
+            for (int m = 1; m < 4; ++m) c = min(c, clearance(v[i][m]));
+            least = fminf(least, (float)c * sp.steps[i]);
+        }
+        *steps = odd ? 0.0f : least;
+    }
     // the few centres that are tested are made again from the frames: kept, all
     // 24 would take 72 registers
 #pragma unroll
@@ -201,7 +236,7 @@ __device__ __forceinline__ bool state_hit8(const GridView &g, float qj, bool liv
     // the link's cells are read together: one round trip
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
-        w[m] = kCellFar;
+        w[m] = 0;
         if (mine)
             w[m] = odd ? kCellScan
                        : cell_word(g, p[0] + Z[0] * sphere_offset(m), p[1] + Z[1] * sphere_offset(m),

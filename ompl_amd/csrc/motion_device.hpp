@@ -65,6 +65,26 @@ __host__ __device__ __forceinline__ int bisection_index(int p, int nd)
     return (a + b) >> 1;
 }
 
+// Which check (0-based) visits index idx (in [1, nd-1]): the inverse of
+// bisection_index.
+__host__ __device__ __forceinline__ int bisection_rank(int idx, int nd)
+{
+    const int L = ilog2_u32((uint32_t)(nd - 1));
+    int a = 1, b = nd - 1, l = 0, i = 0, leaves = 0;
+    for (;;) {
+        const int mid = (a + b) >> 1;
+        if (mid == idx) return l < L ? (1 << l) - 1 + i : (1 << L) - 1 + leaves;
+        i = 2 * i + (idx > mid ? 1 : 0);
+        if (idx > mid) {
+            leaves += ((b - a) >> 1) - ((1 << (L - l - 1)) - 1);
+            a = mid + 1;
+        } else {
+            b = mid - 1;
+        }
+        ++l;
+    }
+}
+
 // StateSpace::validSegmentCount (base/src/StateSpace.cpp:851-854) over
 // RealVectorStateSpace::distance (base/spaces/src/RealVectorStateSpace.cpp:230-242).
 // segments_of: from the squared distance.
