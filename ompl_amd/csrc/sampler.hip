@@ -205,7 +205,9 @@ __global__ void __launch_bounds__(kValidThreads) sample_valid_kernel(ValidArgs A
         }
         __syncthreads(); // the draws are read: their room is free
         const bool live = t < m;
-        const bool valid = live && !state_hit1(A.g, q, live, w.tests[wave]);
+        // every lane of the wave goes in (the exact tests are shared among all 64)
+        const bool hit = state_hit1(A.g, q, live, w.tests[wave]);
+        const bool valid = live && !hit;
         const uint64_t vb = __ballot(valid);
         if (lane == 0) valid_bits[wave] = vb;
         __syncthreads();
