@@ -24,7 +24,7 @@
 // Measured against the kernels that tested every obstacle, in the launch shapes
 // the library starts with: 65,536 states, 64 spheres 35.7 -> 8.7 us; 16,384
 // edges, 16 + 16 obstacles, checked counts 385 -> 44 us; 4,099 edges' lastValid
-// 110 -> 29 us; 61 edges, 128 + 128 obstacles 38 -> 8.8 us.  Against shapes
+// 110 -> 24 us; 61 edges, 128 + 128 obstacles 38 -> 8.8 us.  Against shapes
 // tuned for the scene: 16,384 edges, 128 + 128 obstacles 31 -> 19.0 us on one
 // stream, 12.6 -> 8.3 us a batch on four; 16 + 16 obstacles 77 -> 39 us (no
 // counts).  Large batches are bound by VALU instructions (about 1,100 a wave of
@@ -272,20 +272,6 @@ __device__ __forceinline__ void list_long(const GridWalkArgs &A, int slot)
     A.ticket[l] = 0;
 }
 
-// Keeps an edge for grid_rest_kernel under `slot` (one lane).
-template <Walk MODE>
-__device__ __forceinline__ void keep_edge(const GridWalkArgs &A, const Item<MODE> &I, int slot)
-{
-    A.m.list[slot] = (int32_t)I.id;
-    A.m.surv_nd[slot] = I.nd;
-    double *ab = A.m.surv_ab + (int64_t)slot * 2 * kDof;
-#pragma unroll
-    for (int j = 0; j < kDof; ++j) {
-        ab[j] = I.a[j];
-        ab[kDof + j] = I.b[j];
-    }
-}
-
 __device__ __forceinline__ void clear_next(const GridWalkArgs &A)
 {
     if (blockIdx.x == 0 && threadIdx.x < 2) A.next[threadIdx.x] = 0;
@@ -426,20 +412,22 @@ __device__ __forceinline__ void edge_speeds(const double a[kDof], const double b
     sp.near = kClearReachUnits + units;
 }
 
-// A wave's share of the survivors: pairs of edges first, first + step, ...  It
-// looks at 31 evenly spread positions of two edges at once (the first 31 of the
-// bisection, with s1 beside them for its clearance): how far the arm can move
-// from each before a sphere could touch anything says which of the positions
-// between them are certainly valid.  Only the others are looked at, 64 at a
+// A wave's share of the survivors (kBisect) or edges (kSequence): pairs first,
+// first + step, ...  It looks at 31 evenly spread positions of two edges at once
+// (the first 31 of the bisection; beside them s1, for its clearance, or s2): how
+// far the arm can move from each before a sphere could touch anything says which
+// of the positions between them are certainly valid.  Only the others are looked at, 64 at a
 // time, from as many edges as that takes.  A wave that has taken its last pair
 // waits for the block's others, and they look at what is left together: a pair
 // of long edges leaves ten passes, which would be the launch's end (16,384
 // edges, 16 + 16 obstacles 56 us with every wave for itself, 39 together).
 // Looking at the middle of each gap and then of what that leaves takes fewer
 // states but more passes: 72 us.
+template <Walk MODE>
 __device__ __forceinline__ void wave_edges(const GridWalkArgs &A, int n, int first, int step, BlockEdges &B,
                                            WaveTests &tests)
 {
+    constexpr bool kSeq = MODE == Walk::kSequence;
     const int lane = lane_id(), half = lane >> 5, s = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     WaveEdges &W = B.wave[wave];
@@ -457,7 +445,10 @@ __device__ __forceinline__ void wave_edges(const GridWalkArgs &A, int n, int fir
         const bool more = 2 * (int64_t)next < n; // else the waves of the block go on together
         const int enough = more ? 64 : WaveEdges::kStates - 63;
         if (open) { // list states until there are enough, or no more
-            if (!counts && W.edge[(tail - 2 + half) % WaveEdges::kEdges].bad != INT_MAX) to = -1;
+            // an invalid edge: nothing more, or (in order) what comes before
+            const int bad = W.edge[(tail - 2 + half) % WaveEdges::kEdges].bad;
+            if (kSeq) to = min(to, bad - 1);
+            else if (!counts && bad != INT_MAX) to = -1;
             uint64_t m = wave_ballot(from <= to);
             while (m && listed - looked < enough) {
                 if (from <= to)
@@ -476,9 +467,13 @@ __device__ __forceinline__ void wave_edges(const GridWalkArgs &A, int n, int fir
             const int slot = (head + lane) % WaveEdges::kEdges;
             const bool ready = lane < tail - head && W.edge[slot].end <= looked;
             if (ready && W.edge[slot].id >= 0) {
-                const int id = W.edge[slot].id, bad = W.edge[slot].bad;
+                const int id = W.edge[slot].id, bad = W.edge[slot].bad, nd = W.edge[slot].nd;
                 A.m.out[id] = bad == INT_MAX ? 1 : 0;
-                if (A.m.checked) A.m.checked[id] = bad == INT_MAX ? W.edge[slot].nd : bad + 1;
+                if (kSeq) {
+                    if (bad != INT_MAX) A.last_t[id] = (double)(min(bad, nd) - 1) / (double)nd;
+                } else if (A.m.checked) {
+                    A.m.checked[id] = bad == INT_MAX ? nd : bad + 1;
+                }
             }
             head += __popcll(wave_ballot(ready));
         }
@@ -489,21 +484,43 @@ __device__ __forceinline__ void wave_edges(const GridWalkArgs &A, int n, int fir
         if (pair) {
             const int item = 2 * next + half;
             E = &W.edge[(tail + half) % WaveEdges::kEdges];
-            if (item < n && s < 2 * kDof) E->ab[s] = A.m.surv_ab[(int64_t)item * 2 * kDof + s];
+            if (item < n && s < 2 * kDof)
+                E->ab[s] = !kSeq       ? A.m.surv_ab[(int64_t)item * 2 * kDof + s]
+                           : s < kDof ? A.m.a[(int64_t)s * A.m.n + item]
+                                      : A.m.b[(int64_t)(s - kDof) * A.m.n + item];
+            int nd = 1;
+            if (kSeq) {
+                sync();
+                if (item < n) nd = valid_segment_count<kDof>(E->ab, E->ab + kDof, A.m.lvs, A.m.factor);
+            } else if (item < n && s == 2 * kDof) {
+                nd = A.m.surv_nd[item];
+            }
+            const bool mine = item < n && nd - 1 <= kLongWalk;
             if (s == 2 * kDof) {
-                const int nd = item < n ? A.m.surv_nd[item] : 1;
-                const bool mine = item < n && nd - 1 <= kLongWalk;
                 E->nd = mine ? nd : 1; // a long one's turn comes
-                E->id = mine ? A.m.list[item] : -1;
+                E->id = !mine ? -1 : kSeq ? item : A.m.list[item];
                 E->bad = INT_MAX;
                 E->end = INT_MAX;
             }
+            if (kSeq && item < n && !mine) {
+                if (nd > kMaxSegments) { // reported invalid without a walk
+                    if (s == 0) A.m.out[item] = 0;
+                } else {
+                    if (s < 2 * kDof) A.m.surv_ab[(int64_t)item * 2 * kDof + s] = E->ab[s];
+                    if (s == 2 * kDof) {
+                        A.m.list[item] = item;
+                        A.m.surv_nd[item] = nd;
+                        list_long(A, item);
+                    }
+                }
+            }
             sync();
-            const int nd = E->nd;
-            // slots in order, or (short edges) positions in order
+            nd = E->nd;
+            // in order, or (short edges) all of them; lane 0 of a half: s1 or s2
             position = nd > 32 ? (s ? heap_of_slot(s, 5) : 0) : s;
-            live = position > 0 ? position < nd : nd > 32;
+            live = position > 0 ? position < nd : kSeq ? E->id >= 0 : nd > 32;
             index = live && position > 0 ? bisection_index(position - 1, nd) : 0;
+            if (kSeq && position == 0) index = max(nd, 1);
         } else if (more) {
             // (a ring full of edges whose states are all looked at cannot be: they are retired)
             done = min(64, listed - looked);
@@ -534,6 +551,7 @@ __device__ __forceinline__ void wave_edges(const GridWalkArgs &A, int n, int fir
             index = st & 0xffffff;
         }
         const int nd = live ? E->nd : 1;
+        const bool end = kSeq && index >= nd; // s2 itself
         float q[kDof], steps;
         Speeds sp;
         {
@@ -544,25 +562,30 @@ __device__ __forceinline__ void wave_edges(const GridWalkArgs &A, int n, int fir
                 b[j] = E->ab[kDof + j];
             }
             interpolate_f32<kDof>(a, b, (double)index / (double)nd, q);
+            if (kSeq) {
+#pragma unroll
+                for (int j = 0; j < kDof; ++j) q[j] = end ? (float)b[j] : q[j];
+            }
             sp.far = kFarUnits;
             sp.near = kClearReachUnits;
             if (pair) edge_speeds(a, b, nd, (float)nd * (0.5f / 32.0f) + 1.0f, sp);
         }
         const bool hit = state_hit1<true>(A.g, q, live, tests, sp, &steps);
         if (pair) {
-            if (hit && position > 0) atomicMin(&E->bad, position);
+            if (hit && (kSeq || position > 0)) atomicMin(&E->bad, kSeq ? index : position);
             const int k = hit || !live ? 0 : (int)fminf(steps, 65536.0f);
             sync();
             // what neither this position nor the next one reaches
-            const int right = __shfl(index - k, lane + 1);
-            from = index + k + 1;
-            to = s == 31 ? E->nd - 1 : right - 1;
-            if (E->nd <= 32 || E->bad != INT_MAX) to = -1; // all looked at, or invalid: the first positions come first
+            const int right = __shfl(index - k, s == 31 ? lane - 31 : lane + 1);
+            from = kSeq && s == 0 ? 1 : index + k + 1;
+            to = !kSeq && s == 31 ? E->nd - 1 : right - 1;
+            // all looked at, or invalid: the bisection's first positions come first
+            if (E->nd <= 32 || (!kSeq && E->bad != INT_MAX)) to = -1;
             next += step;
             tail += 2;
             open = true;
         } else {
-            if (hit) atomicMin(&E->bad, 1 + bisection_rank(index, nd));
+            if (hit) atomicMin(&E->bad, kSeq ? index : 1 + bisection_rank(index, nd));
             looked += done;
             sync();
             if (!more) __syncthreads(); // the others have read this ring
@@ -583,7 +606,7 @@ __global__ void __launch_bounds__(256, 4) grid_survivors_kernel(GridWalkArgs A)
     const int n = A.counts[0], n_long = A.counts[1];
     const bool wide = n <= (int)gridDim.x;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (!wide) wave_edges(A, n, blockIdx.x * 4 + wave, gridDim.x * 4, edges, tests[wave]);
+    if (!wide) wave_edges<Walk::kBisect>(A, n, blockIdx.x * 4 + wave, gridDim.x * 4, edges, tests[wave]);
     int turn = 0, l = -1;
     Item<Walk::kBisect> I;
     for (int64_t next = wide ? blockIdx.x : n;;) {
@@ -655,47 +678,48 @@ __global__ void __launch_bounds__(256, 4) grid_wide_kernel(GridWalkArgs A)
     }
 }
 
-// More edges (kSequence) or lists: a wave walks the first 64 positions of each.
-template <Walk MODE>
+// More edges in order (kSequence): waves walk pairs of them.
+__global__ void __launch_bounds__(256, 4) grid_sequence_kernel(GridWalkArgs A)
+{
+    __shared__ WaveTests tests[4];
+    __shared__ BlockEdges edges;
+    clear_next(A);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    wave_edges<Walk::kSequence>(A, (int)A.m.n, blockIdx.x * 4 + wave, gridDim.x * 4, edges, tests[wave]);
+}
+
+// More lists: a wave walks the first 64 states of each.
 __global__ void __launch_bounds__(256, 4) grid_first_kernel(GridWalkArgs A)
 {
     __shared__ WaveTests tests[4];
     clear_next(A);
     const int64_t id = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (id >= A.m.n) return;
-    constexpr int from = MODE == Walk::kSequence ? 1 : 0;
-    Item<MODE> I;
-    if (MODE == Walk::kList) {
-        I.list(A, id);
-    } else {
-        I.edge(A.m, id);
-    }
-    const int slot = (int)id, done = I.nd_too_many() ? 0 : min(I.total, from + 64);
-    const int b = wave_walk(A, I, from, done, tests);
+    Item<Walk::kList> I;
+    I.list(A, id);
+    const int slot = (int)id, done = min(I.total, 64);
+    const int b = wave_walk(A, I, 0, done, tests);
     if (lane_id() != 0) return;
     bool left = false;
-    if (I.nd_too_many()) { // reported invalid without a walk
-        A.m.out[id] = 0;
-    } else if (b != INT_MAX || done == I.total) {
+    if (b != INT_MAX || done == I.total) {
         I.result(A, b);
     } else {
-        if (MODE != Walk::kList) keep_edge(A, I, slot);
         left = I.total - done <= kLongWalk;
         if (!left) list_long(A, slot);
     }
     A.rest[slot] = left;
 }
 
-// What the first kernel left: a block per item; then all blocks together the
-// long ones.
+// What the kernel before left: a block per list; then all blocks together the
+// long edges or lists.
 template <Walk MODE>
 __global__ void __launch_bounds__(256, 4) grid_rest_kernel(GridWalkArgs A)
 {
     __shared__ Rounds R;
     __shared__ WaveTests tests[4];
-    constexpr int from = (MODE == Walk::kSequence ? 1 : 0) + 64;
+    constexpr int from = MODE == Walk::kSequence ? 1 : 64;
     const int n_long = A.counts[1];
-    const int64_t n = A.m.n;
+    const int64_t n = MODE == Walk::kSequence ? 0 : A.m.n;
     Item<MODE> I;
     const int lane = lane_id();
     // the block's slots are blockIdx.x + i gridDim.x (every wave reads the same
@@ -817,12 +841,17 @@ static void launch_wide(const GridWalkArgs &A, hipStream_t s)
     OA_HIP(hipGetLastError());
 }
 
+// Edges in order or lists.
 template <Walk MODE>
 static void launch_items(const GridWalkArgs &A, hipStream_t s)
 {
     if (A.m.n <= kWideItems) return launch_wide<MODE>(A, s);
-    hipLaunchKernelGGL((grid_first_kernel<MODE>), dim3(grid_of(A.m.n, 4)), dim3(256), 0, s, A);
-    hipLaunchKernelGGL((grid_rest_kernel<MODE>), dim3((unsigned)num_cus() * 4), dim3(256), 0, s, A);
+    const unsigned blocks = (unsigned)num_cus();
+    if (MODE == Walk::kSequence)
+        hipLaunchKernelGGL(grid_sequence_kernel, dim3(blocks * 8), dim3(256), 0, s, A);
+    else
+        hipLaunchKernelGGL(grid_first_kernel, dim3(grid_of(A.m.n, 4)), dim3(256), 0, s, A);
+    hipLaunchKernelGGL((grid_rest_kernel<MODE>), dim3(blocks * 4), dim3(256), 0, s, A);
     OA_HIP(hipGetLastError());
 }
 

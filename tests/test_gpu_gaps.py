@@ -1,5 +1,5 @@
 """Walks that leave out the positions which the clearance of their neighbours
-proves valid, against the oracle (validity and checked counts): small obstacles
+proves valid, against the oracle (validity, checked counts, lastValid): small obstacles
 that an edge may touch between the positions looked at first, resolutions from a
 few positions an edge to thousands, the sizes at which a walk changes shape (31,
 32, 33 positions), coordinates at and beyond the range that clearances hold for."""
@@ -48,3 +48,8 @@ def test_edges_between_points(gpu, oracle, lvs, lo, hi, n_obs, offset):
     assert np.array_equal(v.cpu().numpy(), rv) and np.array_equal(c.cpu().numpy(), rc)
     assert np.array_equal(gpu.check_motions(env, A, B, lvs).cpu().numpy(), rv)
     assert 0 < rv.sum() < N
+    lv, lt = gpu.check_motions_last_valid(env, A, B, lvs)
+    lv, lt = lv.cpu().numpy(), lt.cpu().numpy()
+    assert np.array_equal(lv, rv) and np.isnan(lt[rv == 1]).all()
+    for i in np.flatnonzero(rv == 0)[:400]:
+        assert lt[i] == oracle.check_motion_last_valid(oenv, a[i], b[i], lvs)[1], i
