@@ -407,7 +407,7 @@ __device__ __forceinline__ void edge_speeds(const double a[kDof], const double b
         most = fmaxf(most, v);
         sp.steps[i - 1] = plain ? (float)nd / (v * kClearUnits) : 0.0f;
     }
-    const uint32_t units = (uint32_t)(most * kClearUnits * (need / (float)max(nd, 1)));
+    const uint32_t units = plain ? (uint32_t)(most * kClearUnits * (need / (float)max(nd, 1))) : 0u;
     sp.far = kFarUnits + units;
     sp.near = kClearReachUnits + units;
 }
