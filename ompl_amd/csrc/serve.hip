@@ -29,7 +29,7 @@
 // trapped step changes nothing but the draws, so up to 32 of them run at once
 // (16 lanes each), the first valid one is committed, and the pass costs about
 // 9 us.  64 requests over eight scenes of up to 128 obstacles, 48,900 steps,
-// the longest request 2,128 of them: 4.1 ms (11.3 before: eight at
+// the longest request 2,128 of them: 3.3 ms (11.3 before: eight at
 // a time, each tested against every obstacle, and copies of commands, results, end states and
 // paths around every slice, which the kernel now reads and writes in pinned memory).
 //
@@ -610,13 +610,23 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
         // rest are dropped (their draws are not consumed).  Same steps, same
         // results as one at a time.  m stays within the iterations left.
         // (not while a goal state is due: the goal tree would change between
-        // the steps)
+        // the steps)  The first connect step towards a node just added (phase 1)
+        // is usually TRAPPED too, and then likewise changes nothing: it goes
+        // before the sampling steps of a round as its step 0, which saves it a
+        // pass of its own (64 requests over eight scenes 4.1 -> 3.3 ms).
         const bool goal_due = n1 == 0 || (sampled_goals < C.n_goals && sampled_goals < n1 / 2);
         const int lanes = spec_lanes(max(n0, n1));
-        const int m = phase == 0 && !goal_due ? min(min(kSpec, NT / lanes), C.max_iters - iteration) : 0;
+        const int m = phase <= 1 && !goal_due ? min(min(kSpec, NT / lanes), C.max_iters - iteration) : 0;
+        int gs = kTrapped;
+        bool grown = false; // step 0 was a connect step that was not TRAPPED
         if (m >= 2) {
-            need_draws(kDof * m);
-            if (tid < kDof * m) s_samp[tid] = (kPi - -kPi) * draw(tid) + -kPi;
+            const int first = phase; // steps before the sampling steps
+            // whether step j's tgi.start (it grows the start tree)
+            auto from_start = [&](int j, int start) { return j < first ? start : start ^ ((j - first) & 1); };
+            const int start0 = start_tree; // in phase 1 tgi.start, too
+            need_draws(kDof * (m - first));
+            if (tid < kDof * m)
+                s_samp[tid] = tid < kDof * first ? s_rstate[tid] : (kPi - -kPi) * draw(tid - kDof * first) + -kPi;
             __syncthreads();
             if (tid == 0) {
                 c1 = wall_clock64();
@@ -625,7 +635,7 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
             const int wave = tid >> 6, lane = tid & 63;
             if (wave * 64 < m * lanes) {
                 const int step = lanes == 64 ? wave : tid / 16, sub = tid & (lanes - 1), j = min(step, m - 1);
-                const int st_j = start_tree ^ (j & 1);
+                const int st_j = from_start(j, start0);
                 const int tree_j = st_j ? 0 : 1;
                 const Tree Tj = tree(tree_j);
                 double tgt[kDof];
@@ -688,7 +698,7 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
                     for (int r = wave / each; r > 0; --r) rest &= rest - 1;
                     const int j = lowest_bit(rest);
                     const StepMotion M{s_ga + kDof * j, s_gb + kDof * j, s_gx + kDof * j, s_nd[j], s_npos[j],
-                                       ((start_tree ^ j) & 1) == 0};
+                                       !from_start(j, start0)};
                     const int p = checked + 8 * (wave % each) + (lane >> 3);
                     if (wave_ballot(wave_hit8(g, M, p, s_tests[wave])) && lane == 0) s_bad[j] = 1;
                 }
@@ -699,13 +709,15 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
             }
             // take the steps in order: those before the first open one together
             // (all TRAPPED), then that one
+            phase = 0; // where a connect step that was TRAPPED leaves the loop
             for (int taken = 0; taken < steps_here;) {
                 const int j = open ? lowest_bit(open) : steps_here;
                 const uint64_t before = ((uint64_t)1 << j) - 1;
+                const int samples = max(j, first) - max(taken, first);
                 steps += j - taken;
                 checks += __popcll(moved_steps & before & ~(((uint64_t)1 << taken) - 1));
-                pidx += kDof * (j - taken);
-                start_tree ^= (j - taken) & 1; // RRTConnect.cpp:249
+                pidx += kDof * samples;
+                start_tree ^= samples & 1; // RRTConnect.cpp:249
                 iteration += j - taken;
                 taken = j;
                 if (j == steps_here) {
@@ -717,8 +729,10 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
                 ++checks; // an open step has moved
                 const StepMotion M{s_ga + kDof * j, s_gb + kDof * j, s_gx + kDof * j, s_nd[j], s_npos[j], !st_j};
                 const bool valid = block_check<NT>(g, M, checked, s_tests); // what is left of it
-                start_tree = !start_tree;
-                pidx += kDof; // this step's sample is consumed
+                if (j >= first) {
+                    start_tree = !start_tree;
+                    pidx += kDof; // this step's sample is consumed
+                }
                 ++taken;
                 open &= open - 1;
                 if (!valid) {
@@ -738,117 +752,123 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
                     status = OMPL_AMD_PLAN_TREE_FULL;
                     break;
                 }
+                xmotion = last;
+                if (j < first) { // the solve loop goes on below
+                    gs = s_reach[j] ? kReached : kAdvanced;
+                    phase = 1;
+                    grown = true;
+                    break;
+                }
                 // rstate: the sample when reached, else the new state
                 if (tid < kDof) s_rstate[tid] = s_reach[j] ? s_samp[kDof * j + tid] : s_gx[kDof * j + tid];
-                xmotion = last;
                 added = last;
                 tgi_start = start_tree;
                 grow_tree = start_tree ? 0 : 1; // otherTree
                 phase = 1;
                 break;
             }
-            if (tid == 0) {
-                const int64_t c3 = wall_clock64();
-                t_check += c3 - c1;
-                t_step += c3 - c0;
+            if (tid == 0) t_check += wall_clock64() - c1;
+            if (!grown) {
+                if (tid == 0) t_step += wall_clock64() - c0;
+                continue;
             }
-            continue;
         }
-        if (phase == 0) {
-            // RRTConnect.cpp:247-250: pick the tree, flip startTree_
-            grow_tree = start_tree ? 0 : 1;
-            tgi_start = start_tree;
-            start_tree = !start_tree;
-            // RRTConnect.cpp:251-269: goal states (GoalStates, in order) --
-            // every remaining one tried while the goal tree is empty
-            // (nextGoal(ptc)), else one while fewer than half the goal tree's
-            // size have been handed out (nextGoal())
-            if (n1 == 0 || sampled_goals < n1 / 2) {
-                const bool empty = n1 == 0;
-                while (sampled_goals < C.n_goals) {
-                    const int goal = sampled_goals++;
-                    if (endpoint_usable(g, R.ends + (size_t)(kMaxEnds + goal) * kDof, s_x, s_tests)) {
-                        if (n1 >= C.cap) {
-                            status = OMPL_AMD_PLAN_TREE_FULL;
-                        } else {
-                            if (tid < kDof) tree(1).set(tid, n1, s_x[tid]);
-                            if (tid == 0) R.parent[1][n1] = -1;
-                            ++n1;
+        if (!grown) {
+            if (phase == 0) {
+                // RRTConnect.cpp:247-250: pick the tree, flip startTree_
+                grow_tree = start_tree ? 0 : 1;
+                tgi_start = start_tree;
+                start_tree = !start_tree;
+                // RRTConnect.cpp:251-269: goal states (GoalStates, in order) --
+                // every remaining one tried while the goal tree is empty
+                // (nextGoal(ptc)), else one while fewer than half the goal tree's
+                // size have been handed out (nextGoal())
+                if (n1 == 0 || sampled_goals < n1 / 2) {
+                    const bool empty = n1 == 0;
+                    while (sampled_goals < C.n_goals) {
+                        const int goal = sampled_goals++;
+                        if (endpoint_usable(g, R.ends + (size_t)(kMaxEnds + goal) * kDof, s_x, s_tests)) {
+                            if (n1 >= C.cap) {
+                                status = OMPL_AMD_PLAN_TREE_FULL;
+                            } else {
+                                if (tid < kDof) tree(1).set(tid, n1, s_x[tid]);
+                                if (tid == 0) R.parent[1][n1] = -1;
+                                ++n1;
+                            }
+                            __syncthreads();
+                            break;
                         }
                         __syncthreads();
+                        if (!empty) break;
+                    }
+                    if (status == OMPL_AMD_PLAN_RUNNING && n1 == 0) status = OMPL_AMD_PLAN_INVALID_GOAL;
+                    if (status != OMPL_AMD_PLAN_RUNNING) break;
+                }
+                // sampler_->sampleUniform(rstate): RNG::uniformReal(-pi, pi) per joint,
+                // from the next seven draws
+                need_draws(kDof);
+                if (tid < kDof) s_rstate[tid] = (kPi - -kPi) * draw(tid) + -kPi;
+                pidx += kDof;
+                __syncthreads();
+                if (tid == 0) {
+                    c1 = wall_clock64();
+                    t_sample += c1 - c0;
+                }
+            }
+
+            // ---- growTree(tree, tgi, rmotion) (RRTConnect.cpp:116-196)
+            double tgt[kDof];
+#pragma unroll
+            for (int k = 0; k < kDof; ++k) tgt[k] = s_rstate[k];
+            const int nt = grow_tree ? n1 : n0;
+            const Tree T = tree(grow_tree);
+            const Near best = block_nearest<NT>(T, nt, tgt, s_wd, s_wi);
+            if (tid == 0) {
+                const int64_t c2 = wall_clock64();
+                t_nearest += c2 - c1;
+                c1 = c2;
+            }
+            Steer S;
+            S.run(T, nt, best, tgt, C.maxd);
+            if (S.moved) {
+                // tgi.start ? checkMotion(nearest, dst) : isValid(dst) && checkMotion(dst, nearest)
+                const bool from_start = tgi_start != 0;
+                double a[kDof], b[kDof];
+#pragma unroll
+                for (int k = 0; k < kDof; ++k) {
+                    a[k] = from_start ? S.nst[k] : S.x[k];
+                    b[k] = from_start ? S.x[k] : S.nst[k];
+                }
+                const int nd = valid_segment_count<kDof>(a, b, C.lvs, C.factor);
+                if (tid == 0) {
+                    for (int k = 0; k < kDof; ++k) {
+                        s_a[k] = a[k];
+                        s_b[k] = b[k];
+                        s_x[k] = S.x[k];
+                    }
+                }
+                __syncthreads();
+                ++checks;
+                bool valid = false;
+                if (nd <= kMaxSegments) { // longer motions are reported invalid
+                    const StepMotion M{s_a, s_b, s_x, nd, StepMotion::positions(nd, !from_start), !from_start};
+                    valid = !__syncthreads_or(wave_hit8(g, M, tid >> 3, s_tests[tid >> 6])) &&
+                            block_check<NT>(g, M, NT / 8, s_tests);
+                }
+                if (valid) {
+                    const int last = append_step<NT>(T, parents(grow_tree), grow_tree ? n1 : n0, S.nm, s_a, s_b, s_x,
+                                                     nd, from_start, C.inter != 0);
+                    if (last < 0) {
+                        status = OMPL_AMD_PLAN_TREE_FULL;
                         break;
                     }
-                    __syncthreads();
-                    if (!empty) break;
-                }
-                if (status == OMPL_AMD_PLAN_RUNNING && n1 == 0) status = OMPL_AMD_PLAN_INVALID_GOAL;
-                if (status != OMPL_AMD_PLAN_RUNNING) break;
-            }
-            // sampler_->sampleUniform(rstate): RNG::uniformReal(-pi, pi) per joint,
-            // from the next seven draws
-            need_draws(kDof);
-            if (tid < kDof) s_rstate[tid] = (kPi - -kPi) * draw(tid) + -kPi;
-            pidx += kDof;
-            __syncthreads();
-            if (tid == 0) {
-                c1 = wall_clock64();
-                t_sample += c1 - c0;
-            }
-        }
-
-        // ---- growTree(tree, tgi, rmotion) (RRTConnect.cpp:116-196)
-        double tgt[kDof];
-#pragma unroll
-        for (int k = 0; k < kDof; ++k) tgt[k] = s_rstate[k];
-        const int nt = grow_tree ? n1 : n0;
-        const Tree T = tree(grow_tree);
-        const Near best = block_nearest<NT>(T, nt, tgt, s_wd, s_wi);
-        if (tid == 0) {
-            const int64_t c2 = wall_clock64();
-            t_nearest += c2 - c1;
-            c1 = c2;
-        }
-        Steer S;
-        S.run(T, nt, best, tgt, C.maxd);
-        int gs = kTrapped;
-        if (S.moved) {
-            // tgi.start ? checkMotion(nearest, dst) : isValid(dst) && checkMotion(dst, nearest)
-            const bool from_start = tgi_start != 0;
-            double a[kDof], b[kDof];
-#pragma unroll
-            for (int k = 0; k < kDof; ++k) {
-                a[k] = from_start ? S.nst[k] : S.x[k];
-                b[k] = from_start ? S.x[k] : S.nst[k];
-            }
-            const int nd = valid_segment_count<kDof>(a, b, C.lvs, C.factor);
-            if (tid == 0) {
-                for (int k = 0; k < kDof; ++k) {
-                    s_a[k] = a[k];
-                    s_b[k] = b[k];
-                    s_x[k] = S.x[k];
+                    xmotion = last;
+                    gs = S.reach ? kReached : kAdvanced;
                 }
             }
-            __syncthreads();
-            ++checks;
-            bool valid = false;
-            if (nd <= kMaxSegments) { // longer motions are reported invalid
-                const StepMotion M{s_a, s_b, s_x, nd, StepMotion::positions(nd, !from_start), !from_start};
-                valid = !__syncthreads_or(wave_hit8(g, M, tid >> 3, s_tests[tid >> 6])) &&
-                        block_check<NT>(g, M, NT / 8, s_tests);
-            }
-            if (valid) {
-                const int last = append_step<NT>(T, parents(grow_tree), grow_tree ? n1 : n0, S.nm, s_a, s_b, s_x,
-                                                 nd, from_start, C.inter != 0);
-                if (last < 0) {
-                    status = OMPL_AMD_PLAN_TREE_FULL;
-                    break;
-                }
-                xmotion = last;
-                gs = S.reach ? kReached : kAdvanced;
-            }
+            ++steps;
+            if (tid == 0) t_check += wall_clock64() - c1;
         }
-        ++steps;
-        if (tid == 0) t_check += wall_clock64() - c1;
 
         // ---- solve loop (RRTConnect.cpp:245-330)
         bool end_iteration = false;
