@@ -64,8 +64,9 @@ struct Tests {
             const int m = scan ? g.n_obs : (int)(wd >> 24);
 #pragma unroll 1
             for (int k = 0; k < m; ++k) { // once, but for a cell in twenty
-                int o = (int)(wd >> (k == 0 ? 0 : 12)) & 0xfff;
-                if (m > 2) o = scan ? k : (int)g.lists[(wd & 0xffffffu) + k];
+                // (a scan of one or two obstacles, too, goes by k: its word names none)
+                int o = scan ? k : (int)(wd >> (k == 0 ? 0 : 12)) & 0xfff;
+                if (!scan && m > 2) o = (int)g.lists[(wd & 0xffffffu) + k];
                 if (obstacle_hit(g, o, t.x, t.y, t.z)) {
                     atomicOr(&w.hit[owner >> 5], 1u << (owner & 31));
                     break;
