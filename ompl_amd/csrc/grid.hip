@@ -52,11 +52,11 @@ void grid_extent(GridView &g, const double lo[3], const double hi[3], bool empty
         longest = std::max(longest, b[k] - a[k]);
     }
     if (none) { // nothing within reach: one cell, which the build finds far from everything
+        // (the obstacles stay: a state beyond the sine's range is tested against them)
         g.nx = g.ny = g.nz = 1;
         g.ox = g.oy = g.oz = 0.0f;
         g.inv = 0.0f;
         g.sx = g.sy = g.sz = 0.0f;
-        g.n_obs = 0;
         return;
     }
     // two cells more on each side: a point outside the grid takes the border

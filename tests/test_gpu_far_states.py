@@ -1,6 +1,6 @@
 """States beyond the sine's range are tested against every obstacle: in scenes
 of one to three obstacles, where a scan's length is that of a cell that names
-its obstacles.
+its obstacles, and in scenes none of whose obstacles is within the arm's reach.
 GPU parity with the CPU oracle in both lane mappings and through motions,
 lastValid and state lists."""
 import numpy as np
@@ -72,3 +72,19 @@ def test_walks_of_few_obstacles(gpu, oracle, name, n):
     v, f = gpu.check_state_lists(env, dev(b_.T), dev(np.array([0, n // 2, n], np.int64)))
     for i, part in enumerate((ok[:n // 2], ok[n // 2:])):
         assert v.cpu().numpy()[i] == part.all() and f.cpu().numpy()[i] == (-1 if part.all() else np.argmin(part))
+
+
+@pytest.mark.parametrize("n", [500, 140_000])
+def test_nothing_in_reach(gpu, oracle, n):
+    """Beyond 1e8 rad the polynomial's centres leave the workspace, and may
+    meet an obstacle that no arm can reach."""
+    s = np.array([[0, 0, 300.0, 290.0]], np.float32)
+    b = np.array([[-900.0, 0, 0, 890.0, 890.0, 890.0]], np.float32)
+    env, oenv = gpu.Env(s, b), oracle.OracleEnv(s, b)
+    rng = np.random.default_rng(n)
+    q = rng.uniform(-PI, PI, (7, n)).astype(np.float32)
+    far = rng.choice(n, n // 4, replace=False)
+    q[rng.integers(1, 6, n // 4), far] = rng.uniform(1e8, 9e8, n // 4).astype(np.float32)
+    want = oracle.validate_states_mt(oenv, q, 8)
+    assert (want == 0).sum() > 10 and want[np.setdiff1d(np.arange(n), far)].all()
+    assert np.array_equal(gpu.validate_states(env, dev(q)).cpu().numpy(), want)
