@@ -58,10 +58,13 @@ struct NNIndex {
     uint32_t *xn_max = nullptr; // max |x|^2 as FP32 bits (non-negative), then the extents (kStatWords words)
     int64_t n_removed = 0;
     std::vector<uint8_t> removed_host;
-    // spatial index of the first tree.m points; the stream of its last use,
-    // and whether it was used on others since it was built
+    // spatial index of the first tree.m points; whether it was built since its
+    // arrays were allocated, on which stream (an event after the last build, for
+    // calls on other streams), and whether it was used on others since
     NNTree tree;
+    bool tree_live = false;
     hipStream_t tree_stream = nullptr;
+    hipEvent_t tree_built = nullptr;
     bool tree_mixed = false;
     // per-call scratch (grow-only)
     void *scratch = nullptr;
@@ -895,12 +898,20 @@ static void reserve(NNIndex &x, int64_t need, hipStream_t s)
         tree_reserve(x.tree, cap, x.dim, x.tdim);
     else
         tree_free(x.tree);
+    x.tree_live = x.tree_mixed = false;
 }
 
 // Notes a use of the index on stream s.
 static void tree_used(NNIndex &x, hipStream_t s)
 {
-    if (x.tree_stream != s) x.tree_mixed = true;
+    if (x.tree_live && x.tree_stream != s) x.tree_mixed = true;
+}
+
+// Lets stream s wait for the last build, which an ompl_amd_nn_add_dev may have
+// left pending on its own stream.
+static void after_build(NNIndex &x, hipStream_t s)
+{
+    if (x.tree_live && x.tree_stream != s) OA_HIP(hipStreamWaitEvent(s, x.tree_built, 0));
 }
 
 // Brings the index up to date once a tail of 512 points, or of 1/128 of the
@@ -912,9 +923,13 @@ static void tree_update(NNIndex &x, hipStream_t s)
     if (!x.tree.mem || x.n < kTreeMinPoints || x.n - x.tree.m < std::max<int64_t>(512, x.tree.m / 128)) return;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return; // the tail grows
-    // the arrays are rewritten: wait for readers on other streams
-    if (x.tree.m > 0 && (x.tree_mixed || x.tree_stream != s)) OA_HIP(hipDeviceSynchronize());
+    // the arrays are rewritten: wait for readers and for a build on other streams
+    // (also after a clear, which leaves them to finish)
+    if (x.tree_live && (x.tree_mixed || x.tree_stream != s)) OA_HIP(hipDeviceSynchronize());
+    if (!x.tree_built) OA_HIP(hipEventCreateWithFlags(&x.tree_built, hipEventDisableTiming));
     tree_build(x.tree, x.pts, x.removed, x.xn_max + kStatLo, x.xn_max + kStatHi, x.n, x.dim, x.tdim, s);
+    OA_HIP(hipEventRecord(x.tree_built, s));
+    x.tree_live = true;
     x.tree_stream = s;
     x.tree_mixed = false;
 }
@@ -1352,6 +1367,7 @@ int ompl_amd_nn_destroy(ompl_amd_nn h)
         OA_HIP(hipDeviceSynchronize()); // searches on any stream may use the arrays
         for (const DeviceBlock &b : x.blocks) give_block(b);
         if (x.scratch) OA_HIP(hipFree(x.scratch));
+        if (x.tree_built) OA_HIP(hipEventDestroy(x.tree_built));
         tree_free(x.tree);
         delete h;
     });
@@ -1362,6 +1378,7 @@ int ompl_amd_nn_clear(ompl_amd_nn h)
     return guarded([&] {
         NNIndex &x = nn_of(h);
         hipStream_t s = default_stream();
+        after_build(x, s);
         if (x.n && x.removed) OA_HIP(hipMemsetAsync(x.removed, 0, (size_t)x.n, s));
         hipLaunchKernelGGL(clear_stats_kernel, dim3(1), dim3(64), 0, s, x.xn_max);
         OA_HIP(hipStreamSynchronize(s));
@@ -1402,6 +1419,7 @@ int ompl_amd_nn_remove(ompl_amd_nn h, int64_t id, int *removed)
             const uint8_t one = 1;
             hipStream_t s = default_stream();
             OA_HIP(hipMemcpyAsync(x.removed + id, &one, 1, hipMemcpyHostToDevice, s));
+            after_build(x, s); // a pending one would leave the id's place unwritten, or put the point back
             tree_remove(x.tree, id, s);
             OA_HIP(hipStreamSynchronize(s));
             ++x.n_removed;
