@@ -315,10 +315,13 @@ int ompl_amd_nn_add_dev(ompl_amd_nn nn, const float *pts_dev, int64_t n, int64_t
 /* Remove by id (lazy: the id is excluded from every later query). */
 int ompl_amd_nn_remove(ompl_amd_nn nn, int64_t id, int *removed);
 int ompl_amd_nn_size(ompl_amd_nn nn, int64_t *size);
-/* Rebuild the acceleration structure after adds (called implicitly by queries). */
+/* Nothing to do: additions keep the acceleration structure up to date. */
 int ompl_amd_nn_build(ompl_amd_nn nn, void *stream);
 /* k nearest of nq queries (device row-major [nq][dim]); out_idx_dev [nq][k]
- * (-1 past the end), out_dist_dev [nq][k] (+inf past the end). */
+ * (-1 past the end), out_dist_dev [nq][k] (+inf past the end).  A search that
+ * was captured into a graph searches, at each replay, the ids that were there
+ * at its capture, as they then are (removed, or added anew after a clear); it
+ * ends with the structure's capacity (1,024 points, doubled as needed). */
 int ompl_amd_nn_knn_dev(ompl_amd_nn nn, const float *q_dev, int64_t nq, int k, int32_t *out_idx_dev,
                         float *out_dist_dev, void *stream);
 /* Radius search, CSR results sorted by (distance, id) per query:

@@ -71,6 +71,15 @@ inline hipStream_t resolve_stream(void *s)
 }
 void ensure_init();
 
+// Whether launches on s are being recorded into a graph.
+inline bool stream_capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+    (void)hipGetLastError(); // the null stream beside a capture: its launches say so themselves
+    return false;
+}
+
 // Number of compute units of the library's device (for persistent grids).
 int num_cus();
 

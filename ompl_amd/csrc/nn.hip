@@ -55,7 +55,7 @@ struct NNIndex {
     float *pts = nullptr;      // [cap][dim]
     float *xt = nullptr;       // [cap/32][ksteps][64] tiled augmented points
     uint8_t *removed = nullptr;
-    uint32_t *xn_max = nullptr; // max |x|^2 as FP32 bits (non-negative), then the extents (kStatWords words)
+    uint32_t *xn_max = nullptr; // max |x|^2 as FP32 bits (non-negative), the extents, tree.m (kStatWords words)
     int64_t n_removed = 0;
     std::vector<uint8_t> removed_host;
     // spatial index of the first tree.m points; whether it was built since its
@@ -66,6 +66,7 @@ struct NNIndex {
     hipStream_t tree_stream = nullptr;
     hipEvent_t tree_built = nullptr;
     bool tree_mixed = false;
+    bool tree_captured = false; // some search was captured, and may be replayed at any time
     // per-call scratch (grow-only)
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
@@ -668,17 +669,18 @@ __global__ void radius_unpack_kernel(const uint64_t *__restrict__ keys, int64_t 
 
 // Writes tiled augmented rows for points [from, to) and the padding of the
 // last tile; tracks max |x|^2 and the extents of the first coordinates
-// (stats: kStatNorm, kStatLo, kStatHi).  The figures meet in LDS, and a block
+// (stats: kStatNorm, kStatLo, kStatHi; kStatLive, the points in the spatial
+// index, is the build's).  The figures meet in LDS, and a block
 // makes a device-wide atomic only for one that it improves (one atomic per
 // point took 187 us of adding 1,000,000).
-constexpr int kStatNorm = 0, kStatLo = 8, kStatHi = 16, kStatWords = 24;
+constexpr int kStatNorm = 0, kStatLo = 8, kStatHi = 16, kStatTracked = 24, kStatLive = 24, kStatWords = 25;
 
 __global__ void __launch_bounds__(256) build_xt_kernel(const float *__restrict__ pts, int dim, int tdim, int ksteps,
                                                        int64_t from, int64_t to, int64_t n_total,
                                                        float *__restrict__ xt, uint32_t *__restrict__ stats)
 {
-    __shared__ uint32_t blk[kStatWords];
-    if (threadIdx.x < kStatWords) blk[threadIdx.x] = threadIdx.x >= kStatLo && threadIdx.x < kStatHi ? ~0u : 0u;
+    __shared__ uint32_t blk[kStatTracked];
+    if (threadIdx.x < kStatTracked) blk[threadIdx.x] = threadIdx.x >= kStatLo && threadIdx.x < kStatHi ? ~0u : 0u;
     __syncthreads();
     const int64_t p = from + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool real = p < n_total && p < to;
@@ -716,7 +718,7 @@ __global__ void __launch_bounds__(256) build_xt_kernel(const float *__restrict__
         }
     }
     __syncthreads();
-    if (threadIdx.x < kStatWords) {
+    if (threadIdx.x < kStatTracked) {
         const uint32_t v = blk[threadIdx.x];
         const uint32_t have = __hip_atomic_load(&stats[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (threadIdx.x >= kStatLo && threadIdx.x < kStatHi) {
@@ -901,10 +903,13 @@ static void reserve(NNIndex &x, int64_t need, hipStream_t s)
     x.tree_live = x.tree_mixed = false;
 }
 
-// Notes a use of the index on stream s.
-static void tree_used(NNIndex &x, hipStream_t s)
+// Notes a use of the index on stream s, and whether it is being captured.
+static bool tree_used(NNIndex &x, hipStream_t s)
 {
     if (x.tree_live && x.tree_stream != s) x.tree_mixed = true;
+    const bool captured = stream_capturing(s);
+    if (captured) x.tree_captured = true;
+    return captured;
 }
 
 // Lets stream s wait for the last build, which an ompl_amd_nn_add_dev may have
@@ -921,14 +926,15 @@ static void after_build(NNIndex &x, hipStream_t s)
 static void tree_update(NNIndex &x, hipStream_t s)
 {
     if (!x.tree.mem || x.n < kTreeMinPoints || x.n - x.tree.m < std::max<int64_t>(512, x.tree.m / 128)) return;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return; // the tail grows
+    if (stream_capturing(s)) return; // the tail grows
     // the arrays are rewritten: wait for readers and for a build on other streams
     // (also after a clear, which leaves them to finish)
-    if (x.tree_live && (x.tree_mixed || x.tree_stream != s)) OA_HIP(hipDeviceSynchronize());
+    if (x.tree_live && (x.tree_mixed || x.tree_captured || x.tree_stream != s)) OA_HIP(hipDeviceSynchronize());
     if (!x.tree_built) OA_HIP(hipEventCreateWithFlags(&x.tree_built, hipEventDisableTiming));
-    tree_build(x.tree, x.pts, x.removed, x.xn_max + kStatLo, x.xn_max + kStatHi, x.n, x.dim, x.tdim, s);
+    tree_build(x.tree, x.pts, x.removed, x.xn_max + kStatLo, x.xn_max + kStatHi, x.xn_max + kStatLive, x.n,
+               x.dim, x.tdim, s);
     OA_HIP(hipEventRecord(x.tree_built, s));
+    if (x.tree_captured) OA_HIP(hipStreamSynchronize(s)); // a replay need not wait for an addition
     x.tree_live = true;
     x.tree_stream = s;
     x.tree_mixed = false;
@@ -945,9 +951,10 @@ static bool use_tree(const NNIndex &x)
     return tree_supported(x.metric, x.dim) && x.n - x.tree.m <= std::max<int64_t>(kTreeMinPoints, x.tree.m / 8);
 }
 
-static TreeView tree_view(const NNIndex &x)
+static TreeView tree_view(const NNIndex &x, bool captured)
 {
-    return TreeView{x.tree.sp, x.tree.sid, x.tree.b0, x.tree.b1, x.tree.b2, x.tree.m, x.n, x.pts, x.removed};
+    return TreeView{x.tree.sp, x.tree.sid, x.tree.b0, x.tree.b1, x.tree.b2, x.tree.m, x.n,
+                    captured ? x.xn_max + kStatLive : nullptr, x.pts, x.removed};
 }
 
 static void append(NNIndex &x, const float *src, int64_t n, bool src_dev, hipStream_t s)
@@ -1099,9 +1106,9 @@ static void knn(NNIndex &x, const float *q, int64_t nq, int k, const int32_t *kq
         char *buf = head ? (char *)scratch(x, head) : nullptr;
         ProfScope ps("nn_knn", s);
         if (kq) packed_offsets(kq, nq, k, (int64_t *)buf, buf + counts_bytes, cub_bytes, out_off, s);
-        tree_used(x, s);
+        const bool captured = tree_used(x, s);
         tree_knn(x.metric, x.dim,
-                 TreeKnnArgs{tree_view(x), q, nq, k, kq, kq ? out_off : nullptr, out_d, out_i}, s);
+                 TreeKnnArgs{tree_view(x, captured), q, nq, k, kq, kq ? out_off : nullptr, out_d, out_i}, s);
         return;
     }
     const int kmax = k <= 16 ? 16 : (k <= 32 ? 32 : 64);
@@ -1197,7 +1204,8 @@ static void radius(NNIndex &x, const float *q, int64_t nq, float r, const float 
     const size_t order_bytes = tree ? tree_order_bytes(x.tree, nq) : 0;
     const uint32_t *order = nullptr;
     auto tree_search = [&](int64_t *cnt, const int64_t *off, int slot_cap, uint64_t *keys) {
-        tree_radius(x.metric, x.dim, TreeRadiusArgs{tree_view(x), q, order, nq, r, rq, cnt, off, slot_cap, keys}, s);
+        tree_radius(x.metric, x.dim, TreeRadiusArgs{tree_view(x, false), q, order, nq, r, rq, cnt, off, slot_cap, keys},
+                    s); // (a radius search waits for its counts, so none is captured)
     };
     // more splits than k-NN: a radius wave keeps no list, so the launch gains
     // from more waves to hide its latency (SE3 1M x 65,536: 15.8 ms at 16

@@ -256,8 +256,9 @@ __device__ __forceinline__ uint32_t spread_bits(uint32_t v, int dims)
 __global__ void __launch_bounds__(256) tree_gather_kernel(const float *__restrict__ pts,
                                                           const uint8_t *__restrict__ removed, int64_t n, int dim,
                                                           int tdim, int64_t tiles, const uint32_t *__restrict__ perm,
-                                                          NNTree T)
+                                                          NNTree T, uint32_t *__restrict__ live)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *live = (uint32_t)n;
     const int lane = threadIdx.x & 63;
     const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     if (t >= tiles) return;
@@ -507,15 +508,16 @@ struct TreeList {
             thr = bound2(bd);
         }
     }
-    // Adds the lanes' points; the bound follows.
-    __device__ __forceinline__ void add(const TreeQuery<METRIC, DIM> &Q, const TilePoints<DIM> &P, int k, int lane)
+    // Adds the lanes' points (of ids below n); the bound follows.
+    __device__ __forceinline__ void add(const TreeQuery<METRIC, DIM> &Q, const TilePoints<DIM> &P, uint32_t n, int k,
+                                        int lane)
     {
         if (W > 1) {
             const u64 b = __hip_atomic_load(shared, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             take_bound(lane_u64(b, 0));
         }
         const float s = Q.near2(P.e);
-        bool c = P.id >= 0 && s <= thr; // false for NaN
+        bool c = (uint32_t)P.id < n && s <= thr; // false for id -1 and for NaN
         if (METRIC == OMPL_AMD_METRIC_SE3) {
             // the cheap bound first: d^2 >= d_t^2 + d_r^2, d_r^2 >= 2 (1 - |q.x|)
             // (widened past the rounding of the product and of the arc cosine);
@@ -585,13 +587,15 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W) tree_knn_kernel(TreeKnn
     const TreeView &t = A.t;
     TreeList<METRIC, DIM, W> L;
     L.init(&shared_bound);
+    const int64_t in_index = t.live ? (int64_t)*t.live : t.m;
+    const uint32_t ids = (uint32_t)t.n;
     // the points added since the index was built
-    for (int64_t p = t.m + w * kTile; p < t.n; p += W * kTile) {
+    for (int64_t p = in_index + w * kTile; p < t.n; p += W * kTile) {
         TilePoints<DIM> P;
         P.load_tail(t, p, lane);
-        L.add(Q, P, k, lane);
+        L.add(Q, P, ids, k, lane);
     }
-    const int64_t tiles = (t.m + kTile - 1) / kTile, nodes = (tiles + kTile - 1) / kTile,
+    const int64_t tiles = (in_index + kTile - 1) / kTile, nodes = (tiles + kTile - 1) / kTile,
                   supers = (nodes + kTile - 1) / kTile;
     // Picks the remaining child with the nearest box, or -1 when none is
     // within the bound; lb holds the lanes' squared distances as bits.
@@ -632,7 +636,7 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W) tree_knn_kernel(TreeKnn
                 for (;;) {
                     const int nx = pick(open0, lb0);
                     if (nx >= 0) P[1].load(t, t0 + nx, lane);
-                    L.add(Q, P[0], k, lane);
+                    L.add(Q, P[0], ids, k, lane);
                     if (nx < 0) break;
                     P[0] = P[1];
                 }
@@ -811,7 +815,7 @@ void tree_free(NNTree &t)
 }
 
 void tree_build(NNTree &t, const float *pts, const uint8_t *removed, const uint32_t *ext_lo, const uint32_t *ext_hi,
-                int64_t n, int dim, int tdim, hipStream_t s)
+                uint32_t *live, int64_t n, int dim, int tdim, hipStream_t s)
 {
     OA_REQUIRE(n > 0 && n <= t.cap, OMPL_AMD_ERR_INTERNAL, "index build out of range");
     const int64_t tiles = ceil_div(n, kTile), nodes = ceil_div(tiles, kTile), supers = ceil_div(nodes, kTile);
@@ -836,7 +840,7 @@ void tree_build(NNTree &t, const float *pts, const uint8_t *removed, const uint3
                        place, keys);
     hipLaunchKernelGGL(tree_sort_kernel, dim3((unsigned)buckets), dim3(256), 0, s, plan, tdim, counts, keys, perm);
     hipLaunchKernelGGL(tree_gather_kernel, dim3(blocks_of(tiles, 4)), dim3(256), 0, s, pts, removed, n, dim, tdim,
-                       tiles, perm, t);
+                       tiles, perm, t, live);
     hipLaunchKernelGGL(tree_boxes_kernel, dim3(blocks_of(nodes, 4)), dim3(256), 0, s, t.b0, tiles, t.b1, nodes, tdim);
     if (supers > 1) // a single supernode's box is never looked at
         hipLaunchKernelGGL(tree_boxes_kernel, dim3(blocks_of(supers, 4)), dim3(256), 0, s, t.b1, nodes, t.b2, supers,

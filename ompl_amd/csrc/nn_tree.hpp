@@ -1,5 +1,5 @@
 // Spatial index of the nearest-neighbour structure: points in tiles of 64
-// that are compact in space, under two levels of bounding boxes with 64
+// that are compact in space, under three levels of bounding boxes with 64
 // children each, searched by one wave per query (nn_tree.hip).
 #pragma once
 
@@ -41,7 +41,9 @@ struct TreeView {
     const float *sp;
     const int32_t *sid;
     const float *b0, *b1, *b2;
-    int64_t m, n;           // points in the index; all points
+    int64_t m, n;           // points in the index; all points (ids searched are below n)
+    const uint32_t *live;   // a captured k-NN search: where the kernel reads m, since a
+                            // replay may find the index built again with more points
     const float *pts;       // [n][dim], the tail is [m, n)
     const uint8_t *removed; // [n]
 };
@@ -76,9 +78,9 @@ bool tree_supported(int metric, int dim);
 void tree_reserve(NNTree &t, int64_t cap, int dim, int tdim);
 void tree_free(NNTree &t); // nothing on the device uses the arrays any more
 // Indexes points [0, n) of pts ([n][dim]); removed ones get no entry.  ext_lo,
-// ext_hi: extents of the first tdim coordinates (device, ordered_bits).
+// ext_hi: extents of the first tdim coordinates (device, ordered_bits).  live: receives n (device).
 void tree_build(NNTree &t, const float *pts, const uint8_t *removed, const uint32_t *ext_lo, const uint32_t *ext_hi,
-                int64_t n, int dim, int tdim, hipStream_t s);
+                uint32_t *live, int64_t n, int dim, int tdim, hipStream_t s);
 // Drops id from the index.
 void tree_remove(const NNTree &t, int64_t id, hipStream_t s);
 // Scratch bytes for tree_order, 0 when the queries are better left in the caller's order.
