@@ -70,6 +70,8 @@ struct NNIndex {
     // per-call scratch (grow-only)
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
+    bool scratch_captured = false; // a captured search uses it: it is kept when it is outgrown
+    std::vector<void *> scratch_kept;
     // the library's device blocks behind pts, xt, removed and xn_max
     DeviceBlock blocks[4];
 };
@@ -827,11 +829,19 @@ __global__ void fill_i64_kernel(int64_t *p, int64_t n, int64_t v)
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
+static void drop_scratch(NNIndex &x)
+{
+    if (x.scratch && x.scratch_captured) x.scratch_kept.push_back(x.scratch);
+    else if (x.scratch) OA_HIP(hipFree(x.scratch));
+    x.scratch = nullptr;
+    x.scratch_bytes = 0;
+    x.scratch_captured = false;
+}
+
 static void *scratch(NNIndex &x, size_t bytes)
 {
     if (x.scratch_bytes < bytes) {
-        if (x.scratch) OA_HIP(hipFree(x.scratch));
-        x.scratch = nullptr;
+        drop_scratch(x);
         hipError_t e = hipMalloc(&x.scratch, bytes);
         if (e != hipSuccess) fail(OMPL_AMD_ERR_NOMEM, "nn scratch allocation of %zu bytes failed", bytes);
         x.scratch_bytes = bytes;
@@ -850,7 +860,7 @@ static void *scratch_keep(NNIndex &x, size_t bytes, size_t keep, hipStream_t s)
     if (x.scratch) {
         if (keep) OA_HIP(hipMemcpyAsync(fresh, x.scratch, keep, hipMemcpyDeviceToDevice, s));
         OA_HIP(hipStreamSynchronize(s));
-        OA_HIP(hipFree(x.scratch));
+        drop_scratch(x);
     }
     x.scratch = fresh;
     x.scratch_bytes = bytes;
@@ -1107,6 +1117,7 @@ static void knn(NNIndex &x, const float *q, int64_t nq, int k, const int32_t *kq
         ProfScope ps("nn_knn", s);
         if (kq) packed_offsets(kq, nq, k, (int64_t *)buf, buf + counts_bytes, cub_bytes, out_off, s);
         const bool captured = tree_used(x, s);
+        if (captured && head) x.scratch_captured = true;
         tree_knn(x.metric, x.dim,
                  TreeKnnArgs{tree_view(x, captured), q, nq, k, kq, kq ? out_off : nullptr, out_d, out_i}, s);
         return;
@@ -1140,6 +1151,7 @@ static void knn(NNIndex &x, const float *q, int64_t nq, int k, const int32_t *kq
     const size_t cub_span = (cub_bytes + 255) / 256 * 256;
     const size_t per = splits > 1 ? (size_t)splits * nq * k : 0;
     char *buf = (char *)scratch(x, counts_bytes + cub_span + per * (sizeof(float) + sizeof(int32_t)) + 256);
+    if (stream_capturing(s)) x.scratch_captured = true;
     ProfScope ps("nn_knn", s);
     if (kq) packed_offsets(kq, nq, k, (int64_t *)buf, buf + counts_bytes, cub_bytes, out_off, s);
     if (splits == 1) {
@@ -1375,6 +1387,7 @@ int ompl_amd_nn_destroy(ompl_amd_nn h)
         OA_HIP(hipDeviceSynchronize()); // searches on any stream may use the arrays
         for (const DeviceBlock &b : x.blocks) give_block(b);
         if (x.scratch) OA_HIP(hipFree(x.scratch));
+        for (void *p : x.scratch_kept) OA_HIP(hipFree(p));
         if (x.tree_built) OA_HIP(hipEventDestroy(x.tree_built));
         tree_free(x.tree);
         delete h;

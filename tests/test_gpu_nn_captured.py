@@ -1,14 +1,15 @@
 """A k-NN search captured into a graph and replayed while the structure goes on:
 additions that build the index again, removals, a clear, with eager searches
 between the replays.  Every replay against the CPU oracle over the ids that were
-there at the capture."""
+there at the capture.  (9 dimensions: the full scan, whose working space the
+eager searches of more points outgrow.)"""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("metric,dim", [(0, 3), (0, 7), (1, 7)])
+@pytest.mark.parametrize("metric,dim", [(0, 3), (0, 7), (0, 9), (1, 7)])
 @pytest.mark.parametrize("nq", [30, 7000])
 def test_replays(gpu, oracle, metric, dim, nq):
     import torch
