@@ -60,7 +60,7 @@ void ompl_amd::check_motions_tuned(const Tuning &t, const Env &env, const double
     A.checked = checked;
     std::unique_lock<std::mutex> lk; // held until this batch's launches are enqueued
     Workspace &w = own ? *own : workspace(s, (size_t)n, lk);
-    launch_grid_motions(env.grid, A, grid_scratch(w), t.motion_strategy == 2, s);
+    launch_grid_motions(env.grid, A, own ? grid_scratch(w) : stream_grid_scratch(w, s), t.motion_strategy == 2, s);
 }
 
 namespace {
@@ -364,7 +364,7 @@ int ompl_amd_check_motions_last_valid_dev(ompl_amd_env e, const double *a, const
         const hipStream_t st = resolve_stream(stream);
         std::unique_lock<std::mutex> lk; // held until the launches are enqueued
         Workspace &w = workspace(st, (size_t)n, lk);
-        launch_grid_last_valid(env.grid, A, last_t, grid_scratch(w), st);
+        launch_grid_last_valid(env.grid, A, last_t, stream_grid_scratch(w, st), st);
     });
 }
 
@@ -399,7 +399,8 @@ int ompl_amd_check_state_lists_dev(ompl_amd_env e, const double *q_soa, int64_t 
         const hipStream_t st = resolve_stream(stream);
         std::unique_lock<std::mutex> lk; // held until the launches are enqueued
         Workspace &w = workspace(st, (size_t)n_lists, lk);
-        launch_grid_state_lists(env.grid, q_soa, n_states, offsets, n_lists, out, first_invalid, grid_scratch(w), st);
+        launch_grid_state_lists(env.grid, q_soa, n_states, offsets, n_lists, out, first_invalid,
+                                stream_grid_scratch(w, st), st);
     });
 }
 

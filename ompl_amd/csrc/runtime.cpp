@@ -121,22 +121,35 @@ void free_workspace_arrays(Workspace &w)
     w.list_cap = 0;
 }
 
+static GridScratch grid_scratch_with(const Workspace &w, int32_t *counts, int32_t *next)
+{
+    const size_t cap = w.list_cap;
+    return GridScratch{w.list,
+                       w.surv_nd,
+                       w.rest,
+                       w.longs,
+                       w.longs + cap,
+                       w.longs + 2 * cap,
+                       w.surv_ab,
+                       w.counters + 64,
+                       counts,
+                       next};
+}
+
 GridScratch grid_scratch(Workspace &w)
 {
     int32_t *sets = w.counters + 16;
-    const size_t cap = w.list_cap;
-    GridScratch g{w.list,
-                  w.surv_nd,
-                  w.rest,
-                  w.longs,
-                  w.longs + cap,
-                  w.longs + 2 * cap,
-                  w.surv_ab,
-                  w.counters + 64,
-                  sets + 4 * w.grid_parity,
-                  sets + 4 * (1 - w.grid_parity)};
+    const GridScratch g = grid_scratch_with(w, sets + 4 * w.grid_parity, sets + 4 * (1 - w.grid_parity));
     w.grid_parity ^= 1;
     return g;
+}
+
+GridScratch stream_grid_scratch(Workspace &w, hipStream_t s)
+{
+    if (!stream_capturing(s)) return grid_scratch(w);
+    int32_t *set = w.counters + 32;
+    launch_zero(set, 2, s);
+    return grid_scratch_with(w, set, set + 4);
 }
 
 namespace {

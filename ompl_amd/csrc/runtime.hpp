@@ -42,7 +42,9 @@ struct Workspace {
     size_t list_cap = 0;
     // two sets of two at [16..17] and [20..21] (apart from each other's cache
     // sector), used in turn by grid_parity, each cleared by the batch before;
-    // from [64] on a word and a ticket per item of a one-launch batch
+    // a third at [32..33] for batches that a caller captures (and [36..37], which
+    // they clear in place of the next batch's); from [64] on a word and a ticket
+    // per item of a one-launch batch
     int32_t *counters = nullptr;
     int grid_parity = 0;
     // Held by a batch from choosing its counter set to enqueuing its launches
@@ -58,6 +60,10 @@ void alloc_workspace_arrays(Workspace &w, size_t cap);
 void free_workspace_arrays(Workspace &w);
 // The next grid batch's view of a workspace (its lock held).
 GridScratch grid_scratch(Workspace &w);
+// The same of stream s's workspace.  While the caller captures s the batch gets
+// the set for captured batches and a launch that clears it: each replay then
+// starts from zero counts, whatever ran between, and leaves the other sets alone.
+GridScratch stream_grid_scratch(Workspace &w, hipStream_t s);
 Workspace &workspace(hipStream_t s, size_t list_entries, std::unique_lock<std::mutex> &lock);
 
 // Per-thread stream and pinned result slot of the blocking single-call entry
