@@ -12,6 +12,9 @@
  * all others are host pointers.  `stream` is a hipStream_t (NULL = HIP's
  * null stream).  *_dev entry points are asynchronous on `stream`;
  * host-pointer entry points return after the result is in host memory.
+ * A *_dev check that a caller captures into a graph uses the capturing stream's
+ * workspace (sized by an earlier call of its size on that stream): replay it on
+ * that stream, or beside no other call on it.
  *
  * State layouts: joint configurations are structure-of-arrays, dof-major:
  * q[j * n + i] is joint j of state i (coalesced loads: lane i reads q[j*n+i]).

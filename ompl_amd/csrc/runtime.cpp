@@ -147,6 +147,7 @@ GridScratch grid_scratch(Workspace &w)
 GridScratch stream_grid_scratch(Workspace &w, hipStream_t s)
 {
     if (!stream_capturing(s)) return grid_scratch(w);
+    w.captured = true;
     int32_t *set = w.counters + 32;
     launch_zero(set, 2, s);
     return grid_scratch_with(w, set, set + 4);
@@ -228,7 +229,9 @@ Workspace &workspace(hipStream_t s, size_t list_entries, std::unique_lock<std::m
     if (w->list_cap < list_entries) {
         // the stream may still use the old arrays
         OA_HIP(hipStreamSynchronize(s));
-        free_workspace_arrays(*w);
+        if (w->captured) w->list_cap = 0; // captured batches go on with them
+        else free_workspace_arrays(*w);
+        w->captured = false;
         alloc_workspace_arrays(*w, list_entries < 1024 ? 1024 : list_entries);
     }
     return *w;

@@ -47,6 +47,7 @@ struct Workspace {
     // per item of a one-launch batch
     int32_t *counters = nullptr;
     int grid_parity = 0;
+    bool captured = false; // a caller's graph uses the arrays: outgrown, they stay allocated
     // Held by a batch from choosing its counter set to enqueuing its launches
     // (and around resizing), so host threads that share a stream cannot pick
     // the same set or see arrays being replaced.

@@ -126,3 +126,27 @@ def test_state_lists(gpu, oracle, n_lists):
     for _ in range(3):
         replay(graph, side)
         assert np.array_equal(f.cpu().numpy(), want) and np.array_equal(v.cpu().numpy() == 1, want < 0)
+
+
+def test_larger_eager_batches(gpu, oracle):
+    """Eager calls outgrow the stream's workspace, which a captured batch goes on using."""
+    import torch
+
+    s, b = gpu.workload.obstacles(1001, 20, 16)
+    env, oenv = gpu.Env(s, b), oracle.OracleEnv(s, b)
+    side = torch.cuda.Stream()
+    runs = []
+    for n in (2000, 30_000, 200_000):
+        a_, b_ = gpu.workload.edges(n, n, -1.0, 1.2, 0.001, 9.0)
+        sel = np.unique(np.linspace(0, n - 1, 2000).astype(int))
+        want = oracle.check_motions(oenv, a_[sel], b_[sel], 0.05, threads=8)
+        A, B = dev(a_.T), dev(b_.T)
+        with torch.cuda.stream(side):
+            graph, out = captured(lambda: gpu.check_motions(env, A, B, 0.05, exact_count=True), side)
+        runs.append((graph, out, sel, want, (A, B)))
+        for _ in range(2):
+            for graph, (v, c), sel_, (rv, rc), _keep in runs:
+                v.fill_(77)
+                torch.cuda.synchronize()
+                replay(graph, side)
+                assert np.array_equal(v.cpu().numpy()[sel_], rv) and np.array_equal(c.cpu().numpy()[sel_], rc)
