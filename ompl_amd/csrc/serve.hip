@@ -892,6 +892,7 @@ __global__ void __launch_bounds__(NT) plan_slice_kernel(SliceArgs A)
                 // RRTConnect.cpp:301-330: step back once on the start side (or
                 // the goal side at its root), then start chain reversed + goal chain
                 int sm = tgi_start ? xmotion : added, gm = tgi_start ? added : xmotion;
+                __syncthreads(); // a chain of intermediate states has parents from every wave
                 if (tid == 0) {
                     const int32_t *ps = R.parent[0], *pg = R.parent[1];
                     if (ps[sm] >= 0) sm = ps[sm];
