@@ -55,7 +55,7 @@ struct NNIndex {
     float *pts = nullptr;      // [cap][dim]
     float *xt = nullptr;       // [cap/32][ksteps][64] tiled augmented points
     uint8_t *removed = nullptr;
-    uint32_t *xn_max = nullptr; // max |x|^2 as FP32 bits (non-negative), the extents, tree.m (kStatWords words)
+    uint32_t *xn_max = nullptr; // max |x|^2 as FP32 bits (non-negative), then tree.m (kStatWords words)
     int64_t n_removed = 0;
     std::vector<uint8_t> removed_host;
     // spatial index of the first tree.m points; whether it was built since its
@@ -669,20 +669,18 @@ __global__ void radius_unpack_kernel(const uint64_t *__restrict__ keys, int64_t 
     if (dist) dist[i] = __uint_as_float((uint32_t)(k >> 32));
 }
 
-// Writes tiled augmented rows for points [from, to) and the padding of the
-// last tile; tracks max |x|^2 and the extents of the first coordinates
-// (stats: kStatNorm, kStatLo, kStatHi; kStatLive, the points in the spatial
-// index, is the build's).  The figures meet in LDS, and a block
-// makes a device-wide atomic only for one that it improves (one atomic per
-// point took 187 us of adding 1,000,000).
-constexpr int kStatNorm = 0, kStatLo = 8, kStatHi = 16, kStatTracked = 24, kStatLive = 24, kStatWords = 25;
+// Words of xn_max: max |x|^2, and the points in the spatial index (the build's).
+constexpr int kStatLive = 1, kStatWords = 2;
 
+// Writes tiled augmented rows for points [from, to) and the padding of the
+// last tile; tracks max |x|^2.  It meets in LDS, and a block makes a device-wide
+// atomic only if it improves it (one atomic per point took 187 us of adding 1,000,000).
 __global__ void __launch_bounds__(256) build_xt_kernel(const float *__restrict__ pts, int dim, int tdim, int ksteps,
                                                        int64_t from, int64_t to, int64_t n_total,
-                                                       float *__restrict__ xt, uint32_t *__restrict__ stats)
+                                                       float *__restrict__ xt, uint32_t *__restrict__ xn_max)
 {
-    __shared__ uint32_t blk[kStatTracked];
-    if (threadIdx.x < kStatTracked) blk[threadIdx.x] = threadIdx.x >= kStatLo && threadIdx.x < kStatHi ? ~0u : 0u;
+    __shared__ uint32_t blk;
+    if (threadIdx.x == 0) blk = 0;
     __syncthreads();
     const int64_t p = from + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool real = p < n_total && p < to;
@@ -704,36 +702,15 @@ __global__ void __launch_bounds__(256) build_xt_kernel(const float *__restrict__
     uint32_t norm = real ? __float_as_uint(xn) : 0u;
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) norm = max(norm, (uint32_t)__shfl_xor((int)norm, d));
-    if ((threadIdx.x & 63) == 0) atomicMax(&blk[kStatNorm], norm);
-    for (int j = 0; j < tdim && j < 8; ++j) {
-        const float v = real ? pts[p * dim + j] : INFINITY;
-        const bool fin = fabsf(v) < 3e38f; // finite
-        uint32_t lo = fin ? ordered_bits(v) : ~0u, hi = fin ? ordered_bits(v) : 0u;
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) {
-            lo = min(lo, (uint32_t)__shfl_xor((int)lo, d));
-            hi = max(hi, (uint32_t)__shfl_xor((int)hi, d));
-        }
-        if ((threadIdx.x & 63) == 0) {
-            atomicMin(&blk[kStatLo + j], lo);
-            atomicMax(&blk[kStatHi + j], hi);
-        }
-    }
+    if ((threadIdx.x & 63) == 0) atomicMax(&blk, norm);
     __syncthreads();
-    if (threadIdx.x < kStatTracked) {
-        const uint32_t v = blk[threadIdx.x];
-        const uint32_t have = __hip_atomic_load(&stats[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (threadIdx.x >= kStatLo && threadIdx.x < kStatHi) {
-            if (v < have) atomicMin(&stats[threadIdx.x], v);
-        } else if (v > have) {
-            atomicMax(&stats[threadIdx.x], v);
-        }
-    }
+    if (threadIdx.x == 0 && blk > __hip_atomic_load(xn_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(xn_max, blk);
 }
 
 __global__ void clear_stats_kernel(uint32_t *__restrict__ stats)
 {
-    if (threadIdx.x < kStatWords) stats[threadIdx.x] = threadIdx.x >= kStatLo && threadIdx.x < kStatHi ? ~0u : 0u;
+    if (threadIdx.x < kStatWords) stats[threadIdx.x] = 0;
 }
 
 // Each query's radius keys (distance bits << 32 | index; unique per query)
@@ -867,10 +844,8 @@ static void *scratch_keep(NNIndex &x, size_t bytes, size_t keep, hipStream_t s)
     return x.scratch;
 }
 
-// Points from which on the spatial index is kept, and up to which (its places
-// and counts are 32-bit words; beyond, the working space of a build would be
-// more than a gigabyte).
-constexpr int64_t kTreeMinPoints = 2048;
+// Points up to which the spatial index is kept (its places and counts are 32-bit
+// words; beyond, the working space of a build would be more than a gigabyte).
 constexpr int64_t kTreeMaxPoints = (int64_t)1 << 25;
 
 static void reserve(NNIndex &x, int64_t need, hipStream_t s)
@@ -941,8 +916,7 @@ static void tree_update(NNIndex &x, hipStream_t s)
     // (also after a clear, which leaves them to finish)
     if (x.tree_live && (x.tree_mixed || x.tree_captured || x.tree_stream != s)) OA_HIP(hipDeviceSynchronize());
     if (!x.tree_built) OA_HIP(hipEventCreateWithFlags(&x.tree_built, hipEventDisableTiming));
-    tree_build(x.tree, x.pts, x.removed, x.xn_max + kStatLo, x.xn_max + kStatHi, x.xn_max + kStatLive, x.n,
-               x.dim, x.tdim, s);
+    tree_build(x.tree, x.pts, x.removed, x.xn_max + kStatLive, x.n, x.dim, x.tdim, s);
     OA_HIP(hipEventRecord(x.tree_built, s));
     if (x.tree_captured) OA_HIP(hipStreamSynchronize(s)); // a replay need not wait for an addition
     x.tree_live = true;

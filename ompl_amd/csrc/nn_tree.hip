@@ -2,11 +2,11 @@
 //
 // Build: the points are put into one order whose consecutive runs are compact,
 // and cut into tiles of 64.  Every dimension but the last is cut into cells of
-// equal counts (quantiles, from a histogram); the cells, walked in reflected
+// equal counts (quantiles, from a sample); the cells, walked in reflected
 // (boustrophedon) order, are columns along the last dimension, and a column's
 // points are sorted by it, upwards and downwards in turn.  Consecutive points
 // are then neighbours also where a column ends.  A column is dealt to buckets
-// of about a thousand points by counting, and one workgroup sorts each bucket
+// of at most a thousand points or so by counting, and one workgroup sorts each bucket
 // in LDS: 100,000 points in 7 dimensions take 9 launches, where one radix sort
 // per dimension (nested cuts) took about 70 and 440 us; a CPU model gives 40.8
 // tiles per 10-NN query for this order and 38.7 for the nested one (SE3 1M:
@@ -35,15 +35,23 @@ namespace ompl_amd {
 // ---------------------------------------------------------------------------
 // build
 // ---------------------------------------------------------------------------
-constexpr int kBins = 512;         // histogram bins per dimension
-constexpr int kBucketPoints = 1024; // points a bucket is meant to hold
+constexpr int kSample = 2048;       // values per dimension that the cuts are made from,
+constexpr int kSmallSample = 1024;  // and below kSmallPoints, whose cells are fewer (2 us less)
+constexpr int64_t kSmallPoints = 16384;
+static_assert(kSample <= kTreeMinPoints, "a point for every run");
+constexpr int kKnots = 512;         // most quantiles of a dimension that are looked up; finer cuts interpolate
+constexpr int kBins = 512;          // cells per dimension of the queries' search order
+constexpr int kBucketPoints = 768;  // points a bucket is meant to hold
 constexpr int kBucketSort = 4096;   // points sorted at once; a fuller bucket (many equal coordinates) in parts
 
-// A build's cuts and histograms.
+// A build's cuts.  They come from a sample of each coordinate, not from its
+// extent: one far point, or a heavy tail, would leave all others in one cell of
+// equal widths, thus in one bucket (adding 1,000,000 points 32 ms in place of 0.4).
 struct TreePlan {
-    int cuts[8];             // cells per dimension; the last dimension's: buckets per column
-    float base[8], scale[8]; // bin = (x - base) * scale
-    uint32_t hist[8][kBins];
+    int cuts[8];              // cells per dimension; the last dimension's: buckets per column
+    int finite[8];            // finite values of the sample
+    float base[8], scale[8];  // cell of a query = (x - base) * scale
+    float sample[8][kSample]; // ascending
 };
 
 __device__ __forceinline__ float from_ordered(uint32_t u)
@@ -51,23 +59,97 @@ __device__ __forceinline__ float from_ordered(uint32_t u)
     return __uint_as_float(u & 0x80000000u ? u ^ 0x80000000u : ~u);
 }
 
-// Chooses the cuts (one block), and clears the histograms and bucket counts.
-// The dimension whose cells are longest gets one cut more until there are as
-// many cells as tiles; the last dimension is then cut into buckets instead.
-__global__ void __launch_bounds__(256) plan_kernel(const uint32_t *__restrict__ ext_lo,
-                                                   const uint32_t *__restrict__ ext_hi, int64_t n, int tdim,
-                                                   TreePlan *plan, uint32_t *__restrict__ counts, int64_t buckets)
+// One round of a bitonic sort of the block's values, four a thread (value e of
+// thread t is number 4 t + e): exchanges with number ^ J, ascending where K is clear.
+template <int K, int J>
+__device__ __forceinline__ void sample_round(uint32_t v[4], uint32_t *key)
 {
-    for (int i = threadIdx.x; i < 8 * kBins; i += blockDim.x) plan->hist[0][i] = 0;
+    const int i0 = 4 * threadIdx.x;
+    uint32_t o[4];
+    if constexpr (J >= 256) {
+        *reinterpret_cast<uint4 *>(&key[i0]) = make_uint4(v[0], v[1], v[2], v[3]);
+        __syncthreads();
+        const uint4 w = *reinterpret_cast<const uint4 *>(&key[i0 ^ J]);
+        o[0] = w.x, o[1] = w.y, o[2] = w.z, o[3] = w.w;
+        __syncthreads();
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = J >= 4 ? (uint32_t)__shfl_xor((int)v[e], J / 4) : v[e ^ (J & 3)];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int i = i0 + e;
+        v[e] = ((i & J) == 0) == ((i & K) == 0) ? min(v[e], o[e]) : max(v[e], o[e]);
+    }
+    if constexpr (J > 1) sample_round<K, J / 2>(v, key);
+}
+
+template <int K>
+__device__ __forceinline__ void sample_sort(uint32_t v[4], uint32_t *key)
+{
+    if constexpr (K > 2) sample_sort<K / 2>(v, key);
+    sample_round<K, K / 2>(v, key);
+}
+
+// The sorted sample of dimension blockIdx.x: a point at random (by a hash) of
+// each of SAMPLE equal runs, so that no regular order of the points shows.
+// Exchanges within a wave are shuffles: 6 of the sort's 66 rounds (2,048 values)
+// wait for other waves.
+template <int SAMPLE>
+__global__ void __launch_bounds__(SAMPLE / 4) tree_sample_kernel(const float *__restrict__ pts, int64_t n, int dim,
+                                                                 TreePlan *__restrict__ plan)
+{
+    __shared__ uint32_t key[SAMPLE];
+    __shared__ int waves_finite[SAMPLE / 256];
+    const int d = blockIdx.x, i0 = 4 * threadIdx.x;
+    uint32_t v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int64_t from = n * (i0 + e) / SAMPLE, to = n * (i0 + e + 1) / SAMPLE;
+        const uint32_t skip = __umulhi((uint32_t)(i0 + e) * 2654435761u, (uint32_t)(to - from));
+        const float x = pts[(from + skip) * dim + d];
+        v[e] = fabsf(x) < 3e38f ? ordered_bits(x) : ~0u; // not finite: last
+    }
+    sample_sort<SAMPLE>(v, key);
+    int finite = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        plan->sample[d][i0 + e] = from_ordered(v[e]);
+        finite += __popcll(__ballot(v[e] != ~0u));
+    }
+    if ((threadIdx.x & 63) == 0) waves_finite[threadIdx.x >> 6] = finite;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < SAMPLE / 256; ++w) finite += waves_finite[w];
+        plan->finite[d] = finite;
+    }
+}
+
+// Chooses the cuts (one block), and clears the bucket counts.  The dimension
+// whose cells are longest gets one cut more until there are as many cells as
+// tiles; the last dimension is then cut into buckets instead.  A dimension's
+// length is that of its sample without the ends' 64ths.
+__global__ void __launch_bounds__(256) plan_kernel(int64_t n, int tdim, TreePlan *__restrict__ plan,
+                                                   uint32_t *__restrict__ counts, int64_t buckets)
+{
     for (int64_t i = threadIdx.x; i < buckets; i += blockDim.x) counts[i] = 0;
     if (threadIdx.x >= 64) return;
     // lane j holds dimension j
     const int j = threadIdx.x;
     float ext = 0.0f;
     if (j < tdim) {
-        const float lo = from_ordered(ext_lo[j]), e = from_ordered(ext_hi[j]) - lo;
-        if (ext_lo[j] <= ext_hi[j] && e > 0.0f && e < 3e38f) ext = e;
-        plan->base[j] = ext > 0.0f ? lo : 0.0f;
+        const int m = plan->finite[j];
+        float lo = 0.0f;
+        if (m > 0) {
+            lo = plan->sample[j][m / 64];
+            ext = plan->sample[j][m - 1 - m / 64] - lo;
+            if (!(ext > 0.0f)) { // nearly all equal
+                lo = plan->sample[j][0];
+                ext = plan->sample[j][m - 1] - lo;
+            }
+            if (!(ext < 3e38f)) ext = 0.0f;
+        }
+        plan->base[j] = lo;
         plan->scale[j] = ext > 0.0f ? (float)kBins / ext : 0.0f;
     }
     const int64_t tiles = (n + kTile - 1) / kTile;
@@ -106,58 +188,64 @@ __device__ __forceinline__ float bin_of(const TreePlan &plan, int j, float x)
     return fminf(fmaxf((x - plan.base[j]) * plan.scale[j], 0.0f), (float)kBins - 0.001f); // NaN: 0
 }
 
-__global__ void __launch_bounds__(1024) plan_histogram_kernel(const float *__restrict__ pts, int64_t n, int dim,
-                                                              int tdim, TreePlan *plan)
-{
-    __shared__ uint32_t h[kTreeDimMax][kBins];
-    for (int i = threadIdx.x; i < tdim * kBins; i += blockDim.x) h[0][i] = 0;
-    __syncthreads();
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        for (int j = 0; j < tdim; ++j) atomicAdd(&h[j][(int)bin_of(*plan, j, pts[i * dim + j])], 1u);
-    __syncthreads();
-    for (int i = threadIdx.x; i < tdim * kBins; i += blockDim.x)
-        if (h[0][i]) atomicAdd(&plan->hist[0][i], h[0][i]);
-}
-
 // Each point's bucket and its arrival number there.
 __global__ void __launch_bounds__(1024) tree_buckets_kernel(const float *__restrict__ pts, int64_t n, int dim,
                                                             int tdim, const TreePlan *__restrict__ plan,
                                                             uint32_t *__restrict__ counts, uint2 *__restrict__ place)
 {
-    __shared__ float below[kTreeDimMax][kBins + 1]; // points below the bin, all as a fraction
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (w < tdim) { // wave w scans dimension w, 8 bins a lane
-        uint32_t v[kBins / 64], sum = 0;
-#pragma unroll
-        for (int i = 0; i < kBins / 64; ++i) sum += v[i] = plan->hist[w][lane * (kBins / 64) + i];
-        uint32_t incl = sum;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t u = (uint32_t)__shfl_up((int)incl, d);
-            if (lane >= d) incl += u;
-        }
-        uint32_t run = incl - sum;
-        const float inv = 1.0f / (float)n;
-#pragma unroll
-        for (int i = 0; i < kBins / 64; ++i) {
-            below[w][lane * (kBins / 64) + i] = (float)run * inv;
-            run += v[i];
-        }
-        if (lane == 63) below[w][kBins] = (float)run * inv;
+    __shared__ float knot[kTreeDimMax][kKnots + 1]; // ascending; [0] and [knots]: the sample's ends
+    const int lane = threadIdx.x & 63;
+    for (int j = 0; j < tdim; ++j) {
+        const int knots = min(plan->cuts[j], kKnots), m = plan->finite[j];
+        for (int i = threadIdx.x; i <= knots; i += blockDim.x)
+            knot[j][i] = m > 0 ? plan->sample[j][min((int)((int64_t)i * m / knots), m - 1)] : 0.0f;
     }
     __syncthreads();
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        int64_t idx = 0;
-        for (int j = 0; j < tdim; ++j) {
-            const float b = bin_of(*plan, j, pts[i * dim + j]);
-            const int k = (int)b;
-            const float u = below[j][k] + (below[j][k + 1] - below[j][k]) * (b - (float)k);
-            const int c = plan->cuts[j];
-            const int cell = min(c - 1, (int)(u * (float)c));
+        uint32_t idx = 0;
+        float coord[kTreeDimMax]; // read together
+#pragma unroll
+        for (int j = 0; j < kTreeDimMax; ++j)
+            if (j < tdim) coord[j] = pts[i * dim + j];
+#pragma unroll
+        for (int j = 0; j < kTreeDimMax; ++j) {
+            if (j >= tdim) break;
+            const int c = plan->cuts[j], knots = min(c, kKnots);
+            int cell = 0;
+            if (c > 1) {
+                const float x = coord[j];
+                // the last knot at or below x (below the second, or not a number: 0)
+                for (int step = 1 << (31 - __builtin_clz(knots)); step > 0; step >>= 1)
+                    if (cell + step < knots && x >= knot[j][cell + step]) cell += step;
+                if (c > knots) {
+                    const float lo = knot[j][cell], wide = knot[j][cell + 1] - lo;
+                    const float part = wide > 0.0f ? fminf(fmaxf((x - lo) / wide, 0.0f), 1.0f) : 0.0f;
+                    cell = min(c - 1, (int)(((float)cell + part) * ((float)c / (float)knots)));
+                }
+            }
             // reflected order: every other run of a dimension's cells is walked backwards
-            idx = idx * c + ((idx & 1) ? c - 1 - cell : cell);
+            idx = idx * (uint32_t)c + (uint32_t)((idx & 1) ? c - 1 - cell : cell);
         }
-        place[i] = make_uint2((uint32_t)idx, atomicAdd(&counts[idx], 1u));
+        // one atomic for lanes of the same bucket (the first four such groups):
+        // points of equal coordinates would queue up at one address
+        int lead = lane, before = 0, group = 1;
+        bool open = true;
+        for (int r = 0; r < 4; ++r) {
+            const uint64_t m = __ballot(open);
+            if (m == 0) break;
+            const int l = __builtin_ctzll(m);
+            const bool same = open && idx == (uint32_t)__builtin_amdgcn_readlane((int)idx, l);
+            const uint64_t g = __ballot(same);
+            if (same) {
+                lead = l;
+                before = __popcll(g & (((uint64_t)1 << lane) - 1));
+                group = __popcll(g);
+                open = false;
+            }
+        }
+        uint32_t at = 0;
+        if (lead == lane) at = atomicAdd(&counts[idx], (uint32_t)group);
+        place[i] = make_uint2(idx, (uint32_t)__shfl((int)at, lead) + (uint32_t)before);
     }
 }
 
@@ -209,40 +297,59 @@ __global__ void __launch_bounds__(256) tree_scatter_kernel(const float *__restri
     keys[first[p.x] + p.y] = ((unsigned long long)ordered_bits(pts[i * dim + tdim - 1]) << 32) | (uint32_t)i;
 }
 
-// Sorts one bucket by the last coordinate, in the direction of its column.
-__global__ void __launch_bounds__(256) tree_sort_kernel(const TreePlan *__restrict__ plan, int tdim,
+// Sorts the buckets by the last coordinate, each in the direction of its column:
+// block b the first kBucketSort points of bucket b; the blocks after those each
+// the part that starts in a run of kBucketSort places, if any, of the bucket that
+// holds the run's first place (the parts of a bucket start kBucketSort apart, so
+// a run has one at most).
+__global__ void __launch_bounds__(256) tree_sort_kernel(const TreePlan *__restrict__ plan, int tdim, int64_t buckets,
                                                         const uint32_t *__restrict__ first,
                                                         const unsigned long long *__restrict__ keys,
                                                         uint32_t *__restrict__ perm)
 {
     __shared__ unsigned long long buf[kBucketSort];
-    const int64_t b = blockIdx.x;
-    const uint32_t lo = first[b], hi = first[b + 1];
-    const bool down = ((b / plan->cuts[tdim - 1]) & 1) != 0;
-    for (uint32_t at = lo; at < hi; at += kBucketSort) { // block-uniform
-        const int m = (int)min((uint32_t)kBucketSort, hi - at);
-        int np2 = 1;
-        while (np2 < m) np2 <<= 1;
-        for (int i = threadIdx.x; i < np2; i += blockDim.x) {
-            const unsigned long long k = i < m ? keys[at + i] : ~0ull;
-            buf[i] = down && i < m ? k ^ 0xffffffff00000000ull : k;
+    int64_t b = blockIdx.x;
+    uint32_t at;
+    if (b < buckets) {
+        at = first[b];
+    } else {
+        const uint32_t run = (uint32_t)(b - buckets) * kBucketSort;
+        if (run >= first[buckets]) return;
+        int64_t lo = 0, hi = buckets; // first[lo] <= run < first[hi]
+        while (hi - lo > 1) {
+            const int64_t mid = (lo + hi) / 2;
+            if (first[mid] <= run) lo = mid;
+            else hi = mid;
         }
-        __syncthreads();
-        for (int k = 2; k <= np2; k <<= 1)
-            for (int j = k >> 1; j > 0; j >>= 1) {
-                for (int p = threadIdx.x; p < np2 / 2; p += blockDim.x) {
-                    const int i = 2 * p - (p & (j - 1)), o = i + j;
-                    const unsigned long long x = buf[i], y = buf[o];
-                    if ((x > y) == ((i & k) == 0)) {
-                        buf[i] = y;
-                        buf[o] = x;
-                    }
-                }
-                __syncthreads();
-            }
-        for (int i = threadIdx.x; i < m; i += blockDim.x) perm[at + i] = (uint32_t)buf[i];
-        __syncthreads();
+        b = lo;
+        const uint32_t part = (run - first[b] + kBucketSort - 1) / kBucketSort;
+        if (part == 0) return; // block b's
+        at = first[b] + part * kBucketSort;
     }
+    const uint32_t end = first[b + 1];
+    if (at >= end) return; // block-uniform
+    const bool down = ((b / plan->cuts[tdim - 1]) & 1) != 0;
+    const int m = (int)min((uint32_t)kBucketSort, end - at);
+    int np2 = 1;
+    while (np2 < m) np2 <<= 1;
+    for (int i = threadIdx.x; i < np2; i += blockDim.x) {
+        const unsigned long long k = i < m ? keys[at + i] : ~0ull;
+        buf[i] = down && i < m ? k ^ 0xffffffff00000000ull : k;
+    }
+    __syncthreads();
+    for (int k = 2; k <= np2; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int p = threadIdx.x; p < np2 / 2; p += blockDim.x) {
+                const int i = 2 * p - (p & (j - 1)), o = i + j;
+                const unsigned long long x = buf[i], y = buf[o];
+                if ((x > y) == ((i & k) == 0)) {
+                    buf[i] = y;
+                    buf[o] = x;
+                }
+            }
+            __syncthreads();
+        }
+    for (int i = threadIdx.x; i < m; i += blockDim.x) perm[at + i] = (uint32_t)buf[i];
 }
 
 __device__ __forceinline__ uint32_t spread_bits(uint32_t v, int dims)
@@ -814,10 +921,10 @@ void tree_free(NNTree &t)
     t = NNTree{};
 }
 
-void tree_build(NNTree &t, const float *pts, const uint8_t *removed, const uint32_t *ext_lo, const uint32_t *ext_hi,
-                uint32_t *live, int64_t n, int dim, int tdim, hipStream_t s)
+void tree_build(NNTree &t, const float *pts, const uint8_t *removed, uint32_t *live, int64_t n, int dim, int tdim,
+                hipStream_t s)
 {
-    OA_REQUIRE(n > 0 && n <= t.cap, OMPL_AMD_ERR_INTERNAL, "index build out of range");
+    OA_REQUIRE(n >= kSample && n <= t.cap, OMPL_AMD_ERR_INTERNAL, "index build out of range");
     const int64_t tiles = ceil_div(n, kTile), nodes = ceil_div(tiles, kTile), supers = ceil_div(nodes, kTile);
     const int64_t buckets = max_buckets(n);
     char *at = t.build;
@@ -831,14 +938,19 @@ void tree_build(NNTree &t, const float *pts, const uint8_t *removed, const uint3
     uint2 *place = (uint2 *)take((size_t)n * 8);
     unsigned long long *keys = (unsigned long long *)take((size_t)n * 8);
     uint32_t *perm = (uint32_t *)take((size_t)n * 4);
-    const unsigned sweep = (unsigned)std::min<int64_t>(ceil_div(n, 2048), 256);
-    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(256), 0, s, ext_lo, ext_hi, n, tdim, plan, counts, buckets);
-    hipLaunchKernelGGL(plan_histogram_kernel, dim3(sweep), dim3(1024), 0, s, pts, n, dim, tdim, plan);
+    const unsigned sweep = (unsigned)std::min<int64_t>(ceil_div(n, 1024), 256);
+    if (n < kSmallPoints)
+        hipLaunchKernelGGL(tree_sample_kernel<kSmallSample>, dim3((unsigned)tdim), dim3(kSmallSample / 4), 0, s, pts, n,
+                           dim, plan);
+    else
+        hipLaunchKernelGGL(tree_sample_kernel<kSample>, dim3((unsigned)tdim), dim3(kSample / 4), 0, s, pts, n, dim, plan);
+    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(256), 0, s, n, tdim, plan, counts, buckets);
     hipLaunchKernelGGL(tree_buckets_kernel, dim3(sweep), dim3(1024), 0, s, pts, n, dim, tdim, plan, counts, place);
     hipLaunchKernelGGL(tree_scan_kernel, dim3(1), dim3(1024), 0, s, counts, buckets);
     hipLaunchKernelGGL(tree_scatter_kernel, dim3(blocks_of(n, 256)), dim3(256), 0, s, pts, n, dim, tdim, counts,
                        place, keys);
-    hipLaunchKernelGGL(tree_sort_kernel, dim3((unsigned)buckets), dim3(256), 0, s, plan, tdim, counts, keys, perm);
+    hipLaunchKernelGGL(tree_sort_kernel, dim3((unsigned)(buckets + ceil_div(n, kBucketSort))), dim3(256), 0, s, plan,
+                       tdim, buckets, counts, keys, perm);
     hipLaunchKernelGGL(tree_gather_kernel, dim3(blocks_of(tiles, 4)), dim3(256), 0, s, pts, removed, n, dim, tdim,
                        tiles, perm, t, live);
     hipLaunchKernelGGL(tree_boxes_kernel, dim3(blocks_of(nodes, 4)), dim3(256), 0, s, t.b0, tiles, t.b1, nodes, tdim);

@@ -14,6 +14,8 @@ namespace ompl_amd {
 
 constexpr int kTile = 64;   // points per tile, tiles per node, nodes per supernode
 constexpr int kTreeDimMax = 7;
+// Points from which on the index is kept.
+constexpr int64_t kTreeMinPoints = 2048;
 
 // Device arrays of the index; all in one allocation, sized for `cap` points.
 struct NNTree {
@@ -30,7 +32,7 @@ struct NNTree {
     char *build = nullptr;     // the build's own working space (its plan first, kept)
 };
 
-// FP32 bits reordered so that unsigned order is numeric order (the form of extents).
+// FP32 bits reordered so that unsigned order is numeric order.
 __device__ __forceinline__ uint32_t ordered_bits(float v)
 {
     const uint32_t u = __float_as_uint(v);
@@ -77,10 +79,10 @@ bool tree_supported(int metric, int dim);
 // Allocates the arrays for `cap` points (the old ones are dropped: m = 0).
 void tree_reserve(NNTree &t, int64_t cap, int dim, int tdim);
 void tree_free(NNTree &t); // nothing on the device uses the arrays any more
-// Indexes points [0, n) of pts ([n][dim]); removed ones get no entry.  ext_lo,
-// ext_hi: extents of the first tdim coordinates (device, ordered_bits).  live: receives n (device).
-void tree_build(NNTree &t, const float *pts, const uint8_t *removed, const uint32_t *ext_lo, const uint32_t *ext_hi,
-                uint32_t *live, int64_t n, int dim, int tdim, hipStream_t s);
+// Indexes points [0, n) of pts ([n][dim]), n >= kTreeMinPoints; removed ones get no entry.
+// live: receives n (device).
+void tree_build(NNTree &t, const float *pts, const uint8_t *removed, uint32_t *live, int64_t n, int dim, int tdim,
+                hipStream_t s);
 // Drops id from the index.
 void tree_remove(const NNTree &t, int64_t id, hipStream_t s);
 // Scratch bytes for tree_order, 0 when the queries are better left in the caller's order.
