@@ -90,7 +90,7 @@ static void run_work(const char *what, const std::function<void(Work *, hipStrea
 {
     ThreadResources &r = thread_resources();
     Work *acc = nullptr;
-    OA_HIP(hipMalloc(&acc, sizeof(Work)));
+    OA_HIP(device_malloc(&acc, sizeof(Work)));
     OA_HIP(hipMemsetAsync(acc, 0, sizeof(Work), r.stream));
     launch(acc, r.stream);
     OA_HIP(hipGetLastError());

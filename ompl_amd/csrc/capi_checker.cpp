@@ -110,7 +110,7 @@ namespace {
 void graph_workspace(Workspace &w, int64_t n)
 {
     const size_t cap = (size_t)n < 1024 ? 1024 : (size_t)n;
-    OA_HIP(hipMalloc(&w.counters, kWorkspaceCounters * sizeof(int32_t)));
+    OA_HIP(device_malloc(&w.counters, kWorkspaceCounters * sizeof(int32_t)));
     OA_HIP(hipMemset(w.counters, 0, kWorkspaceCounters * sizeof(int32_t)));
     alloc_workspace_arrays(w, cap);
 }
@@ -241,7 +241,7 @@ int ompl_amd_env_create(const float *spheres, int n_spheres, const float *boxes,
                      lists_b = grid_lists_bytes(env.grid);
         env.bytes = obs_b + cells_b + lists_b + 256;
         char *mem = nullptr;
-        const hipError_t err = hipMalloc((void **)&mem, env.bytes);
+        const hipError_t err = device_malloc(&mem, env.bytes);
         if (err != hipSuccess) {
             delete e;
             fail(OMPL_AMD_ERR_NOMEM, "environment allocation failed: %s", hipGetErrorString(err));
@@ -506,7 +506,7 @@ extern "C" int ompl_amd_autotune_motions(ompl_amd_env e, const double *a, const 
         ThreadResources &r = thread_resources();
         hipStream_t s = r.stream;
         uint8_t *out = nullptr;
-        OA_HIP(hipMalloc(&out, (size_t)n));
+        OA_HIP(device_malloc(&out, (size_t)n));
         hipEvent_t e0, e1;
         OA_HIP(hipEventCreate(&e0));
         OA_HIP(hipEventCreate(&e1));
@@ -565,7 +565,7 @@ extern "C" int ompl_amd_autotune_motions_streams(ompl_amd_env e, const double *a
         std::vector<hipStream_t> st((size_t)n_streams);
         for (int j = 0; j < n_streams; ++j) st[(size_t)j] = resolve_stream(streams[j]);
         PipelineScratch S;
-        OA_HIP(hipMalloc(&S.out, (size_t)n * (size_t)n_streams));
+        OA_HIP(device_malloc(&S.out, (size_t)n * (size_t)n_streams));
         OA_HIP(hipEventCreate(&S.e0));
         OA_HIP(hipEventCreate(&S.e1));
         for (int j = 0; j < n_streams; ++j) {

@@ -819,7 +819,7 @@ static void *scratch(NNIndex &x, size_t bytes)
 {
     if (x.scratch_bytes < bytes) {
         drop_scratch(x);
-        hipError_t e = hipMalloc(&x.scratch, bytes);
+        hipError_t e = device_malloc(&x.scratch, bytes);
         if (e != hipSuccess) fail(OMPL_AMD_ERR_NOMEM, "nn scratch allocation of %zu bytes failed", bytes);
         x.scratch_bytes = bytes;
     }
@@ -832,7 +832,7 @@ static void *scratch_keep(NNIndex &x, size_t bytes, size_t keep, hipStream_t s)
 {
     if (x.scratch_bytes >= bytes) return x.scratch;
     void *fresh = nullptr;
-    hipError_t e = hipMalloc(&fresh, bytes);
+    hipError_t e = device_malloc(&fresh, bytes);
     if (e != hipSuccess) fail(OMPL_AMD_ERR_NOMEM, "nn scratch allocation of %zu bytes failed", bytes);
     if (x.scratch) {
         if (keep) OA_HIP(hipMemcpyAsync(fresh, x.scratch, keep, hipMemcpyDeviceToDevice, s));
@@ -1312,7 +1312,7 @@ struct DevBufs {
     template <class T> T *alloc(size_t n)
     {
         void *q = nullptr;
-        OA_HIP(hipMallocAsync(&q, (n ? n : 1) * sizeof(T), s));
+        OA_HIP(device_malloc_async(&q, (n ? n : 1) * sizeof(T), s));
         p.push_back(q);
         return static_cast<T *>(q);
     }

@@ -104,11 +104,11 @@ hipStream_t default_stream()
 
 void alloc_workspace_arrays(Workspace &w, size_t cap)
 {
-    OA_HIP(hipMalloc(&w.list, cap * sizeof(int32_t)));
-    OA_HIP(hipMalloc(&w.rest, cap * sizeof(int32_t)));
-    OA_HIP(hipMalloc(&w.surv_nd, cap * sizeof(int32_t)));
-    OA_HIP(hipMalloc(&w.longs, 3 * cap * sizeof(int32_t)));
-    OA_HIP(hipMalloc(&w.surv_ab, cap * 14 * sizeof(double)));
+    OA_HIP(device_malloc(&w.list, cap * sizeof(int32_t)));
+    OA_HIP(device_malloc(&w.rest, cap * sizeof(int32_t)));
+    OA_HIP(device_malloc(&w.surv_nd, cap * sizeof(int32_t)));
+    OA_HIP(device_malloc(&w.longs, 3 * cap * sizeof(int32_t)));
+    OA_HIP(device_malloc(&w.surv_ab, cap * 14 * sizeof(double)));
     w.list_cap = cap;
 }
 
@@ -177,23 +177,46 @@ DeviceBlock take_block(size_t bytes)
         }
     }
     DeviceBlock b{nullptr, want};
-    hipError_t e = hipMalloc(&b.p, want);
-    if (e == hipErrorOutOfMemory) {
-        std::multimap<size_t, void *> kept;
-        {
-            std::lock_guard<std::mutex> lk(g_blocks_mutex);
-            kept.swap(g_blocks);
-            g_blocks_bytes = 0;
-        }
-        for (const auto &k : kept) (void)hipFree(k.second);
-        (void)hipGetLastError();
-        e = hipMalloc(&b.p, want);
-    }
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
+    const hipError_t e = device_malloc(&b.p, want);
+    if (e != hipSuccess)
         fail(OMPL_AMD_ERR_NOMEM, "device allocation of %zu bytes failed: %s", want, hipGetErrorString(e));
-    }
     return b;
+}
+
+namespace {
+void release_blocks()
+{
+    std::multimap<size_t, void *> kept;
+    {
+        std::lock_guard<std::mutex> lk(g_blocks_mutex);
+        kept.swap(g_blocks);
+        g_blocks_bytes = 0;
+    }
+    for (const auto &k : kept) (void)hipFree(k.second);
+}
+
+template <class Alloc>
+hipError_t malloc_or_release(Alloc alloc)
+{
+    hipError_t e = alloc();
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        release_blocks();
+        e = alloc();
+    }
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+} // namespace
+
+hipError_t device_malloc_bytes(void **p, size_t bytes)
+{
+    return malloc_or_release([&] { return hipMalloc(p, bytes); });
+}
+
+hipError_t device_malloc_async_bytes(void **p, size_t bytes, hipStream_t s)
+{
+    return malloc_or_release([&] { return hipMallocAsync(p, bytes, s); });
 }
 
 void give_block(const DeviceBlock &b)
@@ -218,7 +241,7 @@ Workspace &workspace(hipStream_t s, size_t list_entries, std::unique_lock<std::m
         Workspace *&slot = g_ws[s];
         if (!slot) {
             slot = new Workspace();
-            OA_HIP(hipMalloc(&slot->counters, kWorkspaceCounters * sizeof(int32_t)));
+            OA_HIP(device_malloc(&slot->counters, kWorkspaceCounters * sizeof(int32_t)));
             OA_HIP(hipMemset(slot->counters, 0, kWorkspaceCounters * sizeof(int32_t)));
             OA_HIP(hipDeviceSynchronize());
         }
@@ -424,7 +447,7 @@ int ompl_amd_malloc(void **ptr, size_t bytes)
     return guarded([&] {
         OA_REQUIRE(ptr, OMPL_AMD_ERR_ARG, "null output pointer");
         ensure_init();
-        hipError_t e = hipMalloc(ptr, bytes ? bytes : 1);
+        hipError_t e = device_malloc(ptr, bytes ? bytes : 1);
         if (e == hipErrorOutOfMemory) fail(OMPL_AMD_ERR_NOMEM, "hipMalloc(%zu) out of memory", bytes);
         OA_HIP(e);
     });

@@ -22,7 +22,7 @@ void init_noalloc_scratch(int dev);
 // Device memory of objects that come and go (roadmaps, nearest-neighbour
 // structures): a block given back is kept for the next taker, up to
 // kKeptBlocksBytes in all, and kept blocks go back to the device when an
-// allocation fails.  The giver sees to it that nothing on the device still
+// allocation of the library fails (device_malloc).  The giver sees to it that nothing on the device still
 // uses the block.  Safe from any thread.
 struct DeviceBlock {
     void *p = nullptr;
@@ -31,6 +31,20 @@ struct DeviceBlock {
 constexpr size_t kKeptBlocksBytes = (size_t)768 << 20;
 DeviceBlock take_block(size_t bytes);
 void give_block(const DeviceBlock &b);
+// hipMalloc and hipMallocAsync; when the device is out of memory the kept blocks
+// go back to it and the allocation is tried again.
+hipError_t device_malloc_bytes(void **p, size_t bytes);
+hipError_t device_malloc_async_bytes(void **p, size_t bytes, hipStream_t s);
+template <class T>
+hipError_t device_malloc(T **p, size_t bytes)
+{
+    return device_malloc_bytes(reinterpret_cast<void **>(p), bytes);
+}
+template <class T>
+hipError_t device_malloc_async(T **p, size_t bytes, hipStream_t s)
+{
+    return device_malloc_async_bytes(reinterpret_cast<void **>(p), bytes, s);
+}
 
 // Per-stream scratch of the batched motion path: survivor list + counters.
 struct Workspace {

@@ -344,7 +344,7 @@ static void sample_valid(ompl_amd_env env, const uint32_t *seeds, MtState *gen, 
         }
     } room{s};
     const size_t cursors = (size_t)n_streams * sizeof(ValidCursor), gens = seeds ? (size_t)n_streams * sizeof(MtState) : 0;
-    OA_HIP(hipMallocAsync((void **)&room.p, cursors + gens + 256, s));
+    OA_HIP(device_malloc_async(&room.p, cursors + gens + 256, s));
     A.cursor = (ValidCursor *)room.p;
     A.open = (int32_t *)(room.p + cursors + gens);
     OA_HIP(hipMemsetAsync(A.cursor, 0, cursors, s));
@@ -396,8 +396,8 @@ static MtState *seed_generators(const uint32_t *seeds, int n, hipStream_t s)
 {
     MtState *gen = nullptr;
     uint32_t *dseeds = nullptr;
-    OA_HIP(hipMallocAsync((void **)&gen, (size_t)n * sizeof(MtState), s));
-    OA_HIP(hipMallocAsync((void **)&dseeds, (size_t)n * sizeof(uint32_t), s));
+    OA_HIP(device_malloc_async(&gen, (size_t)n * sizeof(MtState), s));
+    OA_HIP(device_malloc_async(&dseeds, (size_t)n * sizeof(uint32_t), s));
     OA_HIP(hipMemcpyAsync(dseeds, seeds, (size_t)n * sizeof(uint32_t), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(mt_seed_kernel, dim3((n + 63) / 64), dim3(64), 0, s, dseeds, n, gen);
     OA_HIP(hipGetLastError());
@@ -474,7 +474,7 @@ int ompl_amd_rng_sample_se3_dev(ompl_amd_rng rng, int64_t n_per_stream, const do
         const double zero[6] = {0, 0, 0, 0, 0, 0}, one[6] = {1, 1, 1, 1, 1, 1};
         const int64_t n = (int64_t)rng->n * n_per_stream;
         double *u = nullptr;
-        OA_HIP(hipMallocAsync((void **)&u, (size_t)n * 6 * sizeof(double), s));
+        OA_HIP(device_malloc_async(&u, (size_t)n * 6 * sizeof(double), s));
         {
             ProfScope ps("sample_se3", s);
             sample_uniform(nullptr, rng->gen, rng->n, n_per_stream, 6, zero, one, u, nullptr, s);

@@ -1589,7 +1589,7 @@ int ompl_amd_server_create(const ompl_amd_server_config *cfg, ompl_amd_server *o
         if (S.budget_ticks < 1) S.budget_ticks = 1;
         OA_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
         if (cfg->hbm_budget_bytes > 0) {
-            hipError_t e = hipMalloc(&S.pool, cfg->hbm_budget_bytes);
+            hipError_t e = device_malloc(&S.pool, cfg->hbm_budget_bytes);
             if (e != hipSuccess) {
                 (void)hipStreamDestroy(S.stream);
                 delete h;
