@@ -857,9 +857,14 @@ static void reserve(NNIndex &x, int64_t need, hipStream_t s)
     float *pts = nullptr, *xt = nullptr;
     uint8_t *rem = nullptr;
     DeviceBlock fresh[3];
-    fresh[0] = take_block((size_t)cap * x.dim * sizeof(float));
-    fresh[1] = take_block((size_t)cap * x.ksteps * 2 * sizeof(float));
-    fresh[2] = take_block((size_t)cap);
+    try {
+        fresh[0] = take_block((size_t)cap * x.dim * sizeof(float));
+        fresh[1] = take_block((size_t)cap * x.ksteps * 2 * sizeof(float));
+        fresh[2] = take_block((size_t)cap);
+    } catch (...) {
+        for (const DeviceBlock &b : fresh) give_block(b);
+        throw;
+    }
     pts = (float *)fresh[0].p;
     xt = (float *)fresh[1].p;
     rem = (uint8_t *)fresh[2].p;
@@ -881,10 +886,15 @@ static void reserve(NNIndex &x, int64_t need, hipStream_t s)
     x.removed = rem;
     x.cap = cap;
     x.removed_host.resize((size_t)cap, 0);
-    if (tree_supported(x.metric, x.dim) && cap >= kTreeMinPoints && cap <= kTreeMaxPoints)
-        tree_reserve(x.tree, cap, x.dim, x.tdim);
-    else
-        tree_free(x.tree);
+    tree_free(x.tree);
+    if (tree_supported(x.metric, x.dim) && cap >= kTreeMinPoints && cap <= kTreeMaxPoints) {
+        try {
+            tree_reserve(x.tree, cap, x.dim, x.tdim);
+        } catch (const Error &e) {
+            if (e.code != OMPL_AMD_ERR_NOMEM) throw;
+            // no room for the index (about the points' own size again): the full scan serves
+        }
+    }
     x.tree_live = x.tree_mixed = false;
 }
 
