@@ -615,7 +615,8 @@ struct TreeList {
             thr = bound2(bd);
         }
     }
-    // Adds the lanes' points (of ids below n); the bound follows.
+    // Adds the lanes' points (CAPTURED: of ids below n); the bound follows.
+    template <bool CAPTURED>
     __device__ __forceinline__ void add(const TreeQuery<METRIC, DIM> &Q, const TilePoints<DIM> &P, uint32_t n, int k,
                                         int lane)
     {
@@ -624,7 +625,7 @@ struct TreeList {
             take_bound(lane_u64(b, 0));
         }
         const float s = Q.near2(P.e);
-        bool c = (uint32_t)P.id < n && s <= thr; // false for id -1 and for NaN
+        bool c = (CAPTURED ? (uint32_t)P.id < n : P.id >= 0) && s <= thr; // false for NaN
         if (METRIC == OMPL_AMD_METRIC_SE3) {
             // the cheap bound first: d^2 >= d_t^2 + d_r^2, d_r^2 >= 2 (1 - |q.x|)
             // (widened past the rounding of the product and of the arc cosine);
@@ -666,7 +667,10 @@ struct TreeList {
 // against the full scan's 19,700; about 33 tiles and 8 nodes per query, 100
 // instructions a tile and 12 an insertion), by the longest query's read chain
 // in small ones (100,000 x 4,096, k = 10, R^7: 71 us against 247).
-template <int METRIC, int DIM, int W>
+// CAPTURED: the number of indexed points is read from TreeView::live, and ids
+// beyond the view's are left out (a kernel of its own: tests for it in the eager
+// one cost 1 to 1.5% of the small batches).
+template <int METRIC, int DIM, int W, bool CAPTURED>
 __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W) tree_knn_kernel(TreeKnnArgs A)
 {
     constexpr int TD = TreeQuery<METRIC, DIM>::TD;
@@ -694,13 +698,13 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W) tree_knn_kernel(TreeKnn
     const TreeView &t = A.t;
     TreeList<METRIC, DIM, W> L;
     L.init(&shared_bound);
-    const int64_t in_index = t.live ? (int64_t)*t.live : t.m;
+    const int64_t in_index = CAPTURED ? (int64_t)*t.live : t.m;
     const uint32_t ids = (uint32_t)t.n;
     // the points added since the index was built
     for (int64_t p = in_index + w * kTile; p < t.n; p += W * kTile) {
         TilePoints<DIM> P;
         P.load_tail(t, p, lane);
-        L.add(Q, P, ids, k, lane);
+        L.template add<CAPTURED>(Q, P, ids, k, lane);
     }
     const int64_t tiles = (in_index + kTile - 1) / kTile, nodes = (tiles + kTile - 1) / kTile,
                   supers = (nodes + kTile - 1) / kTile;
@@ -743,7 +747,7 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W) tree_knn_kernel(TreeKnn
                 for (;;) {
                     const int nx = pick(open0, lb0);
                     if (nx >= 0) P[1].load(t, t0 + nx, lane);
-                    L.add(Q, P[0], ids, k, lane);
+                    L.template add<CAPTURED>(Q, P[0], ids, k, lane);
                     if (nx < 0) break;
                     P[0] = P[1];
                 }
@@ -1006,21 +1010,29 @@ static int waves_per_query(int64_t nq, bool heavy)
     return nq > 6144 ? 1 : nq > 2048 ? (heavy ? 2 : 1) : nq > 128 ? 4 : 16;
 }
 
+template <int METRIC, int DIM, int W>
+static void launch_knn_waves(const TreeKnnArgs &A, hipStream_t s)
+{
+    const dim3 grid(W == 1 ? blocks_of(A.nq, 4) : (unsigned)A.nq), block(W == 1 ? 256 : 64 * W);
+    if (A.t.live) hipLaunchKernelGGL((tree_knn_kernel<METRIC, DIM, W, true>), grid, block, 0, s, A);
+    else hipLaunchKernelGGL((tree_knn_kernel<METRIC, DIM, W, false>), grid, block, 0, s, A);
+}
+
 template <int METRIC, int DIM>
 static void launch_knn(const TreeKnnArgs &A, hipStream_t s)
 {
     switch (waves_per_query(A.nq, DIM > 3)) {
     case 1:
-        hipLaunchKernelGGL((tree_knn_kernel<METRIC, DIM, 1>), dim3(blocks_of(A.nq, 4)), dim3(256), 0, s, A);
+        launch_knn_waves<METRIC, DIM, 1>(A, s);
         break;
     case 2:
-        hipLaunchKernelGGL((tree_knn_kernel<METRIC, DIM, 2>), dim3((unsigned)A.nq), dim3(128), 0, s, A);
+        launch_knn_waves<METRIC, DIM, 2>(A, s);
         break;
     case 4:
-        hipLaunchKernelGGL((tree_knn_kernel<METRIC, DIM, 4>), dim3((unsigned)A.nq), dim3(256), 0, s, A);
+        launch_knn_waves<METRIC, DIM, 4>(A, s);
         break;
     default:
-        hipLaunchKernelGGL((tree_knn_kernel<METRIC, DIM, 16>), dim3((unsigned)A.nq), dim3(1024), 0, s, A);
+        launch_knn_waves<METRIC, DIM, 16>(A, s);
         break;
     }
 }
