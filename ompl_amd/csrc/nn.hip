@@ -935,9 +935,9 @@ static void tree_update(NNIndex &x, hipStream_t s)
 }
 
 // The index serves a search when the tail it leaves to a scan is small; below
-// kTreeMinPoints everything is tail.  Else (8 and more L2 dimensions, where
-// boxes exclude little, or a tail grown under stream capture) the full scan on
-// the matrix cores does.  Measured, index against full scan, k = 10, one query
+// kTreeMinPoints everything is tail.  Else (8 and more L2 dimensions, for which
+// the index is not built, a tail grown under stream capture, or an index that
+// found no memory) the full scan on the matrix cores does.  Measured, index against full scan, k = 10, one query
 // to 65,536: 2,048 points of R^7 12.9 / 175 us against 46 / 266; 5,000 of SE3
 // 12.6 / 118 against 54 / 418 (the smallest are the call itself).
 static bool use_tree(const NNIndex &x)

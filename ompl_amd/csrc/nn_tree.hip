@@ -41,7 +41,8 @@ constexpr int64_t kSmallPoints = 16384;
 static_assert(kSample <= kTreeMinPoints, "a point for every run");
 constexpr int kKnots = 512;         // most quantiles of a dimension that are looked up; finer cuts interpolate
 constexpr int kBins = 512;          // cells per dimension of the queries' search order
-constexpr int kBucketPoints = 768;  // points a bucket is meant to hold
+constexpr int kBucketPoints = 768;  // points a bucket is meant to hold: the cuts vary with the sample, and a sort of more
+                                    // than 1,024 pads to 2,048 (SE3 1M: sorts 48 us, 63 with 1,024 meant)
 constexpr int kBucketSort = 4096;   // points sorted at once; a fuller bucket (many equal coordinates) in parts
 
 // A build's cuts.  They come from a sample of each coordinate, not from its
@@ -663,8 +664,8 @@ struct TreeList {
 };
 
 // k nearest: W waves per query; with W = 1 a block holds four queries.
-// Bound by VALU instructions in large batches (SE3 1M x 65,536, k = 16: 578 us
-// against the full scan's 19,700; about 33 tiles and 8 nodes per query, 100
+// Bound by VALU instructions (62% of the time) and reads past the L2 (7.3 TB/s)
+// in large batches (SE3 1M x 65,536, k = 16: 578 us against the full scan's 19,700; about 33 tiles and 8 nodes per query, 100
 // instructions a tile and 12 an insertion), by the longest query's read chain
 // in small ones (100,000 x 4,096, k = 10, R^7: 71 us against 247).
 // CAPTURED: the number of indexed points is read from TreeView::live, and ids
@@ -774,8 +775,9 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W) tree_knn_kernel(TreeKnn
 }
 
 // All points within the radius: one wave per query, a block holds four.
-// Bound by reads (SE3 1M x 65,536, r = 0.98: 190 us of a 245 us call; the full
-// scan took 11,862).
+// Bound by VALU instructions once the queries are in space order (SE3 1M x 65,536,
+// r = 0.98: 190 us of a 245 us call, 86% of it issuing them, 98% L2 hits; without
+// the order by reads, 430 us; the full scan took 11,862).
 template <int METRIC, int DIM>
 __global__ void __launch_bounds__(256) tree_radius_kernel(TreeRadiusArgs A)
 {
@@ -973,7 +975,8 @@ void tree_remove(const NNTree &t, int64_t id, hipStream_t s)
 }
 
 // Radius queries are ordered when there are enough of them to share what they
-// read and the points do not fit one XCD's 4 MiB L2: 65,536 queries of 1,000,000
+// read and the points do not fit one XCD's 4 MiB L2 (150,000 of seven coordinates;
+// measured at one size: points of fewer would fit up to more): 65,536 queries of 1,000,000
 // SE3 points took 430 us in the caller's order and 190 us in this one (reads
 // bound it), for 40 us of ordering.  k-NN batches are not: their time is
 // instructions, and ordering (40-60 us) gained at most as much (705 us without,

@@ -13,6 +13,10 @@
 namespace ompl_amd {
 
 constexpr int kTile = 64;   // points per tile, tiles per node, nodes per supernode
+// L2 dimensions with an index: up to the arm's.  Boxes exclude less in more: 100,000
+// even points, k = 10, 64 / 4,096 / 32,768 queries, full scan against index: 8
+// dimensions 149 / 270 / 1,419 against 37 / 149 / 388 us, 10: 148 / 282 / 1,575
+// against 47 / 321 / 1,043, 12: 150 / 305 / 1,757 against 81 / 521 / 2,393.
 constexpr int kTreeDimMax = 7;
 // Points from which on the index is kept.
 constexpr int64_t kTreeMinPoints = 2048;

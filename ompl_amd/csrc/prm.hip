@@ -378,15 +378,15 @@ void build(PrmRoadmap &R, ompl_amd_env env, uint32_t seed, int n_streams, int64_
     OA_HIP(hipStreamSynchronize(s));
     R.stats.ms_candidates = ms(t0);
     if ((flags & OMPL_AMD_PRM_AUTOTUNE) && nu > 0) {
-        // launch shape tuned on (up to) the first 32,768 candidate edges
+        // the autotuner's pass over (up to) the first 32,768 candidate edges
         const int64_t nt = std::min<int64_t>(nu, 32768);
         double *ta = R.alloc<double>((size_t)nt * kDim), *tb = R.alloc<double>((size_t)nt * kDim);
         int32_t *teu = R.alloc<int32_t>((size_t)nt), *tev = R.alloc<int32_t>((size_t)nt);
         hipLaunchKernelGGL(edge_endpoints_kernel, dim3(blocks_for(nt)), dim3(256), 0, s, R.keys, nt, bits, R.nodes, teu,
                            tev, ta, tb);
         OA_HIP(hipStreamSynchronize(s));
-        // the winner becomes the environment's own launch shapes; the
-        // library's tuning (other environments') is left as it was
+        // the shapes become the environment's own, as callers of the flag expect
+        // (every shape runs the same kernels); the library's tuning is left as it was
         ompl_amd_tuning saved, best;
         check(ompl_amd_get_tuning(&saved));
         check(ompl_amd_autotune_motions(env, ta, tb, nt, lvs, factor, 3, &best, nullptr));

@@ -63,7 +63,8 @@ enum GrowStatus { kTrapped = 0, kAdvanced = 1, kReached = 2 };
 constexpr double kPi = 3.141592653589793238462643383279502884;
 constexpr double kEqualEps = 2.220446049250313080847e-16 * 2.0; // StateSpace::equalStates (RealVector)
 // Largest environment a request may name, as the bytes of its obstacles in
-// lists padded to kPlanPad (60 KiB: 2,880 spheres or 1,728 boxes).
+// lists padded to kPlanPad (60 KiB: 2,880 spheres or 1,728 boxes).  The kernel no
+// longer stages them; the limit is what callers know.
 constexpr int kPlanPad = 288;
 constexpr size_t kPlanMaxEnvBytes = 60 * 1024;
 // Start / goal states a request may list (each).
