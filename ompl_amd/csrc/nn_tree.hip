@@ -129,7 +129,8 @@ __global__ void __launch_bounds__(SAMPLE / 4) tree_sample_kernel(const float *__
 // Chooses the cuts (one block), and clears the bucket counts.  The dimension
 // whose cells are longest gets one cut more until there are as many cells as
 // tiles; the last dimension is then cut into buckets instead.  A dimension's
-// length is that of its sample without the ends' 64ths.
+// length is that of its sample without the ends' 64ths (nothing for one that is
+// nearly constant, whatever its few other values).
 __global__ void __launch_bounds__(256) plan_kernel(int64_t n, int tdim, TreePlan *__restrict__ plan,
                                                    uint32_t *__restrict__ counts, int64_t buckets)
 {
@@ -137,19 +138,16 @@ __global__ void __launch_bounds__(256) plan_kernel(int64_t n, int tdim, TreePlan
     if (threadIdx.x >= 64) return;
     // lane j holds dimension j
     const int j = threadIdx.x;
-    float ext = 0.0f;
+    float lo = 0.0f, ext = 0.0f;
+    auto length = [&](int from, int to) {
+        lo = plan->sample[j][from];
+        ext = plan->sample[j][to] - lo;
+        if (!(ext > 0.0f && ext < 3e38f)) ext = 0.0f;
+    };
+    const int m = j < tdim ? plan->finite[j] : 0;
+    if (m > 0) length(m / 64, m - 1 - m / 64);
+    if (__ballot(ext > 0.0f) == 0 && m > 0) length(0, m - 1); // nearly all points equal
     if (j < tdim) {
-        const int m = plan->finite[j];
-        float lo = 0.0f;
-        if (m > 0) {
-            lo = plan->sample[j][m / 64];
-            ext = plan->sample[j][m - 1 - m / 64] - lo;
-            if (!(ext > 0.0f)) { // nearly all equal
-                lo = plan->sample[j][0];
-                ext = plan->sample[j][m - 1] - lo;
-            }
-            if (!(ext < 3e38f)) ext = 0.0f;
-        }
         plan->base[j] = lo;
         plan->scale[j] = ext > 0.0f ? (float)kBins / ext : 0.0f;
     }

@@ -26,6 +26,12 @@ def data(kind, metric, dim):
         x[:N // 2] = x[0]
     elif kind == "all equal":
         x[:] = x[0]
+    elif kind == "nearly constant":  # in one coordinate
+        x[:, 0] = 0.0
+        x[::50, 0] = np.linspace(-1e6, 1e6, N // 50)
+    elif kind == "nearly equal":
+        x[::50] += 1.0
+        x[np.arange(N) % 50 > 0] = x[1]
     elif kind == "line":
         x[:, :t] = x[:, :1] + np.linspace(0, 1, t)
     elif kind == "not finite":
@@ -46,7 +52,8 @@ def add_us(nn, pts):
     return sorted(us)[3]
 
 
-@pytest.mark.parametrize("kind", ["far point", "heavy tail", "half equal", "all equal", "line", "not finite"])
+@pytest.mark.parametrize("kind", ["far point", "heavy tail", "half equal", "all equal", "line", "not finite",
+                                  "nearly constant", "nearly equal"])
 @pytest.mark.parametrize("metric,dim", [(0, 1), (0, 3), (0, 7), (1, 7)])
 def test_skewed_points(gpu, oracle, kind, metric, dim):
     import torch
